@@ -6,36 +6,56 @@
 //       / sqrt((rc |r0|)^4 + |r1 x r2|^4),
 // zero when |r1 x r2|^2 <= eps^2, r/|r| = 0 when |r| <= eps
 // (unitVec, libMath.f90:249-262).  Per segment the library precomputes
-// r0 = b - a, g = gam/(4 pi) and q = rc^2 |r0|^2 (stored squared in the
-// FP64 record); per pair r1 = p - a, r2 = r1 - r0 and r1 x r2 = r0 x r1.
+// r0 = b - a, g = gam/(4 pi) and q = rc^2 |r0|^2; per pair r1 = p - a,
+// r2 = r1 - r0 and r1 x r2 = r0 x r1.
 //
-// Work decomposition: one target point per lane; a workgroup walks one
-// (target tile, segment chunk) work item at a time, staging 256 segments in
-// LDS and reading them back as wave-uniform broadcasts.  Work items are
-// handed out by an atomic counter to a grid sized to the resident capacity
-// of the device, so every CU stays busy to the end of the launch whatever
-// the target count.  Each item writes its own partial sums, which are
-// reduced in a fixed order afterwards: results are bitwise repeatable.  No
-// MFMA: the pair is not a contraction.
+// Work decomposition: segments come in groups of 32 consecutive records
+// with a centre and a far radius (write_group_records); a wave takes 64 or
+// 128 targets and one chunk of groups, and runs a shorter pair on every
+// group that all its targets are far from (pair64_far, pair32_far).  Each
+// (tile, chunk) item writes its own partial sums, which are reduced in a
+// fixed order afterwards: results are bitwise repeatable.
+//
+// What bounds it: vector issue.  No MFMA: n1 and d1 are contractions of
+// depth 4, but FP64 and FP32 MFMA run no faster than the vector units here
+// (64 and 32 cycles per 16x16x4) and do not overlap with them (16 FMAs and
+// one MFMA take the sum of both times).  Measured against pair64 for every
+// pair with LDS broadcasts: 4.0e9 pairs on helices 6.6 -> 5.1 ms, a
+// quad-rotor wake pass (1.58e10 pairs) 25.7 -> 20.0 ms (7.9e11 pairs/s);
+// mixed, 2e10 pairs on helices 14.7 -> 11.4 ms (1.75e12 pairs/s), a rotor
+// wake pass (2.2e9 pairs) 2.00 -> 1.49 ms.
 //
 // Precision modes
 //   FP64  : FP64 throughout; 1/sqrt via v_rsq_f64 plus one third-order
 //           correction.
-//   MIXED : FP32 pair arithmetic on hi/lo-split coordinates
-//           (r1 = (p_hi - a_hi) + (p_lo - a_lo), accurate to FP32 relative
-//           precision of r1 itself), v_rsq_f32, per-tile FP32 sums folded
-//           into a Kahan-compensated accumulator.  Pairs with the target
-//           inside the core (within one core radius of the segment) are
-//           recomputed in FP64 (the regularised core and target-on-filament
-//           terms, where the reference's exact-zero guards act).
+//   MIXED : FP32 pair arithmetic, v_rsq_f32, the sums of each group folded
+//           into FP64.  Far groups use coordinates relative to the group's
+//           centre, the others hi/lo-split coordinates (r1 = (p_hi - a_hi)
+//           + (p_lo - a_lo), accurate to FP32 relative precision of r1
+//           itself).  Pairs with the target inside the core (within one
+//           core radius of the segment) are recomputed in FP64 (the
+//           regularised core and target-on-filament terms, where the
+//           reference's exact-zero guards act).
 //           Launches with fewer than 1024 targets (collocation points, judge
-//           samples) run the FP64 small-target kernel in both modes.
+//           samples) run in FP64 in both modes.
 #include "vlm_internal.h"
 
 namespace vlm {
 namespace {
 
-constexpr int BS_BLOCK = 256;       // wake passes: many targets
+constexpr int BS_BLOCK = 256;
+// constant address space: a load from a wave-uniform address becomes a
+// scalar load.  The records are written by earlier launches only.
+typedef const double __attribute__((address_space(4))) *cdptr;
+typedef const float __attribute__((address_space(4))) *cfptr;
+typedef const long long __attribute__((address_space(4))) *clptr;
+// Whole FP64 records as vectors: one s_load_dwordx16 per eight doubles
+// (field by field the compiler issues five smaller loads: 5.38 against
+// 5.12 ms for 4.0e9 pairs).
+typedef double d8 __attribute__((ext_vector_type(8)));
+typedef const d8 __attribute__((address_space(4))) *cd8ptr;
+
+
 constexpr double EPS2 = kEps * kEps;
 constexpr float EPS2F = 4.93038065763132e-32f;
 constexpr float NEAR_CORE2 = 1.0f;  // h < rc, and |r1|^2 + |r2|^2 < 4 |r0|^2 (stored)
@@ -64,8 +84,7 @@ __device__ __forceinline__ double zero_unless(bool c, double x)
     return __hiloint2double(c ? hi : 0, __double2loint(x));
 }
 
-// FP64 pair; segment record (ax ay az g | r0x r0y r0z qq | n0), qq = (rc |r0|)^4,
-// n0 = |r0|^2 (so r0 . r2 = r0 . r1 - n0).
+// FP64 pair; qq = (rc |r0|)^4, n0 = |r0|^2 (so r0 . r2 = r0 . r1 - n0).
 // The reference's r0 . (r1/|r1| - r2/|r2|) / sqrt(qq + c2^2) is evaluated as
 // d1 / sqrt(n1 den) - d2 / sqrt(n2 den): two reciprocal square roots per
 // pair instead of three.  The pair guard |r1 x r2|^2 <= eps^2 is exact.  The
@@ -75,11 +94,11 @@ __device__ __forceinline__ double zero_unless(bool c, double x)
 // |r1 x r2| <= |r0| |r| lets the pair guard zero the pair whenever
 // |r0| <= 1, and for longer segments the term left over is of the order of
 // the pair's own (eps-sized) contribution.
-__device__ __forceinline__ void pair64(double px, double py, double pz, double4 sa, double4 sb,
-                                       double n0, double &vx, double &vy, double &vz)
+__device__ __forceinline__ void pair64(double px, double py, double pz, double ax, double ay,
+                                       double az, double g, double r0x, double r0y, double r0z,
+                                       double qq, double n0, double &vx, double &vy, double &vz)
 {
-    const double r1x = px - sa.x, r1y = py - sa.y, r1z = pz - sa.z;
-    const double r0x = sb.x, r0y = sb.y, r0z = sb.z;
+    const double r1x = px - ax, r1y = py - ay, r1z = pz - az;
     const double r2x = r1x - r0x, r2y = r1y - r0y, r2z = r1z - r0z;
     const double cx = r0y * r1z - r0z * r1y;
     const double cy = r0z * r1x - r0x * r1z;
@@ -89,27 +108,29 @@ __device__ __forceinline__ void pair64(double px, double py, double pz, double4 
     const double n2 = r2x * r2x + r2y * r2y + r2z * r2z;
     const double d1 = r0x * r1x + r0y * r1y + r0z * r1z;
     const double d2 = d1 - n0;
-    const double den = __builtin_fma(c2, c2, sb.w);
+    const double den = __builtin_fma(c2, c2, qq);
     const double j1 = rsq64(__builtin_fmax(n1, EPS2) * den);
     const double j2 = rsq64(__builtin_fmax(n2, EPS2) * den);
-    const double s = zero_unless(c2 > EPS2, sa.w * (d1 * j1 - d2 * j2));
+    const double s = zero_unless(c2 > EPS2, g * (d1 * j1 - d2 * j2));
     vx += cx * s;
     vy += cy * s;
     vz += cz * s;
 }
 
-// FP32 pair on split coordinates; record (ahx ahy ahz g | alx aly alz q |
-// r0x r0y r0z 4|r0|^2).  Returns true for near-singular pairs, whose
-// contribution is left to the FP64 recompute (zero here).  Same evaluation
-// order as pair64: d1 / sqrt(n1 den) - d2 / sqrt(n2 den).
+// FP32 pair on split coordinates (r: rec32, n: near32).  Returns true for
+// near-singular pairs, whose contribution is left to the FP64 recompute
+// (zero here): targets inside the core and, for segments without a core,
+// every target nearby (c2^2 underflows in FP32 long before the exact guard
+// acts, and den with it).  Same evaluation order as pair64:
+// d1 / sqrt(n1 den) - d2 / sqrt(n2 den).
 __device__ __forceinline__ bool pair32(float phx, float phy, float phz, float plx, float ply,
-                                       float plz, float4 s0, float4 s1, float4 s2, float &vx,
-                                       float &vy, float &vz)
+                                       float plz, cfptr r, cfptr n, float &vx, float &vy,
+                                       float &vz)
 {
-    const float r1x = (phx - s0.x) + (plx - s1.x);
-    const float r1y = (phy - s0.y) + (ply - s1.y);
-    const float r1z = (phz - s0.z) + (plz - s1.z);
-    const float r0x = s2.x, r0y = s2.y, r0z = s2.z;
+    const float r1x = (phx - n[0]) + (plx - n[4]);
+    const float r1y = (phy - n[1]) + (ply - n[5]);
+    const float r1z = (phz - n[2]) + (plz - n[6]);
+    const float r0x = r[4], r0y = r[5], r0z = r[6], n0 = r[3], q = n[3];
     const float r2x = r1x - r0x, r2y = r1y - r0y, r2z = r1z - r0z;
     const float cx = r0y * r1z - r0z * r1y;
     const float cy = r0z * r1x - r0x * r1z;
@@ -117,13 +138,13 @@ __device__ __forceinline__ bool pair32(float phx, float phy, float phz, float pl
     const float c2 = cx * cx + cy * cy + cz * cz;
     const float n1 = r1x * r1x + r1y * r1y + r1z * r1z;
     const float n2 = r2x * r2x + r2y * r2y + r2z * r2z;
-    const bool nearp = (c2 < NEAR_CORE2 * s1.w) && (n1 + n2 < s2.w);
+    const bool nearp = (c2 < NEAR_CORE2 * q) && (n1 + n2 < 4.0f * n0);
     const float d1 = r0x * r1x + r0y * r1y + r0z * r1z;
-    const float d2 = __builtin_fmaf(s2.w, -0.25f, d1);  // d1 - |r0|^2
-    const float den = __builtin_fmaf(c2, c2, s1.w * s1.w);
+    const float d2 = d1 - n0;
+    const float den = __builtin_fmaf(c2, c2, r[7]);
     const float j1 = __builtin_amdgcn_rsqf(__builtin_fmaxf(n1, EPS2F) * den);
     const float j2 = __builtin_amdgcn_rsqf(__builtin_fmaxf(n2, EPS2F) * den);
-    float s = s0.w * (d1 * j1 - d2 * j2);
+    float s = r[11] * (d1 * j1 - d2 * j2);
     s = (c2 > EPS2F && !nearp) ? s : 0.0f;
     vx += cx * s;
     vy += cy * s;
@@ -131,72 +152,175 @@ __device__ __forceinline__ bool pair32(float phx, float phy, float phz, float pl
     return nearp;
 }
 
-struct BsArgs {
-    const double *s64;   // 8 x stride SoA
-    const float *s32;    // 12 x stride SoA
-    int64_t sstride;
-    const long long *nseg;
-    int64_t chunk_len;
-    const double *t;
-    int64_t m;
-    int64_t tstride;
-    double *part;
-    int ntiles;
-    int nitems;
-    int *counter;
-};
-
-__device__ __forceinline__ int next_item(int *counter, int *sh)
+// FP64 pair of a group that every target of the wave is far from (see
+// write_group_records): |r1| >= 2 |r0| and qq > 0, so none of pair64's
+// guards can act, and
+//   n2 = n1 + n0 - 2 d1        (terms at most 2.25 n1, n2 >= n1 / 4)
+//   c2 = n0 n1 - d1^2          (Lagrange's identity)
+//   sum of s c = (sum of s r0) x q - sum of s r0 x (a - c)
+// with q = p - c, the target relative to the group's centre c: the pair
+// accumulates S += w g r0 and T += w g r0 x (a - c) and the cross product is
+// taken once per group.  35 vector instructions (two of them v_rsq_f64, four
+// issue slots each) instead of pair64's 51.  The rounding of n1 and of the
+// cancelling d1 j1 - d2 j2 is shared by n2, so the error against 64-bit
+// references is no larger (quad-precision emulation, relative 2-norm over 60
+// targets: 1.6e-15 against 6.3e-15 on a rotor wake, 2.2e-15 against 6.7e-15
+// on helices).
+__device__ __forceinline__ void pair64_far(double px, double py, double pz, const d8 &u,
+                                           const d8 &v, double &Sx, double &Sy, double &Sz,
+                                           double &Tx, double &Ty, double &Tz)
 {
-    if (threadIdx.x == 0) *sh = atomicAdd(counter, 1);
-    __syncthreads();
-    const int it = *sh;
-    __syncthreads();
-    return it;
+    const double r1x = px - u[0], r1y = py - u[1], r1z = pz - u[2];
+    const double n0 = u[7];
+    const double n1 = r1x * r1x + r1y * r1y + r1z * r1z;
+    const double d1 = u[4] * r1x + u[5] * r1y + u[6] * r1z;
+    const double n2 = __builtin_fma(-2.0, d1, n1 + n0);
+    const double c2 = __builtin_fma(-d1, d1, n0 * n1);
+    const double d2 = d1 - n0;
+    const double den = __builtin_fma(c2, c2, v[3]);
+    const double j1 = rsq64(n1 * den);
+    const double j2 = rsq64(n2 * den);
+    const double w = d1 * j1 - d2 * j2;
+    Sx += w * v[0];
+    Sy += w * v[1];
+    Sz += w * v[2];
+    Tx += w * v[4];
+    Ty += w * v[5];
+    Tz += w * v[6];
 }
 
-template <int TILE>
-__global__ __launch_bounds__(TILE) void bs_fp64_kernel(BsArgs a)
+// The same pair in FP32 on centred coordinates (q = p - c formed in FP64
+// once per group): rounding q and a - c costs eps (|p - c| + |a - c|) <=
+// eps (|r1| + 2 R) for a group of radius R, and groups wider than 64 of
+// their longest segments are never far.  25 vector instructions, two of
+// them v_rsq_f32.
+__device__ __forceinline__ void pair32_far(const float *q, float4 a, float4 b, float4 c, float4 d,
+                                           float *S, float *T)
 {
-    __shared__ double4 sa[TILE];
-    __shared__ double4 sb[TILE];
-    __shared__ double sn[TILE];
-    __shared__ int item_sh;
-    const int tid = threadIdx.x;
-    const int64_t nseg = *a.nseg;
-    const int64_t S = a.sstride;
-    for (;;) {
-        const int item = next_item(a.counter, &item_sh);
-        if (item >= a.nitems) break;
-        const int chunk = item / a.ntiles;
-        const int tile = item - chunk * a.ntiles;
-        const int64_t s0 = (int64_t)chunk * a.chunk_len;
-        const int64_t s1 = min(nseg, s0 + a.chunk_len);
-        const int64_t t = (int64_t)tile * TILE + tid;
-        const bool live = t < a.m;
-        double px = 0.0, py = 0.0, pz = 0.0;
-        if (live) {
-            px = a.t[t];
-            py = a.t[a.tstride + t];
-            pz = a.t[2 * a.tstride + t];
-        }
-        double vx = 0.0, vy = 0.0, vz = 0.0;
-        for (int64_t base = s0; base < s1; base += TILE) {
-            const int cnt = (int)min<int64_t>(TILE, s1 - base);
-            __syncthreads();
-            if (tid < cnt) {
-                const int64_t s = base + tid;
-                sa[tid] = make_double4(a.s64[s], a.s64[S + s], a.s64[2 * S + s], a.s64[3 * S + s]);
-                sb[tid] = make_double4(a.s64[4 * S + s], a.s64[5 * S + s], a.s64[6 * S + s],
-                                       a.s64[7 * S + s]);
-                sn[tid] = a.s64[8 * S + s];
-            }
-            __syncthreads();
+    const float r1x = q[0] - a.x, r1y = q[1] - a.y, r1z = q[2] - a.z;
+    const float n0 = a.w;
+    const float n1 = r1x * r1x + r1y * r1y + r1z * r1z;
+    const float d1 = b.x * r1x + b.y * r1y + b.z * r1z;
+    const float n2 = __builtin_fmaf(-2.0f, d1, n1 + n0);
+    const float c2 = __builtin_fmaf(-d1, d1, n0 * n1);
+    const float d2 = d1 - n0;
+    const float den = __builtin_fmaf(c2, c2, b.w);
+    const float j1 = __builtin_amdgcn_rsqf(n1 * den);
+    const float j2 = __builtin_amdgcn_rsqf(n2 * den);
+    const float w = d1 * j1 - d2 * j2;
+    S[0] += w * c.x;
+    S[1] += w * c.y;
+    S[2] += w * c.z;
+    T[0] += w * d.x;
+    T[1] += w * d.y;
+    T[2] += w * d.z;
+}
+
+// One group for NK targets per lane, all far: records from the wave's LDS
+// copy (broadcast reads), sums folded into FP64 once per group.
+template <int NK>
+__device__ __forceinline__ void group32_far(const float4 *buf, const float (&q)[NK][3],
+                                            double (&v)[NK][3])
+{
+    float S[NK][3] = {}, T[NK][3] = {};
 #pragma unroll 2
-            for (int k = 0; k < cnt; ++k) pair64(px, py, pz, sa[k], sb[k], sn[k], vx, vy, vz);
+    for (int j = 0; j < GRP; ++j) {
+        const float4 a = buf[4 * j], b = buf[4 * j + 1], c = buf[4 * j + 2], d = buf[4 * j + 3];
+#pragma unroll
+        for (int k = 0; k < NK; ++k) pair32_far(q[k], a, b, c, d, S[k], T[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+        v[k][0] += (double)((S[k][1] * q[k][2] - S[k][2] * q[k][1]) - T[k][0]);
+        v[k][1] += (double)((S[k][2] * q[k][0] - S[k][0] * q[k][2]) - T[k][1]);
+        v[k][2] += (double)((S[k][0] * q[k][1] - S[k][1] * q[k][0]) - T[k][2]);
+    }
+}
+
+struct BsArgs {
+    const double *rec64, *grp;
+    const float *rec32, *near32;
+    const long long *nseg;
+    const double *t;
+    double *part;
+    int *counter;
+    int64_t m, tstride;
+    int nchunks, ntiles, nitems, round_robin;
+};
+
+// Work items of both kernels: a wave takes 64 NT targets (NT per lane) and
+// one chunk of groups; no LDS and no barrier, the records are wave-uniform
+// and reach the vector instructions as scalar operands.
+struct Item {
+    int chunk, tile;
+    int64_t g0, g1;
+};
+
+__device__ __forceinline__ Item item_of(const BsArgs &a, int item, int64_t ngroups)
+{
+    Item r;
+    r.chunk = item / a.ntiles;
+    r.tile = item - r.chunk * a.ntiles;
+    const int64_t len = (ngroups + a.nchunks - 1) / a.nchunks;
+    r.g0 = (int64_t)r.chunk * len;
+    r.g1 = min(ngroups, r.g0 + len);
+    return r;
+}
+
+// A wave's first item is its own index; later ones come from the counter,
+// or, in launches of short items (chunks of fewer than LEN_MID groups),
+// round robin: atomics on the one counter complete every 11 ns or so, which
+// bounded those launches (3.4e7 pairs: 258 us with the counter, 107 without).
+// Long launches need the counter: dealing out only their first quarter round
+// robin cost 3-6%, three quarters 15%.
+__device__ __forceinline__ int first_item()
+{
+    return __builtin_amdgcn_readfirstlane((int)blockIdx.x * (BS_BLOCK / 64) +
+                                          ((int)threadIdx.x >> 6));
+}
+__device__ __forceinline__ int next_item(const BsArgs &a, int item)
+{
+    const int nwaves = (int)gridDim.x * (BS_BLOCK / 64);
+    if (a.round_robin) return item + nwaves;
+    int next = 0;
+    if ((threadIdx.x & 63) == 0) next = atomicAdd(a.counter, 1);
+    return nwaves + __builtin_amdgcn_readfirstlane(next);
+}
+
+__global__ __launch_bounds__(BS_BLOCK, 8) void bs_fp64_kernel(BsArgs a)
+{
+    const int lane = threadIdx.x & 63;
+    const int64_t ngroups = (*(clptr)a.nseg + GRP - 1) / GRP;
+    for (int item = first_item(); item < a.nitems; item = next_item(a, item)) {
+        const Item it = item_of(a, item, ngroups);
+        const int64_t t = (int64_t)it.tile * 64 + lane;
+        const int64_t tc = t < a.m ? t : a.m - 1;   // idle lanes repeat the last target
+        const double px = a.t[tc], py = a.t[a.tstride + tc], pz = a.t[2 * a.tstride + tc];
+        double vx = 0.0, vy = 0.0, vz = 0.0;
+        for (int64_t g = it.g0; g < it.g1; ++g) {
+            const cdptr h = (cdptr)a.grp + g * GRPH_N;
+            const double qx = px - h[0], qy = py - h[1], qz = pz - h[2];
+            const bool far = qx * qx + qy * qy + qz * qz > h[3];
+            if (__ballot(!far) == 0) {
+                cd8ptr r = (cd8ptr)(a.rec64 + g * (GRP * REC64_N));
+                double Sx = 0, Sy = 0, Sz = 0, Tx = 0, Ty = 0, Tz = 0;
+#pragma unroll 2
+                for (int j = 0; j < GRP; ++j, r += 2) {
+                    const d8 u = r[0], w = r[1];
+                    pair64_far(px, py, pz, u, w, Sx, Sy, Sz, Tx, Ty, Tz);
+                }
+                vx += (Sy * qz - Sz * qy) - Tx;
+                vy += (Sz * qx - Sx * qz) - Ty;
+                vz += (Sx * qy - Sy * qx) - Tz;
+            } else {
+                cdptr r = (cdptr)a.rec64 + g * (GRP * REC64_N);
+                for (int j = 0; j < GRP; ++j, r += REC64_N)
+                    pair64(px, py, pz, r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[11], r[7], vx,
+                           vy, vz);
+            }
         }
-        if (live) {
-            double *o = a.part + (size_t)chunk * 3 * a.m;
+        if (t < a.m) {
+            double *o = a.part + (size_t)it.chunk * 3 * a.m;
             o[t] = vx;
             o[a.m + t] = vy;
             o[2 * a.m + t] = vz;
@@ -204,187 +328,112 @@ __global__ __launch_bounds__(TILE) void bs_fp64_kernel(BsArgs a)
     }
 }
 
-__device__ __forceinline__ void kahan_add(float &s, float &c, float x)
+// FP32 instructions run at half rate with a scalar operand (4.2 against 2.4
+// cycles per wave instruction, measured), so here the wave copies each
+// group's records to its own 2 KB of LDS (the next group's are loaded while
+// this one is evaluated) and reads them back as broadcasts, each shared by
+// the NT targets of a lane.  Groups that are not far for all 64 NT targets
+// are tested again per 64; the near ones run pair32 with scalar operands,
+// and the lanes recompute their flagged pairs in FP64 after the group.
+template <int NT>
+__global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
 {
-    const float y = x - c;
-    const float tt = s + y;
-    c = (tt - s) - y;
-    s = tt;
-}
-
-// FP32 pair for a group of segments that every target of the wave is far
-// from (see the group test in bs_mixed_kernel), without the near-field
-// handling: no target lies within two segment lengths of a segment, so no
-// pair is near-singular, |r1| and |r2| are bounded away from zero (no
-// unitVec clamp) and every core term q is positive (no zero-denominator
-// guard).  Coordinates are relative to the group's centre c: q = p - c
-// (formed once per group), al = (a - c, (rc^2 |r0|^2)^2), g the
-// circulation factor, s2 = (r0, 4 |r0|^2).  The rounding of q and al is
-// about eps (|p - c| + |a - c|) <= eps (|r1| + 2 R) for a group of radius
-// R; the far test keeps |r1| >= 2 |r0| for every segment, and groups wider
-// than 64 times their longest segment are never far.  A segment's error
-// and its contribution both scale with its |r0|, so no pair's error
-// exceeds about 64 eps of the contribution of the group's longest segment
-// at the same distance, without the hi/lo split.
-__device__ __forceinline__ void pair32_local(float qx, float qy, float qz, float4 al, float g,
-                                             float4 s2, float &vx, float &vy, float &vz)
-{
-    const float r1x = qx - al.x, r1y = qy - al.y, r1z = qz - al.z;
-    const float r0x = s2.x, r0y = s2.y, r0z = s2.z;
-    const float r2x = r1x - r0x, r2y = r1y - r0y, r2z = r1z - r0z;
-    const float cx = r0y * r1z - r0z * r1y;
-    const float cy = r0z * r1x - r0x * r1z;
-    const float cz = r0x * r1y - r0y * r1x;
-    const float c2 = cx * cx + cy * cy + cz * cz;
-    const float n1 = r1x * r1x + r1y * r1y + r1z * r1z;
-    const float n2 = r2x * r2x + r2y * r2y + r2z * r2z;
-    const float d1 = r0x * r1x + r0y * r1y + r0z * r1z;
-    const float d2 = __builtin_fmaf(s2.w, -0.25f, d1);
-    const float den = __builtin_fmaf(c2, c2, al.w);
-    const float j1 = __builtin_amdgcn_rsqf(n1 * den);
-    const float j2 = __builtin_amdgcn_rsqf(n2 * den);
-    const float s = g * (d1 * j1 - d2 * j2);
-    vx += cx * s;
-    vy += cy * s;
-    vz += cz * s;
-}
-
-// MIXED: the staged batch is cut into groups of 32 segments.  At staging,
-// each group gets a far radius around its first segment's start point:
-// the largest |a_i - c| + 2 |r0_i| over the group (plus a rounding
-// margin), or infinity for a short group, one holding a segment with
-// q = rc^2 |r0|^2 below 1e-18, or one wider than 64 of its longest segments.  A wave whose targets all lie outside that
-// radius runs the group with pair32_local (coordinates relative to the
-// group's centre, staged beside the split ones); otherwise it runs pair32, which
-// flags near-singular pairs in a 32-bit mask, and recomputes the flagged
-// ones in FP64 after the group (records read from the FP64 list in global
-// memory), so the FP32 loops stay free of the FP64 branch.  Staged groups
-// are padded with zero records, which contribute exactly zero and are
-// never near (r0 = 0).  __launch_bounds__'s second argument asks for 7
-// waves per SIMD (72 VGPRs), which both pair loops fit.
-template <int TILE>
-__global__ __launch_bounds__(TILE, 7) void bs_mixed_kernel(BsArgs a)
-{
-    static_assert(TILE % 32 == 0, "groups of 32 segments");
-    __shared__ float4 s0v[TILE];
-    __shared__ float4 s1v[TILE];
-    __shared__ float4 s2v[TILE];
-    __shared__ float4 s3v[TILE];          // a - centre of the group, q^2
-    __shared__ float4 far_sh[TILE / 32];  // centre, squared far radius
-    __shared__ int item_sh;
-    const int tid = threadIdx.x;
-    const int64_t nseg = *a.nseg;
-    const int64_t S = a.sstride;
-    for (;;) {
-        const int item = next_item(a.counter, &item_sh);
-        if (item >= a.nitems) break;
-        const int chunk = item / a.ntiles;
-        const int tile = item - chunk * a.ntiles;
-        const int64_t sb0 = (int64_t)chunk * a.chunk_len;
-        const int64_t sb1 = min(nseg, sb0 + a.chunk_len);
-        const int64_t t = (int64_t)tile * TILE + tid;
-        const bool live = t < a.m;
-        double px = 0.0, py = 0.0, pz = 0.0;
-        if (live) {
-            px = a.t[t];
-            py = a.t[a.tstride + t];
-            pz = a.t[2 * a.tstride + t];
-        }
-        const float phx = (float)px, phy = (float)py, phz = (float)pz;
-        const float plx = (float)(px - (double)phx), ply = (float)(py - (double)phy),
-                    plz = (float)(pz - (double)phz);
-        float Sx = 0.f, Sy = 0.f, Sz = 0.f, Cx = 0.f, Cy = 0.f, Cz = 0.f;
-        double nx = 0.0, ny = 0.0, nz = 0.0;
-        for (int64_t base = sb0; base < sb1; base += TILE) {
-            const int cnt = (int)min<int64_t>(TILE, sb1 - base);
-            const int cnt32 = (cnt + 31) & ~31;
-            __syncthreads();
-            {
-                float4 v0 = make_float4(0.f, 0.f, 0.f, 0.f), v1 = v0, v2 = v0;
-                if (tid < cnt) {
-                    const int64_t s = base + tid;
-                    v0 = make_float4(a.s32[s], a.s32[S + s], a.s32[2 * S + s], a.s32[3 * S + s]);
-                    v1 = make_float4(a.s32[4 * S + s], a.s32[5 * S + s], a.s32[6 * S + s],
-                                     a.s32[7 * S + s]);
-                    v2 = make_float4(a.s32[8 * S + s], a.s32[9 * S + s], a.s32[10 * S + s],
-                                     a.s32[11 * S + s]);
-                }
-                // far radius of this lane's group (lanes 32k .. 32k+31)
-                const float cx = __shfl(v0.x, 0, 32), cy = __shfl(v0.y, 0, 32),
-                            cz = __shfl(v0.z, 0, 32);
-                if (tid < cnt32) {
-                    s0v[tid] = v0;
-                    s1v[tid] = v1;
-                    s2v[tid] = v2;
-                    s3v[tid] = make_float4((v0.x - cx) + v1.x, (v0.y - cy) + v1.y,
-                                           (v0.z - cz) + v1.z, v1.w * v1.w);
-                }
-                const float dx = v0.x - cx, dy = v0.y - cy, dz = v0.z - cz;
-                float ex = sqrtf(dx * dx + dy * dy + dz * dz) + sqrtf(v2.w);  // + 2 |r0|
-                float lmax = sqrtf(v2.w);                                     // 2 |r0|
-                if (tid >= cnt || !(v1.w > 1e-18f)) ex = __builtin_inff();
-                for (int o = 16; o > 0; o >>= 1) {
-                    ex = fmaxf(ex, __shfl_xor(ex, o, 32));
-                    lmax = fmaxf(lmax, __shfl_xor(lmax, o, 32));
-                }
-                // a group wider than 64 of its longest segments (records that
-                // jump between distant wake rows; a chain of 32 connected
-                // segments spans at most 34) takes the near path, whose split
-                // coordinates do not lose accuracy with the group's width
-                if (ex > 32.0f * lmax) ex = __builtin_inff();
-                if ((tid & 31) == 0 && tid < cnt32) {
-                    const float cm = fmaxf(fabsf(cx), fmaxf(fabsf(cy), fabsf(cz)));
-                    const float rr = ex * 1.0001f + 1e-5f * cm + 1e-30f;
-                    far_sh[tid >> 5] = make_float4(cx, cy, cz, rr * rr);
-                }
+    __shared__ float4 lds[BS_BLOCK / 64][GRP * 4];
+    const int lane = threadIdx.x & 63;
+    float4 *buf = lds[threadIdx.x >> 6];
+    const int64_t ngroups = (*(clptr)a.nseg + GRP - 1) / GRP;
+    for (int item = first_item(); item < a.nitems; item = next_item(a, item)) {
+        const Item it = item_of(a, item, ngroups);
+        double p[NT][3], v[NT][3];
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            const int64_t t = ((int64_t)it.tile * NT + k) * 64 + lane;
+            const int64_t tc = t < a.m ? t : a.m - 1;   // idle lanes repeat the last target
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+                p[k][d] = a.t[d * a.tstride + tc];
+                v[k][d] = 0.0;
             }
-            __syncthreads();
-            float tx = 0.f, ty = 0.f, tz = 0.f;
-            for (int g = 0; g < cnt32; g += 32) {
-                const float4 f = far_sh[g >> 5];
-                const float qx = phx - f.x, qy = phy - f.y, qz = phz - f.z;
-                const bool far = !live || (qx * qx + qy * qy + qz * qz > f.w);
-                if (__builtin_amdgcn_readfirstlane(__all(far))) {
-                    const float lx = qx + plx, ly = qy + ply, lz = qz + plz;
-#pragma unroll 4
-                    for (int j = 0; j < 32; ++j)
-                        pair32_local(lx, ly, lz, s3v[g + j], s0v[g + j].w, s2v[g + j], tx, ty,
-                                     tz);
+        }
+        const float4 *src = reinterpret_cast<const float4 *>(a.rec32) + lane;
+        float4 n0, n1;
+        if (it.g0 < it.g1) {
+            n0 = src[it.g0 * (GRP * 4)];
+            n1 = src[it.g0 * (GRP * 4) + 64];
+        }
+        for (int64_t g = it.g0; g < it.g1; ++g) {
+            __builtin_amdgcn_wave_barrier();
+            buf[lane] = n0;
+            buf[lane + 64] = n1;
+            __builtin_amdgcn_wave_barrier();
+            const int64_t gn = min(g + 1, it.g1 - 1);
+            n0 = src[gn * (GRP * 4)];
+            n1 = src[gn * (GRP * 4) + 64];
+            const cdptr h = (cdptr)a.grp + g * GRPH_N;
+            float q[NT][3];
+            unsigned near = 0;   // bit k: a target of the k-th 64 is not far
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                double d2 = 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) {
+                    const double x = p[k][d] - h[d];
+                    d2 += x * x;
+                    q[k][d] = (float)x;
+                }
+                if (__ballot(!(d2 > h[3])) != 0) near |= 1u << k;
+            }
+            if (near == 0) {
+                group32_far<NT>(buf, q, v);
+                continue;
+            }
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                if (!(near >> k & 1u)) {
+                    const float qk[1][3] = {{q[k][0], q[k][1], q[k][2]}};
+                    double vk[1][3] = {{v[k][0], v[k][1], v[k][2]}};
+                    group32_far<1>(buf, qk, vk);
+                    for (int d = 0; d < 3; ++d) v[k][d] = vk[0][d];
                     continue;
                 }
+                const double px = p[k][0], py = p[k][1], pz = p[k][2];
+                const float phx = (float)px, phy = (float)py, phz = (float)pz;
+                const float plx = (float)(px - (double)phx), ply = (float)(py - (double)phy),
+                            plz = (float)(pz - (double)phz);
+                cfptr r = (cfptr)a.rec32 + g * (GRP * REC32_N);
+                cfptr n = (cfptr)a.near32 + g * (GRP * NEAR32_N);
+                float tx = 0.f, ty = 0.f, tz = 0.f;
                 unsigned mask = 0u;
-#pragma unroll 4
-                for (int j = 0; j < 32; ++j) {
-                    const bool nearp = pair32(phx, phy, phz, plx, ply, plz, s0v[g + j],
-                                              s1v[g + j], s2v[g + j], tx, ty, tz);
+                for (int j = 0; j < GRP; ++j, r += REC32_N, n += NEAR32_N) {
+                    const bool nearp = pair32(phx, phy, phz, plx, ply, plz, r, n, tx, ty, tz);
                     mask |= (nearp ? 1u : 0u) << j;
                 }
-                if (!live) mask = 0u;
+                v[k][0] += (double)tx;
+                v[k][1] += (double)ty;
+                v[k][2] += (double)tz;
                 while (mask) {
                     const int j = __builtin_ctz(mask);
                     mask &= mask - 1u;
-                    const int64_t s = base + g + j;
-                    pair64(px, py, pz,
-                           make_double4(a.s64[s], a.s64[S + s], a.s64[2 * S + s], a.s64[3 * S + s]),
-                           make_double4(a.s64[4 * S + s], a.s64[5 * S + s], a.s64[6 * S + s],
-                                        a.s64[7 * S + s]),
-                           a.s64[8 * S + s], nx, ny, nz);
+                    const double *s = a.rec64 + (g * GRP + j) * REC64_N;
+                    pair64(px, py, pz, s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[11], s[7],
+                           v[k][0], v[k][1], v[k][2]);
                 }
             }
-            kahan_add(Sx, Cx, tx);
-            kahan_add(Sy, Cy, ty);
-            kahan_add(Sz, Cz, tz);
         }
-        if (live) {
-            double *o = a.part + (size_t)chunk * 3 * a.m;
-            o[t] = ((double)Sx - (double)Cx) + nx;
-            o[a.m + t] = ((double)Sy - (double)Cy) + ny;
-            o[2 * a.m + t] = ((double)Sz - (double)Cz) + nz;
+        double *o = a.part + (size_t)it.chunk * 3 * a.m;
+#pragma unroll
+        for (int k = 0; k < NT; ++k) {
+            const int64_t t = ((int64_t)it.tile * NT + k) * 64 + lane;
+            if (t < a.m) {
+                o[t] = v[k][0];
+                o[a.m + t] = v[k][1];
+                o[2 * a.m + t] = v[k][2];
+            }
         }
     }
 }
 
-// Few targets (collocation points, judge samples: m < 1024): each block
+// Few targets (collocation points, bound vortices, probes): each block
 // takes SM_T targets and one segment chunk; its 256 lanes stride over the
 // chunk (coalesced SoA loads, each record shared by the SM_T targets) and
 // the partial sums are reduced in a fixed order (butterfly within the wave,
@@ -392,6 +441,14 @@ __global__ __launch_bounds__(TILE, 7) void bs_mixed_kernel(BsArgs a)
 // pairs.
 constexpr int SM_T = 4;
 constexpr int SM_BLOCK = 256;
+// fewer targets than this take bs_small_kernel: its lanes are segments, so
+// no lane idles however few the targets (20 targets x 2e5 segments: 54
+// against 92 us with a wave of 64 targets; 90 targets: 92 against 108), but
+// every pair is the long one (300 targets: 186 against 165 us)
+constexpr int SM_MAX = 192;
+constexpr int LEN_MID = 8;
+constexpr int MIXED_NT = 2;       // targets per lane of the mixed kernel
+constexpr int MIXED_MIN = 1024;   // fewer targets than this: FP64 in both modes
 
 __device__ __forceinline__ double wave_sum(double v)
 {
@@ -421,13 +478,13 @@ __global__ __launch_bounds__(SM_BLOCK) void bs_small_kernel(const double *s64, i
         vx[q] = vy[q] = vz[q] = 0.0;
     }
     for (int64_t sg = s0 + tid; sg < s1; sg += SM_BLOCK) {
-        const double4 sa = make_double4(s64[sg], s64[S + sg], s64[2 * S + sg], s64[3 * S + sg]);
-        const double4 sb =
-            make_double4(s64[4 * S + sg], s64[5 * S + sg], s64[6 * S + sg], s64[7 * S + sg]);
-        const double n0 = s64[8 * S + sg];
+        double r[SOA_N];
+#pragma unroll
+        for (int i = 0; i < SOA_N; ++i) r[i] = s64[i * S + sg];
 #pragma unroll
         for (int q = 0; q < SM_T; ++q)
-            pair64(px[q], py[q], pz[q], sa, sb, n0, vx[q], vy[q], vz[q]);
+            pair64(px[q], py[q], pz[q], r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[7], r[8],
+                   vx[q], vy[q], vz[q]);
     }
 #pragma unroll
     for (int q = 0; q < SM_T; ++q) {
@@ -449,31 +506,64 @@ __global__ __launch_bounds__(SM_BLOCK) void bs_small_kernel(const double *s64, i
     }
 }
 
-// Fixed-order sum of the per-chunk partials: one lane per (target,
-// component), chunks added in increasing order; loads are issued eight
-// chunks ahead of the adds.
-constexpr int RED_BLOCK = 64;
-
-__global__ __launch_bounds__(RED_BLOCK) void bs_reduce_kernel(const double *part, int nchunks,
-                                                              int64_t m, double *out,
-                                                              int64_t ostride, int acc)
+// Fixed-order sum of the per-chunk partials: T targets of one component per
+// workgroup, S slices of the chunk range side by side (each in increasing
+// order, loads eight chunks ahead of the adds), the slices added in order.
+// Bound by the dependent round trips to memory of one slice: a lane that
+// walked all chunks alone waited once per eight loads, so many chunks take
+// many slices.  Workgroup 0 clears the work counter for the next launch.
+template <int T, int S>
+__global__ __launch_bounds__(T * S) void bs_reduce_kernel(const double *part, int nchunks,
+                                                          int64_t m, double *out,
+                                                          int64_t ostride, int acc, int *counter)
 {
-    const int64_t t = (int64_t)blockIdx.x * RED_BLOCK + threadIdx.x;
+    __shared__ double sh[S][T];
+    const int l = threadIdx.x % T, w = threadIdx.x / T;
+    const int64_t t = (int64_t)blockIdx.x * T + l;
     const int d = blockIdx.y;
-    if (t >= m) return;
-    const double *p = part + (size_t)d * m + t;
-    const size_t cs = 3 * (size_t)m;
-    double s = acc ? out[d * ostride + t] : 0.0;
-    int c = 0;
-    for (; c + 8 <= nchunks; c += 8) {
-        double v[8];
+    if (counter && blockIdx.x == 0 && d == 0 && threadIdx.x == 0) *counter = 0;
+    const int len = (nchunks + S - 1) / S;
+    const int c1 = min(nchunks, (w + 1) * len);
+    double s = 0.0;
+    if (t < m) {
+        const double *p = part + (size_t)d * m + t;
+        const size_t cs = 3 * (size_t)m;
+        int c = w * len;
+        for (; c + 8 <= c1; c += 8) {
+            double v[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = p[(size_t)(c + k) * cs];
+            for (int k = 0; k < 8; ++k) v[k] = p[(size_t)(c + k) * cs];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) s += v[k];
+            for (int k = 0; k < 8; ++k) s += v[k];
+        }
+        for (; c < c1; ++c) s += p[(size_t)c * cs];
     }
-    for (; c < nchunks; ++c) s += p[(size_t)c * cs];
-    out[d * ostride + t] = s;
+    if constexpr (S > 1) {
+        sh[w][l] = s;
+        __syncthreads();
+        if (w > 0) return;
+        for (int k = 1; k < S; ++k) s += sh[k][l];
+    }
+    if (t < m) out[d * ostride + t] = acc ? out[d * ostride + t] + s : s;
+}
+
+template <int T, int S>
+void reduce_as(vlm_ctx *ctx, const double *part, int nchunks, int64_t m, double *out,
+               int64_t ostride, int acc, int *counter)
+{
+    hipLaunchKernelGGL((bs_reduce_kernel<T, S>), dim3((unsigned)((m + T - 1) / T), 3), dim3(T * S),
+                       0, ctx->stream, part, nchunks, m, out, ostride, acc, counter);
+}
+
+int launch_reduce(vlm_ctx *ctx, const double *part, int nchunks, int64_t m, double *out,
+                  int64_t ostride, int acc, int *counter)
+{
+    if (nchunks >= 256) reduce_as<16, 64>(ctx, part, nchunks, m, out, ostride, acc, counter);
+    else if (nchunks >= 32) reduce_as<64, 8>(ctx, part, nchunks, m, out, ostride, acc, counter);
+    else if (nchunks >= 8) reduce_as<64, 4>(ctx, part, nchunks, m, out, ostride, acc, counter);
+    else reduce_as<64, 1>(ctx, part, nchunks, m, out, ostride, acc, counter);
+    VLM_HIP(hipGetLastError());
+    return VLM_OK;
 }
 
 __global__ void zero_int_kernel(int *p) { *p = 0; }
@@ -513,8 +603,13 @@ int profile_count(vlm_ctx *ctx, const long long *nseg_dev, int64_t m, int kind, 
 
 }  // namespace
 
-int bs_eval(vlm_ctx *ctx, const double *seg64, const float *seg32, int64_t segstride,
-            const long long *nseg_dev, int64_t nseg_max, const double *t, int64_t m,
+int bs_formats(const vlm_ctx *ctx, int64_t m)
+{
+    if (m < SM_MAX) return SEG_SOA;
+    return ctx->precision == VLM_MIXED && m >= MIXED_MIN ? SEG_REC | SEG_F32 : SEG_REC;
+}
+
+int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t, int64_t m,
             int64_t tstride, double *out, int accumulate, const BsWork *ws)
 {
     if (m <= 0) return VLM_OK;
@@ -523,101 +618,101 @@ int bs_eval(vlm_ctx *ctx, const double *seg64, const float *seg32, int64_t segst
     const int64_t max_chunks = ws ? (int64_t)(ws->part_cap / (3 * (size_t)m)) : INT32_MAX;
     if (ws && max_chunks < 1) return fail(ctx, VLM_ERR_ARG, "workspace too small for the targets");
     const bool prof = ctx->profile && !ws;
-    if (m < 1024) {
-        // about 2048 blocks, at least 8 segments per lane
+    if (nseg_est <= 0) return launch_reduce(ctx, nullptr, 0, m, out, tstride, accumulate, nullptr);
+    const int fmt = bs_formats(ctx, m);
+    if (((fmt & SEG_SOA) && !seg.soa) || ((fmt & SEG_REC) && !seg.rec64) ||
+        ((fmt & SEG_F32) && !seg.rec32))
+        return fail(ctx, VLM_ERR_STATE, "segment list lacks the records of this launch");
+    if (fmt == SEG_SOA) {
+        // about 2048 blocks of at least 8 segments per lane; short lists are
+        // split down to 2 per lane, up to 16 chunks (their loads wait on
+        // each other; more chunks only feed the reduction)
         const int64_t groups = (m + SM_T - 1) / SM_T;
         int64_t nc = (2048 + groups - 1) / groups;
-        const int64_t maxc = nseg_max / (8 * SM_BLOCK);
+        const int64_t c2 = nseg_est / (2 * SM_BLOCK), c8 = nseg_est / (8 * SM_BLOCK);
+        const int64_t maxc = c8 > 16 ? c8 : (c2 > 16 ? 16 : c2);
         if (nc > maxc) nc = maxc;
         if (nc > max_chunks) nc = max_chunks;
         if (nc < 1) nc = 1;
-        const int nchunks = nseg_max > 0 ? (int)nc : 0;
+        const int nchunks = (int)nc;
         double *part = ws ? ws->part : nullptr;
-        if (nchunks > 0) {
-            if (!ws) {
-                VLM_HIP(ctx->part.reserve((size_t)nchunks * 3 * (size_t)m));
-                part = ctx->part.p;
-            }
-            hipLaunchKernelGGL(bs_small_kernel, dim3(nchunks, (unsigned)groups), dim3(SM_BLOCK),
-                               0, ctx->stream, seg64, segstride, nseg_dev, nchunks, t, m, tstride,
-                               part);
-            VLM_HIP(hipGetLastError());
-            if (prof) VLM_TRY(profile_count(ctx, nseg_dev, m, 1, nullptr));
-        }
-        hipLaunchKernelGGL(bs_reduce_kernel, dim3((unsigned)((m + RED_BLOCK - 1) / RED_BLOCK), 3),
-                           dim3(RED_BLOCK), 0,
-                           ctx->stream, part, nchunks, m, out, tstride, accumulate);
-        VLM_HIP(hipGetLastError());
-        return VLM_OK;
-    }
-    const int blk = BS_BLOCK;
-    const int ntiles = (int)((m + blk - 1) / blk);
-    const bool mixed = ctx->precision == VLM_MIXED;
-    int cap = mixed ? resident_blocks(ctx, bs_mixed_kernel<BS_BLOCK>, blk, &ctx->occ[1])
-                    : resident_blocks(ctx, bs_fp64_kernel<BS_BLOCK>, blk, &ctx->occ[3]);
-    if (cap <= 0) return fail(ctx, VLM_ERR_HIP, "occupancy query failed");
-    int nchunks = 0;
-    int64_t chunk_len = 1;
-    if (nseg_max > 0) {
-        // about 16 work items per resident workgroup, chunks of at least
-        // four tiles
-        const int64_t min_len = 4 * BS_BLOCK;
-        int64_t nc = ((int64_t)16 * cap + ntiles - 1) / ntiles;
-        const int64_t maxc = (nseg_max + min_len - 1) / min_len;
-        if (nc > maxc) nc = maxc;
-        if (nc > max_chunks) nc = max_chunks;
-        if (nc < 1) nc = 1;
-        chunk_len = (nseg_max + nc - 1) / nc;
-        nchunks = (int)((nseg_max + chunk_len - 1) / chunk_len);
-    }
-    double *part = ws ? ws->part : nullptr;
-    if (nchunks > 0) {
-        int *counter = ws ? ws->counter : nullptr;
         if (!ws) {
             VLM_HIP(ctx->part.reserve((size_t)nchunks * 3 * (size_t)m));
-            VLM_HIP(ctx->counter.reserve(1));
             part = ctx->part.p;
-            counter = ctx->counter.p;
         }
-        BsArgs a;
-        a.s64 = seg64;
-        a.s32 = seg32;
-        a.sstride = segstride;
-        a.nseg = nseg_dev;
-        a.chunk_len = chunk_len;
-        a.t = t;
-        a.m = m;
-        a.tstride = tstride;
-        a.part = part;
-        a.ntiles = ntiles;
-        a.nitems = ntiles * nchunks;
-        a.counter = counter;
-        const int grid = a.nitems < cap ? a.nitems : cap;
-        hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(1), 0, ctx->stream, counter);
-        Timer tm{};
-        const bool timed = prof;
-        if (timed) {
-            VLM_HIP(hipEventCreate(&tm.a));
-            VLM_HIP(hipEventCreate(&tm.b));
-            VLM_HIP(hipEventRecord(tm.a, ctx->stream));
-        }
-        if (mixed)
-            hipLaunchKernelGGL(bs_mixed_kernel<BS_BLOCK>, dim3(grid), dim3(blk), 0, ctx->stream,
-                               a);
-        else
-            hipLaunchKernelGGL(bs_fp64_kernel<BS_BLOCK>, dim3(grid), dim3(blk), 0, ctx->stream,
-                               a);
+        hipLaunchKernelGGL(bs_small_kernel, dim3(nchunks, (unsigned)groups), dim3(SM_BLOCK), 0,
+                           ctx->stream, seg.soa, seg.cap, seg.count, nchunks, t, m, tstride,
+                           part);
         VLM_HIP(hipGetLastError());
-        if (timed) {
-            VLM_HIP(hipEventRecord(tm.b, ctx->stream));
-            VLM_TRY(profile_count(ctx, nseg_dev, m, 0, &tm));
-        }
+        if (prof) VLM_TRY(profile_count(ctx, seg.count, m, 1, nullptr));
+        return launch_reduce(ctx, part, nchunks, m, out, tstride, accumulate, nullptr);
     }
-    hipLaunchKernelGGL(bs_reduce_kernel, dim3((unsigned)((m + RED_BLOCK - 1) / RED_BLOCK), 3),
-                       dim3(RED_BLOCK), 0,
-                       ctx->stream, part, nchunks, m, out, tstride, accumulate);
+    const bool mixed = (fmt & SEG_F32) != 0;
+    const int tile = mixed ? 64 * MIXED_NT : 64;
+    const int ntiles = (int)((m + tile - 1) / tile);
+    const int cap = mixed ? resident_blocks(ctx, bs_mixed_kernel<MIXED_NT>, BS_BLOCK, &ctx->occ[1])
+                          : resident_blocks(ctx, bs_fp64_kernel, BS_BLOCK, &ctx->occ[0]);
+    if (cap <= 0) return fail(ctx, VLM_ERR_HIP, "occupancy query failed");
+    const int64_t W = (int64_t)cap * (BS_BLOCK / 64);   // resident waves
+    const int64_t ngroups = (nseg_est + GRP - 1) / GRP;
+    const int64_t P = ngroups * ntiles;
+    // groups per chunk: two items per wave while that makes chunks shorter
+    // than LEN_MID groups (launches that barely fill the device: an item
+    // costs its latency, not its work), then LEN_MID until there are 16
+    // items per wave (the queue needs them to even out the end: 4 per wave
+    // cost 5% on 4.0e9 pairs, 32 gained nothing), then longer chunks (fewer
+    // partial sums)
+    int64_t len = P / (2 * W);
+    if (len > LEN_MID) len = LEN_MID;
+    if (P / (16 * W) > len) len = P / (16 * W);
+    if (len < 1) len = 1;
+    if ((ngroups + len - 1) / len > max_chunks) len = (ngroups + max_chunks - 1) / max_chunks;
+    const int nchunks = (int)((ngroups + len - 1) / len);
+    double *part = ws ? ws->part : nullptr;
+    int *counter = ws ? ws->counter : nullptr;
+    if (!ws) {
+        VLM_HIP(ctx->part.reserve((size_t)nchunks * 3 * (size_t)m));
+        if (!ctx->counter.p) {
+            VLM_HIP(ctx->counter.reserve(1));
+            hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(1), 0, ctx->stream, ctx->counter.p);
+        }
+        part = ctx->part.p;
+        counter = ctx->counter.p;
+    }
+    BsArgs a;
+    a.rec64 = seg.rec64;
+    a.grp = seg.grp;
+    a.rec32 = seg.rec32;
+    a.near32 = seg.near32;
+    a.nseg = seg.count;
+    a.t = t;
+    a.part = part;
+    a.counter = counter;
+    a.m = m;
+    a.tstride = tstride;
+    a.nchunks = nchunks;
+    a.ntiles = ntiles;
+    const int64_t nitems = (int64_t)ntiles * nchunks;
+    if (nitems > INT32_MAX - W) return fail(ctx, VLM_ERR_ARG, "too many work items");
+    a.nitems = (int)nitems;
+    const int64_t need = (nitems + BS_BLOCK / 64 - 1) / (BS_BLOCK / 64);
+    const int grid = (int)(need < cap ? need : cap);
+    a.round_robin = len < LEN_MID || need <= cap;
+    Timer tm{};
+    const bool timed = prof && m >= MIXED_MIN;
+    if (timed) {
+        VLM_HIP(hipEventCreate(&tm.a));
+        VLM_HIP(hipEventCreate(&tm.b));
+        VLM_HIP(hipEventRecord(tm.a, ctx->stream));
+    }
+    if (mixed)
+        hipLaunchKernelGGL(bs_mixed_kernel<MIXED_NT>, dim3(grid), dim3(BS_BLOCK), 0, ctx->stream, a);
+    else
+        hipLaunchKernelGGL(bs_fp64_kernel, dim3(grid), dim3(BS_BLOCK), 0, ctx->stream, a);
     VLM_HIP(hipGetLastError());
-    return VLM_OK;
+    if (timed) VLM_HIP(hipEventRecord(tm.b, ctx->stream));
+    if (prof) VLM_TRY(profile_count(ctx, seg.count, m, timed ? 0 : 1, timed ? &tm : nullptr));
+    return launch_reduce(ctx, part, nchunks, m, out, tstride, accumulate, counter);
 }
 
 }  // namespace vlm

@@ -20,7 +20,12 @@
 #include "vlm_internal.h"
 
 namespace vlm {
-constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)64 << 20;  // 64 MiB per GPU
+// Inputs are accepted up to 64 MiB at 120 B per filament and 72 B per point
+// (72 + 48 B of records per filament, targets, sums and one chunk).  The
+// records take 225 B per filament, so the array is 64 MiB x 225 / 120 plus
+// room for chunks.
+constexpr size_t NOALLOC_ACCEPTED_BYTES = (size_t)64 << 20;
+constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)192 << 20;
 }
 
 static __device__ __align__(256) unsigned char scratch[vlm::NOALLOC_SCRATCH_BYTES];
@@ -53,30 +58,12 @@ size_t up256(size_t b) { return (b + 255) & ~(size_t)255; }
 
 unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
 
-// Records of an explicit list (every filament kept, as in
-// vlm_filament_vind) at their own index, from 3 x n AoS device arrays.
-__global__ void fil_records_kernel(int64_t n, const double *a, const double *b, const double *g,
-                                   const double *rc, double *d64, float *d32, int64_t cap)
+// AoS device arrays to SoA targets; the first workgroup also clears the
+// work counter of the launch that follows.
+__global__ void aos_to_soa3_kernel(int64_t m, const double *aos, double *soa, int *counter)
 {
     const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    Slot s;
-    s.ax = a[3 * i];
-    s.ay = a[3 * i + 1];
-    s.az = a[3 * i + 2];
-    s.bx = b[3 * i];
-    s.by = b[3 * i + 1];
-    s.bz = b[3 * i + 2];
-    s.gam = g[i];
-    s.rc = rc[i];
-    write_segment_record(s, i, d64, d32, cap);
-}
-
-__global__ void set_count_kernel(long long *count, int64_t n) { *count = (long long)n; }
-
-__global__ void aos_to_soa3_kernel(int64_t m, const double *aos, double *soa)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) *counter = 0;
     if (i >= m) return;
     soa[i] = aos[3 * i];
     soa[m + i] = aos[3 * i + 1];
@@ -108,46 +95,60 @@ int vlm_filament_vind_noalloc(vlm_ctx *ctx, int64_t nfil, const double *a, const
     if (m == 0) return VLM_OK;
     if (!p || !v || (nfil > 0 && (!a || !b || !gam || !rc)))
         return fail(ctx, VLM_ERR_ARG, "null buffer");
-    // workspace layout: d64 | d32 | count | counter | targets | sums | partials
-    const int64_t cap = nfil > 0 ? nfil : 1;
-    const size_t o64 = 0;
-    const size_t o32 = o64 + up256((size_t)SEG64_N * cap * sizeof(double));
-    const size_t ocnt = o32 + up256((size_t)SEG32_N * cap * sizeof(float));
+    // workspace layout: soa | rec64 | grp | rec32 | near32 (the formats that
+    // m targets need) | count | counter |
+    // targets | sums | partials.  The sizes accepted are those of the
+    // documented 64 MiB at 120 B per filament and 72 B per point; the array
+    // itself is larger (225 B per filament, group records included).
+    const int64_t cap = nfil > 0 ? nfil : 1, gcap = (cap + GRP - 1) / GRP, rcap = gcap * GRP;
+    const int fmt = bs_formats(ctx, m);
+    const size_t osoa = 0;
+    const size_t o64 = osoa + (fmt & SEG_SOA ? up256((size_t)SOA_N * rcap * sizeof(double)) : 0);
+    const size_t ogrp = o64 + (fmt & SEG_REC ? up256((size_t)REC64_N * rcap * sizeof(double)) : 0);
+    const size_t o32 = ogrp + (fmt & SEG_REC ? up256((size_t)GRPH_N * gcap * sizeof(double)) : 0);
+    const size_t onear = o32 + (fmt & SEG_F32 ? up256((size_t)REC32_N * rcap * sizeof(float)) : 0);
+    const size_t ocnt = onear + (fmt & SEG_F32 ? up256((size_t)NEAR32_N * rcap * sizeof(float)) : 0);
     const size_t octr = ocnt + 256;
     const size_t otgt = octr + 256;
     const size_t oout = otgt + up256((size_t)3 * m * sizeof(double));
     const size_t opart = oout + up256((size_t)3 * m * sizeof(double));
+    const size_t accepted = up256((size_t)9 * cap * sizeof(double)) +
+                            up256((size_t)12 * cap * sizeof(float)) + 512 +
+                            2 * up256((size_t)3 * m * sizeof(double)) +
+                            (size_t)3 * m * sizeof(double);
     if (nfil > ((int64_t)1 << 32) || m > ((int64_t)1 << 32) ||
-        opart + (size_t)3 * m * sizeof(double) > NOALLOC_SCRATCH_BYTES)
+        accepted > NOALLOC_ACCEPTED_BYTES)
         return fail(ctx, VLM_ERR_ARG,
                     "vlm_filament_vind_noalloc: " + std::to_string(nfil) + " filaments and " +
                         std::to_string(m) + " points exceed the " +
-                        std::to_string(NOALLOC_SCRATCH_BYTES >> 20) +
+                        std::to_string(NOALLOC_ACCEPTED_BYTES >> 20) +
                         " MiB workspace (about 120 B per filament and 72 B per point, plus "
                         "24 B per point for each chunk of partial sums)");
     VLM_DEVICE(ctx);
     unsigned char *w = nullptr;
     VLM_TRY(scratch_address(ctx, &w));
-    double *d64 = reinterpret_cast<double *>(w + o64);
-    float *d32 = reinterpret_cast<float *>(w + o32);
-    long long *count = reinterpret_cast<long long *>(w + ocnt);
-    int *counter = reinterpret_cast<int *>(w + octr);
+    SegPtrs seg;
+    if (fmt & SEG_SOA) seg.soa = reinterpret_cast<double *>(w + osoa);
+    if (fmt & SEG_REC) seg.rec64 = reinterpret_cast<double *>(w + o64);
+    if (fmt & SEG_REC) seg.grp = reinterpret_cast<double *>(w + ogrp);
+    if (fmt & SEG_F32) seg.rec32 = reinterpret_cast<float *>(w + o32);
+    if (fmt & SEG_F32) seg.near32 = reinterpret_cast<float *>(w + onear);
+    seg.count = reinterpret_cast<long long *>(w + ocnt);
+    seg.cap = rcap;
     double *tgt = reinterpret_cast<double *>(w + otgt);
     double *out = reinterpret_cast<double *>(w + oout);
     BsWork ws;
     ws.part = reinterpret_cast<double *>(w + opart);
     ws.part_cap = (NOALLOC_SCRATCH_BYTES - opart) / sizeof(double);
-    ws.counter = counter;
-    if (nfil > 0)
-        hipLaunchKernelGGL(fil_records_kernel, dim3(nblk(nfil)), dim3(256), 0, ctx->stream, nfil,
-                           a, b, gam, rc, d64, d32, cap);
-    hipLaunchKernelGGL(set_count_kernel, dim3(1), dim3(1), 0, ctx->stream, count, nfil);
-    hipLaunchKernelGGL(aos_to_soa3_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, p, tgt);
+    ws.counter = reinterpret_cast<int *>(w + octr);
+    if (nfil > 0) VLM_TRY(explicit_records(ctx, nfil, a, b, gam, rc, seg));
+    hipLaunchKernelGGL(aos_to_soa3_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, p, tgt,
+                       ws.counter);
     if (accumulate)
         hipLaunchKernelGGL(aos_to_soa3_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, v,
-                           out);
+                           out, ws.counter);
     VLM_HIP(hipGetLastError());
-    VLM_TRY(bs_eval(ctx, d64, d32, cap, count, nfil, tgt, m, m, out, accumulate, &ws));
+    VLM_TRY(bs_eval(ctx, seg, nfil, tgt, m, m, out, accumulate, &ws));
     hipLaunchKernelGGL(soa3_to_aos_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, out, v);
     VLM_HIP(hipGetLastError());
     return VLM_OK;

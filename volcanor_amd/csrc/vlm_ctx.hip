@@ -1,7 +1,5 @@
 // Context, error handling, segment compaction, explicit filament sets and
 // kernel timing for libvlm.
-#include <hipcub/hipcub.hpp>
-
 #include <cstring>
 
 #include "vlm_internal.h"
@@ -22,74 +20,19 @@ int hip_fail(vlm_ctx *ctx, hipError_t e, const char *what)
 
 namespace {
 
-// One record per staged slot -> SoA FP64 and FP32 copies at the compacted
-// position.  The last thread publishes the count.
-__global__ void compact_kernel(const Slot *slots, const int *flags, const int *idx,
-                               int64_t n, double *d64, float *d32, int64_t cap,
-                               long long *count)
+unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
+
+// Records of an explicit list (every filament kept, at its own index), one
+// lane per segment of the padded list, and its count.
+__global__ __launch_bounds__(256) void explicit_records_kernel(int64_t n, const double *a,
+                                                               const double *b, const double *g,
+                                                               const double *rc, SegPtrs L)
 {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    if (i == n - 1) *count = (long long)idx[i] + (long long)flags[i];
-    if (!flags[i]) return;
-    write_segment_record(slots[i], idx[i], d64, d32, cap);
-}
-
-__global__ void zero_count_kernel(long long *count) { *count = 0; }
-
-}  // namespace
-
-int ensure_slots(vlm_ctx *ctx, int64_t n)
-{
-    VLM_HIP(ctx->slots.reserve((size_t)n));
-    VLM_HIP(ctx->flags.reserve((size_t)n));
-    VLM_HIP(ctx->idx.reserve((size_t)n));
-    return VLM_OK;
-}
-
-int compact_into(vlm_ctx *ctx, const Slot *slots, const int *flags, int64_t nslots,
-                 DBuf<double> &d64, DBuf<float> &d32, DBuf<long long> &count, int64_t cap)
-{
-    VLM_HIP(count.reserve(1));
-    if (nslots <= 0) {
-        hipLaunchKernelGGL(zero_count_kernel, dim3(1), dim3(1), 0, ctx->stream, count.p);
-        VLM_HIP(hipGetLastError());
-        return VLM_OK;
-    }
-    if (nslots > 0x7fffffff) return fail(ctx, VLM_ERR_ARG, "segment list too large");
-    size_t bytes = 0;
-    VLM_HIP(hipcub::DeviceScan::ExclusiveSum(nullptr, bytes, flags, ctx->idx.p, (int)nslots,
-                                             ctx->stream));
-    if (bytes > ctx->scan_tmp.n) VLM_HIP(ctx->scan_tmp.reserve(bytes));
-    bytes = ctx->scan_tmp.n;
-    VLM_HIP(hipcub::DeviceScan::ExclusiveSum(ctx->scan_tmp.p, bytes, flags, ctx->idx.p,
-                                             (int)nslots, ctx->stream));
-    hipLaunchKernelGGL(compact_kernel, dim3((unsigned)((nslots + 255) / 256)), dim3(256), 0,
-                       ctx->stream, slots, flags, ctx->idx.p, nslots, d64.p, d32.p, cap,
-                       count.p);
-    VLM_HIP(hipGetLastError());
-    return VLM_OK;
-}
-
-int compact_slots(vlm_ctx *ctx, int64_t nslots)
-{
-    const int64_t cap = nslots > 0 ? nslots : 1;
-    if (ctx->seg.cap < cap) {
-        VLM_HIP(ctx->seg.d64.reserve((size_t)SEG64_N * cap));
-        VLM_HIP(ctx->seg.d32.reserve((size_t)SEG32_N * cap));
-        ctx->seg.cap = cap;
-    }
-    return compact_into(ctx, ctx->slots.p, ctx->flags.p, nslots, ctx->seg.d64, ctx->seg.d32,
-                        ctx->seg.count, ctx->seg.cap);
-}
-
-namespace {
-
-__global__ void stage_fil_kernel(int64_t n, const double *a, const double *b, const double *g,
-                                 const double *rc, Slot *slots, int *flags)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
+    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (k == 0) *L.count = (long long)n;
+    if ((k & ~(int64_t)(GRP - 1)) >= n) return;   // whole groups leave together
+    const bool valid = k < n;
+    const int64_t i = valid ? k : n - 1;
     Slot s;
     s.ax = a[3 * i];
     s.ay = a[3 * i + 1];
@@ -99,9 +42,21 @@ __global__ void stage_fil_kernel(int64_t n, const double *a, const double *b, co
     s.bz = b[3 * i + 2];
     s.gam = g[i];
     s.rc = rc[i];
-    slots[i] = s;
-    flags[i] = 1;  // explicit lists keep every filament (no |gam| skip)
+    write_group_records(s, valid, k, L);
 }
+
+}  // namespace
+
+int explicit_records(vlm_ctx *ctx, int64_t n, const double *a, const double *b, const double *g,
+                     const double *rc, const SegPtrs &L)
+{
+    hipLaunchKernelGGL(explicit_records_kernel, dim3(n > 0 ? nblk(n) : 1), dim3(256), 0,
+                       ctx->stream, n, a, b, g, rc, L);
+    VLM_HIP(hipGetLastError());
+    return VLM_OK;
+}
+
+namespace {
 
 // AoS host layout (3 x m) -> SoA device layout
 __global__ void aos_to_soa_kernel(int64_t m, const double *aos, double *soa, int64_t stride)
@@ -122,11 +77,8 @@ __global__ void soa_to_aos_kernel(int64_t m, const double *soa, int64_t stride, 
     aos[3 * i + 2] = soa[2 * stride + i];
 }
 
-unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
-
 int upload_fset(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b,
-                const double *gam, const double *rc, DBuf<double> &d64, DBuf<float> &d32,
-                DBuf<long long> &count)
+                const double *gam, const double *rc, int formats, SegList &seg, SegPtrs *view)
 {
     DBuf<double> raw;
     VLM_HIP(raw.reserve((size_t)8 * nfil));
@@ -138,14 +90,9 @@ int upload_fset(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b,
                            ctx->stream));
     VLM_HIP(hipMemcpyAsync(raw.p + 7 * nfil, rc, sizeof(double) * nfil, hipMemcpyHostToDevice,
                            ctx->stream));
-    VLM_TRY(ensure_slots(ctx, nfil));
-    hipLaunchKernelGGL(stage_fil_kernel, dim3(nblk(nfil)), dim3(256), 0, ctx->stream, nfil,
-                       raw.p, raw.p + 3 * nfil, raw.p + 6 * nfil, raw.p + 7 * nfil,
-                       ctx->slots.p, ctx->flags.p);
-    VLM_HIP(hipGetLastError());
-    VLM_HIP(d64.reserve((size_t)SEG64_N * nfil));
-    VLM_HIP(d32.reserve((size_t)SEG32_N * nfil));
-    VLM_TRY(compact_into(ctx, ctx->slots.p, ctx->flags.p, nfil, d64, d32, count, nfil));
+    VLM_HIP(seg.reserve(nfil, formats, view));
+    VLM_TRY(explicit_records(ctx, nfil, raw.p, raw.p + 3 * nfil, raw.p + 6 * nfil,
+                             raw.p + 7 * nfil, *view));
     VLM_TRY(sync_stream(ctx));  // raw is released on return
     return VLM_OK;
 }
@@ -356,19 +303,13 @@ int vlm_filament_vind(vlm_ctx *ctx, int64_t nfil, const double *a, const double 
         return fail(ctx, VLM_ERR_ARG, "null buffer");
     VLM_HIP(hipSetDevice(ctx->device));
     FSet fs;
-    if (nfil > 0) VLM_TRY(upload_fset(ctx, nfil, a, b, gam, rc, fs.d64, fs.d32, fs.count));
-    else {
-        VLM_HIP(fs.d64.reserve(SEG64_N));
-        VLM_HIP(fs.d32.reserve(SEG32_N));
-        VLM_TRY(compact_into(ctx, nullptr, nullptr, 0, fs.d64, fs.d32, fs.count, 1));
-    }
+    if (nfil > 0)
+        VLM_TRY(upload_fset(ctx, nfil, a, b, gam, rc, bs_formats(ctx, m), fs.seg, &fs.view));
     VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
     VLM_HIP(ctx->out.reserve((size_t)3 * m));
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
-    const int64_t stride = nfil > 0 ? nfil : 1;
-    VLM_TRY(bs_eval(ctx, fs.d64.p, fs.d32.p, stride, fs.count.p, nfil, ctx->tgt.p, m, m,
-                    ctx->out.p, accumulate));
+    VLM_TRY(bs_eval(ctx, fs.view, nfil, ctx->tgt.p, m, m, ctx->out.p, accumulate));
     VLM_TRY(points_to_host(ctx, m, ctx->out.p, m, v));
     return VLM_OK;
 }
@@ -380,7 +321,7 @@ int vlm_fset_create(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b
     if (nfil <= 0 || !a || !b || !gam || !rc) return fail(ctx, VLM_ERR_ARG, "empty filament set");
     VLM_HIP(hipSetDevice(ctx->device));
     FSet *fs = new FSet();
-    int rc_ = upload_fset(ctx, nfil, a, b, gam, rc, fs->d64, fs->d32, fs->count);
+    int rc_ = upload_fset(ctx, nfil, a, b, gam, rc, SEG_ALL, fs->seg, &fs->view);
     if (rc_ != VLM_OK) {
         delete fs;
         return rc_;
@@ -421,8 +362,7 @@ int vlm_fset_vind(vlm_ctx *ctx, int fset, int pset)
     VLM_HIP(hipSetDevice(ctx->device));
     FSet *fs = ctx->fsets[fset];
     PSet *ps = ctx->psets[pset];
-    return bs_eval(ctx, fs->d64.p, fs->d32.p, fs->n, fs->count.p, fs->n, ps->p.p, ps->m, ps->m,
-                   ps->v.p, 0);
+    return bs_eval(ctx, fs->view, fs->n, ps->p.p, ps->m, ps->m, ps->v.p, 0);
 }
 
 int vlm_pset_velocity(vlm_ctx *ctx, int pset, double *v)

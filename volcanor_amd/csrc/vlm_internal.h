@@ -41,20 +41,59 @@ struct DBuf {
     }
 };
 
-// Compacted straight-segment list: structure of arrays (stride cap).
-//   d64 (9):  ax ay az g | r0x r0y r0z q^2 | n0   g = gam/(4 pi), r0 = b - a,
-//                                                 q = rc^2 |r0|^2, n0 = |r0|^2
-//   d32 (12): ahx ahy ahz g | alx aly alz q | r0x r0y r0z 4|r0|^2
-//             (a = a_hi + a_lo split into two floats)
+// Compacted straight-segment list, in groups of GRP consecutive segments.
+// Every segment has one record that a wave reads through the scalar cache
+// (16 values = two or one s_load_dwordx16), so the records are arrays of
+// structures:
+//   rec64 (16 doubles): a(3) g | r0(3) n0 | g r0(3) qq | g r0 x (a - c)(3) -
+//   rec32 (16 floats):  a - c(3) n0 | r0(3) qq | g r0(3) g | g r0 x (a - c)(3) q
+//   near32 (8 floats):  a_hi(3) q' | a_lo(3) -   (a = a_hi + a_lo; q' = q, or
+//                       infinity for q <= 1e-18)
+//   grp (4 doubles per group): centre c, squared far radius
+// Launches with few targets put segments on lanes instead and read one
+// structure of arrays (stride cap):
+//   soa (9): ax ay az g | r0x r0y r0z qq | n0
+// with g = gam / (4 pi), r0 = b - a, n0 = |r0|^2, q = rc^2 n0, qq = q^2 and
+// c the centre of the group's bounding box.  The last group is padded with
+// records of zero circulation and length (qq = 1, so that they give 0).
 // count: device int64 with the number of valid segments.
-constexpr int SEG64_N = 9;   // doubles per FP64 segment record
-constexpr int SEG32_N = 12;  // floats per FP32 segment record
+constexpr int GRP = 32;
+constexpr int SOA_N = 9, REC64_N = 16, REC32_N = 16, NEAR32_N = 8, GRPH_N = 4;
+
+// What a list holds; a launch with m targets needs bs_formats(m).
+enum { SEG_SOA = 1, SEG_REC = 2, SEG_F32 = 4, SEG_ALL = 7 };
+
+// Device pointers of a list (null where a format is absent).
+struct SegPtrs {
+    double *soa = nullptr, *rec64 = nullptr, *grp = nullptr;
+    float *rec32 = nullptr, *near32 = nullptr;
+    long long *count = nullptr;
+    int64_t cap = 0;  // segments, a multiple of GRP (stride of soa)
+};
 
 struct SegList {
-    DBuf<double> d64;
-    DBuf<float> d32;
+    DBuf<double> soa, rec64, grp;
+    DBuf<float> rec32, near32;
     DBuf<long long> count;
-    int64_t cap = 0;
+    // Room for n segments in the given formats.
+    hipError_t reserve(int64_t n, int formats, SegPtrs *out)
+    {
+        const size_t k = (size_t)((n + GRP - 1) / GRP) * GRP;
+        hipError_t e = count.reserve(1);
+        if (e == hipSuccess && (formats & SEG_SOA)) e = soa.reserve(k * SOA_N);
+        if (e == hipSuccess && (formats & SEG_REC)) e = rec64.reserve(k * REC64_N);
+        if (e == hipSuccess && (formats & SEG_REC)) e = grp.reserve(k / GRP * GRPH_N);
+        if (e == hipSuccess && (formats & SEG_F32)) e = rec32.reserve(k * REC32_N);
+        if (e == hipSuccess && (formats & SEG_F32)) e = near32.reserve(k * NEAR32_N);
+        out->soa = formats & SEG_SOA ? soa.p : nullptr;
+        out->rec64 = formats & SEG_REC ? rec64.p : nullptr;
+        out->grp = formats & SEG_REC ? grp.p : nullptr;
+        out->rec32 = formats & SEG_F32 ? rec32.p : nullptr;
+        out->near32 = formats & SEG_F32 ? near32.p : nullptr;
+        out->count = count.p;
+        out->cap = (int64_t)k;
+        return e;
+    }
 };
 
 // Staging slots written by the segment builders before compaction.
@@ -149,9 +188,8 @@ struct Predictor {
 };
 
 struct FSet {
-    DBuf<double> d64;
-    DBuf<float> d32;
-    DBuf<long long> count;
+    SegList seg;
+    SegPtrs view;
     int64_t n = 0;
 };
 
@@ -174,14 +212,12 @@ struct vlm_ctx {
     std::vector<vlm::PSet *> psets;
     // scratch
     vlm::SegList seg;
+    vlm::SegPtrs seg_view;       // the list built last
     vlm::DBuf<vlm::Slot> slots;
-    vlm::DBuf<int> flags, idx;
-    vlm::DBuf<unsigned char> scan_tmp;
-    size_t scan_tmp_bytes = 0;
+    vlm::DBuf<int> seg_counts;   // segments of each staging block
     vlm::DBuf<double> tgt, out, part;
-    vlm::DBuf<int> counter;  // run counts per workgroup of the Biot-Savart launches
-    vlm::DBuf<int4> skruns;  // run lists (tile, first batch, batch count) per workgroup
-    int occ[4] = {0, 0, 0, 0};  // resident workgroups per kernel variant
+    vlm::DBuf<int> counter;  // work counter of the Biot-Savart launches, 0 between them
+    int occ[2] = {0, 0};     // resident workgroups per kernel (FP64, mixed)
     vlm::DBuf<double> hostio;  // device staging for host point lists
     // pinned host arena for host<->device copies: truly asynchronous copies,
     // reset whenever the stream has been synchronised
@@ -240,71 +276,113 @@ constexpr double kPi = 3.141592653589793238462643383279502884;
 constexpr double kInv4Pi = 0.25 / kPi;
 constexpr double kEps = 2.220446049250313080847263336181640625e-16;  // epsilon(1._dp)
 
-// The FP64 and FP32 records of one segment at position k of a compacted
-// list of stride cap (layouts above).
-__device__ __forceinline__ void write_segment_record(const Slot &s, int64_t k, double *d64,
-                                                     float *d32, int64_t cap)
+// Writes the records of one group's GRP consecutive segments: lane l of a
+// 32-lane half wave (every lane active) holds segment k (the group's first
+// plus l); lanes with valid = false write the padding record (none in the
+// structure of arrays).  The far radius: a target further than |a - c| + 2 |r0|
+// from the centre, for every segment, has |r1| >= 2 |r0| for all of them.
+// It is infinite (never far) for a group that holds a segment with
+// q <= 1e-18 (the far pair has no zero-denominator guard) or is wider than
+// 64 of its longest segments (32 consecutive records can jump between wake
+// rows; a chain of 32 connected segments spans 34), whose centred
+// coordinates would lose accuracy against |r1|.
+__device__ __forceinline__ void write_group_records(const Slot &s, bool valid, int64_t k,
+                                                    const SegPtrs &L)
 {
-    const double g = s.gam * kInv4Pi;
     const double r0x = s.bx - s.ax, r0y = s.by - s.ay, r0z = s.bz - s.az;
+    const double g = s.gam * (0.25 / 3.141592653589793238462643383279502884);
     const double n0 = r0x * r0x + r0y * r0y + r0z * r0z;
     const double q = s.rc * s.rc * n0;
-    d64[k] = s.ax;
-    d64[cap + k] = s.ay;
-    d64[2 * cap + k] = s.az;
-    d64[3 * cap + k] = g;
-    d64[4 * cap + k] = r0x;
-    d64[5 * cap + k] = r0y;
-    d64[6 * cap + k] = r0z;
-    d64[7 * cap + k] = q * q;
-    d64[8 * cap + k] = n0;
-    const float hx = (float)s.ax, hy = (float)s.ay, hz = (float)s.az;
-    d32[k] = hx;
-    d32[cap + k] = hy;
-    d32[2 * cap + k] = hz;
-    d32[3 * cap + k] = (float)g;
-    d32[4 * cap + k] = (float)(s.ax - (double)hx);
-    d32[5 * cap + k] = (float)(s.ay - (double)hy);
-    d32[6 * cap + k] = (float)(s.az - (double)hz);
-    d32[7 * cap + k] = (float)q;
-    d32[8 * cap + k] = (float)r0x;
-    d32[9 * cap + k] = (float)r0y;
-    d32[10 * cap + k] = (float)r0z;
-    d32[11 * cap + k] = (float)(4.0 * n0);
+    if (L.soa && valid) {
+        const double v[SOA_N] = {s.ax, s.ay, s.az, g, r0x, r0y, r0z, q * q, n0};
+#pragma unroll
+        for (int i = 0; i < SOA_N; ++i) L.soa[i * L.cap + k] = v[i];
+    }
+    if (!L.rec64) return;
+    float lo[3], hi[3];
+    const float inf = __builtin_inff();
+    lo[0] = valid ? (float)fmin(s.ax, s.bx) : inf;
+    lo[1] = valid ? (float)fmin(s.ay, s.by) : inf;
+    lo[2] = valid ? (float)fmin(s.az, s.bz) : inf;
+    hi[0] = valid ? (float)fmax(s.ax, s.bx) : -inf;
+    hi[1] = valid ? (float)fmax(s.ay, s.by) : -inf;
+    hi[2] = valid ? (float)fmax(s.az, s.bz) : -inf;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            lo[d] = fminf(lo[d], __shfl_xor(lo[d], o, 32));
+            hi[d] = fmaxf(hi[d], __shfl_xor(hi[d], o, 32));
+        }
+    const double cx = 0.5 * ((double)lo[0] + hi[0]), cy = 0.5 * ((double)lo[1] + hi[1]),
+                 cz = 0.5 * ((double)lo[2] + hi[2]);
+    const double lx = s.ax - cx, ly = s.ay - cy, lz = s.az - cz;
+    const double l2 = 2.0 * sqrt(n0);
+    float ex = valid ? (float)((sqrt(lx * lx + ly * ly + lz * lz) + l2) * 1.000001) : 0.f;
+    float lmax = valid ? (float)l2 : 0.f;
+    if (valid && !(q > 1e-18)) ex = inf;
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) {
+        ex = fmaxf(ex, __shfl_xor(ex, o, 32));
+        lmax = fmaxf(lmax, __shfl_xor(lmax, o, 32));
+    }
+    if (!(ex <= 32.0f * lmax)) ex = inf;
+    double v[REC64_N] = {s.ax, s.ay, s.az, g, r0x, r0y, r0z, n0, g * r0x, g * r0y, g * r0z, q * q,
+                         g * (r0y * lz - r0z * ly), g * (r0z * lx - r0x * lz),
+                         g * (r0x * ly - r0y * lx), 0.0};
+    if (!valid)
+        for (int i = 0; i < REC64_N; ++i) v[i] = i == 11 ? 1.0 : 0.0;
+    double2 *o64 = reinterpret_cast<double2 *>(L.rec64 + (size_t)k * REC64_N);
+#pragma unroll
+    for (int i = 0; i < REC64_N / 2; ++i) o64[i] = make_double2(v[2 * i], v[2 * i + 1]);
+    if ((k & (GRP - 1)) == 0) {
+        double2 *h = reinterpret_cast<double2 *>(L.grp + (size_t)(k / GRP) * GRPH_N);
+        h[0] = make_double2(cx, cy);
+        h[1] = make_double2(cz, (double)ex * (double)ex);
+    }
+    if (!L.rec32) return;
+    const float hx = (float)s.ax, hy = (float)s.ay, hz = (float)s.az, qf = (float)q;
+    float4 *o32 = reinterpret_cast<float4 *>(L.rec32 + (size_t)k * REC32_N);
+    float4 *on = reinterpret_cast<float4 *>(L.near32 + (size_t)k * NEAR32_N);
+    if (valid) {
+        o32[0] = make_float4((float)lx, (float)ly, (float)lz, (float)n0);
+        o32[1] = make_float4((float)r0x, (float)r0y, (float)r0z, qf * qf);
+        o32[2] = make_float4((float)v[8], (float)v[9], (float)v[10], (float)g);
+        o32[3] = make_float4((float)v[12], (float)v[13], (float)v[14], qf);
+        on[0] = make_float4(hx, hy, hz, q > 1e-18 ? qf : inf);
+        on[1] = make_float4((float)(s.ax - (double)hx), (float)(s.ay - (double)hy),
+                            (float)(s.az - (double)hz), 0.f);
+    } else {
+        const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
+        o32[0] = o32[2] = on[0] = on[1] = z;
+        o32[1] = make_float4(0.f, 0.f, 0.f, 1.f);
+        o32[3] = make_float4(0.f, 0.f, 0.f, 1.f);
+    }
 }
 
-// Biot-Savart evaluation of a compacted segment list at n targets stored
+// Biot-Savart evaluation of a compacted segment list at m targets stored
 // as SoA (x at t[0..], y at t[tstride..], z at t[2*tstride..]).  Result
-// goes to out (SoA, same stride); accumulate adds into it.  nseg_max is an
-// upper bound of the device count used to size the launch.
+// goes to out (SoA, same stride); accumulate adds into it.  nseg_est is the
+// expected count (0: the list is empty): it sets the number of chunks, and
+// the kernel divides the device count evenly among them.
 // A fixed workspace for bs_eval instead of the context's growing buffers
 // (no allocation): room for part_cap doubles of chunk partial sums (at
-// least 3 m, the chunk count is capped by it) and one int counter.  Such
-// launches are not profiled.
+// least 3 m, the chunk count is capped by it) and one int counter, which is
+// 0 before the call.  Such launches are not profiled.
 struct BsWork {
     double *part;
     size_t part_cap;
     int *counter;
 };
-int bs_eval(vlm_ctx *ctx, const double *seg64, const float *seg32,
-            int64_t segstride, const long long *nseg_dev, int64_t nseg_max,
-            const double *t, int64_t m, int64_t tstride, double *out,
-            int accumulate, const BsWork *ws = nullptr);
+int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t, int64_t m,
+            int64_t tstride, double *out, int accumulate, const BsWork *ws = nullptr);
+// The list formats that a launch with m targets reads.
+int bs_formats(const vlm_ctx *ctx, int64_t m);
 
-// Compact staged slots (flags != 0) into ctx->seg.  nslots on host.
-int compact_slots(vlm_ctx *ctx, int64_t nslots);
-int compact_into(vlm_ctx *ctx, const Slot *slots, const int *flags,
-                 int64_t nslots, DBuf<double> &d64, DBuf<float> &d32,
-                 DBuf<long long> &count, int64_t cap);
-
-// Source-set builders write slots starting at slot offset off; each
-// returns the number of slots it used through *used.
-int stage_wing(vlm_ctx *ctx, Rotor &r, int set, int64_t off, int64_t *used);
-int stage_wake(vlm_ctx *ctx, Rotor &r, int pred, int64_t off, int64_t *used);
-int64_t wing_slots(const Rotor &r, int set);
-int64_t wake_slots(const Rotor &r);
-
-int ensure_slots(vlm_ctx *ctx, int64_t n);
+// Records of an explicit list (every filament kept, at its own index) from
+// 3 x n device arrays, and its count.
+int explicit_records(vlm_ctx *ctx, int64_t n, const double *a, const double *b, const double *g,
+                     const double *rc, const SegPtrs &L);
 
 // Rotor ir of the context (nullptr when out of range).
 Rotor *rotor_of(vlm_ctx *ctx, int ir);

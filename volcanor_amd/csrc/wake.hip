@@ -19,6 +19,7 @@
 // circulation when their core radii are equal (the common case), otherwise
 // both are kept.  Rings with |gam| <= eps are skipped as in
 // blade_vind_bywake (classdef.f90:1450-1456).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
@@ -99,10 +100,28 @@ __device__ __forceinline__ size_t vidx(const RV &v, int b, int i, int j)
     return ((size_t)b * v.nN + i) * (v.ns + 1) + j;
 }
 
-__device__ __forceinline__ void put(Slot *s, int *f, const double *A, const double *B, double g,
-                                    double rc)
+// Entry k of a lattice of rows x cols walked in patches of PATCH rows: each
+// patch column by column, every second patch backwards, so that any run of
+// entries is compact in space whatever the number of columns.  Sources and
+// targets take this order because the Biot-Savart kernel runs its shorter
+// pair on a (wave of 64 targets, group of 32 segments) whose distance
+// exceeds the group's radius: with whole spanwise rows (patch of one row)
+// 54% of them are far on a 3 x 30 rotor after 360 steps of 5 degrees, with
+// 4 rows 96% (8 rows 94%, 2 rows 93%).
+constexpr int PATCH = 4;
+
+__device__ __forceinline__ void patch_entry(int64_t k, int rows, int cols, int *i, int *j)
 {
-    Slot q;
+    const int b = (int)(k / (PATCH * cols));
+    const int w = (int)(k - (int64_t)b * (PATCH * cols));
+    const int h = min(PATCH, rows - PATCH * b);
+    const int c = w / h;
+    *i = PATCH * b + (w - c * h);
+    *j = (b & 1) ? cols - 1 - c : c;
+}
+
+__device__ __forceinline__ bool put(Slot &q, const double *A, const double *B, double g, double rc)
+{
     q.ax = A[0];
     q.ay = A[1];
     q.az = A[2];
@@ -111,136 +130,229 @@ __device__ __forceinline__ void put(Slot *s, int *f, const double *A, const doub
     q.bz = B[2];
     q.gam = g;
     q.rc = rc;
-    *s = q;
-    *f = g != 0.0 ? 1 : 0;
+    return g != 0.0;
 }
 
 __device__ __forceinline__ double skipg(double g) { return fabs(g) > EPS ? g : 0.0; }
 
-// Wing rings (ring form).  set 0: four filaments per ring; set 1: bound
-// vortices vf2 + vf4, without vf2 of the trailing row
-// (blade_vind_bywing_boundVortices, classdef.f90:1376-1395).
-__global__ void stage_wing_kernel(RV v, int set, Slot *slots, int *flags)
-{
-    const int nring = v.nb * v.nc * v.ns;
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= nring) return;
-    const double *c = v.wc + 12 * (size_t)k;
-    const double *rc = v.wrc + 4 * (size_t)k;
-    const double g = v.wg[k];
-    if (set == 0) {
-        for (int f = 0; f < 4; ++f)
-            put(slots + 4 * (size_t)k + f, flags + 4 * (size_t)k + f, c + 3 * f,
-                c + 3 * ((f + 1) & 3), g, rc[f]);
-    } else {
-        const int ic = k % v.nc;
-        put(slots + 2 * (size_t)k, flags + 2 * (size_t)k, c + 3 * 3, c, g, rc[3]);
-        put(slots + 2 * (size_t)k + 1, flags + 2 * (size_t)k + 1, c + 3, c + 6,
-            ic < v.nc - 1 ? g : 0.0, rc[1]);
-    }
-}
+// One source set of a rotor, as the staging kernel sees it: items of at
+// most two segments.
+//   SRC_WING   ring form, items 2k and 2k+1 hold filaments 0-1 and 2-3 of ring k
+//   SRC_BOUND  bound vortices vf4 and vf2 of ring k, without vf2 of the
+//              trailing row (blade_vind_bywing_boundVortices,
+//              classdef.f90:1376-1395)
+//   SRC_WAKE   lattice edges (below); SRC_PRESC prescribed far-wake
+//              filaments (classdef.f90:1471-1476, 1501-1507)
+enum { SRC_WING, SRC_BOUND, SRC_WAKE, SRC_PRESC };
+
+struct SrcDesc {
+    // wing: wc wrc wg; wake: node le gam rc4 ffc fgam frc; prescribed: pf ps
+    const double *p[7];
+    int kind, nc, ns, nN, nF, head, rn, rf, far_exists;
+    int64_t first, per_blade;  // first item in the launch; items per blade (wake)
+};
+
+constexpr int SRC_MAX = 20;            // descriptors per launch (kernel argument space)
+constexpr int STAGE_BLOCKS = 4096;     // staging blocks of one list
+
+struct StageArgs {
+    SrcDesc d[SRC_MAX];
+    int n, iters, block0;
+    int64_t total;
+    Slot *slots;
+    int *counts;
+};
 
 // Near- and far-wake unique segments of every blade.  Edge enumeration per
-// blade (R active rows, F active far filaments):
+// blade (R active rows, F active far filaments; rows and columns in patch
+// order):
 //   [0, R*ns)            trailing spanwise edge of row i: T(i,j) -> T(i,j+1)
 //   [.., + ns)           leading edge of the newest row:  LE(j+1) -> LE(j)
 //   [.., + R*(ns+1))     streamwise edge: U(i,j) -> T(i,j)
 //   [.., + F)            far filament fc1 -> fc2
-// Two slots per edge.
-__global__ void stage_wake_kernel(RV v, int pred, int far_exists, int64_t per_blade,
-                                  Slot *slots, int *flags)
+__device__ __forceinline__ void wake_edge(const SrcDesc &d, int64_t e, Slot (&s)[2], bool (&f)[2])
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= per_blade * v.nb) return;
-    const int b = (int)(e / per_blade);
-    int64_t k = e - (int64_t)b * per_blade;
-    Slot *s = slots + 2 * e;
-    int *f = flags + 2 * e;
-    f[0] = 0;
-    f[1] = 0;
-    const double *N = pred ? v.pnode : v.node;
-    const double *L = (pred ? v.ple : v.le) + 3 * (size_t)b * (v.ns + 1);
-    const double *FC = pred ? v.pffc : v.ffc;
-    const int R = v.nN - v.rn;
-    const int ns = v.ns;
+    const int b = (int)(e / d.per_blade);
+    int64_t k = e - (int64_t)b * d.per_blade;
+    const int ns = d.ns, nN = d.nN;
+    const double *N = d.p[0] + 3 * (size_t)b * nN * (ns + 1);
+    const double *L = d.p[1] + 3 * (size_t)b * (ns + 1);
+    const double *gam = d.p[2] + (size_t)b * nN * ns, *rc4 = d.p[3] + 4 * (size_t)b * nN * ns;
+    const int R = nN - d.rn;
+    auto phys = [&](int i) {
+        const int p = d.head + i;
+        return p >= nN ? p - nN : p;
+    };
     if (k < (int64_t)R * ns) {
-        const int i = v.rn + (int)(k / ns), j = (int)(k % ns);
-        const int p = phys(v, i);
-        const double *A = N + 3 * nidx(v, b, p, j);
-        const double *B = N + 3 * nidx(v, b, p, j + 1);
-        const double ga = skipg(v.gam[ridx(v, b, p, j)]);
-        const double rca = v.rc4[4 * ridx(v, b, p, j) + 1];
+        int i, j;
+        patch_entry(k, R, ns, &i, &j);
+        i += d.rn;
+        const int p = phys(i);
+        const double *A = N + 3 * (p * (ns + 1) + j);
+        const double ga = skipg(gam[p * ns + j]);
+        const double rca = rc4[4 * (p * ns + j) + 1];
         double gb = 0.0, rcb = rca;
         bool hasb = false;
-        if (i + 1 < v.nN) {
-            const int q = phys(v, i + 1);
-            gb = -skipg(v.gam[ridx(v, b, q, j)]);
-            rcb = v.rc4[4 * ridx(v, b, q, j) + 3];
+        if (i + 1 < nN) {
+            const int q = phys(i + 1);
+            gb = -skipg(gam[q * ns + j]);
+            rcb = rc4[4 * (q * ns + j) + 3];
             hasb = true;
-        } else if (far_exists) {
+        } else if (d.far_exists) {
             // open horseshoe (classdef.f90:1458-1463): not |gam|-guarded
-            gb = -v.gam[ridx(v, b, p, j)];
-            rcb = rca;
+            gb = -gam[p * ns + j];
             hasb = true;
         }
         if (!hasb || rca == rcb) {
-            put(s, f, A, B, ga + gb, rca);
+            f[0] = put(s[0], A, A + 3, ga + gb, rca);
         } else {
-            put(s, f, A, B, ga, rca);
-            put(s + 1, f + 1, A, B, gb, rcb);
+            f[0] = put(s[0], A, A + 3, ga, rca);
+            f[1] = put(s[1], A, A + 3, gb, rcb);
         }
         return;
     }
     k -= (int64_t)R * ns;
     if (k < ns) {
-        const int j = (int)k;
-        const int p = phys(v, v.rn);
-        put(s, f, L + 3 * (j + 1), L + 3 * j, skipg(v.gam[ridx(v, b, p, j)]),
-            v.rc4[4 * ridx(v, b, p, j) + 3]);
+        const int j = (int)k, r = phys(d.rn) * ns + j;
+        f[0] = put(s[0], L + 3 * (j + 1), L + 3 * j, skipg(gam[r]), rc4[4 * r + 3]);
         return;
     }
     k -= ns;
     if (k < (int64_t)R * (ns + 1)) {
-        const int i = v.rn + (int)(k / (ns + 1)), j = (int)(k % (ns + 1));
-        const int p = phys(v, i);
-        const double *T = N + 3 * nidx(v, b, p, j);
-        const double *U = (i == v.rn) ? L + 3 * j : N + 3 * nidx(v, b, phys(v, i - 1), j);
+        int i, j;
+        patch_entry(k, R, ns + 1, &i, &j);
+        i += d.rn;
+        const int p = phys(i);
+        const double *T = N + 3 * (p * (ns + 1) + j);
+        const double *U = (i == d.rn) ? L + 3 * j : N + 3 * (phys(i - 1) * (ns + 1) + j);
         double ga = 0.0, rca = 0.0, gb = 0.0, rcb = 0.0;
-        bool hasa = j < ns, hasb = j >= 1;
+        const bool hasa = j < ns, hasb = j >= 1;
         if (hasa) {
-            ga = skipg(v.gam[ridx(v, b, p, j)]);
-            rca = v.rc4[4 * ridx(v, b, p, j) + 0];
+            ga = skipg(gam[p * ns + j]);
+            rca = rc4[4 * (p * ns + j) + 0];
         }
         if (hasb) {
-            gb = -skipg(v.gam[ridx(v, b, p, j - 1)]);
-            rcb = v.rc4[4 * ridx(v, b, p, j - 1) + 2];
+            gb = -skipg(gam[p * ns + j - 1]);
+            rcb = rc4[4 * (p * ns + j - 1) + 2];
         }
         if (hasa && hasb && rca == rcb) {
-            put(s, f, U, T, ga + gb, rca);
+            f[0] = put(s[0], U, T, ga + gb, rca);
         } else {
-            if (hasa) put(s, f, U, T, ga, rca);
-            if (hasb) put(s + 1, f + 1, U, T, gb, rcb);
+            if (hasa) f[0] = put(s[0], U, T, ga, rca);
+            if (hasb) f[1] = put(s[1], U, T, gb, rcb);
         }
         return;
     }
     k -= (int64_t)R * (ns + 1);
-    {
-        const int i = v.rf + (int)k;
-        const size_t q = (size_t)b * v.nF + i;
-        put(s, f, FC + 6 * q, FC + 6 * q + 3, skipg(v.fgam[q]), v.frc[q]);
-    }
+    const size_t q = (size_t)b * d.nF + d.rf + k;
+    f[0] = put(s[0], d.p[4] + 6 * q, d.p[4] + 6 * q + 3, skipg(d.p[5][q]), d.p[6][q]);
 }
 
-// Prescribed far-wake filaments as sources (classdef.f90:1471-1476,
-// 1501-1507), one slot each, while a far wake exists.
-__global__ void stage_presc_kernel(const double *pf, const double *ps, int nb, Slot *slots,
-                                   int *flags)
+// Segments of the items of up to SRC_MAX source sets, compacted within each
+// block (item order) into the block's own slots, and their count.  Bound by
+// latency (a few dependent loads per item); with emit_records_kernel the
+// list of a pass takes two launches, where one launch per set, a device
+// scan and a scatter took 2 nr + 3.
+__global__ __launch_bounds__(256) void stage_kernel(StageArgs a)
 {
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= nb * PF_N) return;
-    const int b = e / PF_N;
-    put(slots + e, flags + e, pf + 6 * (size_t)e, pf + 6 * (size_t)e + 3, skipg(ps[4 * b]),
-        ps[4 * b + 1]);
+    __shared__ int wsum[4];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int blk = a.block0 + blockIdx.x;
+    Slot *dst = a.slots + (size_t)blk * a.iters * 512;
+    int run = 0;
+    for (int it = 0; it < a.iters; ++it) {
+        const int64_t e = ((int64_t)blockIdx.x * a.iters + it) * 256 + tid;
+        Slot s[2];
+        bool f[2] = {false, false};
+        if (e < a.total) {
+            int q = 0;
+            while (q + 1 < a.n && e >= a.d[q + 1].first) ++q;
+            const SrcDesc &d = a.d[q];
+            const int64_t k = e - d.first;
+            if (d.kind == SRC_WAKE) {
+                wake_edge(d, k, s, f);
+            } else if (d.kind == SRC_PRESC) {
+                const int b = (int)(k / PF_N);
+                f[0] = put(s[0], d.p[0] + 6 * k, d.p[0] + 6 * k + 3, skipg(d.p[1][4 * b]),
+                           d.p[1][4 * b + 1]);
+            } else {
+                const int64_t r = d.kind == SRC_WING ? k >> 1 : k;
+                const double *c = d.p[0] + 12 * r, *rc = d.p[1] + 4 * r;
+                const double g = d.p[2][r];
+                if (d.kind == SRC_WING) {
+                    const int h = 2 * (int)(k & 1);
+                    f[0] = put(s[0], c + 3 * h, c + 3 * h + 3, g, rc[h]);
+                    f[1] = put(s[1], c + 3 * h + 3, c + 3 * ((h + 2) & 3), g, rc[h + 1]);
+                } else {
+                    f[0] = put(s[0], c + 9, c, g, rc[3]);
+                    f[1] = put(s[1], c + 3, c + 6, (int)(r % d.nc) < d.nc - 1 ? g : 0.0, rc[1]);
+                }
+            }
+        }
+        const unsigned long long b0 = __ballot(f[0]), b1 = __ballot(f[1]);
+        const unsigned long long lt = (1ull << lane) - 1;
+        if (lane == 0) wsum[w] = __popcll(b0) + __popcll(b1);
+        __syncthreads();
+        int pos = run + __popcll(b0 & lt) + __popcll(b1 & lt);
+        for (int q = 0; q < 4; ++q) {
+            if (q < w) pos += wsum[q];
+            run += wsum[q];
+        }
+        __syncthreads();
+        if (f[0]) dst[pos++] = s[0];
+        if (f[1]) dst[pos] = s[1];
+    }
+    if (tid == 0) a.counts[blk] = run;
+}
+
+// The staged segments in order, as records: each block forms the prefix sum
+// of the staging blocks' counts, and each lane finds the block its record
+// comes from by bisection.
+__global__ __launch_bounds__(256) void emit_records_kernel(const Slot *slots, const int *counts,
+                                                           int nblocks, int stride, SegPtrs L)
+{
+    __shared__ int pre[STAGE_BLOCKS + 1];
+    __shared__ int wsum[4];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int per = (nblocks + 255) / 256;
+    int mine = 0;
+    for (int q = 0; q < per; ++q) {
+        const int b = tid * per + q;
+        if (b < nblocks) mine += counts[b];
+    }
+    int incl = mine;
+    for (int o = 1; o < 64; o <<= 1) {
+        const int v = __shfl_up(incl, o);
+        if (lane >= o) incl += v;
+    }
+    if (lane == 63) wsum[w] = incl;
+    __syncthreads();
+    int excl = incl - mine, total = 0;
+    for (int q = 0; q < 4; ++q) {
+        if (q < w) excl += wsum[q];
+        total += wsum[q];
+    }
+    for (int q = 0; q < per; ++q) {
+        const int b = tid * per + q;
+        if (b < nblocks) {
+            pre[b] = excl;
+            excl += counts[b];
+        }
+    }
+    if (blockIdx.x == 0 && tid == 0) *L.count = total;
+    __syncthreads();
+    const int k = blockIdx.x * 256 + tid;
+    if ((k & ~(GRP - 1)) >= total) return;   // whole groups leave together
+    const bool valid = k < total;
+    const int kk = valid ? k : total - 1;
+    int lo = 0, hi = nblocks;   // last block with pre[lo] <= kk
+    while (hi - lo > 1) {
+        const int mid = (lo + hi) >> 1;
+        if (pre[mid] <= kk) lo = mid;
+        else hi = mid;
+    }
+    const Slot s = slots[(size_t)lo * stride + (kk - pre[lo])];
+    write_group_records(s, valid, k, L);
 }
 
 // pFwake_update (classdef.f90:998-1066) for blade blockIdx.x of wake type
@@ -317,7 +429,9 @@ __global__ void gather_targets_kernel(RV v, int pred, double *t, int64_t stride,
     const int64_t k = e - b * per;
     const double *P;
     if (k < (int64_t)R * (v.ns + 1)) {
-        const int i = v.rn + (int)(k / (v.ns + 1)), j = (int)(k % (v.ns + 1));
+        int i, j;
+        patch_entry(k, R, v.ns + 1, &i, &j);
+        i += v.rn;
         P = (pred ? v.pnode : v.node) + 3 * nidx(v, b, phys(v, i), j);
     } else {
         const int i = v.rf + (int)(k - (int64_t)R * (v.ns + 1));
@@ -338,7 +452,9 @@ __global__ void scatter_vel_kernel(RV v, int which, const double *o, int64_t str
     const int64_t k = e - b * per;
     double *dst;
     if (k < (int64_t)R * (v.ns + 1)) {
-        const int i = v.rn + (int)(k / (v.ns + 1)), j = (int)(k % (v.ns + 1));
+        int i, j;
+        patch_entry(k, R, v.ns + 1, &i, &j);
+        i += v.rn;
         dst = v.vel[which] + 3 * vidx(v, b, i, j);
     } else {
         const int i = v.rf + (int)(k - (int64_t)R * (v.ns + 1));
@@ -967,11 +1083,6 @@ __global__ void mirror_gamma_kernel(const double *src, double *dst, int n)
 // ---------------------------------------------------------------------
 // host-side helpers
 // ---------------------------------------------------------------------
-int64_t wing_slots(const Rotor &r, int set)
-{
-    return (int64_t)r.nring * (set == VLM_SET_WING ? 4 : 2);
-}
-
 static int64_t wake_edges_per_blade(const Rotor &r)
 {
     const int64_t R = r.d.nNwake - (r.rowNear - 1);
@@ -984,43 +1095,6 @@ static int64_t wake_edges_per_blade(const Rotor &r)
 static int64_t presc_slots(const Rotor &r)
 {
     return (r.presc_nt > 0 && r.rowFar <= r.d.nFwake) ? (int64_t)PF_N * r.d.nb : 0;
-}
-
-int64_t wake_slots(const Rotor &r) { return 2 * wake_edges_per_blade(r) * r.d.nb + presc_slots(r); }
-
-int stage_wing(vlm_ctx *ctx, Rotor &r, int set, int64_t off, int64_t *used)
-{
-    *used = wing_slots(r, set);
-    if (*used == 0) return VLM_OK;
-    RV v = view(r);
-    hipLaunchKernelGGL(stage_wing_kernel, dim3(nblk(r.nring)), dim3(256), 0, ctx->stream, v,
-                       set, ctx->slots.p + off, ctx->flags.p + off);
-    VLM_HIP(hipGetLastError());
-    return VLM_OK;
-}
-
-int stage_wake(vlm_ctx *ctx, Rotor &r, int pred, int64_t off, int64_t *used)
-{
-    *used = 0;
-    if (r.d.nNwake <= 0) return VLM_OK;
-    const int64_t per = wake_edges_per_blade(r);
-    if (per <= 0) return VLM_OK;
-    if (r.rowNear - 1 >= r.d.nNwake) return VLM_OK;  // no active near-wake row yet
-    *used = 2 * per * r.d.nb;
-    RV v = view(r);
-    const int far_exists = r.rowFar <= r.d.nFwake ? 1 : 0;
-    hipLaunchKernelGGL(stage_wake_kernel, dim3(nblk(per * r.d.nb)), dim3(256), 0, ctx->stream,
-                       v, pred, far_exists, per, ctx->slots.p + off, ctx->flags.p + off);
-    const int64_t np = presc_slots(r);
-    if (np > 0) {
-        const int t = pred ? 1 : 0;
-        hipLaunchKernelGGL(stage_presc_kernel, dim3(nblk(np)), dim3(256), 0, ctx->stream,
-                           r.pf[t].p, r.ps[t].p, r.d.nb, ctx->slots.p + off + *used,
-                           ctx->flags.p + off + *used);
-        *used += np;
-    }
-    VLM_HIP(hipGetLastError());
-    return VLM_OK;
 }
 
 namespace {
@@ -1040,50 +1114,115 @@ Rotor *get_rotor(vlm_ctx *ctx, int ir)
     return ctx->rotors[ir];
 }
 
-// Build the source list for a set of (rotor, set) pairs.
-int build_sources(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src)
+// Source sets of (rotor, set) pairs as staging descriptors; total receives
+// the number of items, est the expected number of segments (two per wing
+// item, one per wake edge: edges whose two ring filaments differ in core
+// radius are the exception).
+void source_descs(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src,
+                  std::vector<SrcDesc> &ds, int64_t *total, int64_t *est)
 {
+    int64_t n = 0, wing = 0;
+    for (auto &q : src) {
+        Rotor &r = *ctx->rotors[q.first];
+        SrcDesc d;
+        std::memset(&d, 0, sizeof(d));
+        d.nc = r.d.nc;
+        d.ns = r.d.ns;
+        d.first = n;
+        if (q.second == VLM_SET_WING || q.second == VLM_SET_WING_BOUND) {
+            d.kind = q.second == VLM_SET_WING ? SRC_WING : SRC_BOUND;
+            d.p[0] = r.wc.p;
+            d.p[1] = r.wrc.p;
+            d.p[2] = r.wg.p;
+            const int64_t items = (int64_t)r.nring * (d.kind == SRC_WING ? 2 : 1);
+            n += items;
+            wing += items;
+            ds.push_back(d);
+            continue;
+        }
+        const int64_t per = wake_edges_per_blade(r);
+        // no active near-wake row yet: no wake
+        if (r.d.nNwake <= 0 || r.rowNear - 1 >= r.d.nNwake || per <= 0) continue;
+        const int pred = q.second == VLM_SET_WAKE_PRED ? 1 : 0;
+        d.kind = SRC_WAKE;
+        d.p[0] = pred ? r.pnode.p : r.node.p;
+        d.p[1] = pred ? r.ple.p : r.le.p;
+        d.p[2] = r.gam.p;
+        d.p[3] = r.rc4.p;
+        d.p[4] = pred ? r.pffc.p : r.ffc.p;
+        d.p[5] = r.fgam.p;
+        d.p[6] = r.frc.p;
+        d.nN = r.d.nNwake;
+        d.nF = r.d.nFwake;
+        d.head = r.head;
+        d.rn = r.rowNear - 1;
+        d.rf = r.rowFar - 1;
+        d.far_exists = r.rowFar <= r.d.nFwake ? 1 : 0;
+        d.per_blade = per;
+        n += per * r.d.nb;
+        ds.push_back(d);
+        const int64_t np = presc_slots(r);
+        if (np > 0) {
+            std::memset(&d, 0, sizeof(d));
+            d.kind = SRC_PRESC;
+            d.p[0] = r.pf[pred].p;
+            d.p[1] = r.ps[pred].p;
+            d.first = n;
+            n += np;
+            ds.push_back(d);
+        }
+    }
+    *total = n;
+    *est = n + wing;
+}
+
+// Build the source list of (rotor, set) pairs into ctx->seg, in the given
+// formats; *est receives the expected number of segments.
+int build_sources(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src, int formats,
+                  int64_t *est)
+{
+    std::vector<SrcDesc> ds;
     int64_t total = 0;
-    for (auto &s : src) {
-        Rotor &r = *ctx->rotors[s.first];
-        if (s.second == VLM_SET_WING || s.second == VLM_SET_WING_BOUND)
-            total += wing_slots(r, s.second);
-        else if (r.rowNear - 1 < r.d.nNwake)
-            total += wake_slots(r);
+    source_descs(ctx, src, ds, &total, est);
+    if (total == 0) return VLM_OK;
+    const int nlaunch = ((int)ds.size() + SRC_MAX - 1) / SRC_MAX;
+    StageArgs a;
+    a.iters = (int)((total + (int64_t)256 * (STAGE_BLOCKS - nlaunch) - 1) /
+                    ((int64_t)256 * (STAGE_BLOCKS - nlaunch)));
+    const int64_t nb_max = (total + 256 * (int64_t)a.iters - 1) / (256 * (int64_t)a.iters) + nlaunch;
+    if (total > INT32_MAX / 4) return fail(ctx, VLM_ERR_ARG, "segment list too large");
+    VLM_HIP(ctx->slots.reserve((size_t)nb_max * a.iters * 512));
+    VLM_HIP(ctx->seg_counts.reserve(STAGE_BLOCKS));
+    VLM_HIP(ctx->seg.reserve(2 * total, formats, &ctx->seg_view));
+    a.slots = ctx->slots.p;
+    a.counts = ctx->seg_counts.p;
+    int blocks = 0;
+    for (int l = 0; l < nlaunch; ++l) {
+        const int k0 = l * SRC_MAX, k1 = std::min((int)ds.size(), k0 + SRC_MAX);
+        const int64_t first = ds[k0].first;
+        const int64_t end = k1 < (int)ds.size() ? ds[k1].first : total;
+        a.n = k1 - k0;
+        for (int k = k0; k < k1; ++k) {
+            a.d[k - k0] = ds[k];
+            a.d[k - k0].first -= first;
+        }
+        a.block0 = blocks;
+        a.total = end - first;
+        const int nb = (int)((a.total + 256 * (int64_t)a.iters - 1) / (256 * (int64_t)a.iters));
+        if (nb == 0) continue;
+        hipLaunchKernelGGL(stage_kernel, dim3(nb), dim3(256), 0, ctx->stream, a);
+        blocks += nb;
     }
-    VLM_TRY(ensure_slots(ctx, total > 0 ? total : 1));
-    int64_t off = 0, used = 0;
-    for (auto &s : src) {
-        Rotor &r = *ctx->rotors[s.first];
-        if (s.second == VLM_SET_WING || s.second == VLM_SET_WING_BOUND)
-            VLM_TRY(stage_wing(ctx, r, s.second, off, &used));
-        else
-            VLM_TRY(stage_wake(ctx, r, s.second == VLM_SET_WAKE_PRED, off, &used));
-        off += used;
-    }
-    VLM_TRY(compact_slots(ctx, off));
-    ctx->seg.cap = ctx->seg.cap;  // stride of the SoA arrays
+    hipLaunchKernelGGL(emit_records_kernel, dim3(nblk(2 * total)), dim3(256), 0, ctx->stream,
+                       ctx->slots.p, ctx->seg_counts.p, blocks, a.iters * 512, ctx->seg_view);
+    VLM_HIP(hipGetLastError());
     return VLM_OK;
 }
 
 int eval_sources(vlm_ctx *ctx, const double *t, int64_t m, int64_t tstride, double *out, int acc,
-                 int64_t nmax)
+                 int64_t est)
 {
-    return bs_eval(ctx, ctx->seg.d64.p, ctx->seg.d32.p, ctx->seg.cap, ctx->seg.count.p, nmax, t,
-                   m, tstride, out, acc);
-}
-
-int64_t staged_upper_bound(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src)
-{
-    int64_t total = 0;
-    for (auto &s : src) {
-        Rotor &r = *ctx->rotors[s.first];
-        if (s.second == VLM_SET_WING || s.second == VLM_SET_WING_BOUND)
-            total += wing_slots(r, s.second);
-        else if (r.rowNear - 1 < r.d.nNwake)
-            total += wake_slots(r);
-    }
-    return total;
+    return bs_eval(ctx, ctx->seg_view, est, t, m, tstride, out, acc);
 }
 
 int launch_scheme(vlm_ctx *ctx, Rotor &r, int op)
@@ -1277,8 +1416,8 @@ int wake_pass(vlm_ctx *ctx, int pred)
         m += target_count(*ctx->rotors[ir]);
     }
     if (m == 0) return VLM_OK;
-    const int64_t nmax = staged_upper_bound(ctx, src);
-    VLM_TRY(build_sources(ctx, src));
+    int64_t nest = 0;
+    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
     VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
     VLM_HIP(ctx->out.reserve((size_t)3 * m));
     int64_t off = 0;
@@ -1290,7 +1429,7 @@ int wake_pass(vlm_ctx *ctx, int pred)
         VLM_HIP(hipGetLastError());
         off += n;
     }
-    VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 0, nmax));
+    VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 0, nest));
     off = 0;
     for (auto *rp : ctx->rotors) {
         const int64_t n = target_count(*rp);
@@ -1331,7 +1470,9 @@ __global__ void features_kernel(RV v, float *X, int64_t off, double lref_inv,
     const double vinv = 1.0 / vref[0];
     const double *vs, *vp, *va;
     if (k < (int64_t)R * (v.ns + 1)) {
-        const int i = v.rn + (int)(k / (v.ns + 1)), j = (int)(k % (v.ns + 1));
+        int i, j;
+        patch_entry(k, R, v.ns + 1, &i, &j);
+        i += v.rn;
         const double *P = v.pnode + 3 * nidx(v, b, phys(v, i), j);
         for (int q = 0; q < 12; ++q) {
             const int ii = i + kNbr[q][0], jj = j + kNbr[q][1];
@@ -1377,7 +1518,9 @@ __global__ void gather_step_vel_kernel(RV v, double *o, int64_t stride, int64_t 
     const int64_t k = e - b * per;
     const double *V;
     if (k < (int64_t)R * (v.ns + 1)) {
-        const int i = v.rn + (int)(k / (v.ns + 1)), j = (int)(k % (v.ns + 1));
+        int i, j;
+        patch_entry(k, R, v.ns + 1, &i, &j);
+        i += v.rn;
         V = v.vel[VLM_VEL_STEP] + 3 * vidx(v, b, i, j);
     } else {
         V = v.velF[VLM_VEL_STEP] + 3 * ((size_t)b * v.nF + v.rf + (k - (int64_t)R * (v.ns + 1)));
@@ -1531,10 +1674,10 @@ __global__ void full_pairs_kernel(const double *vexact, const double *vn, int64_
 
 // Full Biot-Savart pass 2 of the learned mode, plus training pairs from it
 // (every stride-th target, a quarter of the replay buffer).
-static int full_pass(vlm_ctx *ctx, int64_t m, int64_t nmax)
+static int full_pass(vlm_ctx *ctx, int64_t m, int64_t nest)
 {
     Predictor &P = ctx->pred;
-    VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 0, nmax));
+    VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 0, nest));
     P.full += 1;
     const int64_t stride = (m + P.buf_cap / 4 - 1) / (P.buf_cap / 4);
     const int64_t np = (m + stride - 1) / stride;
@@ -1558,8 +1701,12 @@ int learned_pass(vlm_ctx *ctx)
         m += target_count(*ctx->rotors[ir]);
     }
     if (m == 0) return VLM_OK;
-    const int64_t nmax = staged_upper_bound(ctx, src);
-    VLM_TRY(build_sources(ctx, src));
+    int64_t nest = 0;
+    // the full pass reads m targets, the judge about m / stride of them
+    const int64_t stride0 = P.stride < 1 ? 1 : P.stride;
+    int formats = bs_formats(ctx, m) | bs_formats(ctx, (m + stride0 - 1) / stride0) |
+                  bs_formats(ctx, std::max<int64_t>(1, (m - stride0) / stride0));
+    VLM_TRY(build_sources(ctx, src, formats, &nest));
     VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
     VLM_HIP(ctx->out.reserve((size_t)3 * m));
     VLM_HIP(P.vn.reserve((size_t)3 * m));
@@ -1611,7 +1758,7 @@ int learned_pass(vlm_ctx *ctx)
         VLM_HIP(P.e2.reserve((size_t)3 * ms));
         hipLaunchKernelGGL(gather_sample_kernel, dim3(nblk(ms)), dim3(256), 0, ctx->stream,
                            ctx->tgt.p, m, phase, stride, ms, P.ts.p);
-        VLM_TRY(eval_sources(ctx, P.ts.p, ms, ms, P.vs.p, 0, nmax));
+        VLM_TRY(eval_sources(ctx, P.ts.p, ms, ms, P.vs.p, 0, nest));
         const int64_t take = ms < P.buf_cap ? ms : P.buf_cap;
         hipLaunchKernelGGL(judge_kernel, dim3(nblk(take)), dim3(256), 0, ctx->stream, P.vs.p,
                            take, ctx->out.p, m, phase, stride, P.vn.p, P.X.p, P.scal.p, P.e2.p,
@@ -1634,7 +1781,7 @@ int learned_pass(vlm_ctx *ctx)
         P.buf_head = (P.buf_head + take) % P.buf_cap;
         P.buf_n = P.buf_n + take < P.buf_cap ? P.buf_n + take : P.buf_cap;
     } else {
-        VLM_TRY(full_pass(ctx, m, nmax));
+        VLM_TRY(full_pass(ctx, m, nest));
     }
     // Adam on minibatches: contiguous windows of the replay buffer at a
     // rotating offset (on a judged step before the decision, so the pairs
@@ -1659,7 +1806,7 @@ int learned_pass(vlm_ctx *ctx)
         P.judged += 1;
         if (P.last_err > P.tol) {
             P.fallbacks += 1;
-            VLM_TRY(full_pass(ctx, m, nmax));
+            VLM_TRY(full_pass(ctx, m, nest));
         } else {
             hipLaunchKernelGGL(put_sample_kernel, dim3(nblk(ms)), dim3(256), 0, ctx->stream,
                                P.vs.p, ms, ctx->out.p, m, phase, stride);
@@ -2071,13 +2218,13 @@ int vlm_rotor_induced_velocity(vlm_ctx *ctx, int ir, int set, int64_t m, const d
     if (m <= 0) return VLM_OK;
     if (!p || !v) return fail(ctx, VLM_ERR_ARG, "null buffer");
     std::vector<std::pair<int, int>> src = {{ir, set}};
-    const int64_t nmax = staged_upper_bound(ctx, src);
-    VLM_TRY(build_sources(ctx, src));
+    int64_t nest = 0;
+    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
     VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
     VLM_HIP(ctx->out.reserve((size_t)3 * m));
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
-    VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, accumulate, nmax));
+    VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, accumulate, nest));
     return points_to_host(ctx, m, ctx->out.p, m, v);
 }
 
@@ -2113,9 +2260,9 @@ static int induced_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set
             VLM_HIP(hipGetLastError());
         }
         std::vector<std::pair<int, int>> src = {{ir[k], set[k]}};
-        const int64_t nmax = staged_upper_bound(ctx, src);
-        VLM_TRY(build_sources(ctx, src));
-        VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 1, nmax));
+        int64_t nest = 0;
+        VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
+        VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 1, nest));
     }
     return points_to_host(ctx, m, ctx->out.p, m, v, deferred);
 }
@@ -2144,9 +2291,9 @@ int vlm::induced_terms_soa(vlm_ctx *ctx, int nterms, const int *ir, const int *s
             VLM_HIP(hipGetLastError());
         }
         std::vector<std::pair<int, int>> src = {{ir[k], set[k]}};
-        const int64_t nmax = staged_upper_bound(ctx, src);
-        VLM_TRY(build_sources(ctx, src));
-        VLM_TRY(eval_sources(ctx, tgt, m, m, out, 1, nmax));
+        int64_t nest = 0;
+        VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
+        VLM_TRY(eval_sources(ctx, tgt, m, m, out, 1, nest));
     }
     return VLM_OK;
 }
