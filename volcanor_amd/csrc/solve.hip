@@ -9,6 +9,7 @@
 // refinement on an FP64 residual RHS - AIC . gam.
 //
 // Factorisation: lu_factor_device (lu_mfma.hip).
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <vector>
@@ -73,49 +74,230 @@ __global__ void aic_kernel(int n, const double *wc, const double *wrc, const dou
     A[e] = v[0] * ncap[3 * row] + v[1] * ncap[3 * row + 1] + v[2] * ncap[3 * row + 2];
 }
 
-// Forward/back substitution with the row pivots, one workgroup.
-__global__ __launch_bounds__(1024) void lu_solve_kernel(int n, const double *LU, const int *ipiv,
-                                                        double *x, const int *done)
+// ---------------------------------------------------------------------
+// Systems larger than one wave's (n > 96): substitutions over blocks of
+// TB rows, one workgroup per block and sweep.  A block needs the solved
+// blocks before it (forward: those above; backward: those below), and the
+// workgroups run side by side: each takes a ticket, tickets 0..nb-1 are the
+// forward blocks top down, nb..2nb-1 the backward blocks bottom up, and a
+// block waits only for blocks of lower tickets, whose workgroups have
+// started already, so every wait ends whatever the dispatch order.  A wave
+// polls the solved values themselves: the buffers are filled with a NaN of
+// a payload no value is published with (SENT), and a value arrives as one
+// 64-bit store.  The matrix tile of the next block column is loaded while
+// the values of this one are awaited.
+//
+// Bound by the chain of blocks: one store-to-load trip between compute
+// units and one 64-step substitution in a wave per block.  The sweep this
+// replaces (one workgroup, one column per barrier, pivots applied by one
+// lane) took 99 us per solve at n = 160 and 4.37 ms at n = 2176; the lane
+// per row of the residual 22 and 634 us.
+constexpr int TB = 64;
+constexpr unsigned long long SENT = 0x7FFC0DEADBEEF001ull;
+
+__device__ __forceinline__ unsigned long long load_agent(const unsigned long long *p)
 {
-    if (done && *done) return;
-    const int tid = threadIdx.x;
-    if (tid == 0)
-        for (int k = 0; k < n; ++k)
-            if (ipiv[k] != k) {
-                const double t = x[k];
-                x[k] = x[ipiv[k]];
-                x[ipiv[k]] = t;
-            }
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ void publish(unsigned long long *p, double v)
+{
+    unsigned long long u = (unsigned long long)__double_as_longlong(v);
+    if (u == SENT) u = 0x7FF8000000000000ull;
+    __hip_atomic_store(p, u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__device__ __forceinline__ double readlane_d(double v, int lane)
+{
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(v), lane),
+                            __builtin_amdgcn_readlane(__double2loint(v), lane));
+}
+
+// Device state of one solve: ticket, convergence and the number of
+// corrections, the maximum norms as bit patterns (unsigned order is the
+// order of non-negative doubles), and the two sweeps' block results.
+struct SolveWork {
+    int *ticket, *st;                        // st: converged, corrections applied
+    unsigned long long *rmax, *bmax;         // rmax[2]: residual it writes rmax[it & 1]
+    unsigned long long *y, *z;               // nb * TB each
+};
+
+__global__ __launch_bounds__(256) void solve_init_kernel(int n, const double *b, SolveWork w)
+{
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    const int np = (n + TB - 1) / TB * TB;
+    if (i < np) {
+        w.y[i] = SENT;
+        w.z[i] = SENT;
+    }
+    if (blockIdx.x == 0) {
+        __shared__ double sm[4];
+        if (threadIdx.x == 0) {
+            *w.ticket = 0;
+            w.st[0] = 0;
+            w.st[1] = 0;
+            w.rmax[0] = 0;
+        }
+        double m = 0.0;
+        for (int k = threadIdx.x; k < n; k += 256) m = fmax(m, fabs(b[k]));
+        for (int o = 32; o > 0; o >>= 1) m = fmax(m, __shfl_xor(m, o));
+        if ((threadIdx.x & 63) == 0) sm[threadIdx.x >> 6] = m;
+        __syncthreads();
+        if (threadIdx.x == 0)
+            *w.bmax = (unsigned long long)__double_as_longlong(
+                fmax(fmax(sm[0], sm[1]), fmax(sm[2], sm[3])));
+    }
+}
+
+// x = (LU)^-1 P rhs, or, for a correction (acc), x += it unless the last
+// residual met tol.  perm[i] is the row of the right-hand side that the
+// pivoting moves to row i.
+__global__ __launch_bounds__(256) void lu_sweeps_kernel(int n, const double *LU, const int *perm,
+                                                        const double *rhs, double *x, int acc,
+                                                        int it, double tol, SolveWork w)
+{
+    __shared__ double D[TB * TB];   // diagonal block, column-major
+    __shared__ double part[4][TB];
+    __shared__ int tk;
+    const int tid = threadIdx.x, lane = tid & 63, q = tid >> 6;
+    const bool conv = acc && (w.st[0] || __longlong_as_double((long long)w.rmax[it & 1]) <=
+                                             tol * __longlong_as_double((long long)*w.bmax));
+    if (tid == 0) tk = atomicAdd(w.ticket, 1);
     __syncthreads();
-    for (int j = 0; j < n; ++j) {
-        const double xj = x[j];
-        for (int i = j + 1 + tid; i < n; i += blockDim.x) x[i] -= LU[i + (size_t)n * j] * xj;
-        __syncthreads();
+    if (conv) {
+        // the flag only for the launches that follow: this launch decides by
+        // the norms, which nothing in it changes
+        if (tk == 0 && tid == 0) w.st[0] = 1;
+        return;
     }
-    for (int j = n - 1; j >= 0; --j) {
-        if (tid == 0) x[j] /= LU[j + (size_t)n * j];
-        __syncthreads();
-        const double xj = x[j];
-        for (int i = tid; i < j; i += blockDim.x) x[i] -= LU[i + (size_t)n * j] * xj;
-        __syncthreads();
+    if (tk == 0 && tid == 0 && acc) w.st[1] += 1;
+    const int nb = (n + TB - 1) / TB;
+    const bool back = tk >= nb;
+    const int blk = back ? 2 * nb - 1 - tk : tk;
+    const int r0 = blk * TB, row = r0 + lane;
+    const size_t ld = (size_t)n;
+    for (int e = tid; e < TB * TB; e += 256) {
+        const int i = r0 + (e & 63), j = r0 + (e >> 6);
+        D[e] = (i < n && j < n) ? LU[i + ld * j] : (i == j ? 1.0 : 0.0);
     }
+    // the blocks this one needs, in the order they are solved: this wave
+    // takes 16 columns of each
+    const int nk = back ? nb - 1 - blk : blk;
+    const unsigned long long *src = back ? w.z : w.y;
+    auto col0 = [&](int k) { return (back ? nb - 1 - k : k) * TB + 16 * q; };
+    double t[16], s = 0.0;
+    const int rc = row < n ? row : n - 1;
+    auto load = [&](int k) {
+#pragma unroll
+        for (int c = 0; c < 16; ++c) {
+            const int j = col0(k) + c;
+            const double v = LU[rc + ld * (j < n ? j : n - 1)];
+            t[c] = (row < n && j < n) ? v : 0.0;
+        }
+    };
+    if (nk > 0) load(0);
+    for (int k = 0; k < nk; ++k) {
+        double a[16];
+#pragma unroll
+        for (int c = 0; c < 16; ++c) a[c] = t[c];
+        if (k + 1 < nk) load(k + 1);
+        const unsigned long long *p = src + col0(k) + (lane & 15);
+        unsigned long long u = load_agent(p);
+        while (__any(u == SENT)) {
+            __builtin_amdgcn_s_sleep(1);
+            u = load_agent(p);
+        }
+        const double v = __longlong_as_double((long long)u);
+#pragma unroll
+        for (int c = 0; c < 16; ++c) s += a[c] * readlane_d(v, c);
+    }
+    part[q][lane] = s;
+    __syncthreads();
+    if (q > 0) return;
+    double v;
+    if (back) {   // own forward block
+        unsigned long long u = load_agent(w.y + row);
+        while (__any(u == SENT)) {
+            __builtin_amdgcn_s_sleep(1);
+            u = load_agent(w.y + row);
+        }
+        v = __longlong_as_double((long long)u);
+    } else {
+        v = row < n ? rhs[perm[row]] : 0.0;
+    }
+    v -= (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    constexpr int SU = 8;   // columns whose LDS reads issue ahead of the chain
+    if (!back) {
+        for (int j = 0; j < TB; j += SU) {
+            double l[SU];
+#pragma unroll
+            for (int u = 0; u < SU; ++u) l[u] = lane > j + u ? D[lane + TB * (j + u)] : 0.0;
+#pragma unroll
+            for (int u = 0; u < SU; ++u) v -= l[u] * readlane_d(v, j + u);
+        }
+        publish(w.y + row, v);
+        return;
+    }
+    const double d = D[lane + TB * lane], rd = 1.0 / d;
+    // v / d by the reciprocal and one correction of the remainder, or, where
+    // a reciprocal leaves the normal range, by division
+    const bool plain = __any(!(fabs(rd) < 1e300 && fabs(rd) > 1e-300)) != 0;
+    for (int j = TB - SU; j >= 0; j -= SU) {
+        double l[SU];
+#pragma unroll
+        for (int u = 0; u < SU; ++u) l[u] = lane < j + u ? D[lane + TB * (j + u)] : 0.0;
+#pragma unroll
+        for (int u = SU - 1; u >= 0; --u) {
+            const double g = v * rd;
+            double e = __builtin_fma(__builtin_fma(-g, d, v), rd, g);
+            if (plain) e = v / d;
+            v = lane == j + u ? e : v;
+            v -= l[u] * readlane_d(v, j + u);
+        }
+    }
+    publish(w.z + row, v);
+    if (row < n) x[row] = acc ? x[row] + v : v;
 }
 
-// r = b - A x (one lane per row, FP64); also r_inf via per-row |r|.
-__global__ void residual_kernel(int n, const double *A, const double *x, const double *b,
-                                double *r)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    double s = b[i];
-    for (int j = 0; j < n; ++j) s -= A[i + (size_t)n * j] * x[j];
-    r[i] = s;
-}
+// r = b - A x and its maximum norm: RROWS rows per workgroup, the columns
+// in RSL slices (A is read once, in runs of 256 bytes).  Clears the sweep
+// buffers and the ticket for the correction that follows.
+constexpr int RROWS = 32, RSL = 32;
 
-__global__ void axpy_kernel(int n, const double *d, double *x, const int *done)
+__global__ __launch_bounds__(RROWS * RSL) void residual_kernel(int n, const double *A,
+                                                               const double *x, const double *b,
+                                                               double *r, int it, SolveWork w)
 {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n && !*done) x[i] += d[i];
+    __shared__ double part[RSL][RROWS + 1];
+    const int l = threadIdx.x % RROWS, q = threadIdx.x / RROWS;
+    const int i = blockIdx.x * RROWS + l;
+    if (w.st[0]) return;
+    double s = 0.0;
+    if (i < n)
+        for (int j = q; j < n; j += RSL) s += A[i + (size_t)n * j] * x[j];
+    part[q][l] = s;
+    const int np = (n + TB - 1) / TB * TB;
+    const int e = blockIdx.x * RROWS * RSL + threadIdx.x;
+    for (int k = e; k < np; k += gridDim.x * RROWS * RSL) {
+        w.y[k] = SENT;
+        w.z[k] = SENT;
+    }
+    if (e == 0) {
+        *w.ticket = 0;
+        w.rmax[(it + 1) & 1] = 0;   // read last by the previous correction
+    }
+    __syncthreads();
+    if (q > 0) return;
+    double t = 0.0;
+    for (int k = 0; k < RSL; ++k) t += part[k][l];
+    t = i < n ? b[i] - t : 0.0;
+    if (i < n) r[i] = t;
+    unsigned long long m = (unsigned long long)__double_as_longlong(fabs(t));
+    for (int o = 16; o > 0; o >>= 1) {
+        const unsigned long long v = __shfl_xor(m, o, 32);
+        m = v > m ? v : m;
+    }
+    if (l == 0) atomicMax(w.rmax + (it & 1), m);
 }
 
 // rotor_map_gam (classdef.f90:4181-4196): blades ib <= nbConvect take
@@ -130,44 +312,10 @@ __global__ void map_gam_kernel(const double *x, double *wg, int per_blade, int n
     else if (nbc == 1) wg[e] = x[k];
 }
 
-__global__ void solve_state_init_kernel(int *st)
-{
-    st[0] = 0;  // converged
-    st[1] = 0;  // corrections applied
-}
-
-// Convergence test of the refinement on the device: ||r||_inf against
-// tol ||b||_inf; counts the correction that follows when not converged.
-__global__ void refine_check_kernel(int n, const double *r, const double *b, double tol, int *st)
-{
-    __shared__ double sr[256], sb[256];
-    double mr = 0.0, mb = 0.0;
-    for (int i = threadIdx.x; i < n; i += blockDim.x) {
-        mr = fmax(mr, fabs(r[i]));
-        mb = fmax(mb, fabs(b[i]));
-    }
-    sr[threadIdx.x] = mr;
-    sb[threadIdx.x] = mb;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) {
-            sr[threadIdx.x] = fmax(sr[threadIdx.x], sr[threadIdx.x + w]);
-            sb[threadIdx.x] = fmax(sb[threadIdx.x], sb[threadIdx.x + w]);
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0 && st[0] == 0) {
-        if (sr[0] <= tol * sb[0]) st[0] = 1;
-        else st[1] += 1;
-    }
-}
-
 // The whole solve with refinement in one wave for n <= 64 R: lane l holds
 // rows l + 64 r (r < R) of x, b and r; LU and A are staged in LDS (both fit
 // the 160 KB of a gfx950 CU up to n = 96); values move between lanes by
-// readlane (the index is uniform).  Each row takes the same operations in the same order as in
-// lu_solve_kernel, residual_kernel, refine_check_kernel and axpy_kernel, so
-// the result is bitwise that of the multi-launch path.  The workgroup has
+// readlane (the index is uniform).  The workgroup has
 // SOLVE_STAGE threads so that the staging copy keeps many loads in flight
 // (one wave alone, waiting on each load, took 136 us for n = 90); after it
 // every wave but the first leaves.
@@ -362,15 +510,24 @@ __global__ __launch_bounds__(SOLVE_STAGE) void solve_wave_kernel(int n, const do
 // x = A^-1 rhs by the LU factors plus up to max_iter refinement steps on
 // the FP64 residual.  Everything is enqueued: the convergence test runs on
 // the device (later corrections are skipped once it passes), so the only
-// synchronisation is the final download.  With a rotor given, the solution
-// also becomes its device wing circulation (rotor_map_gam).
-int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const int *ipiv,
+// synchronisation is the final download.  piv: the pivots, or for n >
+// SOLVE_WAVE_N2 the row permutation they compose to.  With a rotor given,
+// the solution also becomes its device wing circulation (rotor_map_gam).
+int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const int *piv,
                  const double *rhs_h, double *x_h, int max_iter, double tol, int *iters,
                  Rotor *rotor = nullptr, bool deferred = false)
 {
-    VLM_HIP(ctx->solve_tmp.reserve((size_t)3 * n + 1));
+    const size_t np = (size_t)(n + TB - 1) / TB * TB;
+    VLM_HIP(ctx->solve_tmp.reserve((size_t)3 * n + 2 * np + 5));
     double *b = ctx->solve_tmp.p, *x = b + n, *r = x + n;
-    int *st = reinterpret_cast<int *>(r + n);
+    SolveWork w;
+    w.y = reinterpret_cast<unsigned long long *>(r + n);
+    w.z = w.y + np;
+    w.rmax = w.z + np;
+    w.bmax = w.rmax + 2;
+    w.st = reinterpret_cast<int *>(w.bmax + 1);
+    w.ticket = w.st + 2;
+    int *st = w.st;
     if (rhs_h) {
         VLM_TRY(h2d(ctx, b, rhs_h, sizeof(double) * n));
     } else {  // the right-hand side left on the device by vlm_rotor_rhs
@@ -379,27 +536,22 @@ int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const i
     }
     if (n <= SOLVE_WAVE_N) {
         hipLaunchKernelGGL((solve_wave_kernel<1, SOLVE_WAVE_N>), dim3(1), dim3(SOLVE_STAGE), 0,
-                           ctx->stream, n, A, LU, ipiv, b, x, max_iter, tol, st);
-        max_iter = 0;
+                           ctx->stream, n, A, LU, piv, b, x, max_iter, tol, st);
     } else if (n <= SOLVE_WAVE_N2) {
         hipLaunchKernelGGL((solve_wave_kernel<2, SOLVE_WAVE_N2>), dim3(1), dim3(SOLVE_STAGE), 0,
-                           ctx->stream, n, A, LU, ipiv, b, x, max_iter, tol, st);
-        max_iter = 0;
+                           ctx->stream, n, A, LU, piv, b, x, max_iter, tol, st);
     } else {
-        VLM_HIP(hipMemcpyAsync(x, b, sizeof(double) * n, hipMemcpyDeviceToDevice, ctx->stream));
-        hipLaunchKernelGGL(solve_state_init_kernel, dim3(1), dim3(1), 0, ctx->stream, st);
-        hipLaunchKernelGGL(lu_solve_kernel, dim3(1), dim3(1024), 0, ctx->stream, n, LU, ipiv, x,
-                           nullptr);
-    }
-    for (int it = 0; it < max_iter; ++it) {
-        hipLaunchKernelGGL(residual_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n,
-                           A, x, b, r);
-        hipLaunchKernelGGL(refine_check_kernel, dim3(1), dim3(256), 0, ctx->stream, n, r, b, tol,
-                           st);
-        hipLaunchKernelGGL(lu_solve_kernel, dim3(1), dim3(1024), 0, ctx->stream, n, LU, ipiv, r,
-                           st);
-        hipLaunchKernelGGL(axpy_kernel, dim3((n + 255) / 256), dim3(256), 0, ctx->stream, n, r, x,
-                           st);
+        const dim3 gs(2 * (unsigned)(np / TB)), gr((n + RROWS - 1) / RROWS);
+        hipLaunchKernelGGL(solve_init_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0,
+                           ctx->stream, n, b, w);
+        hipLaunchKernelGGL(lu_sweeps_kernel, gs, dim3(256), 0, ctx->stream, n, LU, piv, b, x, 0,
+                           0, tol, w);
+        for (int it = 0; it < max_iter; ++it) {
+            hipLaunchKernelGGL(residual_kernel, gr, dim3(RROWS * RSL), 0, ctx->stream, n, A, x, b,
+                               r, it, w);
+            hipLaunchKernelGGL(lu_sweeps_kernel, gs, dim3(256), 0, ctx->stream, n, LU, piv, r, x,
+                               1, it, tol, w);
+        }
     }
     VLM_HIP(hipGetLastError());
     if (rotor) {
@@ -424,6 +576,22 @@ int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const i
     return VLM_OK;
 }
 
+// Row permutation of a pivot sequence: row i of P b is row perm[i] of b.
+// Pivots outside the matrix (a matrix of NaNs has none) move nothing.
+void compose_pivots(int n, const int *piv, int *perm)
+{
+    for (int i = 0; i < n; ++i) perm[i] = i;
+    for (int k = 0; k < n; ++k)
+        if (piv[k] >= 0 && piv[k] < n) std::swap(perm[k], perm[piv[k]]);
+}
+
+// What solve_refine reads of a rotor's pivots at its order.
+const int *solve_pivots(vlm_ctx *ctx, int ir)
+{
+    const int n = ctx->aic_n[ir];
+    return ctx->piv[ir] + (n > SOLVE_WAVE_N2 ? n + 1 : 0);
+}
+
 }  // namespace
 }  // namespace vlm
 
@@ -446,7 +614,7 @@ int vlm_rotor_calc_aic(vlm_ctx *ctx, int ir, const double *cp, const double *nca
         ctx->piv[ir] = nullptr;
         VLM_HIP(hipMalloc(reinterpret_cast<void **>(&ctx->aic[ir]), sizeof(double) * n * n));
         VLM_HIP(hipMalloc(reinterpret_cast<void **>(&ctx->lu[ir]), sizeof(double) * n * n));
-        VLM_HIP(hipMalloc(reinterpret_cast<void **>(&ctx->piv[ir]), sizeof(int) * (n + 1)));
+        VLM_HIP(hipMalloc(reinterpret_cast<void **>(&ctx->piv[ir]), sizeof(int) * (2 * n + 1)));
         ctx->aic_n[ir] = n;
     }
     DBuf<double> geo;
@@ -460,13 +628,19 @@ int vlm_rotor_calc_aic(vlm_ctx *ctx, int ir, const double *cp, const double *nca
     VLM_HIP(hipMemcpyAsync(ctx->lu[ir], ctx->aic[ir], sizeof(double) * nn,
                            hipMemcpyDeviceToDevice, ctx->stream));
     VLM_TRY(lu_factor_device(ctx, n, ctx->lu[ir], ctx->piv[ir], ctx->piv[ir] + n));
-    int info = 0;
-    VLM_HIP(hipMemcpyAsync(&info, ctx->piv[ir] + n, sizeof(int), hipMemcpyDeviceToHost,
+    std::vector<int> piv((size_t)2 * n + 1);   // pivots, info, row permutation
+    char *hp = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(int) * (n + 1), &hp));
+    VLM_HIP(hipMemcpyAsync(hp, ctx->piv[ir], sizeof(int) * (n + 1), hipMemcpyDeviceToHost,
                            ctx->stream));
     if (Aout)
         VLM_HIP(hipMemcpyAsync(Aout, ctx->aic[ir], sizeof(double) * nn, hipMemcpyDeviceToHost,
                                ctx->stream));
     VLM_TRY(sync_stream(ctx));
+    std::memcpy(piv.data(), hp, sizeof(int) * (n + 1));
+    const int info = piv[n];
+    compose_pivots(n, piv.data(), piv.data() + n + 1);
+    VLM_TRY(h2d(ctx, ctx->piv[ir] + n + 1, piv.data() + n + 1, sizeof(int) * n));
     if (info != 0) return fail(ctx, VLM_ERR_SINGULAR, "AIC is singular (zero pivot)");
     return VLM_OK;
 }
@@ -479,8 +653,8 @@ int vlm_rotor_solve(vlm_ctx *ctx, int ir, const double *rhs, double *gam, int ma
     if (!rhs || !gam) return fail(ctx, VLM_ERR_ARG, "null buffer");
     if (!ctx->lu[ir]) return fail(ctx, VLM_ERR_STATE, "vlm_rotor_calc_aic not called");
     const int n = ctx->aic_n[ir];
-    return solve_refine(ctx, n, ctx->aic[ir], ctx->lu[ir], ctx->piv[ir], rhs, gam, max_iter, tol,
-                        iters, ctx->rotors[ir]);
+    return solve_refine(ctx, n, ctx->aic[ir], ctx->lu[ir], solve_pivots(ctx, ir), rhs, gam, max_iter,
+                        tol, iters, ctx->rotors[ir]);
 }
 
 int vlm_rotor_solve_deferred(vlm_ctx *ctx, int ir, const double *rhs, double *gam, int max_iter,
@@ -493,8 +667,8 @@ int vlm_rotor_solve_deferred(vlm_ctx *ctx, int ir, const double *rhs, double *ga
     if (!rhs && !ctx->rotors[ir]->panels_set)
         return fail(ctx, VLM_ERR_STATE, "no right-hand side on the device (vlm_rotor_rhs)");
     const int n = ctx->aic_n[ir];
-    return solve_refine(ctx, n, ctx->aic[ir], ctx->lu[ir], ctx->piv[ir], rhs, gam, max_iter, tol,
-                        iters, ctx->rotors[ir], true);
+    return solve_refine(ctx, n, ctx->aic[ir], ctx->lu[ir], solve_pivots(ctx, ir), rhs, gam, max_iter,
+                        tol, iters, ctx->rotors[ir], true);
 }
 
 int vlm_lu_factor(vlm_ctx *ctx, int n, double *A, int *ipiv)
@@ -520,6 +694,10 @@ int vlm_lu_solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, 
                         const double *rhs, double *x, int max_iter, double tol, int *iters)
 {
     if (!ctx || n <= 0 || !A || !LU || !ipiv || !rhs || !x) return VLM_ERR_ARG;
+    for (int k = 0; k < n; ++k)
+        if (ipiv[k] < 0 || ipiv[k] >= n) return fail(ctx, VLM_ERR_ARG, "pivot out of range");
+    std::vector<int> perm(ipiv, ipiv + n);
+    if (n > SOLVE_WAVE_N2) compose_pivots(n, ipiv, perm.data());
     VLM_DEVICE(ctx);
     DBuf<double> dA, dLU;
     DBuf<int> dp;
@@ -528,7 +706,7 @@ int vlm_lu_solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, 
     VLM_HIP(dp.reserve((size_t)n));
     VLM_HIP(hipMemcpyAsync(dA.p, A, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
     VLM_HIP(hipMemcpyAsync(dLU.p, LU, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
-    VLM_HIP(hipMemcpyAsync(dp.p, ipiv, sizeof(int) * n, hipMemcpyHostToDevice, ctx->stream));
+    VLM_TRY(h2d(ctx, dp.p, perm.data(), sizeof(int) * n));
     return solve_refine(ctx, n, dA.p, dLU.p, dp.p, rhs, x, max_iter, tol, iters);
 }
 
