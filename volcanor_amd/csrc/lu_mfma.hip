@@ -5,10 +5,9 @@
 // info = first zero pivot (1-based) or 0.  Pivot choice follows IDAMAX:
 // the first row of largest magnitude.
 //
-// n <= LU_SMALL (the AIC of one rotor): one workgroup, unblocked.
-// Larger n: right-looking blocked LU.  Panels are 32 columns wide where the
-// panel fits on chip (m <= 2048 rows), 16 columns above that.
-//   1. panel: one workgroup factorises A[k:n, k:k+jb] column by column,
+// Right-looking blocked LU.  Panels are 32 columns wide where the panel has
+// at most 1024 rows, 16 columns above that.
+//   1. panel: one workgroup (one wave up to 256 rows) factorises A[k:n, k:k+jb] column by column,
 //      the panel in registers; rows never move during the panel, each lane
 //      tracks the logical position of its rows, and one barrier per column
 //      publishes every wave's pivot candidate with its row.  16-column
@@ -36,7 +35,6 @@ namespace {
 
 constexpr int LU_THREADS = 1024;
 constexpr int LU_WAVES = LU_THREADS / 64;
-constexpr int LU_SMALL = 256;  // one-workgroup path up to this order
 constexpr int NB = 16;         // panel width of tall panels
 constexpr int NBMAX = 32;      // panel width where the panel fits on chip
 constexpr int PT = 512;        // workgroup of the on-chip panel
@@ -58,63 +56,6 @@ __device__ __forceinline__ void better(double &bv, int &bi, double v, int i)
     bv = take ? v : bv;
     bi = take ? i : bi;
 }
-
-// Unblocked right-looking LU of columns [k0, k1) over rows [k0, n).  Row
-// swaps are applied to columns [s0, s1) (the whole matrix for the
-// one-workgroup path, the panel only in the blocked path), the rank-1
-// updates to columns (k, k1).
-__global__ __launch_bounds__(LU_THREADS) void lu_panel_kernel(int n, double *A, int *ipiv,
-                                                              int *info, int k0, int k1, int s0,
-                                                              int s1)
-{
-    __shared__ double sv[LU_WAVES];
-    __shared__ int si[LU_WAVES];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const size_t ld = (size_t)n;
-    if (*info != 0) {  // an earlier panel hit a zero pivot: keep pivots in range
-        for (int k = k0 + tid; k < k1; k += blockDim.x) ipiv[k] = k;
-        return;
-    }
-    // 2-D split of the trailing update: 64 consecutive rows per wave
-    // (coalesced), LU_WAVES column groups.
-    for (int k = k0; k < k1; ++k) {
-        double bv = -1.0;
-        int bi = k;
-        for (int i = k + tid; i < n; i += LU_THREADS) better(bv, bi, fabs(A[i + ld * k]), i);
-        for (int off = 32; off > 0; off >>= 1)
-            better(bv, bi, __shfl_xor(bv, off), __shfl_xor(bi, off));
-        if (lane == 0) {
-            sv[w] = bv;
-            si[w] = bi;
-        }
-        __syncthreads();
-        bv = sv[0];
-        bi = si[0];
-        for (int q = 1; q < LU_WAVES; ++q) better(bv, bi, sv[q], si[q]);
-        const int p = bi;
-        if (tid == 0) ipiv[k] = p;
-        if (bv == 0.0) {
-            if (tid == 0 && *info == 0) *info = k + 1;
-            for (int j = k + 1 + tid; j < k1; j += LU_THREADS) ipiv[j] = j;
-            return;
-        }
-        if (p != k)
-            for (int j = s0 + tid; j < s1; j += LU_THREADS) {
-                const double t = A[k + ld * j];
-                A[k + ld * j] = A[p + ld * j];
-                A[p + ld * j] = t;
-            }
-        __syncthreads();
-        const double inv = 1.0 / A[k + ld * k];
-        for (int j = k + 1 + w; j < k1; j += LU_WAVES) {
-            const double u = A[k + ld * j];
-            for (int i = k + 1 + lane; i < n; i += 64) A[i + ld * j] -= (A[i + ld * k] * inv) * u;
-        }
-        __syncthreads();
-        for (int i = k + 1 + tid; i < n; i += LU_THREADS) A[i + ld * k] *= inv;
-    }
-}
-
 
 __device__ __forceinline__ double readlane_f64(double v, int lane)
 {
@@ -446,44 +387,42 @@ __global__ __launch_bounds__(PT) void lu_panel_fast_kernel(int n, double *A, int
 
 
 // Panel held in registers, masking design (the 32-column panels, up to
-// 1024 rows): lane t owns the physical panel rows t + PT*q, RPT of
-// them in registers and RL more in LDS (columns [k0, k0+jb), jb <= JB).
-// A pivot row stays in its lane and is masked out of later columns by its
-// logical position.
-// Rows never move during the panel: pos[q] is the logical row (after the
-// swaps so far) of each owned row, so a row swap is two index updates.
-// Per column, each wave finds its candidate (wave argmax), the owning lane
-// copies the candidate row into the wave's LDS slot, and one barrier later
-// every wave picks the winning record (a DPP butterfly over the waves'
-// records) and reads the pivot row from its slot.
-// The slots alternate between two buffers by column parity, so a fast wave
-// writing the next column's slot never overwrites one still being read.
-// The column loop is unrolled by template recursion so that every register
-// index is a constant.
-template <int JB>
+// 1024 rows): W waves, lane t owns the physical panel rows t + 64 W q, RPT
+// of them (columns [k0, k0+JB)).  A pivot row stays in its lane and is
+// masked out of later columns by its logical position.  Rows never move
+// during the panel: pos[q] is the logical row (after the swaps so far) of
+// each owned row, so a row swap is two index updates.  Per column, each
+// wave finds its candidate (wave argmax), the owning lane copies the
+// candidate row into the wave's LDS slot, and one barrier later every wave
+// picks the winning record (a DPP butterfly over the waves' records) and
+// reads the pivot row from its slot.  The slots alternate between two
+// buffers by column parity, so a fast wave writing the next column's slot
+// never overwrites one still being read.  The column loop is unrolled by
+// template recursion so that every register index is a constant (a loop
+// that shifts the columns through the registers instead, small enough for
+// the instruction cache, was slower: 59 against 33 us at 512 rows).
+template <int JB, int W>
 struct WideCtx {
-    double *cand;   // [2][PW][JB]
-    PivRec *rec;    // [2][PW] candidate records
-    double *cinv;   // [2][PW] 1 / candidate value
-    double *L;      // LDS rows: L[(q*JB + j)*PT + tid]
-    int *ipiv, *info, *list;
+    double *cand;   // [2][W][JB]
+    PivRec *rec;    // [2][W] candidate records
+    double *cinv;   // [2][W] 1 / candidate value
+    int *ipiv, *info;
     int tid, lane, w, k0, m;
 };
 
-template <int JB, int RPT, int RL, int C>
-__device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT + RL],
-                                            WideCtx<JB> &P)
+template <int JB, int W, int RPT, int C>
+__device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT],
+                                            WideCtx<JB, W> &P)
 {
     constexpr int par = C & 1;
-    double *L = P.L + P.tid;
     // this lane's candidate: largest |a| among its rows at logical >= C,
     // the lowest logical row on ties (branch-free)
     double bv = -1.0;
     int bi = INT_MAX;
 #pragma unroll
-    for (int q = 0; q < RPT + RL; ++q) {
+    for (int q = 0; q < RPT; ++q) {
         const int p = pos[q];
-        const double x = fabs(q < RPT ? a[q < RPT ? q : 0][C] : L[((q - RPT) * JB + C) * PT]);
+        const double x = fabs(a[q][C]);
         const bool t = (p >= C) & (p < P.m) & ((x > bv) | ((x == bv) & (p < bi)));
         bv = t ? x : bv;
         bi = t ? p : bi;
@@ -495,37 +434,30 @@ __device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT
                                       : wave_min(bv == M ? bi : INT_MAX);
     // its owner publishes the row (columns C..JB-1) and the reciprocal
     if (bi == wi) {
-        double *crow = P.cand + (par * PW + P.w) * JB;
+        double *crow = P.cand + (par * W + P.w) * JB;
 #pragma unroll
         for (int q = 0; q < RPT; ++q)
             if (pos[q] == wi) {
-                P.cinv[par * PW + P.w] = 1.0 / a[q][C];
+                P.cinv[par * W + P.w] = 1.0 / a[q][C];
 #pragma unroll
                 for (int j = C; j < JB; ++j) crow[j] = a[q][j];
-            }
-#pragma unroll
-        for (int q = 0; q < RL; ++q)
-            if (pos[RPT + q] == wi) {
-                P.cinv[par * PW + P.w] = 1.0 / L[(q * JB + C) * PT];
-#pragma unroll
-                for (int j = C; j < JB; ++j) crow[j] = L[(q * JB + j) * PT];
             }
     }
     if (P.lane == 0) {
         // a wave without candidate rows (M = -1) loses to every other
         const bool none = M < 0.0;
-        P.rec[par * PW + P.w] = PivRec{none ? 0u : (unsigned)__double2loint(M),
-                                       none ? 0u : (unsigned)__double2hiint(M),
-                                       none ? INT_MAX : wi * 8 + P.w, 0};
+        P.rec[par * W + P.w] = PivRec{none ? 0u : (unsigned)__double2loint(M),
+                                      none ? 0u : (unsigned)__double2hiint(M),
+                                      none ? INT_MAX : wi * 8 + P.w, 0};
     }
     __syncthreads();
     // the block's pivot: largest wave maximum, lowest row among the waves
-    // holding it, by a butterfly over the PW records in each group of 8
+    // holding it, by a butterfly over the W records in each group of W
     // lanes (half-row mirror, then xor 2 and xor 1)
-    static_assert(PW == 8, "butterfly over 8 waves");
-    PivRec r = P.rec[par * PW + (P.lane & 7)];
-    rec_best<0x141>(r);
-    rec_best<0x4E>(r);
+    static_assert(W == 2 || W == 4 || W == 8, "butterfly over the waves");
+    PivRec r = P.rec[par * W + (P.lane & (W - 1))];
+    if constexpr (W == 8) rec_best<0x141>(r);
+    if constexpr (W >= 4) rec_best<0x4E>(r);
     rec_best<0xB1>(r);
     const double gv = __hiloint2double(__builtin_amdgcn_readfirstlane((int)r.hi),
                                        __builtin_amdgcn_readfirstlane((int)r.lo));
@@ -538,27 +470,20 @@ __device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT
         // and left as it is, as DGETF2 does; the factorisation reports it
         if (gv == 0.0 && *P.info == 0) *P.info = P.k0 + C + 1;
     }
-    const double *prow = P.cand + (par * PW + gw) * JB;
-    const double inv = gv == 0.0 ? 0.0 : P.cinv[par * PW + gw];
+    const double *prow = P.cand + (par * W + gw) * JB;
+    const double inv = gv == 0.0 ? 0.0 : P.cinv[par * W + gw];
 #pragma unroll
-    for (int q = 0; q < RPT + RL; ++q) {
+    for (int q = 0; q < RPT; ++q) {
         if (pos[q] == lp) pos[q] = C;
         else if (pos[q] == C) pos[q] = lp;
     }
-    double l[RPT + RL];
+    double l[RPT];
 #pragma unroll
-    for (int q = 0; q < RPT + RL; ++q) {
+    for (int q = 0; q < RPT; ++q) {
         const bool upd = pos[q] > C && pos[q] < P.m;
-        if (q < RPT) {
-            const double x = a[q < RPT ? q : 0][C];
-            l[q] = upd ? x * inv : 0.0;
-            a[q < RPT ? q : 0][C] = upd ? l[q] : x;
-        } else {
-            double *e = L + ((q - RPT) * JB + C) * PT;
-            const double x = *e;
-            l[q] = upd ? x * inv : 0.0;
-            if (upd) *e = l[q];
-        }
+        const double x = a[q][C];
+        l[q] = upd ? x * inv : 0.0;
+        a[q][C] = upd ? l[q] : x;
     }
     // rank-1 update, CH pivot-row entries at a time (the scheduling barrier
     // keeps later entries' loads from piling up in registers when the
@@ -575,27 +500,23 @@ __device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT
                 const int j = j0 + t < JB ? j0 + t : 0;
 #pragma unroll
                 for (int q = 0; q < RPT; ++q) a[q][j] -= l[q] * u[t];
-#pragma unroll
-                for (int q = 0; q < RL; ++q)
-                    if (l[RPT + q] != 0.0) L[(q * JB + j) * PT] -= l[RPT + q] * u[t];
             }
         }
         __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (C + 1 < JB) wide_column<JB, RPT, RL, C + 1>(a, pos, P);
+    if constexpr (C + 1 < JB) wide_column<JB, W, RPT, C + 1>(a, pos, P);
 }
 
-// Exactly JB columns (the host gives ragged last panels to the tall kernel).
-template <int JB, int RPT, int RL>
-__global__ __launch_bounds__(PT) void lu_panel_wide_kernel(int n, double *A, int *ipiv, int *info,
-                                                           int k0, int *list)
+// Exactly JB columns.
+template <int JB, int W, int RPT>
+__global__ __launch_bounds__(64 * W) void lu_panel_wide_kernel(int n, double *A, int *ipiv,
+                                                               int *info, int k0, int *list)
 {
-    constexpr int S = RPT + RL;
+    constexpr int T = 64 * W;
     constexpr int EMPTY = 1 << 30;   // logical position of a slot past the panel
-    __shared__ double cand[2 * PW * JB];
-    __shared__ PivRec rec[2 * PW];
-    __shared__ double cinv[2 * PW];
-    __shared__ double Lrows[RL > 0 ? RL * JB * PT : 1];
+    __shared__ double cand[2 * W * JB];
+    __shared__ PivRec rec[2 * W];
+    __shared__ double cinv[2 * W];
     __shared__ int moved;
     const int tid = threadIdx.x;
     const size_t ld = (size_t)n;
@@ -605,39 +526,37 @@ __global__ __launch_bounds__(PT) void lu_panel_wide_kernel(int n, double *A, int
         list[LJB] = JB;
     }
     if (*info != 0) {
-        for (int k = tid; k < JB; k += PT) ipiv[k0 + k] = k0 + k;
+        for (int k = tid; k < JB; k += T) ipiv[k0 + k] = k0 + k;
         if (tid == 0) list[0] = 0;
         return;
     }
     if (tid == 0) moved = 0;
     double a[RPT][JB];
-    int pos[S];
+    int pos[RPT];
 #pragma unroll
-    for (int q = 0; q < S; ++q) {
-        const int r = tid + PT * q;
+    for (int q = 0; q < RPT; ++q) {
+        const int r = tid + T * q;
         pos[q] = r < m ? r : EMPTY;
     }
     const double *col = A + ld * (size_t)k0 + k0;
 #pragma unroll
     for (int c = 0; c < JB; ++c) {
 #pragma unroll
-        for (int q = 0; q < S; ++q) {
+        for (int q = 0; q < RPT; ++q) {
             // unconditional load from a clamped row, then the select: no
             // branch, so every load of the panel is in flight at once
-            const int r = tid + PT * q;
+            const int r = tid + T * q;
             const double x = col[ld * c + (r < m ? r : m - 1)];
-            const double v = r < m ? x : 0.0;
-            if (q < RPT) a[q < RPT ? q : 0][c] = v;
-            else Lrows[((q - RPT) * JB + c) * PT + tid] = v;
+            a[q][c] = r < m ? x : 0.0;
         }
         __builtin_amdgcn_sched_barrier(0);   // one column's addresses live at a time
     }
     __syncthreads();   // moved = 0 visible
-    WideCtx<JB> P{cand, rec, cinv, Lrows, ipiv, info, list, tid, tid & 63, tid >> 6, k0, m};
-    wide_column<JB, RPT, RL, 0>(a, pos, P);
+    WideCtx<JB, W> P{cand, rec, cinv, ipiv, info, tid, tid & 63, tid >> 6, k0, m};
+    wide_column<JB, W, RPT, 0>(a, pos, P);
 #pragma unroll
-    for (int q = 0; q < S; ++q) {
-        const int r = tid + PT * q;
+    for (int q = 0; q < RPT; ++q) {
+        const int r = tid + T * q;
         if (r < m && pos[q] != r) {
             const int e = atomicAdd(&moved, 1);
             if (e < LPAIRS) {
@@ -652,12 +571,106 @@ __global__ __launch_bounds__(PT) void lu_panel_wide_kernel(int n, double *A, int
 #pragma unroll
     for (int c = 0; c < JB; ++c) {
 #pragma unroll
-        for (int q = 0; q < S; ++q)
-            if (pos[q] < m)
-                out[ld * c + pos[q]] = q < RPT ? a[q < RPT ? q : 0][c]
-                                               : Lrows[((q - RPT) * JB + c) * PT + tid];
+        for (int q = 0; q < RPT; ++q)
+            if (pos[q] < m) out[ld * c + pos[q]] = a[q][c];
         __builtin_amdgcn_sched_barrier(0);
     }
+}
+
+// Panel of at most 64 rows held by one wave: lane l owns physical row l,
+// and no step leaves the wave: the pivot by a DPP maximum and ballots, its
+// row by readlane (scalar operands of the update), no LDS and no barrier.
+// The arithmetic per element is that of the panels above.  Bound by the
+// chain of one column; 18 us for 32 columns, where 2, 4 and 8 waves of the
+// panel above (one row per lane: 128, 256, 512 rows) take 24, 29 and 37 us
+// for their LDS round trips and barrier.  With two and three rows per lane
+// it took 38 and 53 us, so taller panels stay above.  Takes any width jb <=
+// NBMAX, so the last columns of a matrix need no other kernel.
+struct WaveCtx {
+    int *ipiv, *info;
+    int lane, k0, m, jb;
+};
+
+template <int C>
+__device__ __forceinline__ void wave_column(double (&a)[NBMAX], int &pos, const WaveCtx &P)
+{
+    if (C >= P.jb) return;
+    // candidates: rows at logical >= C; the row at C counts as zero if it
+    // holds a NaN, so that a column of zeros or NaNs pivots on its diagonal
+    const double x = fabs(a[C]);
+    const bool live = pos >= C && pos < P.m;
+    const bool cand = live && (x >= 0.0 || pos == C);
+    const double bv = x >= 0.0 ? x : 0.0;
+    const unsigned hi = cand ? (unsigned)__double2hiint(bv) : 0u;
+    const unsigned M = wave_umax(hi);
+    unsigned long long hit = __ballot(cand && hi == M);
+    if (__popcll(hit) != 1) {
+        const bool th = cand && hi == M;
+        const unsigned lo = th ? (unsigned)__double2loint(bv) : 0u;
+        const unsigned Ml = wave_umax(lo);
+        const bool top = th && lo == Ml;
+        const int r = wave_min(top ? pos : INT_MAX);
+        hit = __ballot(top && pos == r);
+    }
+    const int wl = __ffsll((long long)hit) - 1;
+    const int lp = __builtin_amdgcn_readlane(pos, wl);
+    double u[NBMAX];
+#pragma unroll
+    for (int j = C; j < NBMAX; ++j) u[j] = readlane_f64(a[j], wl);
+    const bool zero = u[C] == 0.0;
+    if (P.lane == 0) {
+        P.ipiv[P.k0 + C] = P.k0 + lp;
+        // a zero column (lp = C, no swap) is recorded and left as it is, as
+        // DGETF2 does; the factorisation reports it
+        if (zero && *P.info == 0) *P.info = P.k0 + C + 1;
+    }
+    const double inv = zero ? 0.0 : 1.0 / u[C];
+    pos = pos == lp ? C : (pos == C ? lp : pos);
+    const bool upd = pos > C && pos < P.m;
+    const double l = upd ? a[C] * inv : 0.0;
+    a[C] = upd ? l : a[C];
+#pragma unroll
+    for (int j = C + 1; j < NBMAX; ++j) a[j] -= l * u[j];
+    if constexpr (C + 1 < NBMAX) wave_column<C + 1>(a, pos, P);
+}
+
+__global__ __launch_bounds__(64, 1) void lu_panel_wave_kernel(int n, double *A, int *ipiv,
+                                                              int *info, int k0, int jb,
+                                                              int *list)
+{
+    const int lane = threadIdx.x;
+    const size_t ld = (size_t)n;
+    const int m = n - k0;
+    if (lane == 0) {
+        list[LK0] = k0;
+        list[LJB] = jb;
+    }
+    if (*info != 0) {
+        if (lane < jb) ipiv[k0 + lane] = k0 + lane;
+        if (lane == 0) list[0] = 0;
+        return;
+    }
+    double a[NBMAX];
+    int pos = lane;   // logical row; lanes past the panel stay out by pos >= m
+    double *col = A + ld * (size_t)k0 + k0;
+#pragma unroll
+    for (int c = 0; c < NBMAX; ++c) {
+        const double x = col[ld * (c < jb ? c : jb - 1) + (lane < m ? lane : m - 1)];
+        a[c] = (lane < m && c < jb) ? x : 0.0;
+    }
+    const WaveCtx P{ipiv, info, lane, k0, m, jb};
+    wave_column<0>(a, pos, P);
+#pragma unroll
+    for (int c = 0; c < NBMAX; ++c)
+        if (c < jb && pos < m) col[ld * c + pos] = a[c];
+    const bool mv = lane < m && pos != lane;
+    const unsigned long long b = __ballot(mv);
+    if (mv) {
+        const int e = __popcll(b & ((1ull << lane) - 1));
+        list[1 + 2 * e] = k0 + pos;    // destination (logical) row
+        list[2 + 2 * e] = k0 + lane;   // source (physical) row
+    }
+    if (lane == 0) list[0] = __popcll(b);
 }
 
 // Panel of the blocked path too tall to be held on chip (jb <= NB): one
@@ -933,20 +946,14 @@ namespace {
 int lu_launch(vlm_ctx *ctx, int n, double *A, int *ipiv, int *info_dev)
 {
     hipLaunchKernelGGL(zero_info_kernel, dim3(1), dim3(1), 0, ctx->stream, info_dev);
-    if (n <= LU_SMALL) {
-        hipLaunchKernelGGL(lu_panel_kernel, dim3(1), dim3(LU_THREADS), 0, ctx->stream, n, A,
-                           ipiv, info_dev, 0, n, 0, n);
-        VLM_HIP(hipGetLastError());
-        return VLM_OK;
-    }
     // panel schedule: 16 columns while the panel is taller than the
-    // 32-column on-chip panel, 32 after; a last panel of fewer than 32
-    // rows goes 16 columns at a time through the tall kernel
+    // 32-column on-chip panel, 32 after (fewer only for the last columns,
+    // whose panel one wave holds)
     std::vector<int> k0s;
     for (int k = 0; k < n;) {
         k0s.push_back(k);
         const int m = n - k;
-        k += m > WIDE_ROWS ? NB : (m >= NBMAX ? NBMAX : (m < NB ? m : NB));
+        k += m > WIDE_ROWS ? NB : (m >= NBMAX ? NBMAX : m);
     }
     const int npanels = (int)k0s.size();
     VLM_HIP(ctx->lu_work.reserve((size_t)npanels * LSTRIDE));
@@ -955,8 +962,8 @@ int lu_launch(vlm_ctx *ctx, int n, double *A, int *ipiv, int *info_dev)
         const int k = k0s[p], m = n - k;
         const int jb = (p + 1 < npanels ? k0s[p + 1] : n) - k;
         int *list = lists + (size_t)p * LSTRIDE;
-        const dim3 g1(1), bp(PT);
-        if (m > MID_ROWS || jb < NB || (m <= WIDE_ROWS && jb < NBMAX))
+        const dim3 g1(1), bp(PT), bw(64);
+        if (m > MID_ROWS)
             hipLaunchKernelGGL(lu_panel_tall_kernel, g1, dim3(LU_THREADS), 0, ctx->stream, n, A,
                                ipiv, info_dev, k, jb, list);
         else if (m > 4 * PT)
@@ -968,12 +975,21 @@ int lu_launch(vlm_ctx *ctx, int n, double *A, int *ipiv, int *info_dev)
         else if (m > WIDE_ROWS)
             hipLaunchKernelGGL((lu_panel_fast_kernel<NB, 3>), g1, bp, 0, ctx->stream, n, A,
                                ipiv, info_dev, k, list);
-        else if (m > PT)
-            hipLaunchKernelGGL((lu_panel_wide_kernel<NBMAX, 2, 0>), g1, bp, 0, ctx->stream, n,
-                               A, ipiv, info_dev, k, list);
+        else if (m > 512)
+            hipLaunchKernelGGL((lu_panel_wide_kernel<NBMAX, 8, 2>), g1, dim3(512), 0, ctx->stream,
+                               n, A, ipiv, info_dev, k, list);
+        else if (m > 256)
+            hipLaunchKernelGGL((lu_panel_wide_kernel<NBMAX, 8, 1>), g1, dim3(512), 0,
+                               ctx->stream, n, A, ipiv, info_dev, k, list);
+        else if (m > 128)
+            hipLaunchKernelGGL((lu_panel_wide_kernel<NBMAX, 4, 1>), g1, dim3(256), 0,
+                               ctx->stream, n, A, ipiv, info_dev, k, list);
+        else if (m > 64)
+            hipLaunchKernelGGL((lu_panel_wide_kernel<NBMAX, 2, 1>), g1, dim3(128), 0, ctx->stream,
+                               n, A, ipiv, info_dev, k, list);
         else
-            hipLaunchKernelGGL((lu_panel_wide_kernel<NBMAX, 1, 0>), g1, bp, 0, ctx->stream, n,
-                               A, ipiv, info_dev, k, list);
+            hipLaunchKernelGGL(lu_panel_wave_kernel, g1, bw, 0, ctx->stream, n, A, ipiv,
+                               info_dev, k, jb, list);
         const int rest = n - k - jb;
         if (rest > 0) {
             if (jb <= NB)
