@@ -456,18 +456,30 @@ __device__ __forceinline__ double wave_sum(double v)
     return v;
 }
 
+// Chunks of the lists of one launch: list k has chunks chunk0[k] to
+// chunk0[k + 1] - 1.
+struct TermTab {
+    int n, neg;   // neg: bit k set where the sum is negated before list k
+    int chunk0[TERM_MAX + 1];
+    int64_t off[TERM_MAX];
+};
+
 __global__ __launch_bounds__(SM_BLOCK) void bs_small_kernel(const double *s64, int64_t S,
-                                                            const long long *nseg_p, int nchunks,
+                                                            const long long *counts, TermTab tt,
                                                             const double *t, int64_t m,
                                                             int64_t tstride, double *part)
 {
     __shared__ double red[3 * SM_T][SM_BLOCK / 64];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int64_t nseg = *nseg_p;
+    int k = 0;
+    while (k + 1 < tt.n && (int)blockIdx.x >= tt.chunk0[k + 1]) ++k;
+    const int64_t nseg = counts[k];
+    const int nchunks = tt.chunk0[k + 1] - tt.chunk0[k];
     const int64_t len = (nseg + nchunks - 1) / nchunks;
-    const int64_t s0 = (int64_t)blockIdx.x * len;
+    const int64_t s0 = (int64_t)((int)blockIdx.x - tt.chunk0[k]) * len;
     const int64_t s1 = min(nseg, s0 + len);
     const int64_t g0 = (int64_t)blockIdx.y * SM_T;
+    s64 += tt.off[k];
     double px[SM_T], py[SM_T], pz[SM_T], vx[SM_T], vy[SM_T], vz[SM_T];
 #pragma unroll
     for (int q = 0; q < SM_T; ++q) {
@@ -504,6 +516,52 @@ __global__ __launch_bounds__(SM_BLOCK) void bs_small_kernel(const double *s64, i
             part[((size_t)blockIdx.x * 3 + d) * m + g0 + q] = v;
         }
     }
+}
+
+// Sum of the lists' chunk partials at one component of 64 targets, then the
+// term recurrence (TermLists): RT_S slices of a list's chunks side by side,
+// each in increasing order, the slices and then the lists added in order, so
+// that a list contributes the same bits however many share the launch.
+constexpr int RT_S = 8, RT_W = 16;
+
+__global__ __launch_bounds__(64 * RT_W) void bs_reduce_terms_kernel(const double *part,
+                                                                    TermTab tt, int64_t m,
+                                                                    double *out, int64_t ostride,
+                                                                    int acc)
+{
+    __shared__ double sh[TERM_MAX * RT_S][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int64_t t = (int64_t)blockIdx.x * 64 + l;
+    const int d = blockIdx.y;
+    const size_t cs = 3 * (size_t)m;
+    for (int u = w; u < tt.n * RT_S; u += RT_W) {
+        const int k = u / RT_S, q = u % RT_S;
+        const int nc = tt.chunk0[k + 1] - tt.chunk0[k], len = (nc + RT_S - 1) / RT_S;
+        const int c1 = min(nc, (q + 1) * len);
+        double s = 0.0;
+        if (t < m) {
+            const double *p = part + (size_t)tt.chunk0[k] * cs + (size_t)d * m + t;
+            int c = q * len;
+            for (; c + 8 <= c1; c += 8) {
+                double v[8];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = p[(size_t)(c + i) * cs];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) s += v[i];
+            }
+            for (; c < c1; ++c) s += p[(size_t)c * cs];
+        }
+        sh[u][l] = s;
+    }
+    __syncthreads();
+    if (w > 0 || t >= m) return;
+    double v = acc ? out[d * ostride + t] : 0.0;
+    for (int k = 0; k < tt.n; ++k) {
+        double s = sh[k * RT_S][l];
+        for (int q = 1; q < RT_S; ++q) s += sh[k * RT_S + q][l];
+        v = (tt.neg >> k & 1 ? -v : v) + s;
+    }
+    out[d * ostride + t] = v;
 }
 
 // Fixed-order sum of the per-chunk partials: T targets of one component per
@@ -609,6 +667,49 @@ int bs_formats(const vlm_ctx *ctx, int64_t m)
     return ctx->precision == VLM_MIXED && m >= MIXED_MIN ? SEG_REC | SEG_F32 : SEG_REC;
 }
 
+int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, const double *t,
+                  int64_t m, int64_t tstride, double *out, int accumulate, const BsWork *ws)
+{
+    if (m <= 0) return VLM_OK;
+    if (terms.n < 1 || terms.n > TERM_MAX) return fail(ctx, VLM_ERR_ARG, "bad term count");
+    const int64_t max_chunks = ws ? (int64_t)(ws->part_cap / (3 * (size_t)m)) : INT32_MAX;
+    if (max_chunks < terms.n) return fail(ctx, VLM_ERR_ARG, "workspace too small for the targets");
+    // per list about 2048 blocks of at least 8 segments per lane; short
+    // lists are split down to 2 per lane, up to 16 chunks (their loads wait
+    // on each other; more chunks only feed the reduction)
+    const int64_t groups = (m + SM_T - 1) / SM_T;
+    TermTab tt;
+    tt.n = terms.n;
+    tt.neg = 0;
+    tt.chunk0[0] = 0;
+    for (int k = 0; k < terms.n; ++k) {
+        int64_t nc = (2048 + groups - 1) / groups;
+        const int64_t c2 = terms.est[k] / (2 * SM_BLOCK), c8 = terms.est[k] / (8 * SM_BLOCK);
+        const int64_t maxc = c8 > 16 ? c8 : (c2 > 16 ? 16 : c2);
+        if (nc > maxc) nc = maxc;
+        if (nc > max_chunks / terms.n) nc = max_chunks / terms.n;
+        if (nc < 1) nc = 1;
+        tt.chunk0[k + 1] = tt.chunk0[k] + (int)nc;
+        tt.off[k] = terms.off[k];
+        if (terms.neg[k]) tt.neg |= 1 << k;
+    }
+    const int nchunks = tt.chunk0[tt.n];
+    double *part = ws ? ws->part : nullptr;
+    if (!ws) {
+        VLM_HIP(ctx->part.reserve((size_t)nchunks * 3 * (size_t)m));
+        part = ctx->part.p;
+    }
+    hipLaunchKernelGGL(bs_small_kernel, dim3(nchunks, (unsigned)groups), dim3(SM_BLOCK), 0,
+                       ctx->stream, seg.soa, seg.cap, seg.count, tt, t, m, tstride, part);
+    hipLaunchKernelGGL(bs_reduce_terms_kernel, dim3((unsigned)((m + 63) / 64), 3),
+                       dim3(64 * RT_W), 0, ctx->stream, part, tt, m, out, tstride, accumulate);
+    VLM_HIP(hipGetLastError());
+    if (ctx->profile && !ws)
+        for (int k = 0; k < terms.n; ++k)
+            VLM_TRY(profile_count(ctx, seg.count + k, m, 1, nullptr));
+    return VLM_OK;
+}
+
 int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t, int64_t m,
             int64_t tstride, double *out, int accumulate, const BsWork *ws)
 {
@@ -624,28 +725,12 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
         ((fmt & SEG_F32) && !seg.rec32))
         return fail(ctx, VLM_ERR_STATE, "segment list lacks the records of this launch");
     if (fmt == SEG_SOA) {
-        // about 2048 blocks of at least 8 segments per lane; short lists are
-        // split down to 2 per lane, up to 16 chunks (their loads wait on
-        // each other; more chunks only feed the reduction)
-        const int64_t groups = (m + SM_T - 1) / SM_T;
-        int64_t nc = (2048 + groups - 1) / groups;
-        const int64_t c2 = nseg_est / (2 * SM_BLOCK), c8 = nseg_est / (8 * SM_BLOCK);
-        const int64_t maxc = c8 > 16 ? c8 : (c2 > 16 ? 16 : c2);
-        if (nc > maxc) nc = maxc;
-        if (nc > max_chunks) nc = max_chunks;
-        if (nc < 1) nc = 1;
-        const int nchunks = (int)nc;
-        double *part = ws ? ws->part : nullptr;
-        if (!ws) {
-            VLM_HIP(ctx->part.reserve((size_t)nchunks * 3 * (size_t)m));
-            part = ctx->part.p;
-        }
-        hipLaunchKernelGGL(bs_small_kernel, dim3(nchunks, (unsigned)groups), dim3(SM_BLOCK), 0,
-                           ctx->stream, seg.soa, seg.cap, seg.count, nchunks, t, m, tstride,
-                           part);
-        VLM_HIP(hipGetLastError());
-        if (prof) VLM_TRY(profile_count(ctx, seg.count, m, 1, nullptr));
-        return launch_reduce(ctx, part, nchunks, m, out, tstride, accumulate, nullptr);
+        TermLists one;
+        one.n = 1;
+        one.off[0] = 0;
+        one.est[0] = nseg_est;
+        one.neg[0] = 0;
+        return bs_eval_terms(ctx, seg, one, t, m, tstride, out, accumulate, ws);
     }
     const bool mixed = (fmt & SEG_F32) != 0;
     const int tile = mixed ? 64 * MIXED_NT : 64;

@@ -79,7 +79,7 @@ struct SegList {
     hipError_t reserve(int64_t n, int formats, SegPtrs *out)
     {
         const size_t k = (size_t)((n + GRP - 1) / GRP) * GRP;
-        hipError_t e = count.reserve(1);
+        hipError_t e = count.reserve(16);
         if (e == hipSuccess && (formats & SEG_SOA)) e = soa.reserve(k * SOA_N);
         if (e == hipSuccess && (formats & SEG_REC)) e = rec64.reserve(k * REC64_N);
         if (e == hipSuccess && (formats & SEG_REC)) e = grp.reserve(k / GRP * GRPH_N);
@@ -378,6 +378,21 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
             int64_t tstride, double *out, int accumulate, const BsWork *ws = nullptr);
 // The list formats that a launch with m targets reads.
 int bs_formats(const vlm_ctx *ctx, int64_t m);
+
+// Few targets (bs_formats(m) == SEG_SOA), up to TERM_MAX lists in one
+// structure of arrays: list k starts at segment off[k] and has seg.count[k]
+// segments (about est[k]).
+//   u = accumulate ? out : 0;  for k: u = (neg[k] ? -u : u) + velocity of k;
+//   out = u
+constexpr int TERM_MAX = 16;
+struct TermLists {
+    int n = 0;
+    int64_t off[TERM_MAX], est[TERM_MAX];
+    int neg[TERM_MAX];
+};
+int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, const double *t,
+                  int64_t m, int64_t tstride, double *out, int accumulate,
+                  const BsWork *ws = nullptr);
 
 // Records of an explicit list (every filament kept, at its own index) from
 // 3 x n device arrays, and its count.

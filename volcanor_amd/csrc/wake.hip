@@ -149,7 +149,8 @@ struct SrcDesc {
     // wing: wc wrc wg; wake: node le gam rc4 ffc fgam frc; prescribed: pf ps
     const double *p[7];
     int kind, nc, ns, nN, nF, head, rn, rf, far_exists;
-    int64_t first, per_blade;  // first item in the launch; items per blade (wake)
+    int64_t first, count;      // its items, among those of the launch
+    int64_t per_blade;         // items per blade (wake)
 };
 
 constexpr int SRC_MAX = 20;            // descriptors per launch (kernel argument space)
@@ -269,7 +270,9 @@ __global__ __launch_bounds__(256) void stage_kernel(StageArgs a)
             while (q + 1 < a.n && e >= a.d[q + 1].first) ++q;
             const SrcDesc &d = a.d[q];
             const int64_t k = e - d.first;
-            if (d.kind == SRC_WAKE) {
+            if (k >= d.count) {
+                // between the last set of a list and the next list's block
+            } else if (d.kind == SRC_WAKE) {
                 wake_edge(d, k, s, f);
             } else if (d.kind == SRC_PRESC) {
                 const int b = (int)(k / PF_N);
@@ -306,14 +309,27 @@ __global__ __launch_bounds__(256) void stage_kernel(StageArgs a)
 }
 
 // The staged segments in order, as records: each block forms the prefix sum
-// of the staging blocks' counts, and each lane finds the block its record
-// comes from by bisection.
+// of its list's staging counts, and each lane finds the block its record
+// comes from by bisection.  List t was staged in blocks sb[t] to sb[t+1]-1,
+// is emitted by the blocks from eb[t] and starts at record off[t].
+struct EmitTab {
+    int n, stride;
+    int sb[TERM_MAX + 1], eb[TERM_MAX + 1];
+    int64_t off[TERM_MAX];
+};
+
 __global__ __launch_bounds__(256) void emit_records_kernel(const Slot *slots, const int *counts,
-                                                           int nblocks, int stride, SegPtrs L)
+                                                           EmitTab tab, SegPtrs L)
 {
     __shared__ int pre[STAGE_BLOCKS + 1];
     __shared__ int wsum[4];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    int t = 0;
+    while (t + 1 < tab.n && (int)blockIdx.x >= tab.eb[t + 1]) ++t;
+    const int blk = (int)blockIdx.x - tab.eb[t];
+    const int nblocks = tab.sb[t + 1] - tab.sb[t];
+    counts += tab.sb[t];
+    slots += (size_t)tab.sb[t] * tab.stride;
     const int per = (nblocks + 255) / 256;
     int mine = 0;
     for (int q = 0; q < per; ++q) {
@@ -339,9 +355,9 @@ __global__ __launch_bounds__(256) void emit_records_kernel(const Slot *slots, co
             excl += counts[b];
         }
     }
-    if (blockIdx.x == 0 && tid == 0) *L.count = total;
+    if (blk == 0 && tid == 0) L.count[t] = total;
     __syncthreads();
-    const int k = blockIdx.x * 256 + tid;
+    const int k = blk * 256 + tid;
     if ((k & ~(GRP - 1)) >= total) return;   // whole groups leave together
     const bool valid = k < total;
     const int kk = valid ? k : total - 1;
@@ -351,8 +367,8 @@ __global__ __launch_bounds__(256) void emit_records_kernel(const Slot *slots, co
         if (pre[mid] <= kk) lo = mid;
         else hi = mid;
     }
-    const Slot s = slots[(size_t)lo * stride + (kk - pre[lo])];
-    write_group_records(s, valid, k, L);
+    const Slot s = slots[(size_t)lo * tab.stride + (kk - pre[lo])];
+    write_group_records(s, valid, tab.off[t] + k, L);
 }
 
 // pFwake_update (classdef.f90:998-1066) for blade blockIdx.x of wake type
@@ -1135,6 +1151,7 @@ void source_descs(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src,
             d.p[1] = r.wrc.p;
             d.p[2] = r.wg.p;
             const int64_t items = (int64_t)r.nring * (d.kind == SRC_WING ? 2 : 1);
+            d.count = items;
             n += items;
             wing += items;
             ds.push_back(d);
@@ -1159,7 +1176,8 @@ void source_descs(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src,
         d.rf = r.rowFar - 1;
         d.far_exists = r.rowFar <= r.d.nFwake ? 1 : 0;
         d.per_blade = per;
-        n += per * r.d.nb;
+        d.count = per * r.d.nb;
+        n += d.count;
         ds.push_back(d);
         const int64_t np = presc_slots(r);
         if (np > 0) {
@@ -1168,6 +1186,7 @@ void source_descs(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src,
             d.p[0] = r.pf[pred].p;
             d.p[1] = r.ps[pred].p;
             d.first = n;
+            d.count = np;
             n += np;
             ds.push_back(d);
         }
@@ -1176,46 +1195,85 @@ void source_descs(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src,
     *est = n + wing;
 }
 
-// Build the source list of (rotor, set) pairs into ctx->seg, in the given
-// formats; *est receives the expected number of segments.
-int build_sources(vlm_ctx *ctx, const std::vector<std::pair<int, int>> &src, int formats,
-                  int64_t *est)
+typedef std::vector<std::pair<int, int>> Sources;   // (rotor, set) pairs
+
+// Build up to TERM_MAX source lists into ctx->seg, in the given formats:
+// where each starts and its expected number of segments go to *lists (empty
+// sets give lists of no segments).
+int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, TermLists *lists)
 {
-    std::vector<SrcDesc> ds;
-    int64_t total = 0;
-    source_descs(ctx, src, ds, &total, est);
-    if (total == 0) return VLM_OK;
-    const int nlaunch = ((int)ds.size() + SRC_MAX - 1) / SRC_MAX;
+    const int nt = (int)terms.size();
+    std::vector<std::vector<SrcDesc>> ds(nt);
+    std::vector<int64_t> total(nt);
+    int64_t all = 0, nd = 0, cap = 0;
+    lists->n = nt;
+    for (int t = 0; t < nt; ++t) {
+        source_descs(ctx, terms[t], ds[t], &total[t], &lists->est[t]);
+        lists->off[t] = cap;
+        cap += (2 * total[t] + GRP - 1) / GRP * GRP;
+        all += total[t];
+        nd += (int64_t)ds[t].size();
+    }
+    if (all > INT32_MAX / 4) return fail(ctx, VLM_ERR_ARG, "segment list too large");
+    // items per staging block; a list starts on a block of its own, and a
+    // launch (SRC_MAX sets) ends with one
+    const int64_t spare = nt + nd / SRC_MAX + 1;
     StageArgs a;
-    a.iters = (int)((total + (int64_t)256 * (STAGE_BLOCKS - nlaunch) - 1) /
-                    ((int64_t)256 * (STAGE_BLOCKS - nlaunch)));
-    const int64_t nb_max = (total + 256 * (int64_t)a.iters - 1) / (256 * (int64_t)a.iters) + nlaunch;
-    if (total > INT32_MAX / 4) return fail(ctx, VLM_ERR_ARG, "segment list too large");
-    VLM_HIP(ctx->slots.reserve((size_t)nb_max * a.iters * 512));
+    a.iters = (int)((all + 256 * (STAGE_BLOCKS - spare) - 1) / (256 * (STAGE_BLOCKS - spare)));
+    if (a.iters < 1) a.iters = 1;
+    const int64_t bi = 256 * (int64_t)a.iters;   // items per block
+    VLM_HIP(ctx->slots.reserve((size_t)(all / bi + spare + 1) * a.iters * 512));
     VLM_HIP(ctx->seg_counts.reserve(STAGE_BLOCKS));
-    VLM_HIP(ctx->seg.reserve(2 * total, formats, &ctx->seg_view));
+    VLM_HIP(ctx->seg.reserve(cap, formats, &ctx->seg_view));
     a.slots = ctx->slots.p;
     a.counts = ctx->seg_counts.p;
+    a.n = 0;
+    a.block0 = 0;
+    a.total = 0;
     int blocks = 0;
-    for (int l = 0; l < nlaunch; ++l) {
-        const int k0 = l * SRC_MAX, k1 = std::min((int)ds.size(), k0 + SRC_MAX);
-        const int64_t first = ds[k0].first;
-        const int64_t end = k1 < (int)ds.size() ? ds[k1].first : total;
-        a.n = k1 - k0;
-        for (int k = k0; k < k1; ++k) {
-            a.d[k - k0] = ds[k];
-            a.d[k - k0].first -= first;
-        }
+    auto flush = [&]() {
+        const int nb = (int)((a.total + bi - 1) / bi);
+        if (nb > 0)
+            hipLaunchKernelGGL(stage_kernel, dim3(nb), dim3(256), 0, ctx->stream, a);
+        blocks = a.block0 + nb;
         a.block0 = blocks;
-        a.total = end - first;
-        const int nb = (int)((a.total + 256 * (int64_t)a.iters - 1) / (256 * (int64_t)a.iters));
-        if (nb == 0) continue;
-        hipLaunchKernelGGL(stage_kernel, dim3(nb), dim3(256), 0, ctx->stream, a);
-        blocks += nb;
+        a.n = 0;
+        a.total = 0;
+    };
+    EmitTab tab;
+    tab.n = nt;
+    tab.stride = a.iters * 512;
+    int eb = 0;
+    for (int t = 0; t < nt; ++t) {
+        a.total = (a.total + bi - 1) / bi * bi;
+        tab.sb[t] = a.block0 + (int)(a.total / bi);
+        tab.eb[t] = eb;
+        tab.off[t] = lists->off[t];
+        for (auto &d : ds[t]) {
+            if (a.n == SRC_MAX) flush();
+            a.d[a.n] = d;
+            a.d[a.n++].first = a.total;
+            a.total += d.count;
+        }
+        // at least one block writes the count
+        eb += (int)std::max<int64_t>(1, (2 * total[t] + 255) / 256);
     }
-    hipLaunchKernelGGL(emit_records_kernel, dim3(nblk(2 * total)), dim3(256), 0, ctx->stream,
-                       ctx->slots.p, ctx->seg_counts.p, blocks, a.iters * 512, ctx->seg_view);
+    a.total = (a.total + bi - 1) / bi * bi;
+    tab.sb[nt] = a.block0 + (int)(a.total / bi);
+    flush();
+    tab.eb[nt] = eb;
+    hipLaunchKernelGGL(emit_records_kernel, dim3(eb), dim3(256), 0, ctx->stream, ctx->slots.p,
+                       ctx->seg_counts.p, tab, ctx->seg_view);
     VLM_HIP(hipGetLastError());
+    return VLM_OK;
+}
+
+// One list; *est receives its expected number of segments.
+int build_sources(vlm_ctx *ctx, const Sources &src, int formats, int64_t *est)
+{
+    TermLists one;
+    VLM_TRY(build_lists(ctx, {src}, formats, &one));
+    *est = one.est[0];
     return VLM_OK;
 }
 
@@ -1408,7 +1466,7 @@ int rotor_convect(vlm_ctx *ctx, Rotor &r, double dt, int pred)
 
 int wake_pass(vlm_ctx *ctx, int pred)
 {
-    std::vector<std::pair<int, int>> src;
+    Sources src;
     int64_t m = 0;
     for (int ir = 0; ir < (int)ctx->rotors.size(); ++ir) {
         src.push_back({ir, VLM_SET_WING});
@@ -1693,7 +1751,7 @@ static int full_pass(vlm_ctx *ctx, int64_t m, int64_t nest)
 int learned_pass(vlm_ctx *ctx)
 {
     Predictor &P = ctx->pred;
-    std::vector<std::pair<int, int>> src;
+    Sources src;
     int64_t m = 0;
     for (int ir = 0; ir < (int)ctx->rotors.size(); ++ir) {
         src.push_back({ir, VLM_SET_WING});
@@ -2217,7 +2275,7 @@ int vlm_rotor_induced_velocity(vlm_ctx *ctx, int ir, int set, int64_t m, const d
     if (set < VLM_SET_WING || set > VLM_SET_WAKE_PRED) return fail(ctx, VLM_ERR_ARG, "bad set");
     if (m <= 0) return VLM_OK;
     if (!p || !v) return fail(ctx, VLM_ERR_ARG, "null buffer");
-    std::vector<std::pair<int, int>> src = {{ir, set}};
+    Sources src = {{ir, set}};
     int64_t nest = 0;
     VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
     VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
@@ -2226,6 +2284,46 @@ int vlm_rotor_induced_velocity(vlm_ctx *ctx, int ir, int set, int64_t m, const d
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
     VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, accumulate, nest));
     return points_to_host(ctx, m, ctx->out.p, m, v);
+}
+
+// The ordered term sum at m device targets (SoA, stride m) into out: with
+// few targets TERM_MAX lists share four launches, otherwise each list gets
+// its own.  A list of a few thousand segments is about 5 us per launch
+// whatever the launch does: a step of four rotors, 32 lists of right-hand
+// sides and 20 of loads, took 6194 us with four launches per list and takes
+// 5370 us.  With many targets the pairs of one list fill the chip.
+static int ordered_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set,
+                         const int *flags, int64_t m, const double *tgt, double *out,
+                         int accumulate)
+{
+    const int fmt = bs_formats(ctx, m);
+    if (nterms == 0 && !accumulate) {
+        hipLaunchKernelGGL(fill_kernel, dim3(nblk(3 * m)), dim3(256), 0, ctx->stream, out, 3 * m,
+                           0.0);
+        VLM_HIP(hipGetLastError());
+    }
+    int acc = accumulate;
+    for (int k = 0; k < nterms;) {
+        const int n = fmt == SEG_SOA ? std::min(TERM_MAX, nterms - k) : 1;
+        std::vector<Sources> src;
+        TermLists lists;
+        for (int q = 0; q < n; ++q) src.push_back({{ir[k + q], set[k + q]}});
+        VLM_TRY(build_lists(ctx, src, fmt, &lists));
+        for (int q = 0; q < n; ++q) lists.neg[q] = (flags[k + q] & VLM_TERM_NEGATE) != 0;
+        if (fmt == SEG_SOA) {
+            VLM_TRY(bs_eval_terms(ctx, ctx->seg_view, lists, tgt, m, m, out, acc));
+        } else {
+            if (lists.neg[0] && acc) {
+                hipLaunchKernelGGL(negate_kernel, dim3(nblk(3 * m)), dim3(256), 0, ctx->stream,
+                                   out, 3 * m);
+                VLM_HIP(hipGetLastError());
+            }
+            VLM_TRY(bs_eval(ctx, ctx->seg_view, lists.est[0], tgt, m, m, out, acc));
+        }
+        acc = 1;
+        k += n;
+    }
+    return VLM_OK;
 }
 
 static int induced_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set,
@@ -2246,24 +2344,8 @@ static int induced_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set
     VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
     VLM_HIP(ctx->out.reserve((size_t)3 * m));
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
-    if (accumulate) {
-        VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
-    } else {
-        hipLaunchKernelGGL(fill_kernel, dim3(nblk(3 * m)), dim3(256), 0, ctx->stream,
-                           ctx->out.p, 3 * m, 0.0);
-        VLM_HIP(hipGetLastError());
-    }
-    for (int k = 0; k < nterms; ++k) {
-        if (flags[k] & VLM_TERM_NEGATE) {
-            hipLaunchKernelGGL(negate_kernel, dim3(nblk(3 * m)), dim3(256), 0, ctx->stream,
-                               ctx->out.p, 3 * m);
-            VLM_HIP(hipGetLastError());
-        }
-        std::vector<std::pair<int, int>> src = {{ir[k], set[k]}};
-        int64_t nest = 0;
-        VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
-        VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 1, nest));
-    }
+    if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
+    VLM_TRY(ordered_terms(ctx, nterms, ir, set, flags, m, ctx->tgt.p, ctx->out.p, accumulate));
     return points_to_host(ctx, m, ctx->out.p, m, v, deferred);
 }
 
@@ -2281,21 +2363,7 @@ int vlm::induced_terms_soa(vlm_ctx *ctx, int nterms, const int *ir, const int *s
             return fail(ctx, VLM_ERR_ARG, "bad set");
     }
     if (m <= 0) return VLM_OK;
-    hipLaunchKernelGGL(fill_kernel, dim3(nblk(3 * m)), dim3(256), 0, ctx->stream, out, 3 * m,
-                       0.0);
-    VLM_HIP(hipGetLastError());
-    for (int k = 0; k < nterms; ++k) {
-        if (flags[k] & VLM_TERM_NEGATE) {
-            hipLaunchKernelGGL(negate_kernel, dim3(nblk(3 * m)), dim3(256), 0, ctx->stream, out,
-                               3 * m);
-            VLM_HIP(hipGetLastError());
-        }
-        std::vector<std::pair<int, int>> src = {{ir[k], set[k]}};
-        int64_t nest = 0;
-        VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
-        VLM_TRY(eval_sources(ctx, tgt, m, m, out, 1, nest));
-    }
-    return VLM_OK;
+    return ordered_terms(ctx, nterms, ir, set, flags, m, tgt, out, 0);
 }
 
 vlm::Rotor *vlm::rotor_of(vlm_ctx *ctx, int ir) { return get_rotor(ctx, ir); }
