@@ -156,13 +156,51 @@ struct SrcDesc {
 constexpr int SRC_MAX = 20;            // descriptors per launch (kernel argument space)
 constexpr int STAGE_BLOCKS = 4096;     // staging blocks of one list
 
+// The N-body targets of a rotor, written as SoA by blocks of their own in the
+// staging launch: near-wake nodes of rows rn..nN-1 then far trailing ends,
+// for its nbc convected blades.
+struct TgtDesc {
+    const double *node, *ffc;
+    int ns, nN, nF, head, rn, rf, nbc;
+    int block0;                // first target block of the launch
+    int64_t off;               // of its targets
+};
+
+constexpr int TGT_MAX = 12;
+
 struct StageArgs {
     SrcDesc d[SRC_MAX];
-    int n, iters, block0;
-    int64_t total;
+    TgtDesc t[TGT_MAX];
+    int n, nt, iters, block0, tblock0;
+    int64_t total, tstride;
     Slot *slots;
     int *counts;
+    double *tgt;
 };
+static_assert(sizeof(StageArgs) <= 4096, "kernel argument space");
+
+__device__ void gather_target(const TgtDesc &d, int64_t e, double *t, int64_t stride)
+{
+    const int R = d.nN - d.rn, F = max(d.nF - d.rf, 0), cols = d.ns + 1;
+    const int64_t nnear = (int64_t)R * cols, per = nnear + F;
+    if (e >= per * d.nbc) return;
+    const int b = (int)(e / per);
+    const int64_t k = e - b * per;
+    const double *P;
+    if (k < nnear) {
+        int i, j;
+        patch_entry(k, R, cols, &i, &j);
+        int p = d.head + d.rn + i;
+        if (p >= d.nN) p -= d.nN;
+        P = d.node + 3 * (((size_t)b * d.nN + p) * cols + j);
+    } else {
+        P = d.ffc + 6 * ((size_t)b * d.nF + d.rf + (k - nnear));
+    }
+    t += d.off + e;
+    t[0] = P[0];
+    t[stride] = P[1];
+    t[2 * stride] = P[2];
+}
 
 // Near- and far-wake unique segments of every blade.  Edge enumeration per
 // blade (R active rows, F active far filaments; rows and columns in patch
@@ -258,6 +296,13 @@ __global__ __launch_bounds__(256) void stage_kernel(StageArgs a)
 {
     __shared__ int wsum[4];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if ((int)blockIdx.x >= a.tblock0) {
+        const int tb = (int)blockIdx.x - a.tblock0;
+        int q = 0;
+        while (q + 1 < a.nt && tb >= a.t[q + 1].block0) ++q;
+        gather_target(a.t[q], (int64_t)(tb - a.t[q].block0) * 256 + tid, a.tgt, a.tstride);
+        return;
+    }
     const int blk = a.block0 + blockIdx.x;
     Slot *dst = a.slots + (size_t)blk * a.iters * 512;
     int run = 0;
@@ -433,96 +478,190 @@ __global__ __launch_bounds__(256) void presc_update_kernel(RV v, int pred, int s
     }
 }
 
-// Targets: near-wake nodes of rows rn..nN-1 then far trailing ends, for
-// blades < nbConvect, written as SoA at t[off..].
-__global__ void gather_targets_kernel(RV v, int pred, double *t, int64_t stride, int64_t off)
+// Everything a velocity pass leads to, per lattice node and far filament and
+// for all rotors of the launch: the pass's velocity (SoA, target order) into
+// its array, the initial wake velocity, the predicted wake as a copy of the
+// current one (main.f90:1028-1035), the scheme algebra and the convection.
+// Bound by launches (about 5 us each): these were six to ten kernels per
+// rotor and pass, each of a few kB to a few MB.
+//
+// Scheme algebra over whole velocity arrays of the convected blades, rows
+// outside the wake included, as the reference has it (main.f90:968-1404):
+// v = velNwake, v1..v3 = velNwake1..3, p = velNwakePredicted,
+// s = velNwakeStep; statements after the bar follow the convection.
+enum AdvOp {
+    ADV_NONE,
+    ADV_AB2,         // s = (3 v - v1) / 2; v1 = s; v = s
+    ADV_AM2_PRED,    // s = v; v = (3 v - v1) / 2
+    ADV_AM2_CORR,    // v = (p + s) / 2                           | v1 = s
+    ADV_AM3_PRED,    // 1160-1171
+    ADV_AM3_CORR,    // 1219-1235                                 | v1 = v2; v2 = s
+    ADV_AM4_PRED,    // 1307-1320
+    ADV_AM4_CORR,    // 1365-1385                                 | v1 = v2; v2 = v3; v3 = s
+    ADV_KEEP1, ADV_KEEP2, ADV_KEEP3   //                          | v1, v2 or v3 = v
+};
+
+struct AdvRotor {
+    double *node, *pnode, *le, *ple, *ffc, *pffc, *vel[NVEL], *velF[NVEL];
+    double un[3], uf[3];             // initial wake velocity, near and far
+    int ns, nN, nF, nbc, head, rn, rf;
+    int i0, i1;                      // near rows convected
+    int scatter, init, copy;
+    int block0;                      // first block of the launch
+    int64_t off;                     // of its targets
+};
+
+constexpr int ADV_MAX = 12;
+
+struct AdvArgs {
+    AdvRotor r[ADV_MAX];
+    int n, slot, op, convect;        // slot: VLM_VEL or VLM_VEL_PRED;
+                                     // convect: -1 none, 0 current, 1 predicted wake
+    double dt;
+    const double *o;
+    int64_t stride;
+};
+static_assert(sizeof(AdvArgs) <= 4096, "kernel argument space");
+
+// Nodes, far filaments and (copy) shed line points per blade.
+__host__ __device__ __forceinline__ int64_t adv_per(const AdvRotor &r)
 {
-    const int R = v.nN - v.rn, F = v.nF - v.rf;
-    const int64_t per = (int64_t)R * (v.ns + 1) + F;
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= per * v.nbc) return;
-    const int b = (int)(e / per);
-    const int64_t k = e - b * per;
-    const double *P;
-    if (k < (int64_t)R * (v.ns + 1)) {
-        int i, j;
-        patch_entry(k, R, v.ns + 1, &i, &j);
-        i += v.rn;
-        P = (pred ? v.pnode : v.node) + 3 * nidx(v, b, phys(v, i), j);
-    } else {
-        const int i = v.rf + (int)(k - (int64_t)R * (v.ns + 1));
-        P = (pred ? v.pffc : v.ffc) + 6 * ((size_t)b * v.nF + i);
-    }
-    t[off + e] = P[0];
-    t[stride + off + e] = P[1];
-    t[2 * stride + off + e] = P[2];
+    return (int64_t)r.nN * (r.ns + 1) + r.nF + (r.copy ? r.ns + 1 : 0);
 }
 
-__global__ void scatter_vel_kernel(RV v, int which, const double *o, int64_t stride, int64_t off)
+__global__ __launch_bounds__(256) void advance_kernel(AdvArgs a)
 {
-    const int R = v.nN - v.rn, F = v.nF - v.rf;
-    const int64_t per = (int64_t)R * (v.ns + 1) + F;
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= per * v.nbc) return;
+    int q = 0;
+    while (q + 1 < a.n && (int)blockIdx.x >= a.r[q + 1].block0) ++q;
+    const AdvRotor &r = a.r[q];
+    const int64_t e = (int64_t)((int)blockIdx.x - r.block0) * 256 + threadIdx.x;
+    const int64_t per = adv_per(r);
+    if (e >= per * r.nbc) return;
     const int b = (int)(e / per);
-    const int64_t k = e - b * per;
-    double *dst;
-    if (k < (int64_t)R * (v.ns + 1)) {
-        int i, j;
-        patch_entry(k, R, v.ns + 1, &i, &j);
-        i += v.rn;
-        dst = v.vel[which] + 3 * vidx(v, b, i, j);
+    int64_t k = e - b * per;
+    // per blade: the targets in their order, the rows and filaments outside
+    // the wake, the shed line
+    const int cols = r.ns + 1, R = max(r.nN - r.rn, 0), F = max(r.nF - r.rf, 0);
+    const int64_t nnear = (int64_t)R * cols, nwin = nnear + F;
+    const int64_t nout = (int64_t)(r.nN - R) * cols;
+    const bool win = k < nwin;
+    bool near;
+    int i, j = 0;
+    if (win) {
+        near = k < nnear;
+        if (near) {
+            patch_entry(k, R, cols, &i, &j);
+            i += r.rn;
+        } else {
+            i = r.rf + (int)(k - nnear);
+        }
+    } else if (k - nwin < nout) {
+        near = true;
+        i = (int)((k - nwin) / cols);
+        j = (int)((k - nwin) % cols);
+    } else if (k - nwin - nout < r.nF - F) {
+        near = false;
+        i = (int)(k - nwin - nout);
     } else {
-        const int i = v.rf + (int)(k - (int64_t)R * (v.ns + 1));
-        dst = v.velF[which] + 3 * ((size_t)b * v.nF + i);
+        const size_t n = 3 * ((size_t)b * cols + (k - nwin - nout - (r.nF - F)));
+        for (int d = 0; d < 3; ++d) r.ple[n + d] = r.le[n + d];
+        return;
     }
-    dst[0] = o[off + e];
-    dst[1] = o[stride + off + e];
-    dst[2] = o[2 * stride + off + e];
-}
-
-// blade_convectwake (classdef.f90:1515-1575): nodes of logical rows
-// [i0, i1) move by velNwake*dt; far trailing ends of rows rf.. move by
-// velFwake*dt.  Both 'C' and 'P' use velNwake, as the reference does.
-__global__ void convect_kernel(RV v, int pred, int i0, int i1, double dt)
-{
-    const int rows = i1 - i0;
-    const int64_t nnear = (int64_t)rows * (v.ns + 1);
-    const int F = v.nF - v.rf;
-    const int64_t per = nnear + F;
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= per * v.nbc) return;
-    const int b = (int)(e / per);
-    const int64_t k = e - b * per;
-    if (k < nnear) {
-        const int i = i0 + (int)(k / (v.ns + 1)), j = (int)(k % (v.ns + 1));
-        double *P = (pred ? v.pnode : v.node) + 3 * nidx(v, b, phys(v, i), j);
-        const double *V = v.vel[VLM_VEL] + 3 * vidx(v, b, i, j);
-        P[0] += V[0] * dt;
-        P[1] += V[1] * dt;
-        P[2] += V[2] * dt;
-    } else {
-        const int i = v.rf + (int)(k - nnear);
-        double *P = (pred ? v.pffc : v.ffc) + 6 * ((size_t)b * v.nF + i);
-        const double *V = v.velF[VLM_VEL] + 3 * ((size_t)b * v.nF + i);
-        P[0] += V[0] * dt;
-        P[1] += V[1] * dt;
-        P[2] += V[2] * dt;
+    const size_t iv = near ? ((size_t)b * r.nN + i) * cols + j : (size_t)b * r.nF + i;
+    auto arr = [&](int s) { return (near ? r.vel[s] : r.velF[s]) + 3 * iv; };
+    double *V = arr(VLM_VEL), *X = arr(a.slot);
+    double x[3], v[3];
+    for (int d = 0; d < 3; ++d) {
+        x[d] = win && r.scatter ? a.o[d * a.stride + r.off + b * nwin + k] : X[d];
+        if (win && r.init) x[d] += near ? r.un[d] : r.uf[d];
+        if (win && (r.scatter || r.init)) X[d] = x[d];
+        v[d] = x[d];   // with slot VLM_VEL
     }
-}
-
-// Far-wake continuity: fc2(i) <- fc1(i-1) for i = rf+1 .. nF-1.
-__global__ void far_continuity_kernel(RV v, int pred)
-{
-    const int F = v.nF - v.rf - 1;
-    const int e = blockIdx.x * blockDim.x + threadIdx.x;
-    if (F <= 0 || e >= F * v.nbc) return;
-    const int b = e / F, i = v.rf + 1 + e % F;
-    double *FC = pred ? v.pffc : v.ffc;
-    const size_t q = (size_t)b * v.nF + i;
-    FC[6 * q + 3] = FC[6 * (q - 1) + 0];
-    FC[6 * q + 4] = FC[6 * (q - 1) + 1];
-    FC[6 * q + 5] = FC[6 * (q - 1) + 2];
+    if (a.op == ADV_NONE && a.convect < 0) return;
+    double *V1 = arr(VLM_VEL_PREV), *V2 = arr(VEL_H2), *V3 = arr(VEL_H3), *S = arr(VLM_VEL_STEP);
+    for (int d = 0; d < 3; ++d) {
+        switch (a.op) {
+        case ADV_AB2: {
+            const double s = 0.5 * (3.0 * v[d] - V1[d]);
+            S[d] = s;
+            V1[d] = s;
+            v[d] = s;
+            break;
+        }
+        case ADV_AM2_PRED:
+            S[d] = v[d];
+            v[d] = 0.5 * (3.0 * v[d] - V1[d]);
+            break;
+        case ADV_AM3_PRED:
+            S[d] = v[d];
+            v[d] = (23.0 * v[d] - 16.0 * V2[d] + 5.0 * V1[d]) / 12.0;
+            break;
+        case ADV_AM4_PRED:
+            S[d] = v[d];
+            v[d] = (55.0 * v[d] - 59.0 * V3[d] + 37.0 * V2[d] - 9.0 * V1[d]) / 24.0;
+            break;
+        case ADV_AM2_CORR: {
+            const double s = S[d];
+            v[d] = (x[d] + s) * 0.5;
+            V1[d] = s;
+            break;
+        }
+        case ADV_AM3_CORR: {
+            const double s = S[d], v2 = V2[d];
+            v[d] = (5.0 * x[d] + 8.0 * s - v2) / 12.0;
+            V1[d] = v2;
+            V2[d] = s;
+            break;
+        }
+        case ADV_AM4_CORR: {
+            const double s = S[d], v2 = V2[d], v3 = V3[d];
+            v[d] = (9.0 * x[d] + 19.0 * s - 5.0 * v3 + v2) / 24.0;
+            V1[d] = v2;
+            V2[d] = v3;
+            V3[d] = s;
+            break;
+        }
+        case ADV_KEEP1:
+            V1[d] = v[d];
+            break;
+        case ADV_KEEP2:
+            V2[d] = v[d];
+            break;
+        case ADV_KEEP3:
+            V3[d] = v[d];
+            break;
+        default:
+            break;
+        }
+        if (a.op >= ADV_AB2 && a.op <= ADV_AM4_CORR) V[d] = v[d];
+    }
+    if (a.convect < 0) return;
+    // blade_convectwake (classdef.f90:1515-1575): nodes of rows [i0, i1) and
+    // far trailing ends move by v dt; both wakes use velNwake, as the
+    // reference does.  Far-wake continuity: fc2(i+1) <- fc1(i).
+    const bool copied = win && r.copy;
+    if (near) {
+        const bool moves = i >= r.i0 && i < r.i1;
+        if (!moves && !copied) return;
+        int p = r.head + i;
+        if (p >= r.nN) p -= r.nN;
+        const size_t n = 3 * (((size_t)b * r.nN + p) * cols + j);
+        double *P = (a.convect ? r.pnode : r.node) + n;
+        const double *B = copied ? r.node + n : P;
+        for (int d = 0; d < 3; ++d) {
+            const double p0 = B[d];
+            P[d] = moves ? p0 + v[d] * a.dt : p0;
+        }
+    } else if (win) {
+        double *P = (a.convect ? r.pffc : r.ffc) + 6 * iv;
+        const double *B = copied ? r.ffc + 6 * iv : P;
+        for (int d = 0; d < 3; ++d) {
+            const double p1 = B[d] + v[d] * a.dt;
+            P[d] = p1;
+            if (i + 1 < r.nF) P[9 + d] = p1;
+            if (copied && i == r.rf) P[3 + d] = B[3 + d];
+        }
+    }
 }
 
 struct RotMats {
@@ -848,137 +987,6 @@ __global__ void shift_copy_kernel(RV v)
     }
 }
 
-// Predicted wake := current wake on the active rows (main.f90:1028-1035).
-__global__ void copy_pred_kernel(RV v)
-{
-    const int R = v.nN - v.rn, F = v.nF - v.rf;
-    const int64_t per = (int64_t)R * (v.ns + 1) + (v.ns + 1) + F;
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= per * v.nbc) return;
-    const int b = (int)(e / per);
-    int64_t k = e - b * per;
-    if (k < (int64_t)R * (v.ns + 1)) {
-        const int i = v.rn + (int)(k / (v.ns + 1)), j = (int)(k % (v.ns + 1));
-        const size_t n = 3 * nidx(v, b, phys(v, i), j);
-        v.pnode[n] = v.node[n];
-        v.pnode[n + 1] = v.node[n + 1];
-        v.pnode[n + 2] = v.node[n + 2];
-        return;
-    }
-    k -= (int64_t)R * (v.ns + 1);
-    if (k < v.ns + 1) {
-        const size_t n = 3 * ((size_t)b * (v.ns + 1) + k);
-        v.ple[n] = v.le[n];
-        v.ple[n + 1] = v.le[n + 1];
-        v.ple[n + 2] = v.le[n + 2];
-        return;
-    }
-    k -= v.ns + 1;
-    const size_t q = 6 * ((size_t)b * v.nF + v.rf + k);
-    for (int d = 0; d < 6; ++d) v.pffc[q + d] = v.ffc[q + d];
-}
-
-// Scheme algebra over whole velocity arrays of blades < nbConvect, as the
-// reference applies it to whole arrays (main.f90:968-1115).
-//   op 0: AB2  step = 1.5 v - 0.5 v1; v1 = step; v = step
-//   op 1: AM2 predictor  step = v; v = 0.5 (3 v - v1)
-//   op 2: AM2 corrector  v = (pred + step) * 0.5
-//   op 3: history        v1 = step
-//   op 4: first step     v1 = v
-__global__ void scheme_kernel(double *v, double *v1, double *vp, double *vs, int64_t n, int op)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    switch (op) {
-    case 0: {
-        const double s = 0.5 * (3.0 * v[k] - v1[k]);
-        vs[k] = s;
-        v1[k] = s;
-        v[k] = s;
-        break;
-    }
-    case 1:
-        vs[k] = v[k];
-        v[k] = 0.5 * (3.0 * v[k] - v1[k]);
-        break;
-    case 2:
-        v[k] = (vp[k] + vs[k]) * 0.5;
-        break;
-    case 3:
-        v1[k] = vs[k];
-        break;
-    default:
-        v1[k] = v[k];
-        break;
-    }
-}
-
-// AM3 and AM4 velocity algebra (main.f90:1117-1404) on whole logical-row
-// arrays: v = velNwake, v1..v3 = velNwake1..3, vp = velNwakePredicted,
-// vs = velNwakeStep.
-enum AmOp {
-    AM3_PRED, AM3_CORR, AM3_ROTATE,  // 1160-1171, 1219-1235
-    AM4_PRED, AM4_CORR, AM4_ROTATE,  // 1307-1320, 1365-1385
-    AM_START1, AM_START2, AM_START3  // start-up copies v1|v2|v3 = v
-};
-
-__global__ void am_kernel(double *v, double *v1, double *v2, double *v3, const double *vp,
-                          double *vs, int64_t n, int op)
-{
-    const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    switch (op) {
-    case AM3_PRED:
-        vs[k] = v[k];
-        v[k] = (23.0 * v[k] - 16.0 * v2[k] + 5.0 * v1[k]) / 12.0;
-        break;
-    case AM3_CORR:
-        v[k] = (5.0 * vp[k] + 8.0 * vs[k] - v2[k]) / 12.0;
-        break;
-    case AM3_ROTATE:
-        v1[k] = v2[k];
-        v2[k] = vs[k];
-        break;
-    case AM4_PRED:
-        vs[k] = v[k];
-        v[k] = (55.0 * v[k] - 59.0 * v3[k] + 37.0 * v2[k] - 9.0 * v1[k]) / 24.0;
-        break;
-    case AM4_CORR:
-        v[k] = (9.0 * vp[k] + 19.0 * vs[k] - 5.0 * v3[k] + v2[k]) / 24.0;
-        break;
-    case AM4_ROTATE:
-        v1[k] = v2[k];
-        v2[k] = v3[k];
-        v3[k] = vs[k];
-        break;
-    case AM_START1:
-        v1[k] = v[k];
-        break;
-    case AM_START2:
-        v2[k] = v[k];
-        break;
-    default:
-        v3[k] = v[k];
-        break;
-    }
-}
-
-// vel(:, row0:nrows-1, :) += a for blades 0..nbc-1 of a logical-row
-// velocity array (cols = ns+1 for the near wake, 1 for the far wake).
-__global__ void add_uniform_kernel(double *vel, int nbc, int nrows, int cols, int row0,
-                                   double ax, double ay, double az)
-{
-    const int64_t per = (int64_t)(nrows - row0) * cols;
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= per * nbc) return;
-    const int b = (int)(e / per);
-    const int64_t k = e - b * per;
-    double *V = vel + 3 * (((size_t)b * nrows + row0) * cols + k);
-    V[0] += ax;
-    V[1] += ay;
-    V[2] += az;
-}
-
 // vel_order2_Nwake / vel_order2_Fwake (libCommon.f90:213-258) on the
 // active window, written to `out` (logical rows).
 __global__ void order2_kernel(const double *vn, const double *vnp1, double *out, int nbc,
@@ -1200,7 +1208,10 @@ typedef std::vector<std::pair<int, int>> Sources;   // (rotor, set) pairs
 // Build up to TERM_MAX source lists into ctx->seg, in the given formats:
 // where each starts and its expected number of segments go to *lists (empty
 // sets give lists of no segments).
-int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, TermLists *lists)
+// With pred >= 0 the staging launches also gather the N-body targets on the
+// current (0) or predicted (1) wake, m in total, into ctx->tgt.
+int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, TermLists *lists,
+                int pred = -1, int64_t m = 0)
 {
     const int nt = (int)terms.size();
     std::vector<std::vector<SrcDesc>> ds(nt);
@@ -1228,18 +1239,46 @@ int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, Te
     a.slots = ctx->slots.p;
     a.counts = ctx->seg_counts.p;
     a.n = 0;
+    a.nt = 0;
     a.block0 = 0;
     a.total = 0;
-    int blocks = 0;
+    int tblocks = 0;
     auto flush = [&]() {
         const int nb = (int)((a.total + bi - 1) / bi);
-        if (nb > 0)
-            hipLaunchKernelGGL(stage_kernel, dim3(nb), dim3(256), 0, ctx->stream, a);
-        blocks = a.block0 + nb;
-        a.block0 = blocks;
+        a.tblock0 = nb;
+        if (nb + tblocks > 0)
+            hipLaunchKernelGGL(stage_kernel, dim3(nb + tblocks), dim3(256), 0, ctx->stream, a);
+        a.block0 += nb;
         a.n = 0;
+        a.nt = 0;
         a.total = 0;
+        tblocks = 0;
     };
+    if (pred >= 0) {
+        VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
+        a.tgt = ctx->tgt.p;
+        a.tstride = m;
+        int64_t off = 0;
+        for (auto *r : ctx->rotors) {
+            const int64_t n = target_count(*r);
+            if (n == 0) continue;
+            if (a.nt == TGT_MAX) flush();
+            TgtDesc &d = a.t[a.nt++];
+            d.node = pred ? r->pnode.p : r->node.p;
+            d.ffc = pred ? r->pffc.p : r->ffc.p;
+            d.ns = r->d.ns;
+            d.nN = r->d.nNwake;
+            d.nF = r->d.nFwake;
+            d.head = r->head;
+            d.rn = r->rowNear - 1;
+            d.rf = r->rowFar - 1;
+            d.nbc = r->d.nbConvect;
+            d.block0 = tblocks;
+            d.off = off;
+            tblocks += (int)nblk(n);
+            off += n;
+        }
+    }
     EmitTab tab;
     tab.n = nt;
     tab.stride = a.iters * 512;
@@ -1269,10 +1308,11 @@ int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, Te
 }
 
 // One list; *est receives its expected number of segments.
-int build_sources(vlm_ctx *ctx, const Sources &src, int formats, int64_t *est)
+int build_sources(vlm_ctx *ctx, const Sources &src, int formats, int64_t *est, int pred = -1,
+                  int64_t m = 0)
 {
     TermLists one;
-    VLM_TRY(build_lists(ctx, {src}, formats, &one));
+    VLM_TRY(build_lists(ctx, {src}, formats, &one, pred, m));
     *est = one.est[0];
     return VLM_OK;
 }
@@ -1281,66 +1321,6 @@ int eval_sources(vlm_ctx *ctx, const double *t, int64_t m, int64_t tstride, doub
                  int64_t est)
 {
     return bs_eval(ctx, ctx->seg_view, est, t, m, tstride, out, acc);
-}
-
-int launch_scheme(vlm_ctx *ctx, Rotor &r, int op)
-{
-    const int64_t nn = (int64_t)3 * r.d.nbConvect * r.d.nNwake * (r.d.ns + 1);
-    const int64_t nf = (int64_t)3 * r.d.nbConvect * r.d.nFwake;
-    if (nn > 0)
-        hipLaunchKernelGGL(scheme_kernel, dim3(nblk(nn)), dim3(256), 0, ctx->stream,
-                           r.velN[VLM_VEL].p, r.velN[VLM_VEL_PREV].p, r.velN[VLM_VEL_PRED].p,
-                           r.velN[VLM_VEL_STEP].p, nn, op);
-    if (nf > 0)
-        hipLaunchKernelGGL(scheme_kernel, dim3(nblk(nf)), dim3(256), 0, ctx->stream,
-                           r.velF[VLM_VEL].p, r.velF[VLM_VEL_PREV].p, r.velF[VLM_VEL_PRED].p,
-                           r.velF[VLM_VEL_STEP].p, nf, op);
-    VLM_HIP(hipGetLastError());
-    return VLM_OK;
-}
-
-int launch_am(vlm_ctx *ctx, Rotor &r, int op)
-{
-    const int64_t nn = (int64_t)3 * r.d.nbConvect * r.d.nNwake * (r.d.ns + 1);
-    const int64_t nf = (int64_t)3 * r.d.nbConvect * r.d.nFwake;
-    if (nn > 0)
-        hipLaunchKernelGGL(am_kernel, dim3(nblk(nn)), dim3(256), 0, ctx->stream,
-                           r.velN[VLM_VEL].p, r.velN[VLM_VEL_PREV].p, r.velN[VEL_H2].p,
-                           r.velN[VEL_H3].p, r.velN[VLM_VEL_PRED].p, r.velN[VLM_VEL_STEP].p, nn,
-                           op);
-    if (nf > 0)
-        hipLaunchKernelGGL(am_kernel, dim3(nblk(nf)), dim3(256), 0, ctx->stream,
-                           r.velF[VLM_VEL].p, r.velF[VLM_VEL_PREV].p, r.velF[VEL_H2].p,
-                           r.velF[VEL_H3].p, r.velF[VLM_VEL_PRED].p, r.velF[VLM_VEL_STEP].p, nf,
-                           op);
-    VLM_HIP(hipGetLastError());
-    return VLM_OK;
-}
-
-// initWakeVel of pass 1 (main.f90:829-838: + near, - far) or of pass 2
-// (902-913 and the AM blocks: - near, - far) on the active windows.
-int add_init_wake_vel(vlm_ctx *ctx, Rotor &r, int iter, bool pass2)
-{
-    if (iter >= r.init_wake_vel_nt || r.init_wake_vel == 0.0) return VLM_OK;
-    const int slot = pass2 ? VLM_VEL_PRED : VLM_VEL;
-    const double u = r.init_wake_vel;
-    const double sn = pass2 ? -1.0 : 1.0;
-    const int nbc = r.d.nbConvect;
-    const int rn = r.rowNear - 1, rf = r.rowFar - 1;
-    if (r.d.nNwake > rn) {
-        const int64_t n = (int64_t)nbc * (r.d.nNwake - rn) * (r.d.ns + 1);
-        hipLaunchKernelGGL(add_uniform_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                           r.velN[slot].p, nbc, r.d.nNwake, r.d.ns + 1, rn, sn * u * r.shaft[0],
-                           sn * u * r.shaft[1], sn * u * r.shaft[2]);
-    }
-    if (r.d.nFwake > rf) {
-        const int64_t n = (int64_t)nbc * (r.d.nFwake - rf);
-        hipLaunchKernelGGL(add_uniform_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                           r.velF[slot].p, nbc, r.d.nFwake, 1, rf, -u * r.shaft[0],
-                           -u * r.shaft[1], -u * r.shaft[2]);
-    }
-    VLM_HIP(hipGetLastError());
-    return VLM_OK;
 }
 
 // getTransformAxis, libMath.f90:695-726 (column-major)
@@ -1358,18 +1338,6 @@ void transform_axis(double theta, const double *ax, double *T)
     T[6] = a1 * st + a0 * a2 * om;
     T[7] = -a0 * st + a1 * a2 * om;
     T[8] = ct + a2 * a2 * om;
-}
-
-int copy_predicted(vlm_ctx *ctx, Rotor &r)
-{
-    const int64_t R = r.d.nNwake - (r.rowNear - 1);
-    const int64_t F = r.d.nFwake - (r.rowFar - 1);
-    const int64_t per = R * (r.d.ns + 1) + (r.d.ns + 1) + (F > 0 ? F : 0);
-    const int64_t n = per * r.d.nbConvect;
-    if (R <= 0 || n <= 0) return VLM_OK;
-    hipLaunchKernelGGL(copy_pred_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream, view(r));
-    VLM_HIP(hipGetLastError());
-    return VLM_OK;
 }
 
 }  // namespace
@@ -1420,30 +1388,10 @@ int mirror_wake(vlm_ctx *ctx, Rotor &r, int mode)
     return VLM_OK;
 }
 
-int rotor_convect(vlm_ctx *ctx, Rotor &r, double dt, int pred)
+// What follows the convection of a rotor of its own: the axisymmetric copy
+// of blade 1's wake and the prescribed far wake (classdef.f90:4826-4829).
+static int after_convect(vlm_ctx *ctx, Rotor &r, int pred)
 {
-    // an image's convection is the mirror of its source's wake
-    if (r.image_of >= 0) return mirror_wake(ctx, r, pred ? 1 : 0);
-    if (r.d.nNwake <= 0) return VLM_OK;
-    RV v = view(r);
-    int i0 = r.rowNear - 1, i1 = r.d.nNwake;
-    if (pred && ctx->bug_compat) {
-        i0 = 0;  // `do i = 1, rowNear, nNwake` runs for row 1 only
-        i1 = 1;
-    }
-    if (i0 >= r.d.nNwake) i1 = i0;  // nothing shed yet
-    const int64_t F = r.d.nFwake - (r.rowFar - 1);
-    const int64_t per = (int64_t)(i1 - i0) * (r.d.ns + 1) + (F > 0 ? F : 0);
-    if (per > 0) {
-        hipLaunchKernelGGL(convect_kernel, dim3(nblk(per * r.d.nbConvect)), dim3(256), 0,
-                           ctx->stream, v, pred, i0, i1, dt);
-        VLM_HIP(hipGetLastError());
-    }
-    if (F > 1) {
-        hipLaunchKernelGGL(far_continuity_kernel, dim3(nblk((F - 1) * r.d.nbConvect)), dim3(256),
-                           0, ctx->stream, v, pred);
-        VLM_HIP(hipGetLastError());
-    }
     if (r.d.nbConvect == 1 && r.d.nb > 1) {
         if (r.d.nb > 16) return fail(ctx, VLM_ERR_ARG, "axisymmetric copy supports <= 16 blades");
         RotMats M;
@@ -1452,19 +1400,109 @@ int rotor_convect(vlm_ctx *ctx, Rotor &r, double dt, int pred)
             const double theta = 2.0 * kPi / r.d.nb * b;
             transform_axis(theta, r.shaft, M.T[b]);
         }
-        const int64_t R = r.d.nNwake - (r.rowNear - 1);
+        const int64_t R = r.d.nNwake - (r.rowNear - 1), F = r.d.nFwake - (r.rowFar - 1);
         const int64_t per2 = (R > 0 ? R : 0) * (r.d.ns + 1) + (r.d.ns + 1) + (F > 0 ? F : 0) +
                              (R > 0 ? R : 0) * r.d.ns;
         hipLaunchKernelGGL(axisym_kernel, dim3(nblk(per2 * (r.d.nb - 1))), dim3(256), 0,
-                           ctx->stream, v, pred, M, r.hub[0], r.hub[1], r.hub[2]);
+                           ctx->stream, view(r), pred, M, r.hub[0], r.hub[1], r.hub[2]);
         VLM_HIP(hipGetLastError());
     }
-    // the prescribed far wake after the convection (classdef.f90:4826-4829)
     if (r.presc_nt > 0 && r.iter > r.presc_nt) VLM_TRY(presc_update(ctx, r, pred));
     return VLM_OK;
 }
 
-int wake_pass(vlm_ctx *ctx, int pred)
+// One advance of every rotor, or of rotor `only`.
+struct Advance {
+    int slot = VLM_VEL, op = ADV_NONE, convect = -1;
+    bool scatter = false;   // ctx->out holds the pass's velocities, m targets
+    bool init = false;      // add the initial wake velocity of step iter
+    bool copy = false;      // predicted wake := current wake before it moves
+    double dt = 0.0;
+    int iter = 0;
+    int64_t m = 0;
+    const Rotor *only = nullptr;
+};
+
+static int advance(vlm_ctx *ctx, const Advance &p)
+{
+    AdvArgs a;
+    a.n = 0;
+    a.slot = p.slot;
+    a.op = p.op;
+    a.convect = p.convect;
+    a.dt = p.dt;
+    a.o = ctx->out.p;
+    a.stride = p.m;
+    int blocks = 0;
+    Rotor *batch[ADV_MAX];
+    auto flush = [&]() -> int {
+        if (blocks > 0)
+            hipLaunchKernelGGL(advance_kernel, dim3(blocks), dim3(256), 0, ctx->stream, a);
+        VLM_HIP(hipGetLastError());
+        if (p.convect >= 0)
+            for (int q = 0; q < a.n; ++q) VLM_TRY(after_convect(ctx, *batch[q], p.convect));
+        a.n = 0;
+        blocks = 0;
+        return VLM_OK;
+    };
+    int64_t off = 0;
+    for (auto *r : ctx->rotors) {
+        const int64_t nt = p.scatter ? target_count(*r) : 0, toff = off;
+        off += nt;
+        if ((p.only && r != p.only) || r->d.nNwake <= 0) continue;
+        if (r->image_of >= 0) {
+            // an image mirrors its source's wake at its place in the order
+            if (p.convect < 0) continue;
+            VLM_TRY(flush());
+            VLM_TRY(mirror_wake(ctx, *r, p.convect));
+            continue;
+        }
+        if (a.n == ADV_MAX) VLM_TRY(flush());
+        batch[a.n] = r;
+        AdvRotor &d = a.r[a.n++];
+        d.node = r->node.p;
+        d.pnode = r->pnode.p;
+        d.le = r->le.p;
+        d.ple = r->ple.p;
+        d.ffc = r->ffc.p;
+        d.pffc = r->pffc.p;
+        for (int k = 0; k < NVEL; ++k) {
+            d.vel[k] = r->velN[k].p;
+            d.velF[k] = r->velF[k].p;
+        }
+        // initWakeVel of pass 1 (main.f90:829-838: + near, - far) or of pass
+        // 2 (902-913 and the AM blocks: - near, - far)
+        const double u = r->init_wake_vel, un = p.slot == VLM_VEL ? u : -u;
+        d.init = p.init && p.iter < r->init_wake_vel_nt && u != 0.0;
+        for (int k = 0; k < 3; ++k) {
+            d.un[k] = un * r->shaft[k];
+            d.uf[k] = -u * r->shaft[k];
+        }
+        d.ns = r->d.ns;
+        d.nN = r->d.nNwake;
+        d.nF = r->d.nFwake;
+        d.nbc = r->d.nbConvect;
+        d.head = r->head;
+        d.rn = r->rowNear - 1;
+        d.rf = r->rowFar - 1;
+        d.i0 = d.rn;
+        d.i1 = d.nN;
+        if (p.convect == 1 && ctx->bug_compat) {
+            d.i0 = 0;  // `do i = 1, rowNear, nNwake` runs for row 1 only
+            d.i1 = 1;
+        }
+        d.scatter = nt > 0;
+        d.copy = p.copy && d.nN > d.rn;
+        d.block0 = blocks;
+        d.off = toff;
+        blocks += (int)nblk(adv_per(d) * d.nbc);
+    }
+    return flush();
+}
+
+// Velocities of all targets on the current or predicted wake into ctx->out;
+// *m receives their number.
+static int wake_pass(vlm_ctx *ctx, int pred, int64_t *mp)
 {
     Sources src;
     int64_t m = 0;
@@ -1473,31 +1511,12 @@ int wake_pass(vlm_ctx *ctx, int pred)
         src.push_back({ir, pred ? VLM_SET_WAKE_PRED : VLM_SET_WAKE});
         m += target_count(*ctx->rotors[ir]);
     }
+    *mp = m;
     if (m == 0) return VLM_OK;
     int64_t nest = 0;
-    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
-    VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
+    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest, pred, m));
     VLM_HIP(ctx->out.reserve((size_t)3 * m));
-    int64_t off = 0;
-    for (auto *rp : ctx->rotors) {
-        const int64_t n = target_count(*rp);
-        if (n == 0) continue;
-        hipLaunchKernelGGL(gather_targets_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                           view(*rp), pred, ctx->tgt.p, m, off);
-        VLM_HIP(hipGetLastError());
-        off += n;
-    }
-    VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 0, nest));
-    off = 0;
-    for (auto *rp : ctx->rotors) {
-        const int64_t n = target_count(*rp);
-        if (n == 0) continue;
-        hipLaunchKernelGGL(scatter_vel_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                           view(*rp), pred ? VLM_VEL_PRED : VLM_VEL, ctx->out.p, m, off);
-        VLM_HIP(hipGetLastError());
-        off += n;
-    }
-    return VLM_OK;
+    return eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 0, nest);
 }
 
 
@@ -1748,7 +1767,7 @@ static int full_pass(vlm_ctx *ctx, int64_t m, int64_t nest)
     return VLM_OK;
 }
 
-int learned_pass(vlm_ctx *ctx)
+int learned_pass(vlm_ctx *ctx, int64_t *mp)
 {
     Predictor &P = ctx->pred;
     Sources src;
@@ -1758,14 +1777,14 @@ int learned_pass(vlm_ctx *ctx)
         src.push_back({ir, VLM_SET_WAKE_PRED});
         m += target_count(*ctx->rotors[ir]);
     }
+    *mp = m;
     if (m == 0) return VLM_OK;
     int64_t nest = 0;
     // the full pass reads m targets, the judge about m / stride of them
     const int64_t stride0 = P.stride < 1 ? 1 : P.stride;
     int formats = bs_formats(ctx, m) | bs_formats(ctx, (m + stride0 - 1) / stride0) |
                   bs_formats(ctx, std::max<int64_t>(1, (m - stride0) / stride0));
-    VLM_TRY(build_sources(ctx, src, formats, &nest));
-    VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
+    VLM_TRY(build_sources(ctx, src, formats, &nest, 1, m));
     VLM_HIP(ctx->out.reserve((size_t)3 * m));
     VLM_HIP(P.vn.reserve((size_t)3 * m));
     VLM_HIP(P.X.reserve((size_t)45 * m));
@@ -1780,8 +1799,6 @@ int learned_pass(vlm_ctx *ctx)
     for (auto *rp : ctx->rotors) {
         const int64_t n = target_count(*rp);
         if (n == 0) continue;
-        hipLaunchKernelGGL(gather_targets_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                           view(*rp), 1, ctx->tgt.p, m, off);
         hipLaunchKernelGGL(gather_step_vel_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
                            view(*rp), P.vn.p, m, off);
         off += n;
@@ -1872,15 +1889,6 @@ int learned_pass(vlm_ctx *ctx)
             P.learned += 1;
         }
     }
-    off = 0;
-    for (auto *rp : ctx->rotors) {
-        const int64_t n = target_count(*rp);
-        if (n == 0) continue;
-        hipLaunchKernelGGL(scatter_vel_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                           view(*rp), VLM_VEL_PRED, ctx->out.p, m, off);
-        off += n;
-    }
-    VLM_HIP(hipGetLastError());
     return VLM_OK;
 }
 
@@ -2263,7 +2271,11 @@ int vlm_rotor_convectwake(vlm_ctx *ctx, int ir, double dt, int wakeType)
     VLM_DEVICE(ctx);
     if (wakeType != VLM_WAKE_C && wakeType != VLM_WAKE_P)
         return fail(ctx, VLM_ERR_ARG, "wakeType must be VLM_WAKE_C or VLM_WAKE_P");
-    return rotor_convect(ctx, *r, dt, wakeType == VLM_WAKE_P);
+    Advance p;
+    p.convect = wakeType == VLM_WAKE_P;
+    p.dt = dt;
+    p.only = r;
+    return advance(ctx, p);
 }
 
 int vlm_rotor_induced_velocity(vlm_ctx *ctx, int ir, int set, int64_t m, const double *p,
@@ -2390,7 +2402,11 @@ int vlm_wake_velocity(vlm_ctx *ctx, int wakeType)
     VLM_DEVICE(ctx);
     if (wakeType != VLM_WAKE_C && wakeType != VLM_WAKE_P)
         return fail(ctx, VLM_ERR_ARG, "wakeType must be VLM_WAKE_C or VLM_WAKE_P");
-    return wake_pass(ctx, wakeType == VLM_WAKE_P);
+    Advance p;
+    VLM_TRY(wake_pass(ctx, wakeType == VLM_WAKE_P, &p.m));
+    p.slot = wakeType == VLM_WAKE_P ? VLM_VEL_PRED : VLM_VEL;
+    p.scatter = true;
+    return advance(ctx, p);
 }
 
 int vlm_convect(vlm_ctx *ctx, int scheme, int iter, double dt)
@@ -2399,144 +2415,75 @@ int vlm_convect(vlm_ctx *ctx, int scheme, int iter, double dt)
     VLM_DEVICE(ctx);
     if (scheme < VLM_SCHEME_FT1 || scheme > VLM_SCHEME_AM4)
         return fail(ctx, VLM_ERR_ARG, "fdScheme must be 0..5");
-    VLM_TRY(wake_pass(ctx, 0));
-    // lifting rotors convect; an image mirrors its source's wake at the
-    // same place in the rotor order (rotor_convect does the mirror), and
-    // takes no part in the velocity algebra
-    auto active = [](Rotor *r) { return r->d.nNwake > 0 && r->image_of < 0; };
-    auto image = [](Rotor *r) { return r->d.nNwake > 0 && r->image_of >= 0; };
-    auto init_vel = [&](bool pass2) -> int {
-        for (auto *r : ctx->rotors)
-            if (active(r)) VLM_TRY(add_init_wake_vel(ctx, *r, iter, pass2));
-        return VLM_OK;
-    };
-    VLM_TRY(init_vel(false));
-    if (scheme == VLM_SCHEME_AM3 || scheme == VLM_SCHEME_AM4) {
-        // start-up steps convect with pass 1 and keep it as history.  AM3's
-        // first start-up branch tests iter == 0, which the time loop never
-        // reaches (main.f90:1118), so its step 1 runs the full scheme on the
-        // zero-initialised histories.
-        const bool am3 = scheme == VLM_SCHEME_AM3;
-        int start = -1;
-        if (am3 && iter == 2) start = AM_START2;
-        if (!am3 && iter >= 1 && iter <= 3) start = AM_START1 + (iter - 1);
-        if (start >= 0) {
-            for (auto *r : ctx->rotors)
-                if (active(r)) {
-                    VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-                    VLM_TRY(launch_am(ctx, *r, start));
-                } else if (image(r)) {
-                    VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-                }
-            return VLM_OK;
+    Advance p1, p2;
+    VLM_TRY(wake_pass(ctx, 0, &p1.m));
+    p1.scatter = p1.init = true;
+    p1.iter = iter;
+    p1.dt = dt;
+    p1.convect = 0;
+    // pass 1 alone: explicit schemes and start-up steps, which convect with
+    // pass 1 and keep it as history.  AM3's first start-up branch tests
+    // iter == 0, which the time loop never reaches (main.f90:1118), so its
+    // step 1 runs the full scheme on the zero-initialised histories.
+    bool start = true;
+    if (scheme == VLM_SCHEME_AM3 && iter == 2) p1.op = ADV_KEEP2;
+    else if (scheme == VLM_SCHEME_AM4 && iter >= 1 && iter <= 3) p1.op = ADV_KEEP1 + (iter - 1);
+    else if ((scheme == VLM_SCHEME_AB2 || scheme == VLM_SCHEME_AM2) && iter == 1) p1.op = ADV_KEEP1;
+    else if (scheme == VLM_SCHEME_AB2) p1.op = ADV_AB2;
+    else start = scheme == VLM_SCHEME_FT1;
+    if (start) return advance(ctx, p1);
+    // predictor, then pass 2 on the predicted wake and the corrector
+    p1.convect = 1;
+    p1.copy = true;
+    if (scheme == VLM_SCHEME_AM2) p1.op = ADV_AM2_PRED;
+    if (scheme == VLM_SCHEME_AM3) p1.op = ADV_AM3_PRED;
+    if (scheme == VLM_SCHEME_AM4) p1.op = ADV_AM4_PRED;
+    VLM_TRY(advance(ctx, p1));
+    if (scheme == VLM_SCHEME_AM2 && ctx->pred.mode == 1) VLM_TRY(learned_pass(ctx, &p2.m));
+    else VLM_TRY(wake_pass(ctx, 1, &p2.m));
+    p2.slot = VLM_VEL_PRED;
+    p2.scatter = p2.init = true;
+    p2.iter = iter;
+    p2.dt = dt;
+    p2.convect = 0;
+    if (scheme == VLM_SCHEME_AM2) p2.op = ADV_AM2_CORR;
+    if (scheme == VLM_SCHEME_AM3) p2.op = ADV_AM3_CORR;
+    if (scheme == VLM_SCHEME_AM4) p2.op = ADV_AM4_CORR;
+    if (scheme != VLM_SCHEME_PC2) return advance(ctx, p2);
+    // PC2 averages the two passes over neighbouring rows before it convects
+    p2.convect = -1;
+    VLM_TRY(advance(ctx, p2));
+    for (auto *r : ctx->rotors) {
+        if (r->d.nNwake <= 0 || r->image_of >= 0) continue;
+        const int rows = r->d.nNwake - (r->rowNear - 1);
+        const int frows = r->d.nFwake - (r->rowFar - 1);
+        const int nbc = r->d.nbConvect;
+        if (rows > 0) {
+            const int64_t n = (int64_t)nbc * rows * (r->d.ns + 1) * 3;
+            hipLaunchKernelGGL(order2_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
+                               r->velN[VLM_VEL].p, r->velN[VLM_VEL_PRED].p,
+                               r->velN[VLM_VEL_STEP].p, nbc, rows, r->d.nNwake, r->d.ns + 1,
+                               r->rowNear - 1);
+            hipLaunchKernelGGL(copy_window_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
+                               r->velN[VLM_VEL_STEP].p, r->velN[VLM_VEL].p, nbc, rows,
+                               r->d.nNwake, r->d.ns + 1, r->rowNear - 1);
         }
-        for (auto *r : ctx->rotors)
-            if (active(r)) {
-                VLM_TRY(copy_predicted(ctx, *r));
-                VLM_TRY(launch_am(ctx, *r, am3 ? AM3_PRED : AM4_PRED));
-                VLM_TRY(rotor_convect(ctx, *r, dt, 1));
-            } else if (image(r)) {
-                VLM_TRY(rotor_convect(ctx, *r, dt, 1));
-            }
-        VLM_TRY(wake_pass(ctx, 1));
-        VLM_TRY(init_vel(true));
-        for (auto *r : ctx->rotors)
-            if (active(r)) {
-                VLM_TRY(launch_am(ctx, *r, am3 ? AM3_CORR : AM4_CORR));
-                VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-                VLM_TRY(launch_am(ctx, *r, am3 ? AM3_ROTATE : AM4_ROTATE));
-            } else if (image(r)) {
-                VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-            }
-        return VLM_OK;
-    }
-    if (scheme == VLM_SCHEME_FT1) {
-        for (auto *r : ctx->rotors)
-            if (active(r) || image(r)) VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-        return VLM_OK;
-    }
-    if (scheme == VLM_SCHEME_PC2) {
-        for (auto *r : ctx->rotors)
-            if (active(r)) {
-                VLM_TRY(copy_predicted(ctx, *r));
-                VLM_TRY(rotor_convect(ctx, *r, dt, 1));
-            } else if (image(r)) {
-                VLM_TRY(rotor_convect(ctx, *r, dt, 1));
-            }
-        VLM_TRY(wake_pass(ctx, 1));
-        VLM_TRY(init_vel(true));
-        for (auto *r : ctx->rotors) {
-            if (image(r)) VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-            if (!active(r)) continue;
-            const int rows = r->d.nNwake - (r->rowNear - 1);
-            const int frows = r->d.nFwake - (r->rowFar - 1);
-            const int nbc = r->d.nbConvect;
-            if (rows > 0) {
-                const int64_t n = (int64_t)nbc * rows * (r->d.ns + 1) * 3;
-                hipLaunchKernelGGL(order2_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                                   r->velN[VLM_VEL].p, r->velN[VLM_VEL_PRED].p,
-                                   r->velN[VLM_VEL_STEP].p, nbc, rows, r->d.nNwake, r->d.ns + 1,
-                                   r->rowNear - 1);
-                hipLaunchKernelGGL(copy_window_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                                   r->velN[VLM_VEL_STEP].p, r->velN[VLM_VEL].p, nbc, rows,
-                                   r->d.nNwake, r->d.ns + 1, r->rowNear - 1);
-            }
-            if (frows > 0) {
-                const int64_t n = (int64_t)nbc * frows * 3;
-                hipLaunchKernelGGL(order2_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                                   r->velF[VLM_VEL].p, r->velF[VLM_VEL_PRED].p,
-                                   r->velF[VLM_VEL_STEP].p, nbc, frows, r->d.nFwake, 1,
-                                   r->rowFar - 1);
-                hipLaunchKernelGGL(copy_window_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
-                                   r->velF[VLM_VEL_STEP].p, r->velF[VLM_VEL].p, nbc, frows,
-                                   r->d.nFwake, 1, r->rowFar - 1);
-            }
-            VLM_HIP(hipGetLastError());
-            VLM_TRY(rotor_convect(ctx, *r, dt, 0));
+        if (frows > 0) {
+            const int64_t n = (int64_t)nbc * frows * 3;
+            hipLaunchKernelGGL(order2_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
+                               r->velF[VLM_VEL].p, r->velF[VLM_VEL_PRED].p,
+                               r->velF[VLM_VEL_STEP].p, nbc, frows, r->d.nFwake, 1,
+                               r->rowFar - 1);
+            hipLaunchKernelGGL(copy_window_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream,
+                               r->velF[VLM_VEL_STEP].p, r->velF[VLM_VEL].p, nbc, frows,
+                               r->d.nFwake, 1, r->rowFar - 1);
         }
-        return VLM_OK;
+        VLM_HIP(hipGetLastError());
     }
-    if (iter == 1) {
-        for (auto *r : ctx->rotors)
-            if (active(r)) {
-                VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-                VLM_TRY(launch_scheme(ctx, *r, 4));
-            } else if (image(r)) {
-                VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-            }
-        return VLM_OK;
-    }
-    if (scheme == VLM_SCHEME_AB2) {
-        for (auto *r : ctx->rotors)
-            if (active(r)) {
-                VLM_TRY(launch_scheme(ctx, *r, 0));
-                VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-            } else if (image(r)) {
-                VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-            }
-        return VLM_OK;
-    }
-    // AM2
-    for (auto *r : ctx->rotors)
-        if (active(r)) {
-            VLM_TRY(copy_predicted(ctx, *r));
-            VLM_TRY(launch_scheme(ctx, *r, 1));
-            VLM_TRY(rotor_convect(ctx, *r, dt, 1));
-        } else if (image(r)) {
-            VLM_TRY(rotor_convect(ctx, *r, dt, 1));
-        }
-    if (ctx->pred.mode == 1) VLM_TRY(learned_pass(ctx));
-    else VLM_TRY(wake_pass(ctx, 1));
-    VLM_TRY(init_vel(true));
-    for (auto *r : ctx->rotors)
-        if (active(r)) {
-            VLM_TRY(launch_scheme(ctx, *r, 2));
-            VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-            VLM_TRY(launch_scheme(ctx, *r, 3));
-        } else if (image(r)) {
-            VLM_TRY(rotor_convect(ctx, *r, dt, 0));
-        }
-    return VLM_OK;
+    Advance p3;
+    p3.convect = 0;
+    p3.dt = dt;
+    return advance(ctx, p3);
 }
 
 int vlm_rotor_set_image(vlm_ctx *ctx, int ir, int source, int imagePlane)
