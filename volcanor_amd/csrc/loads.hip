@@ -71,11 +71,27 @@ __device__ __forceinline__ double angle_tan(const double *a, const double *b)
 // secArea 15.
 // Blade records (BLADE_N): xAxisAziFlap 0-2, yAxisAziFlap 3-5, zAxisAziFlap 6-8.
 
-__global__ void cp_soa_kernel(const double *pan, int64_t n, double *cps)
+// Panel, section and blade records of a rotor from pinned host memory (one
+// after the other) into their arrays, and the collocation points as SoA.
+// One launch instead of three copies and a kernel of about 5 us each.
+__global__ __launch_bounds__(256) void panels_kernel(const double *h, int64_t n, int64_t nsec,
+                                                     int64_t nb, double *pan, double *sec,
+                                                     double *bla, double *cps)
 {
-    const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (e >= n) return;
-    for (int i = 0; i < 3; ++i) cps[i * n + e] = pan[PANEL_N * e + i];
+    int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int64_t np = PANEL_N * n, ns = SECTION_N * nsec;
+    if (e >= np + ns + BLADE_N * nb) return;
+    const double x = h[e];
+    if (e < np) {
+        pan[e] = x;
+        const int64_t k = e / PANEL_N;
+        const int i = (int)(e - PANEL_N * k);
+        if (i < 3) cps[i * n + k] = x;
+    } else if (e < np + ns) {
+        sec[e - np] = x;
+    } else {
+        bla[e - np - ns] = x;
+    }
 }
 
 // main.f90:528-591: velCPm of the rigid motion, velCP = velCPm + the
@@ -163,14 +179,16 @@ __device__ double lsq2_solve(double xq, const double *s, double b0, double b1, d
 // blade_calc_force 1704-1896 and rotor_calc_force 4607-4671).  One
 // workgroup: one thread per (convected blade, section) computes the
 // section's resultant velocity, angles, lift direction and panel pressure
-// loop in the reference's order, then one thread per blade sums its
-// sections and thread 0 the rotor.  Section results go to out as
-// LOADS_SEC_N-double records, the rotor's forceInertial, lift and
-// liftUnsteady after them.
+// loop in the reference's order, then one thread
+// per blade and component sums the sections and nine threads the rotor.
+// Section results go to out as LOADS_SEC_N-double records, the rotor's
+// forceInertial, lift and liftUnsteady after them, and all of it to host
+// (pinned memory).  Bound by the latency of its chains.
 __global__ __launch_bounds__(256) void loads_kernel(const double *pan, const double *sec,
                                                     const double *bla, const double *vcp,
                                                     const double *vld, const double *wg,
-                                                    double *gprev, double *out, LoadPar p)
+                                                    double *gprev, double *out, double *host,
+                                                    LoadPar p)
 {
     extern __shared__ double sh[];  // per section: forceInertial, liftUnsteady; per blade: 9
     const int nsec = p.nbc * p.ns, nc = p.nc, ns = p.ns;
@@ -287,29 +305,27 @@ __global__ __launch_bounds__(256) void loads_kernel(const double *pan, const dou
         o[18] = clu;
     }
     __syncthreads();
-    for (int b = threadIdx.x; b < p.nbc; b += blockDim.x) {
-        double s[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-        for (int is = 0; is < ns; ++is) {
-            const int t = b * ns + is;
-            for (int i = 0; i < 3; ++i) {
-                s[i] += sh[6 * t + i];
-                s[3 + i] += out[LOADS_SEC_N * (int64_t)t + 8 + i];
-                s[6 + i] += sh[6 * t + 3 + i];
-            }
-        }
-        for (int k = 0; k < 9; ++k) shb[9 * b + k] = s[k];
+    for (int t = threadIdx.x; t < 9 * p.nbc; t += blockDim.x) {
+        const int b = t / 9, k = t - 9 * b, c = k % 3, g = k / 3;
+        const double *src = g == 1 ? out + LOADS_SEC_N * (int64_t)b * ns + 8 + c
+                                   : sh + 6 * b * ns + (g == 0 ? c : 3 + c);
+        const int st = g == 1 ? LOADS_SEC_N : 6;
+        double s = 0.0;
+        for (int is = 0; is < ns; ++is) s += src[st * is];
+        shb[t] = s;
     }
+    for (int t = threadIdx.x; t < LOADS_SEC_N * nsec; t += blockDim.x) host[t] = out[t];
     __syncthreads();
-    if (threadIdx.x == 0) {
-        double r[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+    if (threadIdx.x < 9) {
+        const int k = threadIdx.x;
+        double r = 0.0;
         if (p.nbc == 1 && p.nb > 1) {
-            for (int k = 0; k < 9; ++k) r[k] = (double)p.nb * shb[k];
+            r = (double)p.nb * shb[k];
         } else {
-            for (int b = 0; b < p.nbc; ++b)
-                for (int k = 0; k < 9; ++k) r[k] = r[k] + shb[9 * b + k];
+            for (int b = 0; b < p.nbc; ++b) r = r + shb[9 * b + k];
         }
-        double *o = out + LOADS_SEC_N * (int64_t)nsec;
-        for (int k = 0; k < 9; ++k) o[k] = r[k];
+        out[LOADS_SEC_N * (int64_t)nsec + k] = r;
+        host[LOADS_SEC_N * (int64_t)nsec + k] = r;
     }
 }
 
@@ -328,10 +344,16 @@ int vlm_rotor_set_panels(vlm_ctx *ctx, int ir, const double *panel, const double
     if (!panel || !section || !blade) return fail(ctx, VLM_ERR_ARG, "null buffer");
     VLM_DEVICE(ctx);
     const int64_t n = r->nring, nsec = (int64_t)r->d.nb * r->d.ns;
-    VLM_TRY(h2d(ctx, r->pan.p, panel, sizeof(double) * PANEL_N * n));
-    VLM_TRY(h2d(ctx, r->sec.p, section, sizeof(double) * SECTION_N * nsec));
-    VLM_TRY(h2d(ctx, r->bla.p, blade, sizeof(double) * BLADE_N * r->d.nb));
-    hipLaunchKernelGGL(cp_soa_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream, r->pan.p, n,
+    const size_t np = PANEL_N * (size_t)n, ns = SECTION_N * (size_t)nsec;
+    const size_t nbl = BLADE_N * (size_t)r->d.nb;
+    char *hp = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(double) * (np + ns + nbl), &hp));
+    double *h = reinterpret_cast<double *>(hp);
+    std::memcpy(h, panel, sizeof(double) * np);
+    std::memcpy(h + np, section, sizeof(double) * ns);
+    std::memcpy(h + np + ns, blade, sizeof(double) * nbl);
+    hipLaunchKernelGGL(panels_kernel, dim3(nblk((int64_t)(np + ns + nbl))), dim3(256), 0,
+                       ctx->stream, h, n, nsec, (int64_t)r->d.nb, r->pan.p, r->sec.p, r->bla.p,
                        r->cps.p);
     VLM_HIP(hipGetLastError());
     r->panels_set = 1;
@@ -406,11 +428,14 @@ int vlm_rotor_loads(vlm_ctx *ctx, int ir, int nterms, const int *irs, const int 
     const size_t shmem = sizeof(double) * (6 * (size_t)p.nbc * p.ns + 9 * (size_t)p.nbc);
     if (shmem > 64 * 1024) return fail(ctx, VLM_ERR_ARG, "too many blade sections for the loads");
     VLM_TRY(induced_terms_soa(ctx, nterms, irs, sets, flags, n, r->cps.p, r->vld.p));
-    hipLaunchKernelGGL(loads_kernel, dim3(1), dim3(256), shmem, ctx->stream, r->pan.p, r->sec.p,
-                       r->bla.p, r->vcp.p, r->vld.p, r->wg.p, r->gprev.p, r->lout.p, p);
-    VLM_HIP(hipGetLastError());
     const size_t nout = (size_t)LOADS_SEC_N * p.nbc * p.ns + LOADS_ROTOR_N;
-    return d2h_deferred(ctx, out, r->lout.p, sizeof(double) * nout);
+    char *hp = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(double) * nout, &hp));
+    hipLaunchKernelGGL(loads_kernel, dim3(1), dim3(256), shmem, ctx->stream, r->pan.p, r->sec.p,
+                       r->bla.p, r->vcp.p, r->vld.p, r->wg.p, r->gprev.p, r->lout.p,
+                       reinterpret_cast<double *>(hp), p);
+    VLM_HIP(hipGetLastError());
+    return defer(ctx, {{out, hp, sizeof(double) * nout}});
 }
 
 }  // extern "C"

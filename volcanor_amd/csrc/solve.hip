@@ -428,12 +428,19 @@ __device__ void wave_lu_solve(int n, const double *sLU, const int *spiv, double 
     }
 }
 
+// Where the one-wave solve leaves its results: x and (converged, corrections)
+// in pinned host memory, and with wg the wing circulation of a rotor of nb
+// blades (nbc of them convected) of per panels each.
+struct SolveOut {
+    double *x, *wg;
+    int *st, per, nb, nbc;
+};
+
 template <int R, int NMAX>
 __global__ __launch_bounds__(SOLVE_STAGE) void solve_wave_kernel(int n, const double *A,
                                                                  const double *LU,
                                                         const int *ipiv, const double *b,
-                                                        double *x, int max_iter, double tol,
-                                                        int *st)
+                                                        int max_iter, double tol, SolveOut o)
 {
     __shared__ double sLU[NMAX * NMAX], sA[NMAX * NMAX];
     __shared__ int spiv[NMAX];
@@ -500,10 +507,23 @@ __global__ __launch_bounds__(SOLVE_STAGE) void solve_wave_kernel(int n, const do
     }
 #pragma unroll
     for (int q = 0; q < R; ++q)
-        if (l + 64 * q < n) x[l + 64 * q] = xv[q];
+        if (l + 64 * q < n) o.x[l + 64 * q] = xv[q];
     if (l == 0) {
-        st[0] = conv;
-        st[1] = corr;
+        o.st[0] = conv;
+        o.st[1] = corr;
+    }
+    if (!o.wg) return;
+    // rotor_map_gam: blade 1 for every blade of an axisymmetric rotor
+    for (int e = 0; e < o.per * o.nb; e += 64) {
+        const int k = e + l, blade = k / o.per;
+        const int src = blade < o.nbc ? k : o.nbc == 1 ? k - blade * o.per : n;
+        double g = 0.0;
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const double t = __shfl(xv[q], src & 63);
+            if (src >> 6 == q) g = t;
+        }
+        if (k < o.per * o.nb && src < n) o.wg[k] = g;
     }
 }
 
@@ -519,28 +539,38 @@ int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const i
 {
     const size_t np = (size_t)(n + TB - 1) / TB * TB;
     VLM_HIP(ctx->solve_tmp.reserve((size_t)3 * n + 2 * np + 5));
-    double *b = ctx->solve_tmp.p, *x = b + n, *r = x + n;
-    SolveWork w;
-    w.y = reinterpret_cast<unsigned long long *>(r + n);
-    w.z = w.y + np;
-    w.rmax = w.z + np;
-    w.bmax = w.rmax + 2;
-    w.st = reinterpret_cast<int *>(w.bmax + 1);
-    w.ticket = w.st + 2;
-    int *st = w.st;
-    if (rhs_h) {
-        VLM_TRY(h2d(ctx, b, rhs_h, sizeof(double) * n));
-    } else {  // the right-hand side left on the device by vlm_rotor_rhs
-        VLM_HIP(hipMemcpyAsync(b, rotor->rhs.p, sizeof(double) * n, hipMemcpyDeviceToDevice,
-                               ctx->stream));
-    }
-    if (n <= SOLVE_WAVE_N) {
-        hipLaunchKernelGGL((solve_wave_kernel<1, SOLVE_WAVE_N>), dim3(1), dim3(SOLVE_STAGE), 0,
-                           ctx->stream, n, A, LU, piv, b, x, max_iter, tol, st);
-    } else if (n <= SOLVE_WAVE_N2) {
-        hipLaunchKernelGGL((solve_wave_kernel<2, SOLVE_WAVE_N2>), dim3(1), dim3(SOLVE_STAGE), 0,
-                           ctx->stream, n, A, LU, piv, b, x, max_iter, tol, st);
+    double *x = ctx->solve_tmp.p + n, *r = x + n;
+    const double *b = ctx->solve_tmp.p;
+    if (rhs_h) VLM_TRY(h2d(ctx, ctx->solve_tmp.p, rhs_h, sizeof(double) * n));
+    else b = rotor->rhs.p;   // left on the device by vlm_rotor_rhs
+    const int per = rotor ? rotor->d.nc * rotor->d.ns : 0;
+    // x and (converged, corrections) on the host
+    char *hp = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(double) * n + 2 * sizeof(int), &hp));
+    int *hst = reinterpret_cast<int *>(hp + sizeof(double) * n);
+    if (n <= SOLVE_WAVE_N2) {
+        SolveOut o;
+        o.x = reinterpret_cast<double *>(hp);
+        o.st = hst;
+        o.wg = rotor ? rotor->wg.p : nullptr;
+        o.per = per;
+        o.nb = rotor ? rotor->d.nb : 0;
+        o.nbc = rotor ? rotor->d.nbConvect : 0;
+        if (n <= SOLVE_WAVE_N)
+            hipLaunchKernelGGL((solve_wave_kernel<1, SOLVE_WAVE_N>), dim3(1), dim3(SOLVE_STAGE),
+                               0, ctx->stream, n, A, LU, piv, b, max_iter, tol, o);
+        else
+            hipLaunchKernelGGL((solve_wave_kernel<2, SOLVE_WAVE_N2>), dim3(1), dim3(SOLVE_STAGE),
+                               0, ctx->stream, n, A, LU, piv, b, max_iter, tol, o);
+        VLM_HIP(hipGetLastError());
     } else {
+        SolveWork w;
+        w.y = reinterpret_cast<unsigned long long *>(r + n);
+        w.z = w.y + np;
+        w.rmax = w.z + np;
+        w.bmax = w.rmax + 2;
+        w.st = reinterpret_cast<int *>(w.bmax + 1);
+        w.ticket = w.st + 2;
         const dim3 gs(2 * (unsigned)(np / TB)), gr((n + RROWS - 1) / RROWS);
         hipLaunchKernelGGL(solve_init_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0,
                            ctx->stream, n, b, w);
@@ -552,27 +582,22 @@ int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const i
             hipLaunchKernelGGL(lu_sweeps_kernel, gs, dim3(256), 0, ctx->stream, n, LU, piv, r, x,
                                1, it, tol, w);
         }
-    }
-    VLM_HIP(hipGetLastError());
-    if (rotor) {
-        const int per = rotor->d.nc * rotor->d.ns;
-        hipLaunchKernelGGL(map_gam_kernel, dim3((per * rotor->d.nb + 255) / 256), dim3(256), 0,
-                           ctx->stream, x, rotor->wg.p, per, rotor->d.nb, rotor->d.nbConvect);
+        if (rotor)
+            hipLaunchKernelGGL(map_gam_kernel, dim3((per * rotor->d.nb + 255) / 256), dim3(256),
+                               0, ctx->stream, x, rotor->wg.p, per, rotor->d.nb,
+                               rotor->d.nbConvect);
         VLM_HIP(hipGetLastError());
+        VLM_HIP(hipMemcpyAsync(hp, x, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
+        VLM_HIP(hipMemcpyAsync(hst, w.st, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     }
     if (deferred) {
-        VLM_TRY(d2h_deferred(ctx, x_h, x, sizeof(double) * n));
-        if (iters) VLM_TRY(d2h_deferred(ctx, iters, st + 1, sizeof(int)));
-        return VLM_OK;
+        if (!iters) return defer(ctx, {{x_h, hp, sizeof(double) * n}});
+        return defer(ctx, {{x_h, hp, sizeof(double) * n},
+                           {iters, reinterpret_cast<const char *>(hst + 1), sizeof(int)}});
     }
-    char *px = nullptr, *ps = nullptr;
-    VLM_TRY(pin_take(ctx, sizeof(double) * n, &px));
-    VLM_TRY(pin_take(ctx, 2 * sizeof(int), &ps));
-    VLM_HIP(hipMemcpyAsync(px, x, sizeof(double) * n, hipMemcpyDeviceToHost, ctx->stream));
-    VLM_HIP(hipMemcpyAsync(ps, st, 2 * sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
     VLM_TRY(sync_stream(ctx));
-    std::memcpy(x_h, px, sizeof(double) * n);
-    if (iters) *iters = reinterpret_cast<const int *>(ps)[1];
+    std::memcpy(x_h, hp, sizeof(double) * n);
+    if (iters) *iters = hst[1];
     return VLM_OK;
 }
 

@@ -113,16 +113,21 @@ int sync_stream(vlm_ctx *ctx)
     return VLM_OK;
 }
 
+int defer(vlm_ctx *ctx, std::initializer_list<vlm_ctx::Deferred> d)
+{
+    if (!ctx->defer_ev) VLM_HIP(hipEventCreateWithFlags(&ctx->defer_ev, hipEventDisableTiming));
+    VLM_HIP(hipEventRecord(ctx->defer_ev, ctx->stream));
+    ctx->deferred.insert(ctx->deferred.end(), d);
+    return VLM_OK;
+}
+
 int d2h_deferred(vlm_ctx *ctx, void *dst, const void *src, size_t bytes)
 {
     if (bytes == 0) return VLM_OK;
     char *p = nullptr;
     VLM_TRY(pin_take(ctx, bytes, &p));
     VLM_HIP(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    if (!ctx->defer_ev) VLM_HIP(hipEventCreateWithFlags(&ctx->defer_ev, hipEventDisableTiming));
-    VLM_HIP(hipEventRecord(ctx->defer_ev, ctx->stream));
-    ctx->deferred.push_back({dst, p, bytes});
-    return VLM_OK;
+    return defer(ctx, {{dst, p, bytes}});
 }
 
 // Waits only for the work enqueued up to the last deferred copy; the arena

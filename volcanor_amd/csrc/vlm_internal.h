@@ -128,7 +128,6 @@ struct Rotor {
     // far wake
     DBuf<double> ffc, pffc;       // 6*nb*nF
     DBuf<double> fgam, frc, frc0, fl0, flc, fage;  // nb*nF
-    DBuf<double> ftmp;            // shift staging, 11*nb*nF
     // velocities, logical rows: [VLM_VEL, PREV, PRED, STEP] and the older
     // histories of AM3/AM4 (velNwake2, velNwake3; PREV is velNwake1)
     DBuf<double> velN[NVEL], velF[NVEL];
@@ -419,6 +418,8 @@ int sync_stream(vlm_ctx *ctx);
 // Deferred download: the copy is enqueued now, dst is written at
 // wait_deferred or at the next sync_stream (whichever comes first).
 int d2h_deferred(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);
+// The same for pinned memory (pin_take) that work already enqueued writes.
+int defer(vlm_ctx *ctx, std::initializer_list<vlm_ctx::Deferred> d);
 int wait_deferred(vlm_ctx *ctx);
 int mlp_forward_dev(vlm_ctx *ctx, int64_t m, const float *X, float *Y);
 // Training step on a device batch; loss_host downloads the loss (and
