@@ -433,7 +433,7 @@ __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
     }
 }
 
-// Few targets (collocation points, bound vortices, probes): each block
+// Few targets or short lists (few_pairs): each block
 // takes SM_T targets and one segment chunk; its 256 lanes stride over the
 // chunk (coalesced SoA loads, each record shared by the SM_T targets) and
 // the partial sums are reduced in a fixed order (butterfly within the wave,
@@ -441,11 +441,6 @@ __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
 // pairs.
 constexpr int SM_T = 4;
 constexpr int SM_BLOCK = 256;
-// fewer targets than this take bs_small_kernel: its lanes are segments, so
-// no lane idles however few the targets (20 targets x 2e5 segments: 54
-// against 92 us with a wave of 64 targets; 90 targets: 92 against 108), but
-// every pair is the long one (300 targets: 186 against 165 us)
-constexpr int SM_MAX = 192;
 constexpr int LEN_MID = 8;
 constexpr int MIXED_NT = 2;       // targets per lane of the mixed kernel
 constexpr int MIXED_MIN = 1024;   // fewer targets than this: FP64 in both modes
@@ -518,6 +513,12 @@ __global__ __launch_bounds__(SM_BLOCK) void bs_small_kernel(const double *s64, i
     }
 }
 
+// Component d of target t lies at out[d ds + t ts]: SoA (stride, 1) or the
+// host's order (1, 3).
+struct OutMap {
+    int64_t ds, ts;
+};
+
 // Sum of the lists' chunk partials at one component of 64 targets, then the
 // term recurrence (TermLists): RT_S slices of a list's chunks side by side,
 // each in increasing order, the slices and then the lists added in order, so
@@ -526,8 +527,7 @@ constexpr int RT_S = 8, RT_W = 16;
 
 __global__ __launch_bounds__(64 * RT_W) void bs_reduce_terms_kernel(const double *part,
                                                                     TermTab tt, int64_t m,
-                                                                    double *out, int64_t ostride,
-                                                                    int acc)
+                                                                    double *out, OutMap o, int acc)
 {
     __shared__ double sh[TERM_MAX * RT_S][64];
     const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
@@ -555,13 +555,14 @@ __global__ __launch_bounds__(64 * RT_W) void bs_reduce_terms_kernel(const double
     }
     __syncthreads();
     if (w > 0 || t >= m) return;
-    double v = acc ? out[d * ostride + t] : 0.0;
+    out += d * o.ds + t * o.ts;
+    double v = acc ? *out : 0.0;
     for (int k = 0; k < tt.n; ++k) {
         double s = sh[k * RT_S][l];
         for (int q = 1; q < RT_S; ++q) s += sh[k * RT_S + q][l];
         v = (tt.neg >> k & 1 ? -v : v) + s;
     }
-    out[d * ostride + t] = v;
+    *out = v;
 }
 
 // Fixed-order sum of the per-chunk partials: T targets of one component per
@@ -572,8 +573,8 @@ __global__ __launch_bounds__(64 * RT_W) void bs_reduce_terms_kernel(const double
 // many slices.  Workgroup 0 clears the work counter for the next launch.
 template <int T, int S>
 __global__ __launch_bounds__(T * S) void bs_reduce_kernel(const double *part, int nchunks,
-                                                          int64_t m, double *out,
-                                                          int64_t ostride, int acc, int *counter)
+                                                          int64_t m, double *out, OutMap o,
+                                                          int acc, int *counter)
 {
     __shared__ double sh[S][T];
     const int l = threadIdx.x % T, w = threadIdx.x / T;
@@ -602,24 +603,27 @@ __global__ __launch_bounds__(T * S) void bs_reduce_kernel(const double *part, in
         if (w > 0) return;
         for (int k = 1; k < S; ++k) s += sh[k][l];
     }
-    if (t < m) out[d * ostride + t] = acc ? out[d * ostride + t] + s : s;
+    if (t < m) {
+        double *q = out + d * o.ds + t * o.ts;
+        *q = acc ? *q + s : s;
+    }
 }
 
 template <int T, int S>
-void reduce_as(vlm_ctx *ctx, const double *part, int nchunks, int64_t m, double *out,
-               int64_t ostride, int acc, int *counter)
+void reduce_as(vlm_ctx *ctx, const double *part, int nchunks, int64_t m, double *out, OutMap o,
+               int acc, int *counter)
 {
     hipLaunchKernelGGL((bs_reduce_kernel<T, S>), dim3((unsigned)((m + T - 1) / T), 3), dim3(T * S),
-                       0, ctx->stream, part, nchunks, m, out, ostride, acc, counter);
+                       0, ctx->stream, part, nchunks, m, out, o, acc, counter);
 }
 
 int launch_reduce(vlm_ctx *ctx, const double *part, int nchunks, int64_t m, double *out,
-                  int64_t ostride, int acc, int *counter)
+                  OutMap o, int acc, int *counter)
 {
-    if (nchunks >= 256) reduce_as<16, 64>(ctx, part, nchunks, m, out, ostride, acc, counter);
-    else if (nchunks >= 32) reduce_as<64, 8>(ctx, part, nchunks, m, out, ostride, acc, counter);
-    else if (nchunks >= 8) reduce_as<64, 4>(ctx, part, nchunks, m, out, ostride, acc, counter);
-    else reduce_as<64, 1>(ctx, part, nchunks, m, out, ostride, acc, counter);
+    if (nchunks >= 256) reduce_as<16, 64>(ctx, part, nchunks, m, out, o, acc, counter);
+    else if (nchunks >= 32) reduce_as<64, 8>(ctx, part, nchunks, m, out, o, acc, counter);
+    else if (nchunks >= 8) reduce_as<64, 4>(ctx, part, nchunks, m, out, o, acc, counter);
+    else reduce_as<64, 1>(ctx, part, nchunks, m, out, o, acc, counter);
     VLM_HIP(hipGetLastError());
     return VLM_OK;
 }
@@ -661,14 +665,30 @@ int profile_count(vlm_ctx *ctx, const long long *nseg_dev, int64_t m, int kind, 
 
 }  // namespace
 
-int bs_formats(const vlm_ctx *ctx, int64_t m)
+// bs_small_kernel has segments on its lanes, so no lane idles however few the
+// targets and short lists spread over the device, but every pair is the long
+// one.  Whole calls, small against 64 targets per wave, us:
+//   m    20 x 2e5      54   92    90 x 2e5     92  108   192 x 1e5     67   59
+//   m   200 x 2000     22   27   300 x 4e4     46   50   300 x 1e5     82   81
+//   m   300 x 2000     22   27   400 x 4e4     54   56   512 x 4e4     61   57
+//   m   600 x 2000     24   27   600 x 8000    36   35   192 x 4e5    229  151
+//   m  1200 x 500      24   27  1200 x 2000    28   31   400 x 4e5    357  306
+static bool few_pairs(int64_t m, int64_t nseg)
 {
-    if (m < SM_MAX) return SEG_SOA;
-    return ctx->precision == VLM_MIXED && m >= MIXED_MIN ? SEG_REC | SEG_F32 : SEG_REC;
+    if (m < 192 && 5 * m < 4 * 64 * ((m + 63) / 64)) return true;   // waves not 4/5 full
+    if (nseg > 16000000 || m > 2048) return false;
+    return m * nseg <= (m <= 400 ? 16000000 : 3000000);
+}
+
+int bs_formats(const vlm_ctx *ctx, int64_t m, int64_t nseg)
+{
+    if (ctx->precision == VLM_MIXED && m >= MIXED_MIN) return SEG_REC | SEG_F32;
+    return few_pairs(m, nseg) ? SEG_SOA : SEG_REC;
 }
 
 int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, const double *t,
-                  int64_t m, int64_t tstride, double *out, int accumulate, const BsWork *ws)
+                  int64_t m, int64_t tstride, double *out, int accumulate, const BsWork *ws,
+                  bool aos)
 {
     if (m <= 0) return VLM_OK;
     if (terms.n < 1 || terms.n > TERM_MAX) return fail(ctx, VLM_ERR_ARG, "bad term count");
@@ -696,13 +716,14 @@ int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, cons
     const int nchunks = tt.chunk0[tt.n];
     double *part = ws ? ws->part : nullptr;
     if (!ws) {
-        VLM_HIP(ctx->part.reserve((size_t)nchunks * 3 * (size_t)m));
+        VLM_HIP(ctx->part.reserve(ws_size<double>((size_t)nchunks * 3 * (size_t)m)));
         part = ctx->part.p;
     }
     hipLaunchKernelGGL(bs_small_kernel, dim3(nchunks, (unsigned)groups), dim3(SM_BLOCK), 0,
                        ctx->stream, seg.soa, seg.cap, seg.count, tt, t, m, tstride, part);
     hipLaunchKernelGGL(bs_reduce_terms_kernel, dim3((unsigned)((m + 63) / 64), 3),
-                       dim3(64 * RT_W), 0, ctx->stream, part, tt, m, out, tstride, accumulate);
+                       dim3(64 * RT_W), 0, ctx->stream, part, tt, m, out,
+                       aos ? OutMap{1, 3} : OutMap{tstride, 1}, accumulate);
     VLM_HIP(hipGetLastError());
     if (ctx->profile && !ws)
         for (int k = 0; k < terms.n; ++k)
@@ -711,16 +732,17 @@ int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, cons
 }
 
 int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t, int64_t m,
-            int64_t tstride, double *out, int accumulate, const BsWork *ws)
+            int64_t tstride, double *out, int accumulate, const BsWork *ws, bool aos)
 {
     if (m <= 0) return VLM_OK;
+    const OutMap o = aos ? OutMap{1, 3} : OutMap{tstride, 1};
     // chunk partial sums: the context's growing buffer, or a fixed
     // workspace that caps the chunk count
     const int64_t max_chunks = ws ? (int64_t)(ws->part_cap / (3 * (size_t)m)) : INT32_MAX;
     if (ws && max_chunks < 1) return fail(ctx, VLM_ERR_ARG, "workspace too small for the targets");
     const bool prof = ctx->profile && !ws;
-    if (nseg_est <= 0) return launch_reduce(ctx, nullptr, 0, m, out, tstride, accumulate, nullptr);
-    const int fmt = bs_formats(ctx, m);
+    if (nseg_est <= 0) return launch_reduce(ctx, nullptr, 0, m, out, o, accumulate, nullptr);
+    const int fmt = bs_formats(ctx, m, nseg_est);
     if (((fmt & SEG_SOA) && !seg.soa) || ((fmt & SEG_REC) && !seg.rec64) ||
         ((fmt & SEG_F32) && !seg.rec32))
         return fail(ctx, VLM_ERR_STATE, "segment list lacks the records of this launch");
@@ -730,7 +752,7 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
         one.off[0] = 0;
         one.est[0] = nseg_est;
         one.neg[0] = 0;
-        return bs_eval_terms(ctx, seg, one, t, m, tstride, out, accumulate, ws);
+        return bs_eval_terms(ctx, seg, one, t, m, tstride, out, accumulate, ws, aos);
     }
     const bool mixed = (fmt & SEG_F32) != 0;
     const int tile = mixed ? 64 * MIXED_NT : 64;
@@ -756,7 +778,7 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
     double *part = ws ? ws->part : nullptr;
     int *counter = ws ? ws->counter : nullptr;
     if (!ws) {
-        VLM_HIP(ctx->part.reserve((size_t)nchunks * 3 * (size_t)m));
+        VLM_HIP(ctx->part.reserve(ws_size<double>((size_t)nchunks * 3 * (size_t)m)));
         if (!ctx->counter.p) {
             VLM_HIP(ctx->counter.reserve(1));
             hipLaunchKernelGGL(zero_int_kernel, dim3(1), dim3(1), 0, ctx->stream, ctx->counter.p);
@@ -797,7 +819,7 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
     VLM_HIP(hipGetLastError());
     if (timed) VLM_HIP(hipEventRecord(tm.b, ctx->stream));
     if (prof) VLM_TRY(profile_count(ctx, seg.count, m, timed ? 0 : 1, timed ? &tm : nullptr));
-    return launch_reduce(ctx, part, nchunks, m, out, tstride, accumulate, counter);
+    return launch_reduce(ctx, part, nchunks, m, out, o, accumulate, counter);
 }
 
 }  // namespace vlm

@@ -4,7 +4,7 @@
 //
 // Every intermediate buffer of the call lives in one file-scope device
 // array, `scratch`, of NOALLOC_SCRATCH_BYTES: the segment records (FP64
-// and FP32 structure of arrays, the count), the targets and sums in
+// and FP32 formats, the count), the targets in
 // structure-of-arrays form, the chunk partial sums of the Biot-Savart
 // launch and its work counter.  The call enqueues kernels on the context's
 // stream and returns; it calls no hipMalloc, no hipFree, no allocating
@@ -21,7 +21,7 @@
 
 namespace vlm {
 // Inputs are accepted up to 64 MiB at 120 B per filament and 72 B per point
-// (72 + 48 B of records per filament, targets, sums and one chunk).  The
+// (the sizes of an earlier layout, kept as the limit of the call).  The
 // records take 225 B per filament, so the array is 64 MiB x 225 / 120 plus
 // room for chunks.
 constexpr size_t NOALLOC_ACCEPTED_BYTES = (size_t)64 << 20;
@@ -70,15 +70,6 @@ __global__ void aos_to_soa3_kernel(int64_t m, const double *aos, double *soa, in
     soa[2 * m + i] = aos[3 * i + 2];
 }
 
-__global__ void soa3_to_aos_kernel(int64_t m, const double *soa, double *aos)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    aos[3 * i] = soa[i];
-    aos[3 * i + 1] = soa[m + i];
-    aos[3 * i + 2] = soa[2 * m + i];
-}
-
 }  // namespace
 }  // namespace vlm
 
@@ -97,11 +88,11 @@ int vlm_filament_vind_noalloc(vlm_ctx *ctx, int64_t nfil, const double *a, const
         return fail(ctx, VLM_ERR_ARG, "null buffer");
     // workspace layout: soa | rec64 | grp | rec32 | near32 (the formats that
     // m targets need) | count | counter |
-    // targets | sums | partials.  The sizes accepted are those of the
+    // targets | partials.  The sizes accepted are those of the
     // documented 64 MiB at 120 B per filament and 72 B per point; the array
     // itself is larger (225 B per filament, group records included).
     const int64_t cap = nfil > 0 ? nfil : 1, gcap = (cap + GRP - 1) / GRP, rcap = gcap * GRP;
-    const int fmt = bs_formats(ctx, m);
+    const int fmt = bs_formats(ctx, m, nfil);
     const size_t osoa = 0;
     const size_t o64 = osoa + (fmt & SEG_SOA ? up256((size_t)SOA_N * rcap * sizeof(double)) : 0);
     const size_t ogrp = o64 + (fmt & SEG_REC ? up256((size_t)REC64_N * rcap * sizeof(double)) : 0);
@@ -110,8 +101,7 @@ int vlm_filament_vind_noalloc(vlm_ctx *ctx, int64_t nfil, const double *a, const
     const size_t ocnt = onear + (fmt & SEG_F32 ? up256((size_t)NEAR32_N * rcap * sizeof(float)) : 0);
     const size_t octr = ocnt + 256;
     const size_t otgt = octr + 256;
-    const size_t oout = otgt + up256((size_t)3 * m * sizeof(double));
-    const size_t opart = oout + up256((size_t)3 * m * sizeof(double));
+    const size_t opart = otgt + up256((size_t)3 * m * sizeof(double));
     const size_t accepted = up256((size_t)9 * cap * sizeof(double)) +
                             up256((size_t)12 * cap * sizeof(float)) + 512 +
                             2 * up256((size_t)3 * m * sizeof(double)) +
@@ -136,7 +126,6 @@ int vlm_filament_vind_noalloc(vlm_ctx *ctx, int64_t nfil, const double *a, const
     seg.count = reinterpret_cast<long long *>(w + ocnt);
     seg.cap = rcap;
     double *tgt = reinterpret_cast<double *>(w + otgt);
-    double *out = reinterpret_cast<double *>(w + oout);
     BsWork ws;
     ws.part = reinterpret_cast<double *>(w + opart);
     ws.part_cap = (NOALLOC_SCRATCH_BYTES - opart) / sizeof(double);
@@ -144,13 +133,8 @@ int vlm_filament_vind_noalloc(vlm_ctx *ctx, int64_t nfil, const double *a, const
     if (nfil > 0) VLM_TRY(explicit_records(ctx, nfil, a, b, gam, rc, seg));
     hipLaunchKernelGGL(aos_to_soa3_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, p, tgt,
                        ws.counter);
-    if (accumulate)
-        hipLaunchKernelGGL(aos_to_soa3_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, v,
-                           out, ws.counter);
     VLM_HIP(hipGetLastError());
-    VLM_TRY(bs_eval(ctx, seg, nfil, tgt, m, m, out, accumulate, &ws));
-    hipLaunchKernelGGL(soa3_to_aos_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, out, v);
-    VLM_HIP(hipGetLastError());
+    VLM_TRY(bs_eval(ctx, seg, nfil, tgt, m, m, v, accumulate, &ws, true));
     return VLM_OK;
 }
 

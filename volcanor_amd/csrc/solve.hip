@@ -642,13 +642,13 @@ int vlm_rotor_calc_aic(vlm_ctx *ctx, int ir, const double *cp, const double *nca
         VLM_HIP(hipMalloc(reinterpret_cast<void **>(&ctx->piv[ir]), sizeof(int) * (2 * n + 1)));
         ctx->aic_n[ir] = n;
     }
-    DBuf<double> geo;
-    VLM_HIP(geo.reserve((size_t)6 * n));
-    VLM_TRY(h2d(ctx, geo.p, cp, sizeof(double) * 3 * n));
-    VLM_TRY(h2d(ctx, geo.p + 3 * n, ncap, sizeof(double) * 3 * n));
+    VLM_HIP(ctx->hostio.reserve((size_t)6 * n));
+    double *geo = ctx->hostio.p;
+    VLM_TRY(h2d(ctx, geo, cp, sizeof(double) * 3 * n));
+    VLM_TRY(h2d(ctx, geo + 3 * n, ncap, sizeof(double) * 3 * n));
     const int64_t nn = (int64_t)n * n;
     hipLaunchKernelGGL(aic_kernel, dim3((unsigned)((nn + 255) / 256)), dim3(256), 0, ctx->stream,
-                       n, r.wc.p, r.wrc.p, geo.p, geo.p + 3 * n, ctx->aic[ir]);
+                       n, r.wc.p, r.wrc.p, geo, geo + 3 * n, ctx->aic[ir]);
     VLM_HIP(hipGetLastError());
     VLM_HIP(hipMemcpyAsync(ctx->lu[ir], ctx->aic[ir], sizeof(double) * nn,
                            hipMemcpyDeviceToDevice, ctx->stream));
@@ -658,11 +658,9 @@ int vlm_rotor_calc_aic(vlm_ctx *ctx, int ir, const double *cp, const double *nca
     VLM_TRY(pin_take(ctx, sizeof(int) * (n + 1), &hp));
     VLM_HIP(hipMemcpyAsync(hp, ctx->piv[ir], sizeof(int) * (n + 1), hipMemcpyDeviceToHost,
                            ctx->stream));
-    if (Aout)
-        VLM_HIP(hipMemcpyAsync(Aout, ctx->aic[ir], sizeof(double) * nn, hipMemcpyDeviceToHost,
-                               ctx->stream));
     VLM_TRY(sync_stream(ctx));
     std::memcpy(piv.data(), hp, sizeof(int) * (n + 1));
+    if (Aout) VLM_TRY(d2h(ctx, Aout, ctx->aic[ir], sizeof(double) * nn));
     const int info = piv[n];
     compose_pivots(n, piv.data(), piv.data() + n + 1);
     VLM_TRY(h2d(ctx, ctx->piv[ir] + n + 1, piv.data() + n + 1, sizeof(int) * n));
@@ -700,17 +698,18 @@ int vlm_lu_factor(vlm_ctx *ctx, int n, double *A, int *ipiv)
 {
     if (!ctx || n <= 0 || !A || !ipiv) return VLM_ERR_ARG;
     VLM_DEVICE(ctx);
-    DBuf<double> dA;
-    DBuf<int> dp;
-    VLM_HIP(dA.reserve((size_t)n * n));
-    VLM_HIP(dp.reserve((size_t)n + 1));
-    VLM_HIP(hipMemcpyAsync(dA.p, A, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
-    VLM_TRY(lu_factor_device(ctx, n, dA.p, dp.p, dp.p + n));
-    int info = 0;
-    VLM_HIP(hipMemcpyAsync(A, dA.p, sizeof(double) * n * n, hipMemcpyDeviceToHost, ctx->stream));
-    VLM_HIP(hipMemcpyAsync(ipiv, dp.p, sizeof(int) * n, hipMemcpyDeviceToHost, ctx->stream));
-    VLM_HIP(hipMemcpyAsync(&info, dp.p + n, sizeof(int), hipMemcpyDeviceToHost, ctx->stream));
-    VLM_TRY(sync_stream(ctx));
+    const size_t nn = (size_t)n * n;
+    VLM_HIP(ctx->hostio.reserve(nn));
+    VLM_HIP(ctx->hostio_i.reserve((size_t)n + 1));
+    double *dA = ctx->hostio.p;
+    int *dp = ctx->hostio_i.p;
+    VLM_TRY(h2d(ctx, dA, A, sizeof(double) * nn));
+    VLM_TRY(lu_factor_device(ctx, n, dA, dp, dp + n));
+    std::vector<int> piv((size_t)n + 1);   // pivots, info
+    VLM_TRY(d2h(ctx, A, dA, sizeof(double) * nn));
+    VLM_TRY(d2h(ctx, piv.data(), dp, sizeof(int) * (n + 1)));
+    std::memcpy(ipiv, piv.data(), sizeof(int) * n);
+    const int info = piv[n];
     if (info != 0) return fail(ctx, VLM_ERR_SINGULAR, "matrix is singular (zero pivot)");
     return VLM_OK;
 }
@@ -724,15 +723,15 @@ int vlm_lu_solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, 
     std::vector<int> perm(ipiv, ipiv + n);
     if (n > SOLVE_WAVE_N2) compose_pivots(n, ipiv, perm.data());
     VLM_DEVICE(ctx);
-    DBuf<double> dA, dLU;
-    DBuf<int> dp;
-    VLM_HIP(dA.reserve((size_t)n * n));
-    VLM_HIP(dLU.reserve((size_t)n * n));
-    VLM_HIP(dp.reserve((size_t)n));
-    VLM_HIP(hipMemcpyAsync(dA.p, A, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
-    VLM_HIP(hipMemcpyAsync(dLU.p, LU, sizeof(double) * n * n, hipMemcpyHostToDevice, ctx->stream));
-    VLM_TRY(h2d(ctx, dp.p, perm.data(), sizeof(int) * n));
-    return solve_refine(ctx, n, dA.p, dLU.p, dp.p, rhs, x, max_iter, tol, iters);
+    const size_t nn = (size_t)n * n;
+    VLM_HIP(ctx->hostio.reserve(2 * nn));
+    VLM_HIP(ctx->hostio_i.reserve((size_t)n + 1));
+    double *dA = ctx->hostio.p, *dLU = dA + nn;
+    int *dp = ctx->hostio_i.p;
+    VLM_TRY(h2d(ctx, dA, A, sizeof(double) * nn));
+    VLM_TRY(h2d(ctx, dLU, LU, sizeof(double) * nn));
+    VLM_TRY(h2d(ctx, dp, perm.data(), sizeof(int) * n));
+    return solve_refine(ctx, n, dA, dLU, dp, rhs, x, max_iter, tol, iters);
 }
 
 }  // extern "C"

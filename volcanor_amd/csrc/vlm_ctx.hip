@@ -1,5 +1,6 @@
 // Context, error handling, segment compaction, explicit filament sets and
 // kernel timing for libvlm.
+#include <algorithm>
 #include <cstring>
 
 #include "vlm_internal.h"
@@ -22,27 +23,110 @@ namespace {
 
 unsigned nblk(int64_t n) { return (unsigned)((n + 255) / 256); }
 
+constexpr size_t CALL_BYTES = (size_t)4 << 20;
+
 // Records of an explicit list (every filament kept, at its own index), one
 // lane per segment of the padded list, and its count.
+__device__ void explicit_record(int64_t n, int64_t k, const double *a, const double *b, double g,
+                                double rc, const SegPtrs &L)
+{
+    if (k == 0) *L.count = (long long)n;
+    if ((k & ~(int64_t)(GRP - 1)) >= n) return;   // whole groups leave together
+    Slot s;
+    s.ax = a[0];
+    s.ay = a[1];
+    s.az = a[2];
+    s.bx = b[0];
+    s.by = b[1];
+    s.bz = b[2];
+    s.gam = g;
+    s.rc = rc;
+    write_group_records(s, k < n, k, L);
+}
+
 __global__ __launch_bounds__(256) void explicit_records_kernel(int64_t n, const double *a,
                                                                const double *b, const double *g,
                                                                const double *rc, SegPtrs L)
 {
     const int64_t k = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (k == 0) *L.count = (long long)n;
-    if ((k & ~(int64_t)(GRP - 1)) >= n) return;   // whole groups leave together
-    const bool valid = k < n;
-    const int64_t i = valid ? k : n - 1;
-    Slot s;
-    s.ax = a[3 * i];
-    s.ay = a[3 * i + 1];
-    s.az = a[3 * i + 2];
-    s.bx = b[3 * i];
-    s.by = b[3 * i + 1];
-    s.bz = b[3 * i + 2];
-    s.gam = g[i];
-    s.rc = rc[i];
-    write_group_records(s, valid, k, L);
+    const int64_t i = k < n ? k : n - 1;
+    if (n > 0) explicit_record(n, k, a + 3 * i, b + 3 * i, g[i], rc[i], L);
+    else if (k == 0) *L.count = 0;
+}
+
+// 256 points of a host list (xyz per point) on their way to LDS, so that
+// reads of pinned memory are whole lines; the loads issue together (a round
+// trip to the host takes some 2 us).
+struct Triples {
+    double x[3];
+    __device__ Triples(const double *p, int64_t i0, int64_t m)
+    {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) x[q] = p[min(3 * i0 + q * 256 + threadIdx.x, 3 * m - 1)];
+    }
+    __device__ void put(double *sh) const
+    {
+#pragma unroll
+        for (int q = 0; q < 3; ++q) sh[q * 256 + threadIdx.x] = x[q];
+    }
+};
+
+__device__ void points_block(const double *p, int64_t blk, int64_t m, double *soa, int64_t stride,
+                             double *sh)
+{
+    const int64_t i0 = blk * 256, i = i0 + threadIdx.x;
+    const Triples t(p, i0, m);
+    t.put(sh);
+    __syncthreads();
+    if (i >= m) return;
+    for (int d = 0; d < 3; ++d) soa[d * stride + i] = sh[3 * threadIdx.x + d];
+}
+
+// xyz per point -> SoA
+__global__ __launch_bounds__(256) void aos_to_soa_kernel(int64_t m, const double *aos,
+                                                         double *soa, int64_t stride)
+{
+    __shared__ double sh[768];
+    points_block(aos, blockIdx.x, m, soa, stride, sh);
+}
+
+// SoA -> xyz per point
+__global__ __launch_bounds__(256) void soa_to_aos_kernel(int64_t m, const double *soa,
+                                                         int64_t stride, double *aos)
+{
+    __shared__ double sh[768];
+    const int64_t i0 = (int64_t)blockIdx.x * 256, i = i0 + threadIdx.x;
+    if (i < m)
+        for (int d = 0; d < 3; ++d) sh[3 * threadIdx.x + d] = soa[d * stride + i];
+    __syncthreads();
+    const int64_t left = 3 * (m - i0);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) {
+        const int e = q * 256 + threadIdx.x;
+        if (e < left) aos[3 * i0 + e] = sh[e];
+    }
+}
+
+// The filaments (a | b | circulations | radii) and points of one call, in
+// pinned memory, as records and SoA targets: blocks below fblocks take 256
+// filaments each.
+__global__ __launch_bounds__(256) void call_inputs_kernel(const double *h, int64_t n, SegPtrs L,
+                                                          int fblocks, const double *p, int64_t m,
+                                                          double *t)
+{
+    __shared__ double sa[768], sb[768];
+    if ((int)blockIdx.x >= fblocks) {
+        points_block(p, (int)blockIdx.x - fblocks, m, t, m, sa);
+        return;
+    }
+    const int64_t i0 = (int64_t)blockIdx.x * 256, k = i0 + threadIdx.x;
+    const int64_t i = k < n ? k : n - 1;
+    const Triples a(h, i0, n), b(h + 3 * n, i0, n);
+    const double g = h[6 * n + i], rc = h[7 * n + i];
+    a.put(sa);
+    b.put(sb);
+    __syncthreads();
+    explicit_record(n, k, sa + 3 * (i - i0), sb + 3 * (i - i0), g, rc, L);
 }
 
 }  // namespace
@@ -58,43 +142,17 @@ int explicit_records(vlm_ctx *ctx, int64_t n, const double *a, const double *b, 
 
 namespace {
 
-// AoS host layout (3 x m) -> SoA device layout
-__global__ void aos_to_soa_kernel(int64_t m, const double *aos, double *soa, int64_t stride)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    soa[i] = aos[3 * i];
-    soa[stride + i] = aos[3 * i + 1];
-    soa[2 * stride + i] = aos[3 * i + 2];
-}
-
-__global__ void soa_to_aos_kernel(int64_t m, const double *soa, int64_t stride, double *aos)
-{
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
-    aos[3 * i] = soa[i];
-    aos[3 * i + 1] = soa[stride + i];
-    aos[3 * i + 2] = soa[2 * stride + i];
-}
-
 int upload_fset(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b,
                 const double *gam, const double *rc, int formats, SegList &seg, SegPtrs *view)
 {
-    DBuf<double> raw;
-    VLM_HIP(raw.reserve((size_t)8 * nfil));
-    VLM_HIP(hipMemcpyAsync(raw.p, a, sizeof(double) * 3 * nfil, hipMemcpyHostToDevice,
-                           ctx->stream));
-    VLM_HIP(hipMemcpyAsync(raw.p + 3 * nfil, b, sizeof(double) * 3 * nfil,
-                           hipMemcpyHostToDevice, ctx->stream));
-    VLM_HIP(hipMemcpyAsync(raw.p + 6 * nfil, gam, sizeof(double) * nfil, hipMemcpyHostToDevice,
-                           ctx->stream));
-    VLM_HIP(hipMemcpyAsync(raw.p + 7 * nfil, rc, sizeof(double) * nfil, hipMemcpyHostToDevice,
-                           ctx->stream));
+    VLM_HIP(ctx->hostio.reserve((size_t)8 * nfil));
+    double *raw = ctx->hostio.p;
+    VLM_TRY(h2d(ctx, raw, a, sizeof(double) * 3 * nfil));
+    VLM_TRY(h2d(ctx, raw + 3 * nfil, b, sizeof(double) * 3 * nfil));
+    VLM_TRY(h2d(ctx, raw + 6 * nfil, gam, sizeof(double) * nfil));
+    VLM_TRY(h2d(ctx, raw + 7 * nfil, rc, sizeof(double) * nfil));
     VLM_HIP(seg.reserve(nfil, formats, view));
-    VLM_TRY(explicit_records(ctx, nfil, raw.p, raw.p + 3 * nfil, raw.p + 6 * nfil,
-                             raw.p + 7 * nfil, *view));
-    VLM_TRY(sync_stream(ctx));  // raw is released on return
-    return VLM_OK;
+    return explicit_records(ctx, nfil, raw, raw + 3 * nfil, raw + 6 * nfil, raw + 7 * nfil, *view);
 }
 
 }  // namespace
@@ -162,13 +220,29 @@ int pin_take(vlm_ctx *ctx, size_t bytes, char **out)
     return VLM_OK;
 }
 
+static int piece_event(vlm_ctx *ctx, int slot)
+{
+    if (!ctx->io_ev[slot])
+        VLM_HIP(hipEventCreateWithFlags(&ctx->io_ev[slot], hipEventDisableTiming));
+    VLM_HIP(hipEventRecord(ctx->io_ev[slot], ctx->stream));
+    return VLM_OK;
+}
+
 int h2d(vlm_ctx *ctx, void *dst, const void *src, size_t bytes)
 {
     if (bytes == 0) return VLM_OK;
     char *p = nullptr;
-    VLM_TRY(pin_take(ctx, bytes, &p));
-    std::memcpy(p, src, bytes);
-    VLM_HIP(hipMemcpyAsync(dst, p, bytes, hipMemcpyHostToDevice, ctx->stream));
+    const size_t piece = bytes < PIN_PIECE ? bytes : PIN_PIECE;
+    VLM_TRY(pin_take(ctx, bytes <= piece ? bytes : 2 * piece, &p));
+    int k = 0;
+    for (size_t o = 0; o < bytes; o += piece, ++k) {
+        const size_t n = std::min(piece, bytes - o);
+        char *q = p + (k & 1) * piece;
+        if (k >= 2) VLM_HIP(hipEventSynchronize(ctx->io_ev[k & 1]));
+        std::memcpy(q, (const char *)src + o, n);
+        VLM_HIP(hipMemcpyAsync((char *)dst + o, q, n, hipMemcpyHostToDevice, ctx->stream));
+        if (bytes > piece) VLM_TRY(piece_event(ctx, k & 1));
+    }
     return VLM_OK;
 }
 
@@ -176,19 +250,38 @@ int d2h(vlm_ctx *ctx, void *dst, const void *src, size_t bytes)
 {
     if (bytes == 0) return sync_stream(ctx);
     char *p = nullptr;
-    VLM_TRY(pin_take(ctx, bytes, &p));
-    VLM_HIP(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    VLM_TRY(sync_stream(ctx));
-    std::memcpy(dst, p, bytes);
-    return VLM_OK;
+    const size_t piece = bytes < PIN_PIECE ? bytes : PIN_PIECE;
+    VLM_TRY(pin_take(ctx, bytes <= piece ? bytes : 2 * piece, &p));
+    if (bytes <= piece) {
+        VLM_HIP(hipMemcpyAsync(p, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+        VLM_TRY(sync_stream(ctx));
+        std::memcpy(dst, p, bytes);
+        return VLM_OK;
+    }
+    const size_t np = (bytes + piece - 1) / piece;
+    for (size_t k = 0; k <= np; ++k) {
+        if (k < np) {
+            VLM_HIP(hipMemcpyAsync(p + (k & 1) * piece, (const char *)src + k * piece,
+                                   std::min(piece, bytes - k * piece), hipMemcpyDeviceToHost,
+                                   ctx->stream));
+            VLM_TRY(piece_event(ctx, k & 1));
+        }
+        if (k > 0) {
+            VLM_HIP(hipEventSynchronize(ctx->io_ev[(k - 1) & 1]));
+            std::memcpy((char *)dst + (k - 1) * piece, p + ((k - 1) & 1) * piece,
+                        std::min(piece, bytes - (k - 1) * piece));
+        }
+    }
+    return sync_stream(ctx);
 }
 
 int points_to_device(vlm_ctx *ctx, int64_t m, const double *p, double *soa, int64_t stride)
 {
-    VLM_HIP(ctx->hostio.reserve((size_t)3 * m));
-    VLM_TRY(h2d(ctx, ctx->hostio.p, p, sizeof(double) * 3 * m));
+    char *h = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(double) * 3 * m, &h));
+    std::memcpy(h, p, sizeof(double) * 3 * m);
     hipLaunchKernelGGL(aos_to_soa_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m,
-                       ctx->hostio.p, soa, stride);
+                       reinterpret_cast<const double *>(h), soa, stride);
     VLM_HIP(hipGetLastError());
     return VLM_OK;
 }
@@ -196,12 +289,15 @@ int points_to_device(vlm_ctx *ctx, int64_t m, const double *p, double *soa, int6
 int points_to_host(vlm_ctx *ctx, int64_t m, const double *soa, int64_t stride, double *p,
                    bool deferred = false)
 {
-    VLM_HIP(ctx->hostio.reserve((size_t)3 * m));
+    char *h = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(double) * 3 * m, &h));
     hipLaunchKernelGGL(soa_to_aos_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, soa,
-                       stride, ctx->hostio.p);
+                       stride, reinterpret_cast<double *>(h));
     VLM_HIP(hipGetLastError());
-    if (deferred) return d2h_deferred(ctx, p, ctx->hostio.p, sizeof(double) * 3 * m);
-    return d2h(ctx, p, ctx->hostio.p, sizeof(double) * 3 * m);
+    if (deferred) return defer(ctx, {{p, h, sizeof(double) * 3 * m}});
+    VLM_TRY(sync_stream(ctx));
+    std::memcpy(p, h, sizeof(double) * 3 * m);
+    return VLM_OK;
 }
 
 }  // namespace vlm
@@ -256,6 +352,8 @@ int vlm_destroy(vlm_ctx *ctx)
     if (ctx->pin) (void)hipHostFree(ctx->pin);
     if (ctx->judge_ev) (void)hipEventDestroy(ctx->judge_ev);
     if (ctx->defer_ev) (void)hipEventDestroy(ctx->defer_ev);
+    for (auto e : ctx->io_ev)
+        if (e) (void)hipEventDestroy(e);
     if (ctx->judge_pin) (void)hipHostFree(ctx->judge_pin);
     (void)hipStreamDestroy(ctx->stream);
     delete ctx;
@@ -307,16 +405,44 @@ int vlm_filament_vind(vlm_ctx *ctx, int64_t nfil, const double *a, const double 
     if (!p || !v || (nfil > 0 && (!a || !b || !gam || !rc)))
         return fail(ctx, VLM_ERR_ARG, "null buffer");
     VLM_HIP(hipSetDevice(ctx->device));
-    FSet fs;
+    const int formats = bs_formats(ctx, m, nfil);
+    VLM_HIP(ctx->tgt.reserve(ws_size<double>((size_t)3 * m)));
+    VLM_HIP(ctx->seg.reserve(std::max<int64_t>(nfil, 4096), formats, &ctx->seg_view));
+    // Inputs of up to CALL_BYTES are read, and the result is written, by
+    // kernels in pinned memory: three launches and one wait (300 points,
+    // 2000 filaments: 39 us a call, against 88 with allocations and four
+    // copies).  Larger ones are copied first (a kernel that gathers them from the host loses what the
+    // copy of one piece beside the host's copy of the next gains).
+    const size_t fil = (size_t)8 * nfil, pts = (size_t)3 * m;
+    if (sizeof(double) * (fil + 2 * pts) <= CALL_BYTES) {
+        char *hp = nullptr;
+        VLM_TRY(pin_take(ctx, sizeof(double) * (fil + 2 * pts), &hp));
+        double *h = reinterpret_cast<double *>(hp), *ph = h + fil, *vh = ph + pts;
+        if (nfil > 0) {
+            std::memcpy(h, a, sizeof(double) * 3 * nfil);
+            std::memcpy(h + 3 * nfil, b, sizeof(double) * 3 * nfil);
+            std::memcpy(h + 6 * nfil, gam, sizeof(double) * nfil);
+            std::memcpy(h + 7 * nfil, rc, sizeof(double) * nfil);
+        }
+        std::memcpy(ph, p, sizeof(double) * pts);
+        if (accumulate) std::memcpy(vh, v, sizeof(double) * pts);
+        const unsigned fb = nblk(nfil);
+        hipLaunchKernelGGL(call_inputs_kernel, dim3(fb + nblk(m)), dim3(256), 0, ctx->stream, h,
+                           nfil, ctx->seg_view, (int)fb, ph, m, ctx->tgt.p);
+        VLM_HIP(hipGetLastError());
+        VLM_TRY(bs_eval(ctx, ctx->seg_view, nfil, ctx->tgt.p, m, m, vh, accumulate, nullptr,
+                        true));
+        VLM_TRY(sync_stream(ctx));
+        std::memcpy(v, vh, sizeof(double) * pts);
+        return VLM_OK;
+    }
     if (nfil > 0)
-        VLM_TRY(upload_fset(ctx, nfil, a, b, gam, rc, bs_formats(ctx, m), fs.seg, &fs.view));
-    VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
-    VLM_HIP(ctx->out.reserve((size_t)3 * m));
+        VLM_TRY(upload_fset(ctx, nfil, a, b, gam, rc, formats, ctx->seg, &ctx->seg_view));
+    VLM_HIP(ctx->out.reserve(ws_size<double>(pts)));
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
-    VLM_TRY(bs_eval(ctx, fs.view, nfil, ctx->tgt.p, m, m, ctx->out.p, accumulate));
-    VLM_TRY(points_to_host(ctx, m, ctx->out.p, m, v));
-    return VLM_OK;
+    VLM_TRY(bs_eval(ctx, ctx->seg_view, nfil, ctx->tgt.p, m, m, ctx->out.p, accumulate));
+    return points_to_host(ctx, m, ctx->out.p, m, v);
 }
 
 int vlm_fset_create(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b,

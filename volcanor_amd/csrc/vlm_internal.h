@@ -41,6 +41,16 @@ struct DBuf {
     }
 };
 
+// Elements to reserve for a workspace that grows with a run: at least 256 kB,
+// so that a short list grows it once and not at each doubling (hipFree waits
+// for the device).
+template <typename T>
+inline size_t ws_size(size_t n)
+{
+    const size_t least = ((size_t)256 << 10) / sizeof(T);
+    return n > least ? n : least;
+}
+
 // Compacted straight-segment list, in groups of GRP consecutive segments.
 // Every segment has one record that a wave reads through the scalar cache
 // (16 values = two or one s_load_dwordx16), so the records are arrays of
@@ -50,7 +60,7 @@ struct DBuf {
 //   near32 (8 floats):  a_hi(3) q' | a_lo(3) -   (a = a_hi + a_lo; q' = q, or
 //                       infinity for q <= 1e-18)
 //   grp (4 doubles per group): centre c, squared far radius
-// Launches with few targets put segments on lanes instead and read one
+// Launches of few pairs put segments on lanes instead and read one
 // structure of arrays (stride cap):
 //   soa (9): ax ay az g | r0x r0y r0z qq | n0
 // with g = gam / (4 pi), r0 = b - a, n0 = |r0|^2, q = rc^2 n0, qq = q^2 and
@@ -60,7 +70,7 @@ struct DBuf {
 constexpr int GRP = 32;
 constexpr int SOA_N = 9, REC64_N = 16, REC32_N = 16, NEAR32_N = 8, GRPH_N = 4;
 
-// What a list holds; a launch with m targets needs bs_formats(m).
+// What a list holds; a launch with m targets needs bs_formats(m, its segments).
 enum { SEG_SOA = 1, SEG_REC = 2, SEG_F32 = 4, SEG_ALL = 7 };
 
 // Device pointers of a list (null where a format is absent).
@@ -217,7 +227,9 @@ struct vlm_ctx {
     vlm::DBuf<double> tgt, out, part;
     vlm::DBuf<int> counter;  // work counter of the Biot-Savart launches, 0 between them
     int occ[2] = {0, 0};     // resident workgroups per kernel (FP64, mixed)
-    vlm::DBuf<double> hostio;  // device staging for host point lists
+    vlm::DBuf<double> hostio;  // device copy of host filament lists and matrices
+    vlm::DBuf<int> hostio_i;
+    hipEvent_t io_ev[2] = {nullptr, nullptr};  // pieces of a copy in flight (h2d, d2h)
     // pinned host arena for host<->device copies: truly asynchronous copies,
     // reset whenever the stream has been synchronised
     char *pin = nullptr;
@@ -361,7 +373,8 @@ __device__ __forceinline__ void write_group_records(const Slot &s, bool valid, i
 
 // Biot-Savart evaluation of a compacted segment list at m targets stored
 // as SoA (x at t[0..], y at t[tstride..], z at t[2*tstride..]).  Result
-// goes to out (SoA, same stride); accumulate adds into it.  nseg_est is the
+// goes to out (SoA of stride tstride, or with aos xyz per target, also in
+// pinned host memory); accumulate adds into it.  nseg_est is the
 // expected count (0: the list is empty): it sets the number of chunks, and
 // the kernel divides the device count evenly among them.
 // A fixed workspace for bs_eval instead of the context's growing buffers
@@ -374,11 +387,13 @@ struct BsWork {
     int *counter;
 };
 int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t, int64_t m,
-            int64_t tstride, double *out, int accumulate, const BsWork *ws = nullptr);
-// The list formats that a launch with m targets reads.
-int bs_formats(const vlm_ctx *ctx, int64_t m);
+            int64_t tstride, double *out, int accumulate, const BsWork *ws = nullptr,
+            bool aos = false);
+// The list formats that a launch with m targets and (about) nseg segments
+// reads.
+int bs_formats(const vlm_ctx *ctx, int64_t m, int64_t nseg);
 
-// Few targets (bs_formats(m) == SEG_SOA), up to TERM_MAX lists in one
+// Short work (bs_formats == SEG_SOA), up to TERM_MAX lists in one
 // structure of arrays: list k starts at segment off[k] and has seg.count[k]
 // segments (about est[k]).
 //   u = accumulate ? out : 0;  for k: u = (neg[k] ? -u : u) + velocity of k;
@@ -391,7 +406,7 @@ struct TermLists {
 };
 int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, const double *t,
                   int64_t m, int64_t tstride, double *out, int accumulate,
-                  const BsWork *ws = nullptr);
+                  const BsWork *ws = nullptr, bool aos = false);
 
 // Records of an explicit list (every filament kept, at its own index) from
 // 3 x n device arrays, and its count.
@@ -410,7 +425,12 @@ void mlp_release(vlm_ctx *ctx);
 // host bytes into the arena and enqueues an asynchronous copy, so the
 // caller's buffer is free on return without a stream synchronisation;
 // sync_stream waits for the stream and recycles the arena; d2h enqueues the
-// copy, synchronises and copies out of the arena.
+// copy, synchronises and copies out of the arena.  Copies above PIN_PIECE
+// go piece by piece, the host's copy of one piece beside the transfer of the
+// other (38 MB: 1.4 ms from and 2.2 ms to unpinned memory, 1.3 ms so).
+// Kernels may read and write the arena themselves, which spares a small
+// call the copies' launches.
+constexpr size_t PIN_PIECE = (size_t)2 << 20;
 int pin_take(vlm_ctx *ctx, size_t bytes, char **out);
 int h2d(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);
 int d2h(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);

@@ -1239,9 +1239,9 @@ int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, Te
     a.iters = (int)((all + 256 * (STAGE_BLOCKS - spare) - 1) / (256 * (STAGE_BLOCKS - spare)));
     if (a.iters < 1) a.iters = 1;
     const int64_t bi = 256 * (int64_t)a.iters;   // items per block
-    VLM_HIP(ctx->slots.reserve((size_t)(all / bi + spare + 1) * a.iters * 512));
+    VLM_HIP(ctx->slots.reserve(ws_size<Slot>((size_t)(all / bi + spare + 1) * a.iters * 512)));
     VLM_HIP(ctx->seg_counts.reserve(STAGE_BLOCKS));
-    VLM_HIP(ctx->seg.reserve(cap, formats, &ctx->seg_view));
+    VLM_HIP(ctx->seg.reserve(std::max<int64_t>(cap, 4096), formats, &ctx->seg_view));
     a.slots = ctx->slots.p;
     a.counts = ctx->seg_counts.p;
     a.n = 0;
@@ -1261,7 +1261,7 @@ int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, Te
         tblocks = 0;
     };
     if (pred >= 0) {
-        VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
+        VLM_HIP(ctx->tgt.reserve(ws_size<double>((size_t)3 * m)));
         a.tgt = ctx->tgt.p;
         a.tstride = m;
         int64_t off = 0;
@@ -1311,6 +1311,15 @@ int build_lists(vlm_ctx *ctx, const std::vector<Sources> &terms, int formats, Te
                        ctx->seg_counts.p, tab, ctx->seg_view);
     VLM_HIP(hipGetLastError());
     return VLM_OK;
+}
+
+// The expected number of segments of a list.
+int64_t expected(vlm_ctx *ctx, const Sources &src)
+{
+    std::vector<SrcDesc> ds;
+    int64_t n = 0, est = 0;
+    source_descs(ctx, src, ds, &n, &est);
+    return est;
 }
 
 // One list; *est receives its expected number of segments.
@@ -1520,8 +1529,8 @@ static int wake_pass(vlm_ctx *ctx, int pred, int64_t *mp)
     *mp = m;
     if (m == 0) return VLM_OK;
     int64_t nest = 0;
-    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest, pred, m));
-    VLM_HIP(ctx->out.reserve((size_t)3 * m));
+    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m, expected(ctx, src)), &nest, pred, m));
+    VLM_HIP(ctx->out.reserve(ws_size<double>((size_t)3 * m)));
     return eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, 0, nest);
 }
 
@@ -1788,10 +1797,11 @@ int learned_pass(vlm_ctx *ctx, int64_t *mp)
     int64_t nest = 0;
     // the full pass reads m targets, the judge about m / stride of them
     const int64_t stride0 = P.stride < 1 ? 1 : P.stride;
-    int formats = bs_formats(ctx, m) | bs_formats(ctx, (m + stride0 - 1) / stride0) |
-                  bs_formats(ctx, std::max<int64_t>(1, (m - stride0) / stride0));
+    const int64_t est = expected(ctx, src);
+    int formats = bs_formats(ctx, m, est) | bs_formats(ctx, (m + stride0 - 1) / stride0, est) |
+                  bs_formats(ctx, std::max<int64_t>(1, (m - stride0) / stride0), est);
     VLM_TRY(build_sources(ctx, src, formats, &nest, 1, m));
-    VLM_HIP(ctx->out.reserve((size_t)3 * m));
+    VLM_HIP(ctx->out.reserve(ws_size<double>((size_t)3 * m)));
     VLM_HIP(P.vn.reserve((size_t)3 * m));
     VLM_HIP(P.X.reserve((size_t)45 * m));
     VLM_HIP(P.Y.reserve((size_t)3 * m));
@@ -2281,9 +2291,9 @@ int vlm_rotor_induced_velocity(vlm_ctx *ctx, int ir, int set, int64_t m, const d
     if (!p || !v) return fail(ctx, VLM_ERR_ARG, "null buffer");
     Sources src = {{ir, set}};
     int64_t nest = 0;
-    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m), &nest));
-    VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
-    VLM_HIP(ctx->out.reserve((size_t)3 * m));
+    VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m, expected(ctx, src)), &nest));
+    VLM_HIP(ctx->tgt.reserve(ws_size<double>((size_t)3 * m)));
+    VLM_HIP(ctx->out.reserve(ws_size<double>((size_t)3 * m)));
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
     VLM_TRY(eval_sources(ctx, ctx->tgt.p, m, m, ctx->out.p, accumulate, nest));
@@ -2300,7 +2310,6 @@ static int ordered_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set
                          const int *flags, int64_t m, const double *tgt, double *out,
                          int accumulate)
 {
-    const int fmt = bs_formats(ctx, m);
     if (nterms == 0 && !accumulate) {
         hipLaunchKernelGGL(fill_kernel, dim3(nblk(3 * m)), dim3(256), 0, ctx->stream, out, 3 * m,
                            0.0);
@@ -2308,10 +2317,16 @@ static int ordered_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set
     }
     int acc = accumulate;
     for (int k = 0; k < nterms;) {
-        const int n = fmt == SEG_SOA ? std::min(TERM_MAX, nterms - k) : 1;
+        int fmt = 0, n = 0;
         std::vector<Sources> src;
         TermLists lists;
-        for (int q = 0; q < n; ++q) src.push_back({{ir[k + q], set[k + q]}});
+        for (; n < TERM_MAX && k + n < nterms; ++n) {
+            const Sources s = {{ir[k + n], set[k + n]}};
+            const int f = bs_formats(ctx, m, expected(ctx, s));
+            if (n > 0 && (f != SEG_SOA || fmt != SEG_SOA)) break;
+            fmt = f;
+            src.push_back(s);
+        }
         VLM_TRY(build_lists(ctx, src, fmt, &lists));
         for (int q = 0; q < n; ++q) lists.neg[q] = (flags[k + q] & VLM_TERM_NEGATE) != 0;
         if (fmt == SEG_SOA) {
@@ -2345,8 +2360,8 @@ static int induced_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set
     }
     if (m <= 0) return VLM_OK;
     if (!p || !v) return fail(ctx, VLM_ERR_ARG, "null buffer");
-    VLM_HIP(ctx->tgt.reserve((size_t)3 * m));
-    VLM_HIP(ctx->out.reserve((size_t)3 * m));
+    VLM_HIP(ctx->tgt.reserve(ws_size<double>((size_t)3 * m)));
+    VLM_HIP(ctx->out.reserve(ws_size<double>((size_t)3 * m)));
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
     VLM_TRY(ordered_terms(ctx, nterms, ir, set, flags, m, ctx->tgt.p, ctx->out.p, accumulate));
