@@ -8,13 +8,18 @@
 // Parameter packing (row-major W[out][in]):
 //   W1 64x45 | b1 64 | W2 64x64 | b2 64 | W3 64x64 | b3 64 | W4 3x64 | b4 3
 //
-// Every layer is a small matrix product on the matrix cores (FP32 MFMA):
-// a workgroup takes a tile of 64 samples, each of its four waves 16 of
-// them, with the parameters and activations in LDS.  Training runs the
-// forward pass, the loss, the backward deltas and the tile's weight
-// gradients in one kernel per tile; a second kernel adds the tile
-// gradients in a fixed order (deterministic, no atomics) and applies Adam.
+// Every layer is a small matrix product on the matrix cores (FP32 MFMA).  A
+// workgroup takes tiles of 16 samples; each of its four waves owns 16
+// columns of every layer and keeps their weights (and, for training, the
+// weight gradients) in registers, and activations and deltas pass between
+// the waves through LDS.  Both kernels are bound by the latency of that chain
+// (six products, six barriers), so tiles are small and many: with 64 samples
+// per workgroup, weights staged in LDS and a gradient row per tile, a batch
+// of 2048 took 50 us on 32 CUs and its reduction and loss 14 us.
+// Training writes one partial gradient per workgroup; a second kernel adds
+// them in a fixed order (deterministic, no atomics) and applies Adam.
 #include <cmath>
+#include <cstring>
 #include <vector>
 
 #include "vlm_internal.h"
@@ -31,6 +36,8 @@ constexpr int OFF_B3 = OFF_W3 + MLP_H * MLP_H;
 constexpr int OFF_W4 = OFF_B3 + MLP_H;
 constexpr int OFF_B4 = OFF_W4 + MLP_OUT * MLP_H;
 constexpr int MLP_NP = OFF_B4 + MLP_OUT;  // 11459
+// Host batches up to this size are read by the kernels in pinned memory.
+constexpr size_t MLP_DIRECT = (size_t)4 << 20;
 
 namespace {
 
@@ -39,247 +46,328 @@ namespace {
 // register r of lane l is D[4*(l/16) + r][l%16].
 typedef float fx4 __attribute__((ext_vector_type(4)));
 
-constexpr int TS = 64;            // samples per tile (one workgroup, four waves)
-constexpr int K1 = 48;            // MLP_IN padded to a multiple of 4
-constexpr int LW1 = K1 + 1;       // LDS row strides
-constexpr int LH = MLP_H + 1;
-constexpr int LDY = 16 + 1;
-// LDS image of the parameters: W1 64 x LW1 | W2 64 x LH | W3 64 x LH |
-// W4 16 x LH (rows 3..15 zero) | b1 b2 b3 (64 each) | b4 (16, padded)
-constexpr int S_W1 = 0;
-constexpr int S_W2 = S_W1 + MLP_H * LW1;
-constexpr int S_W3 = S_W2 + MLP_H * LH;
-constexpr int S_W4 = S_W3 + MLP_H * LH;
-constexpr int S_B1 = S_W4 + 16 * LH;
-constexpr int S_B2 = S_B1 + MLP_H;
-constexpr int S_B3 = S_B2 + MLP_H;
-constexpr int S_B4 = S_B3 + MLP_H;
-constexpr int S_NP = S_B4 + 16;
+constexpr int TS = 16;            // samples per tile (one workgroup, four waves)
+constexpr int LX = 52;            // LDS row strides: multiples of 4 (b128 reads) that
+constexpr int LH = 68;            // spread the 16 rows of a fragment over all banks
+constexpr int LDY = 20;
+constexpr int XE = 3;             // X elements per lane: TS x MLP_IN / 256, rounded up
+constexpr int MLP_ROWS = 512;     // workgroups (partial gradients) of a training launch
 
-__device__ void stage_params(const float *params, float *sp)
+// A product over K values runs as K / 4 steps in any order that A and B
+// share: step t takes k = lk K/4 + t, so that a lane's values are contiguous.
+template <int NT>
+__device__ __forceinline__ fx4 product(const float *row, const float (&b)[NT], fx4 acc)
 {
-    for (int k = threadIdx.x; k < S_NP; k += blockDim.x) {
-        float v = 0.f;
-        if (k < S_W2) {
-            const int o = k / LW1, i = k % LW1;
-            if (i < MLP_IN) v = params[OFF_W1 + o * MLP_IN + i];
-        } else if (k < S_W3) {
-            const int o = (k - S_W2) / LH, i = (k - S_W2) % LH;
-            if (i < MLP_H) v = params[OFF_W2 + o * MLP_H + i];
-        } else if (k < S_W4) {
-            const int o = (k - S_W3) / LH, i = (k - S_W3) % LH;
-            if (i < MLP_H) v = params[OFF_W3 + o * MLP_H + i];
-        } else if (k < S_B1) {
-            const int o = (k - S_W4) / LH, i = (k - S_W4) % LH;
-            if (o < MLP_OUT && i < MLP_H) v = params[OFF_W4 + o * MLP_H + i];
-        } else if (k < S_B2) {
-            v = params[OFF_B1 + (k - S_B1)];
-        } else if (k < S_B3) {
-            v = params[OFF_B2 + (k - S_B2)];
-        } else if (k < S_B4) {
-            v = params[OFF_B3 + (k - S_B3)];
-        } else if (k - S_B4 < MLP_OUT) {
-            v = params[OFF_B4 + (k - S_B4)];
+    float a[NT];
+#pragma unroll
+    for (int t = 0; t < NT; t += 4) {
+        const float4 v = *reinterpret_cast<const float4 *>(row + t);
+        a[t] = v.x;
+        a[t + 1] = v.y;
+        a[t + 2] = v.z;
+        a[t + 3] = v.w;
+    }
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(a[t], b[t], acc, 0, 0, 0);
+    return acc;
+}
+
+// D^T Act over the tile's samples: A[o][s] = D[s][o], B[s][i] = Act[s][i].
+__device__ __forceinline__ fx4 outer(const float (&d)[4], const float *act, int la, fx4 acc)
+{
+#pragma unroll
+    for (int t = 0; t < 4; ++t)
+        acc = __builtin_amdgcn_mfma_f32_16x16x4f32(d[t], act[t * la], acc, 0, 0, 0);
+    return acc;
+}
+
+__device__ __forceinline__ void load16(const float *p, float (&w)[16])
+{
+#pragma unroll
+    for (int t = 0; t < 16; t += 4) {
+        const float4 v = *reinterpret_cast<const float4 *>(p + t);
+        w[t] = v.x;
+        w[t + 1] = v.y;
+        w[t + 2] = v.z;
+        w[t + 3] = v.w;
+    }
+}
+
+// The forward weights of a lane: column 16 w + li of layers 1 to 3, column li
+// of layer 4 (zero beyond the third).
+struct Forward {
+    float w1[12], w2[16], w3[16], w4[16], b1, b2, b3, b4;
+    __device__ Forward(const float *P, int w, int li, int lk)
+    {
+        const int c = 16 * w + li;
+#pragma unroll
+        for (int t = 0; t < 12; ++t) {
+            const int k = 12 * lk + t;
+            const float v = P[OFF_W1 + c * MLP_IN + min(k, MLP_IN - 1)];
+            w1[t] = k < MLP_IN ? v : 0.f;
         }
-        sp[k] = v;
+        load16(P + OFF_W2 + c * MLP_H + 16 * lk, w2);
+        load16(P + OFF_W3 + c * MLP_H + 16 * lk, w3);
+        load16(P + OFF_W4 + min(li, MLP_OUT - 1) * MLP_H + 16 * lk, w4);
+        b1 = P[OFF_B1 + c];
+        b2 = P[OFF_B2 + c];
+        b3 = P[OFF_B3 + c];
+        b4 = P[OFF_B4 + min(li, MLP_OUT - 1)];
+#pragma unroll
+        for (int t = 0; t < 16; ++t) w4[t] = li < MLP_OUT ? w4[t] : 0.f;
+    }
+};
+
+// The tile's elements of X (row-major), for LDS: requested one tile ahead.
+__device__ __forceinline__ void fetch_x(const float *X, int64_t s0, int64_t m, float (&x)[XE])
+{
+    const int64_t left = (m - s0) * MLP_IN;   // may be <= 0 past the last tile
+#pragma unroll
+    for (int q = 0; q < XE; ++q) {
+        const int e = q * 256 + threadIdx.x;
+        x[q] = e < TS * MLP_IN && e < left ? X[s0 * MLP_IN + e] : 0.f;
     }
 }
 
-// X tile (TS x MLP_IN, row-major in global) into LDS, zero padded.
-__device__ void stage_x(const float *X, int64_t s0, int64_t m, float *Xs)
+__device__ __forceinline__ void put_x(const float (&x)[XE], float *Xs)
 {
-    for (int e = threadIdx.x; e < TS * LW1; e += blockDim.x) {
-        const int s = e / LW1, k = e % LW1;
-        Xs[e] = (k < MLP_IN && s0 + s < m) ? X[(s0 + s) * MLP_IN + k] : 0.f;
+#pragma unroll
+    for (int q = 0; q < XE; ++q) {
+        const int e = q * 256 + threadIdx.x;
+        if (e < TS * MLP_IN) Xs[e / MLP_IN * LX + e % MLP_IN] = x[q];
     }
 }
 
-// Rows [16w, 16w+16) of O = act(A . W^T + b): A is TS x K (stride LA), W is
-// NOB*16 x K (stride LWt), O stride LO.
-template <int K, int LA, int LWt, int NOB, bool TANH>
-__device__ __forceinline__ void dense_fwd(const float *A, const float *W, const float *b, float *O,
-                                          int LO, int w, int l)
+// Zero padding of the input rows (columns 45 to 47).
+__device__ __forceinline__ void pad_x(float *Xs)
 {
-    const int li = l & 15, lk = l >> 4;
-#pragma unroll
-    for (int ob = 0; ob < NOB; ++ob) {
-        fx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k0 = 0; k0 < K; k0 += 4)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(A[(16 * w + li) * LA + k0 + lk],
-                                                       W[(16 * ob + li) * LWt + k0 + lk], acc, 0,
-                                                       0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int srow = 16 * w + 4 * lk + r, j = 16 * ob + li;
-            const float v = acc[r] + b[j];
-            O[srow * LO + j] = TANH ? tanhf(v) : v;
-        }
-    }
+    if (threadIdx.x < 3 * TS) Xs[threadIdx.x / 3 * LX + MLP_IN + threadIdx.x % 3] = 0.f;
 }
 
-// Rows [16w, 16w+16) of the backward delta: H <- (D . W) * (1 - H^2), where
-// D is TS x K (stride LD) and W is K x 64 (stride LWt); H holds tanh
-// outputs on entry and the deltas on exit.
-template <int K, int LD, int LWt>
-__device__ __forceinline__ void dense_bwd(const float *D, const float *W, float *H, int w, int l)
+// tanh layer: the lane's values are samples 4 lk + r of column c.
+template <int NT>
+__device__ __forceinline__ void layer(const float *row, const float (&w)[NT], float b, float *O,
+                                      int c, int lk, float (&h)[4])
 {
-    const int li = l & 15, lk = l >> 4;
+    const fx4 acc = product<NT>(row, w, fx4{0.f, 0.f, 0.f, 0.f});
 #pragma unroll
-    for (int ib = 0; ib < 4; ++ib) {
-        fx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k0 = 0; k0 < K; k0 += 4)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(D[(16 * w + li) * LD + k0 + lk],
-                                                       W[(k0 + lk) * LWt + 16 * ib + li], acc, 0,
-                                                       0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int srow = 16 * w + 4 * lk + r, j = 16 * ib + li;
-            const float h = H[srow * LH + j];
-            H[srow * LH + j] = acc[r] * (1.f - h * h);
-        }
-    }
-}
-
-// Tile gradient of one layer: dW[o][i] = sum_s D[s][o] Act[s][i] for the
-// 16 outputs of block ob and NIB input blocks, written to the tile's
-// partial-gradient row; bias gradients by lanes of wave 0.
-template <int NIB, int LD, int LA>
-__device__ __forceinline__ void dense_grad(const float *D, const float *Act, int ob, int nout,
-                                           int nin, float *gw, int l)
-{
-    const int li = l & 15, lk = l >> 4;
-#pragma unroll
-    for (int ib = 0; ib < NIB; ++ib) {
-        fx4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int k0 = 0; k0 < TS; k0 += 4)
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(D[(k0 + lk) * LD + 16 * ob + li],
-                                                       Act[(k0 + lk) * LA + 16 * ib + li], acc, 0,
-                                                       0, 0);
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int o = 16 * ob + 4 * lk + r, i = 16 * ib + li;
-            if (o < nout && i < nin) gw[o * nin + i] = acc[r];
-        }
-    }
-}
-
-__device__ __forceinline__ void bias_grad(const float *D, int LD, int nout, float *gb)
-{
-    const int o = threadIdx.x;
-    if (o < nout) {
-        float g = 0.f;
-        for (int s = 0; s < TS; ++s) g += D[s * LD + o];
-        gb[o] = g;
+    for (int r = 0; r < 4; ++r) {
+        h[r] = tanhf(acc[r] + b);
+        O[(4 * lk + r) * LH + c] = h[r];
     }
 }
 
 __global__ __launch_bounds__(256) void mlp_forward_kernel(const float *params, int64_t m,
                                                           const float *X, float *Y)
 {
-    __shared__ float sp[S_NP];
-    __shared__ float Xs[TS * LW1];
-    __shared__ float Ha[TS * LH], Hb[TS * LH];
-    __shared__ float Ys[TS * LDY];
-    stage_params(params, sp);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
+    __shared__ __align__(16) float Xs[TS * LX], Ha[TS * LH], Hb[TS * LH];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, li = l & 15, lk = l >> 4;
+    const int c = 16 * w + li;
     const int64_t ntiles = (m + TS - 1) / TS;
+    float x[XE], h[4];
+    fetch_x(X, (int64_t)blockIdx.x * TS, m, x);
+    const Forward f(params, w, li, lk);
+    pad_x(Xs);
     for (int64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
         const int64_t s0 = t * TS;
+        put_x(x, Xs);
+        fetch_x(X, s0 + (int64_t)gridDim.x * TS, m, x);
         __syncthreads();
-        stage_x(X, s0, m, Xs);
+        layer<12>(Xs + li * LX + 12 * lk, f.w1, f.b1, Ha, c, lk, h);
         __syncthreads();
-        dense_fwd<K1, LW1, LW1, 4, true>(Xs, sp + S_W1, sp + S_B1, Ha, LH, w, l);
+        layer<16>(Ha + li * LH + 16 * lk, f.w2, f.b2, Hb, c, lk, h);
         __syncthreads();
-        dense_fwd<MLP_H, LH, LH, 4, true>(Ha, sp + S_W2, sp + S_B2, Hb, LH, w, l);
+        layer<16>(Hb + li * LH + 16 * lk, f.w3, f.b3, Ha, c, lk, h);
         __syncthreads();
-        dense_fwd<MLP_H, LH, LH, 4, true>(Hb, sp + S_W3, sp + S_B3, Ha, LH, w, l);
-        __syncthreads();
-        dense_fwd<MLP_H, LH, LH, 1, false>(Ha, sp + S_W4, sp + S_B4, Ys, LDY, w, l);
-        __syncthreads();
-        for (int e = threadIdx.x; e < TS * MLP_OUT; e += blockDim.x) {
-            const int sl = e / MLP_OUT, o = e % MLP_OUT;
-            if (s0 + sl < m) Y[(s0 + sl) * MLP_OUT + o] = Ys[sl * LDY + o];
+        if (w == 0) {
+            const fx4 y = product<16>(Ha + li * LH + 16 * lk, f.w4, fx4{0.f, 0.f, 0.f, 0.f});
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int64_t s = s0 + 4 * lk + r;
+                if (li < MLP_OUT && s < m) Y[s * MLP_OUT + li] = y[r] + f.b4;
+            }
         }
     }
 }
 
-// One tile of a training batch: forward, loss 0.5 |y - t|^2 / m, backward
-// deltas and the tile's partial gradient (row `tile` of part).
+// Tiles of a training batch: forward, loss 0.5 |y - t|^2 / m, backward deltas
+// and the workgroup's partial gradient (row blockIdx.x of part).
 __global__ __launch_bounds__(256) void mlp_train_tile_kernel(const float *params, int64_t m,
                                                              const float *X, const float *T,
                                                              float *part, float *loss)
 {
-    __shared__ float sp[S_NP];
-    __shared__ float Xs[TS * LW1];
-    __shared__ float H1[TS * LH], H2[TS * LH], H3[TS * LH];
-    __shared__ float DY[TS * LDY];
-    __shared__ float red[256];
-    stage_params(params, sp);
-    const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
-    const int64_t tile = blockIdx.x, s0 = tile * TS;
-    float *g = part + (size_t)tile * MLP_NP;
-    stage_x(X, s0, m, Xs);
-    __syncthreads();
-    dense_fwd<K1, LW1, LW1, 4, true>(Xs, sp + S_W1, sp + S_B1, H1, LH, w, l);
-    __syncthreads();
-    dense_fwd<MLP_H, LH, LH, 4, true>(H1, sp + S_W2, sp + S_B2, H2, LH, w, l);
-    __syncthreads();
-    dense_fwd<MLP_H, LH, LH, 4, true>(H2, sp + S_W3, sp + S_B3, H3, LH, w, l);
-    __syncthreads();
-    dense_fwd<MLP_H, LH, LH, 1, false>(H3, sp + S_W4, sp + S_B4, DY, LDY, w, l);
-    __syncthreads();
-    // dy = (y - t) / m on real samples and outputs, zero elsewhere
+    __shared__ __align__(16) float Xs[TS * LX], H1[TS * LH], H2[TS * LH], H3[TS * LH];
+    __shared__ __align__(16) float D1[TS * LH], D2[TS * LH], D3[TS * LH], DYs[4][TS * LDY];
+    const int w = threadIdx.x >> 6, l = threadIdx.x & 63, li = l & 15, lk = l >> 4;
+    const int c = 16 * w + li;
+    const int64_t ntiles = (m + TS - 1) / TS;
     const float inv_m = 1.0f / (float)m;
-    float lsum = 0.f;
-    for (int e = threadIdx.x; e < TS * 16; e += blockDim.x) {
-        const int sl = e / 16, o = e % 16;
-        float d = 0.f;
-        if (o < MLP_OUT && s0 + sl < m) {
-            const float err = DY[sl * LDY + o] - T[(s0 + sl) * MLP_OUT + o];
-            lsum += 0.5f * err * err * inv_m;
-            d = err * inv_m;
+    const fx4 zero = {0.f, 0.f, 0.f, 0.f};
+    float x[XE], y[4];
+    fetch_x(X, (int64_t)blockIdx.x * TS, m, x);
+    auto fetch_t = [&](int64_t s0) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int64_t s = s0 + 4 * lk + r;
+            y[r] = li < MLP_OUT && s < m ? T[s * MLP_OUT + li] : 0.f;
         }
-        DY[sl * LDY + o] = d;
+    };
+    fetch_t((int64_t)blockIdx.x * TS);
+    const Forward f(params, w, li, lk);
+    // backward weights: rows k of W_{l+1} at the lane's column
+    float u2[16], u3[16], u4[4];
+#pragma unroll
+    for (int t = 0; t < 16; ++t) {
+        u2[t] = params[OFF_W2 + (16 * lk + t) * MLP_H + c];
+        u3[t] = params[OFF_W3 + (16 * lk + t) * MLP_H + c];
     }
-    red[threadIdx.x] = lsum;
-    __syncthreads();
-    for (int k = 128; k > 0; k >>= 1) {
-        if (threadIdx.x < k) red[threadIdx.x] += red[threadIdx.x + k];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const int o = 4 * lk + t;
+        const float v = params[OFF_W4 + min(o, MLP_OUT - 1) * MLP_H + c];
+        u4[t] = o < MLP_OUT ? v : 0.f;
+    }
+    fx4 g1[3] = {zero, zero, zero}, g2[4] = {zero, zero, zero, zero};
+    fx4 g3[4] = {zero, zero, zero, zero}, g4 = zero;
+    float gb1 = 0.f, gb2 = 0.f, gb3 = 0.f, gb4 = 0.f, lsum = 0.f;
+    float *DY = DYs[w];   // each wave has the output deltas for itself
+    pad_x(Xs);
+    for (int64_t tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
+        const int64_t s0 = tile * TS, s1 = s0 + (int64_t)gridDim.x * TS;
+        float h1[4], h2[4], h3[4], d[4];
+        put_x(x, Xs);
+        fetch_x(X, s1, m, x);
+        __syncthreads();
+        layer<12>(Xs + li * LX + 12 * lk, f.w1, f.b1, H1, c, lk, h1);
+        __syncthreads();
+        layer<16>(H1 + li * LH + 16 * lk, f.w2, f.b2, H2, c, lk, h2);
+        __syncthreads();
+        layer<16>(H2 + li * LH + 16 * lk, f.w3, f.b3, H3, c, lk, h3);
+        __syncthreads();
+        // dy = (y - t) / m on real samples and outputs, zero elsewhere
+        fx4 acc = product<16>(H3 + li * LH + 16 * lk, f.w4, zero);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float e = 0.f;
+            if (li < MLP_OUT && s0 + 4 * lk + r < m) {
+                const float err = acc[r] + f.b4 - y[r];
+                lsum += 0.5f * err * err * inv_m;
+                e = err * inv_m;
+            }
+            DY[(4 * lk + r) * LDY + li] = e;
+            gb4 += e;
+        }
+        fetch_t(s1);
+        // layer 4: gradient of the wave's 16 columns, delta of layer 3
+#pragma unroll
+        for (int t = 0; t < 4; ++t) d[t] = DY[(4 * lk + t) * LDY + li];
+        g4 = outer(d, H3 + 4 * lk * LH + c, LH, g4);
+        auto delta = [&](const fx4 &p, const float (&h)[4], float *D, float &gb) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float v = p[r] * (1.f - h[r] * h[r]);
+                D[(4 * lk + r) * LH + c] = v;
+                gb += v;
+            }
+            // the wave's columns, as the other factor of its gradients
+#pragma unroll
+            for (int t = 0; t < 4; ++t) d[t] = D[(4 * lk + t) * LH + c];
+        };
+        delta(product<4>(DY + li * LDY + 4 * lk, u4, zero), h3, D3, gb3);
+        __syncthreads();
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib)
+            g3[ib] = outer(d, H2 + 4 * lk * LH + 16 * ib + li, LH, g3[ib]);
+        delta(product<16>(D3 + li * LH + 16 * lk, u3, zero), h2, D2, gb2);
+        __syncthreads();
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib)
+            g2[ib] = outer(d, H1 + 4 * lk * LH + 16 * ib + li, LH, g2[ib]);
+        delta(product<16>(D2 + li * LH + 16 * lk, u2, zero), h1, D1, gb1);
+#pragma unroll
+        for (int ib = 0; ib < 3; ++ib)
+            g1[ib] = outer(d, Xs + 4 * lk * LX + 16 * ib + li, LX, g1[ib]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) loss[tile] = red[0];
-    // layer 4
-    if (w == 0) dense_grad<4, LDY, LH>(DY, H3, 0, MLP_OUT, MLP_H, g + OFF_W4, l);
-    bias_grad(DY, LDY, MLP_OUT, g + OFF_B4);
-    __syncthreads();
-    dense_bwd<16, LDY, LH>(DY, sp + S_W4, H3, w, l);       // H3 <- delta3
-    __syncthreads();
-    dense_grad<4, LH, LH>(H3, H2, w, MLP_H, MLP_H, g + OFF_W3, l);
-    bias_grad(H3, LH, MLP_H, g + OFF_B3);
-    __syncthreads();
-    dense_bwd<MLP_H, LH, LH>(H3, sp + S_W3, H2, w, l);     // H2 <- delta2
-    __syncthreads();
-    dense_grad<4, LH, LH>(H2, H1, w, MLP_H, MLP_H, g + OFF_W2, l);
-    bias_grad(H2, LH, MLP_H, g + OFF_B2);
-    __syncthreads();
-    dense_bwd<MLP_H, LH, LH>(H2, sp + S_W2, H1, w, l);     // H1 <- delta1
-    __syncthreads();
-    dense_grad<3, LH, LW1>(H1, Xs, w, MLP_H, MLP_IN, g + OFF_W1, l);
-    bias_grad(H1, LH, MLP_H, g + OFF_B1);
+    // gradients: lane l holds outputs 16 w + 4 lk + r of input 16 ib + li
+    float *g = part + (size_t)blockIdx.x * MLP_NP;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int o = 16 * w + 4 * lk + r;
+#pragma unroll
+        for (int ib = 0; ib < 4; ++ib) {
+            const int i = 16 * ib + li;
+            if (ib < 3 && i < MLP_IN) g[OFF_W1 + o * MLP_IN + i] = g1[ib < 3 ? ib : 0][r];
+            g[OFF_W2 + o * MLP_H + i] = g2[ib][r];
+            g[OFF_W3 + o * MLP_H + i] = g3[ib][r];
+        }
+        if (lk == 0 && r < MLP_OUT) g[OFF_W4 + r * MLP_H + c] = g4[r];
+    }
+    auto over_lk = [](float v) {
+        v += __shfl_xor(v, 16);
+        return v + __shfl_xor(v, 32);
+    };
+    gb1 = over_lk(gb1);
+    gb2 = over_lk(gb2);
+    gb3 = over_lk(gb3);
+    gb4 = over_lk(gb4);
+    lsum = over_lk(lsum);
+    for (int o = 1; o < 16; o <<= 1) lsum += __shfl_xor(lsum, o);
+    if (lk == 0) {
+        g[OFF_B1 + c] = gb1;
+        g[OFF_B2 + c] = gb2;
+        g[OFF_B3 + c] = gb3;
+        if (w == 0 && li < MLP_OUT) g[OFF_B4 + li] = gb4;
+    }
+    if (threadIdx.x == 0) loss[blockIdx.x] = lsum;
 }
 
-// Sum of the tile gradients in tile order, then (optionally) Adam.
-__global__ void mlp_grad_kernel(float *params, const float *part, int ntiles, float *grad,
-                                float *mom, float *var, int adam, float lr, float b1, float b2,
-                                float bc1, float bc2, float epsa)
+// Sum of the partial gradients, then (optionally) Adam: GS slices of rows side
+// by side, each in order, the slices added in order (one lane per parameter
+// over 32 rows: 9 us).  The last workgroup sums the loss, also to loss_host
+// (pinned) when given.
+constexpr int GS = 8;
+
+__global__ __launch_bounds__(64 * GS) void mlp_grad_kernel(float *params, const float *part,
+                                                           int rows, float *grad, float *mom,
+                                                           float *var, int adam, float lr,
+                                                           float b1, float b2, float bc1,
+                                                           float bc2, float epsa,
+                                                           const float *loss, float *lsum,
+                                                           float *loss_host)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= MLP_NP) return;
+    __shared__ float sh[GS][64];
+    const int l = threadIdx.x & 63, w = threadIdx.x >> 6;
+    if (blockIdx.x == gridDim.x - 1) {
+        float s = 0.f;
+        for (int c = threadIdx.x; c < rows; c += 64 * GS) s += loss[c];
+        for (int o = 1; o < 64; o <<= 1) s += __shfl_xor(s, o);
+        if (l == 0) sh[w][0] = s;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int q = 1; q < GS; ++q) s += sh[q][0];
+            *lsum = s;
+            if (loss_host) *loss_host = s;
+        }
+        return;
+    }
+    const int k = blockIdx.x * 64 + l, kc = min(k, MLP_NP - 1);
+    const int len = (rows + GS - 1) / GS, c1 = min(rows, (w + 1) * len);
     float g = 0.f;
-    for (int c = 0; c < ntiles; ++c) g += part[(size_t)c * MLP_NP + k];
+    int c = w * len;
+    for (; c + 8 <= c1; c += 8) {
+        float v[8];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) v[q] = part[(size_t)(c + q) * MLP_NP + kc];
+#pragma unroll
+        for (int q = 0; q < 8; ++q) g += v[q];
+    }
+    for (; c < c1; ++c) g += part[(size_t)c * MLP_NP + kc];
+    sh[w][l] = g;
+    __syncthreads();
+    if (w > 0 || k >= MLP_NP) return;
+    for (int q = 1; q < GS; ++q) g += sh[q][l];
     grad[k] = g;
     if (adam) {
         const float mk = b1 * mom[k] + (1.f - b1) * g;
@@ -288,20 +376,6 @@ __global__ void mlp_grad_kernel(float *params, const float *part, int ntiles, fl
         var[k] = vk;
         params[k] -= lr * (mk / bc1) / (sqrtf(vk / bc2) + epsa);
     }
-}
-
-__global__ void sum_kernel(const float *x, int64_t n, float *out)
-{
-    __shared__ float sh[256];
-    float s = 0.f;
-    for (int64_t k = threadIdx.x; k < n; k += blockDim.x) s += x[k];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if (threadIdx.x < w) sh[threadIdx.x] += sh[threadIdx.x + w];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) *out = sh[0];
 }
 
 }  // namespace
@@ -338,9 +412,12 @@ int mlp_train_dev(vlm_ctx *ctx, int64_t m, const float *X, const float *T, int a
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
     if (m <= 0) return VLM_OK;
     const int64_t ntiles = (m + TS - 1) / TS;
-    VLM_HIP(M->part.reserve((size_t)ntiles * MLP_NP));
-    VLM_HIP(M->loss.reserve((size_t)ntiles));
-    hipLaunchKernelGGL(mlp_train_tile_kernel, dim3((unsigned)ntiles), dim3(256), 0, ctx->stream,
+    const int rows = (int)(ntiles < MLP_ROWS ? ntiles : MLP_ROWS);
+    VLM_HIP(M->part.reserve((size_t)rows * MLP_NP));
+    VLM_HIP(M->loss.reserve((size_t)rows));
+    char *hp = nullptr;
+    if (loss_host) VLM_TRY(pin_take(ctx, sizeof(float), &hp));
+    hipLaunchKernelGGL(mlp_train_tile_kernel, dim3((unsigned)rows), dim3(256), 0, ctx->stream,
                        M->params.p, m, X, T, M->part.p, M->loss.p);
     VLM_HIP(hipGetLastError());
     float bc1 = 1.f, bc2 = 1.f;
@@ -350,18 +427,18 @@ int mlp_train_dev(vlm_ctx *ctx, int64_t m, const float *X, const float *T, int a
         bc1 = 1.f - std::pow(b1, (float)M->steps);
         bc2 = 1.f - std::pow(b2, (float)M->steps);
     }
-    hipLaunchKernelGGL(mlp_grad_kernel, dim3((MLP_NP + 255) / 256), dim3(256), 0, ctx->stream,
-                       M->params.p, M->part.p, (int)ntiles, M->grad.p, M->mom.p, M->var.p, adam,
-                       lr, b1, b2, bc1, bc2, 1e-8f);
+    const bool want_loss = loss_host || keep_loss;
+    float *lsum = want_loss ? M->lsum.p : M->lsum.p + 1;
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3((MLP_NP + 63) / 64 + 1), dim3(64 * GS), 0,
+                       ctx->stream, M->params.p, M->part.p, rows, M->grad.p, M->mom.p, M->var.p,
+                       adam, lr, b1, b2, bc1, bc2, 1e-8f, M->loss.p, lsum,
+                       reinterpret_cast<float *>(hp));
     VLM_HIP(hipGetLastError());
-    if (loss_host || keep_loss) {
-        VLM_HIP(M->lsum.reserve(1));
-        hipLaunchKernelGGL(sum_kernel, dim3(1), dim3(256), 0, ctx->stream, M->loss.p, ntiles,
-                           M->lsum.p);
-        VLM_HIP(hipGetLastError());
-        M->have_loss = true;
+    if (want_loss) M->have_loss = true;
+    if (loss_host) {
+        VLM_TRY(sync_stream(ctx));
+        *loss_host = *reinterpret_cast<const float *>(hp);
     }
-    if (loss_host) VLM_TRY(d2h(ctx, loss_host, M->lsum.p, sizeof(float)));
     return VLM_OK;
 }
 
@@ -401,7 +478,7 @@ static Mlp *get_mlp(vlm_ctx *ctx)
     Mlp *M = new Mlp();
     if (M->params.reserve(MLP_NP) != hipSuccess || M->mom.reserve(MLP_NP) != hipSuccess ||
         M->var.reserve(MLP_NP) != hipSuccess || M->grad.reserve(MLP_NP) != hipSuccess ||
-        M->lsum.reserve(1) != hipSuccess) {
+        M->lsum.reserve(2) != hipSuccess) {   // kept, not kept
         delete M;
         return nullptr;
     }
@@ -452,9 +529,7 @@ int vlm_mlp_get_params(vlm_ctx *ctx, float *params)
     VLM_DEVICE(ctx);
     Mlp *M = get_mlp(ctx);
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
-    VLM_TRY(sync_stream(ctx));
-    VLM_HIP(hipMemcpy(params, M->params.p, MLP_NP * sizeof(float), hipMemcpyDeviceToHost));
-    return VLM_OK;
+    return d2h(ctx, params, M->params.p, MLP_NP * sizeof(float));
 }
 
 int vlm_mlp_forward(vlm_ctx *ctx, int64_t m, const float *x, float *y)
@@ -464,14 +539,43 @@ int vlm_mlp_forward(vlm_ctx *ctx, int64_t m, const float *x, float *y)
     Mlp *M = get_mlp(ctx);
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
     if (m == 0) return VLM_OK;
+    const size_t nx = sizeof(float) * (size_t)m * MLP_IN, ny = sizeof(float) * (size_t)m * MLP_OUT;
+    if (nx + ny <= MLP_DIRECT) {
+        char *hp = nullptr;
+        VLM_TRY(pin_take(ctx, nx + ny, &hp));
+        std::memcpy(hp, x, nx);
+        VLM_TRY(mlp_forward_dev(ctx, m, reinterpret_cast<const float *>(hp),
+                                reinterpret_cast<float *>(hp + nx)));
+        VLM_TRY(sync_stream(ctx));
+        std::memcpy(y, hp + nx, ny);
+        return VLM_OK;
+    }
     VLM_HIP(M->xin.reserve((size_t)m * MLP_IN));
     VLM_HIP(M->yout.reserve((size_t)m * MLP_OUT));
-    VLM_HIP(hipMemcpyAsync(M->xin.p, x, sizeof(float) * m * MLP_IN, hipMemcpyHostToDevice,
-                           ctx->stream));
+    VLM_TRY(h2d(ctx, M->xin.p, x, nx));
     VLM_TRY(mlp_forward_dev(ctx, m, M->xin.p, M->yout.p));
-    VLM_HIP(hipMemcpyAsync(y, M->yout.p, sizeof(float) * m * MLP_OUT, hipMemcpyDeviceToHost,
-                           ctx->stream));
-    VLM_TRY(sync_stream(ctx));
+    return d2h(ctx, y, M->yout.p, ny);
+}
+
+// A host batch where the training kernel reads it (each value once): in the
+// pinned arena up to MLP_DIRECT bytes, else in a device copy.
+static int batch_in(vlm_ctx *ctx, Mlp *M, int64_t m, const float *x, const float *t,
+                    const float **X, const float **T)
+{
+    const size_t nx = sizeof(float) * (size_t)m * MLP_IN, nt = sizeof(float) * (size_t)m * MLP_OUT;
+    if (nx + nt <= MLP_DIRECT) {
+        char *hp = nullptr;
+        VLM_TRY(pin_take(ctx, nx + nt, &hp));
+        std::memcpy(hp, x, nx);
+        std::memcpy(hp + nx, t, nt);
+        *X = reinterpret_cast<const float *>(hp);
+    } else {
+        VLM_HIP(M->xin.reserve((size_t)m * (MLP_IN + MLP_OUT)));
+        VLM_TRY(h2d(ctx, M->xin.p, x, nx));
+        VLM_TRY(h2d(ctx, M->xin.p + m * MLP_IN, t, nt));
+        *X = M->xin.p;
+    }
+    *T = *X + m * MLP_IN;
     return VLM_OK;
 }
 
@@ -482,17 +586,12 @@ int vlm_mlp_loss_grad(vlm_ctx *ctx, int64_t m, const float *x, const float *t, f
     VLM_DEVICE(ctx);
     Mlp *M = get_mlp(ctx);
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
-    VLM_HIP(M->xin.reserve((size_t)m * (MLP_IN + MLP_OUT)));
-    VLM_HIP(hipMemcpyAsync(M->xin.p, x, sizeof(float) * m * MLP_IN, hipMemcpyHostToDevice,
-                           ctx->stream));
-    VLM_HIP(hipMemcpyAsync(M->xin.p + m * MLP_IN, t, sizeof(float) * m * MLP_OUT,
-                           hipMemcpyHostToDevice, ctx->stream));
+    const float *X, *T;
+    VLM_TRY(batch_in(ctx, M, m, x, t, &X, &T));
     float l = 0.f;
-    VLM_TRY(mlp_train_dev(ctx, m, M->xin.p, M->xin.p + m * MLP_IN, 0, 0.f, &l));
+    VLM_TRY(mlp_train_dev(ctx, m, X, T, 0, 0.f, &l));
     if (loss) *loss = l;
-    if (grad) {
-        VLM_HIP(hipMemcpy(grad, M->grad.p, MLP_NP * sizeof(float), hipMemcpyDeviceToHost));
-    }
+    if (grad) return d2h(ctx, grad, M->grad.p, MLP_NP * sizeof(float));
     return VLM_OK;
 }
 
@@ -503,13 +602,10 @@ int vlm_mlp_train_step(vlm_ctx *ctx, int64_t m, const float *x, const float *t, 
     VLM_DEVICE(ctx);
     Mlp *M = get_mlp(ctx);
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
-    VLM_HIP(M->xin.reserve((size_t)m * (MLP_IN + MLP_OUT)));
-    VLM_HIP(hipMemcpyAsync(M->xin.p, x, sizeof(float) * m * MLP_IN, hipMemcpyHostToDevice,
-                           ctx->stream));
-    VLM_HIP(hipMemcpyAsync(M->xin.p + m * MLP_IN, t, sizeof(float) * m * MLP_OUT,
-                           hipMemcpyHostToDevice, ctx->stream));
+    const float *X, *T;
+    VLM_TRY(batch_in(ctx, M, m, x, t, &X, &T));
     float l = 0.f;
-    VLM_TRY(mlp_train_dev(ctx, m, M->xin.p, M->xin.p + m * MLP_IN, 1, lr, &l));
+    VLM_TRY(mlp_train_dev(ctx, m, X, T, 1, lr, &l));
     if (loss) *loss = l;
     return VLM_OK;
 }
