@@ -313,12 +313,16 @@ __global__ void map_gam_kernel(const double *x, double *wg, int per_blade, int n
 }
 
 // The whole solve with refinement in one wave for n <= 64 R: lane l holds
-// rows l + 64 r (r < R) of x, b and r; LU and A are staged in LDS (both fit
-// the 160 KB of a gfx950 CU up to n = 96); values move between lanes by
-// readlane (the index is uniform).  The workgroup has
-// SOLVE_STAGE threads so that the staging copy keeps many loads in flight
-// (one wave alone, waiting on each load, took 136 us for n = 90); after it
-// every wave but the first leaves.
+// rows l + 64 r (r < R) of x, b and r in the pivoted order; LU and the
+// pivoted A are staged in LDS (both fit the 160 KB of a gfx950 CU up to n =
+// 96).  The workgroup has SOLVE_STAGE threads so that the staging copy keeps
+// many loads in flight; after it every wave but the first leaves.
+// Bound by the instructions of that wave, one every four cycles: a column of
+// a substitution is two readlanes (x_j), two writelanes (x_j kept, so that
+// rows already solved may be overwritten and need no mask) and R FMAs, and U
+// is scaled by its diagonal off that chain.  Order 90 with three
+// corrections takes 38 us; with masks, a division per column and the row
+// swaps in the wave it took 56.
 constexpr int SOLVE_STAGE = 512;
 constexpr int SOLVE_WAVE_N = 64;   // one row per lane
 constexpr int SOLVE_WAVE_N2 = 96;  // two rows per lane
@@ -329,103 +333,84 @@ __device__ __forceinline__ double wave_max(double v)
     return v;
 }
 
-// element i (uniform over the wave) of a vector held as v[r] at row l + 64 r,
-// by readlane (no LDS round trip on the substitution's dependency chain)
-template <int R>
-__device__ __forceinline__ double wave_get(const double (&v)[R], int i)
+// One column of a substitution: x_j of v[r], the rows of v[Q0..Q1].
+template <int R, int Q0, int Q1>
+__device__ __forceinline__ void wave_column(double xj, const double (&c)[R], double (&v)[R])
 {
-    const int r = i >> 6;
-    double x = v[0];
 #pragma unroll
-    for (int q = 1; q < R; ++q)
-        if (r == q) x = v[q];
-    const int lane = __builtin_amdgcn_readfirstlane(i & 63);
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), lane),
-                            __builtin_amdgcn_readlane(__double2loint(x), lane));
+    for (int q = Q0; q <= Q1; ++q) v[q] -= c[q] * xj;
 }
 
-template <int R>
-__device__ void wave_lu_solve(int n, const double *sLU, const int *spiv, double (&v)[R])
+constexpr int WSU = 8;   // columns whose LDS reads issue ahead of the chain
+
+// Columns [64 r, min(n, 64 r + 64)) forward with the unit lower triangle.
+template <int R, int r>
+__device__ __forceinline__ void wave_forward(int n, const double *sLU, double (&v)[R],
+                                             double (&x)[R])
+{
+    const int l = threadIdx.x, j1 = min(n, 64 * r + 64);
+    for (int j = 64 * r; j < j1; j += WSU) {
+        double c[WSU][R];
+#pragma unroll
+        for (int u = 0; u < WSU; ++u)
+#pragma unroll
+            for (int q = r; q < R; ++q)
+                c[u][q] = sLU[min(l + 64 * q, n - 1) + n * min(j + u, n - 1)];
+#pragma unroll
+        for (int u = 0; u < WSU; ++u) {
+            if (j + u >= j1) break;
+            const double xj = readlane_d(v[r], (j + u) & 63);
+            x[r] = l == ((j + u) & 63) ? xj : x[r];
+            wave_column<R, r, R - 1>(xj, c[u], v);
+        }
+    }
+}
+
+// The same columns backward with the upper triangle, its rows scaled by rd
+// (v already divided by the diagonal), or, plain, with a division by d_j.
+template <int R, int r>
+__device__ __forceinline__ void wave_backward(int n, const double *sLU, const double (&d)[R],
+                                              const double (&rd)[R], bool plain, double (&v)[R],
+                                              double (&x)[R])
 {
     const int l = threadIdx.x;
-    for (int k = 0; k < n; ++k) {
-        const int p = spiv[k];
-        if (p != k) {
-            const double vk = wave_get<R>(v, k), vp = wave_get<R>(v, p);
+    for (int j = min(n, 64 * r + 64) - 1; j >= 64 * r; j -= WSU) {
+        double c[WSU][R];
 #pragma unroll
-            for (int q = 0; q < R; ++q) {
-                const int row = l + 64 * q;
-                if (row == k) v[q] = vp;
-                else if (row == p) v[q] = vk;
+        for (int u = 0; u < WSU; ++u)
+#pragma unroll
+            for (int q = 0; q <= r; ++q) {
+                const double t = sLU[min(l + 64 * q, n - 1) + n * max(j - u, 0)];
+                c[u][q] = plain ? t : t * rd[q];
             }
+#pragma unroll
+        for (int u = 0; u < WSU; ++u) {
+            if (j - u < 64 * r) break;
+            double xj = readlane_d(v[r], (j - u) & 63);
+            if (plain) xj /= readlane_d(d[r], (j - u) & 63);
+            x[r] = l == ((j - u) & 63) ? xj : x[r];
+            wave_column<R, 0, r>(xj, c[u], v);
         }
     }
-    // Substitutions in blocks of SU steps whose LDS reads issue first, off
-    // the dependency chain through v (a loop holding readlane is not
-    // unrolled by the compiler); reads are unconditional, from clamped rows.
-    constexpr int SU = 4;
-    int j = 0;
-    for (; j + SU <= n; j += SU) {
-        double L[SU][R];
+}
+
+// v <- (LU)^-1 v.  plain: a reciprocal of the diagonal leaves the normal
+// range.
+template <int R>
+__device__ void wave_lu_solve(int n, const double *sLU, const double (&d)[R],
+                              const double (&rd)[R], bool plain, double (&v)[R])
+{
+    double x[R];
 #pragma unroll
-        for (int u = 0; u < SU; ++u)
+    for (int q = 0; q < R; ++q) x[q] = 0.0;
+    wave_forward<R, 0>(n, sLU, v, x);
+    if constexpr (R > 1) wave_forward<R, R - 1>(n, sLU, v, x);
 #pragma unroll
-            for (int q = 0; q < R; ++q) L[u][q] = sLU[min(l + 64 * q, n - 1) + n * (j + u)];
+    for (int q = 0; q < R; ++q) v[q] = plain ? x[q] : x[q] / d[q];
+    if constexpr (R > 1) wave_backward<R, R - 1>(n, sLU, d, rd, plain, v, x);
+    wave_backward<R, 0>(n, sLU, d, rd, plain, v, x);
 #pragma unroll
-        for (int u = 0; u < SU; ++u) {
-            const double xj = wave_get<R>(v, j + u);
-#pragma unroll
-            for (int q = 0; q < R; ++q) {
-                const int row = l + 64 * q;
-                const double t = v[q] - L[u][q] * xj;
-                v[q] = (row > j + u && row < n) ? t : v[q];
-            }
-        }
-    }
-    for (; j < n; ++j) {
-        const double xj = wave_get<R>(v, j);
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int row = l + 64 * q;
-            const double t = v[q] - sLU[min(row, n - 1) + n * j] * xj;
-            v[q] = (row > j && row < n) ? t : v[q];
-        }
-    }
-    j = n - 1;
-    for (; j - SU + 1 >= 0; j -= SU) {
-        double U[SU][R], D[SU];
-#pragma unroll
-        for (int u = 0; u < SU; ++u) {
-            D[u] = sLU[(j - u) + n * (j - u)];
-#pragma unroll
-            for (int q = 0; q < R; ++q) U[u][q] = sLU[min(l + 64 * q, n - 1) + n * (j - u)];
-        }
-#pragma unroll
-        for (int u = 0; u < SU; ++u) {
-#pragma unroll
-            for (int q = 0; q < R; ++q)
-                if (l + 64 * q == j - u) v[q] /= D[u];
-            const double xj = wave_get<R>(v, j - u);
-#pragma unroll
-            for (int q = 0; q < R; ++q) {
-                const int row = l + 64 * q;
-                const double t = v[q] - U[u][q] * xj;
-                v[q] = row < j - u ? t : v[q];
-            }
-        }
-    }
-    for (; j >= 0; --j) {
-#pragma unroll
-        for (int q = 0; q < R; ++q)
-            if (l + 64 * q == j) v[q] /= sLU[j + n * j];
-        const double xj = wave_get<R>(v, j);
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-            const int row = l + 64 * q;
-            const double t = v[q] - sLU[min(row, n - 1) + n * j] * xj;
-            v[q] = row < j ? t : v[q];
-        }
-    }
+    for (int q = 0; q < R; ++q) v[q] = x[q];
 }
 
 // Where the one-wave solve leaves its results: x and (converged, corrections)
@@ -439,60 +424,72 @@ struct SolveOut {
 template <int R, int NMAX>
 __global__ __launch_bounds__(SOLVE_STAGE) void solve_wave_kernel(int n, const double *A,
                                                                  const double *LU,
-                                                        const int *ipiv, const double *b,
-                                                        int max_iter, double tol, SolveOut o)
+                                                                 const int *perm, const double *b,
+                                                                 int max_iter, double tol,
+                                                                 SolveOut o)
 {
+    static_assert(R <= 2, "two blocks of columns");
     __shared__ double sLU[NMAX * NMAX], sA[NMAX * NMAX];
-    __shared__ int spiv[NMAX];
+    __shared__ int sperm[NMAX];
     const int l = threadIdx.x;
-#pragma unroll 4
-    for (int k = l; k < n * n; k += SOLVE_STAGE) {
-        sLU[k] = LU[k];
-        sA[k] = A[k];
+    for (int k = l; k < n; k += SOLVE_STAGE) sperm[k] = perm[k];
+    __syncthreads();
+    // eight loads of each matrix in flight per lane
+    for (int k0 = 0; k0 < n * n; k0 += 8 * SOLVE_STAGE) {
+        double u[8], a[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int k = min(k0 + i * SOLVE_STAGE + l, n * n - 1), j = k / n;
+            u[i] = LU[k];
+            a[i] = A[sperm[k - n * j] + n * j];
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int k = k0 + i * SOLVE_STAGE + l;
+            if (k < n * n) {
+                sLU[k] = u[i];
+                sA[k] = a[i];
+            }
+        }
     }
-    for (int k = l; k < n; k += SOLVE_STAGE) spiv[k] = ipiv[k];
     __syncthreads();
     if (l >= 64) return;
-    double bl[R], xv[R], rl[R];
+    double bl[R], xv[R], rl[R], d[R], rd[R];
     double bm = 0.0;
+    bool odd = false;
 #pragma unroll
     for (int q = 0; q < R; ++q) {
         const int row = l + 64 * q;
-        bl[q] = row < n ? b[row] : 0.0;
+        bl[q] = row < n ? b[sperm[row]] : 0.0;
         bm = fmax(bm, fabs(bl[q]));
         xv[q] = bl[q];
+        d[q] = row < n ? sLU[row + n * row] : 1.0;
+        rd[q] = 1.0 / d[q];
+        odd = odd || !(fabs(rd[q]) < 1e300 && fabs(rd[q]) > 1e-300);
     }
+    const bool plain = __any(odd) != 0;
     const double bmax = wave_max(bm);
-    wave_lu_solve<R>(n, sLU, spiv, xv);
+    wave_lu_solve<R>(n, sLU, d, rd, plain, xv);
     int conv = 0, corr = 0;
     for (int it = 0; it < max_iter; ++it) {
 #pragma unroll
         for (int q = 0; q < R; ++q) rl[q] = l + 64 * q < n ? bl[q] : 0.0;
-        int j = 0;
-        for (; j + 4 <= n; j += 4) {
-            double a[4][R];
+        for (int j = 0; j < n; j += 8) {
+            double a[8][R];
 #pragma unroll
-            for (int u = 0; u < 4; ++u)
+            for (int u = 0; u < 8; ++u)
 #pragma unroll
-                for (int q = 0; q < R; ++q) a[u][q] = sA[min(l + 64 * q, n - 1) + n * (j + u)];
+                for (int q = 0; q < R; ++q)
+                    a[u][q] = sA[min(l + 64 * q, n - 1) + n * min(j + u, n - 1)];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const double xj = wave_get<R>(xv, j + u);
-#pragma unroll
-                for (int q = 0; q < R; ++q) {
-                    const double t = rl[q] - a[u][q] * xj;
-                    rl[q] = l + 64 * q < n ? t : rl[q];
-                }
+            for (int u = 0; u < 8; ++u) {
+                if (j + u >= n) break;
+                const double xj = readlane_d(R == 1 || j < 64 ? xv[0] : xv[R - 1], (j + u) & 63);
+                wave_column<R, 0, R - 1>(xj, a[u], rl);
             }
         }
-        for (; j < n; ++j) {
-            const double xj = wave_get<R>(xv, j);
 #pragma unroll
-            for (int q = 0; q < R; ++q) {
-                const double t = rl[q] - sA[min(l + 64 * q, n - 1) + n * j] * xj;
-                rl[q] = l + 64 * q < n ? t : rl[q];
-            }
-        }
+        for (int q = 0; q < R; ++q) rl[q] = l + 64 * q < n ? rl[q] : 0.0;
         double rm = 0.0;
 #pragma unroll
         for (int q = 0; q < R; ++q) rm = fmax(rm, fabs(rl[q]));
@@ -501,7 +498,7 @@ __global__ __launch_bounds__(SOLVE_STAGE) void solve_wave_kernel(int n, const do
             break;
         }
         ++corr;
-        wave_lu_solve<R>(n, sLU, spiv, rl);
+        wave_lu_solve<R>(n, sLU, d, rd, plain, rl);
 #pragma unroll
         for (int q = 0; q < R; ++q) xv[q] += rl[q];
     }
@@ -530,10 +527,10 @@ __global__ __launch_bounds__(SOLVE_STAGE) void solve_wave_kernel(int n, const do
 // x = A^-1 rhs by the LU factors plus up to max_iter refinement steps on
 // the FP64 residual.  Everything is enqueued: the convergence test runs on
 // the device (later corrections are skipped once it passes), so the only
-// synchronisation is the final download.  piv: the pivots, or for n >
-// SOLVE_WAVE_N2 the row permutation they compose to.  With a rotor given,
+// synchronisation is the final download.  perm: the row permutation that
+// the pivots compose to.  With a rotor given,
 // the solution also becomes its device wing circulation (rotor_map_gam).
-int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const int *piv,
+int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const int *perm,
                  const double *rhs_h, double *x_h, int max_iter, double tol, int *iters,
                  Rotor *rotor = nullptr, bool deferred = false)
 {
@@ -558,10 +555,10 @@ int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const i
         o.nbc = rotor ? rotor->d.nbConvect : 0;
         if (n <= SOLVE_WAVE_N)
             hipLaunchKernelGGL((solve_wave_kernel<1, SOLVE_WAVE_N>), dim3(1), dim3(SOLVE_STAGE),
-                               0, ctx->stream, n, A, LU, piv, b, max_iter, tol, o);
+                               0, ctx->stream, n, A, LU, perm, b, max_iter, tol, o);
         else
             hipLaunchKernelGGL((solve_wave_kernel<2, SOLVE_WAVE_N2>), dim3(1), dim3(SOLVE_STAGE),
-                               0, ctx->stream, n, A, LU, piv, b, max_iter, tol, o);
+                               0, ctx->stream, n, A, LU, perm, b, max_iter, tol, o);
         VLM_HIP(hipGetLastError());
     } else {
         SolveWork w;
@@ -574,12 +571,12 @@ int solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, const i
         const dim3 gs(2 * (unsigned)(np / TB)), gr((n + RROWS - 1) / RROWS);
         hipLaunchKernelGGL(solve_init_kernel, dim3((unsigned)((np + 255) / 256)), dim3(256), 0,
                            ctx->stream, n, b, w);
-        hipLaunchKernelGGL(lu_sweeps_kernel, gs, dim3(256), 0, ctx->stream, n, LU, piv, b, x, 0,
+        hipLaunchKernelGGL(lu_sweeps_kernel, gs, dim3(256), 0, ctx->stream, n, LU, perm, b, x, 0,
                            0, tol, w);
         for (int it = 0; it < max_iter; ++it) {
             hipLaunchKernelGGL(residual_kernel, gr, dim3(RROWS * RSL), 0, ctx->stream, n, A, x, b,
                                r, it, w);
-            hipLaunchKernelGGL(lu_sweeps_kernel, gs, dim3(256), 0, ctx->stream, n, LU, piv, r, x,
+            hipLaunchKernelGGL(lu_sweeps_kernel, gs, dim3(256), 0, ctx->stream, n, LU, perm, r, x,
                                1, it, tol, w);
         }
         if (rotor)
@@ -610,11 +607,10 @@ void compose_pivots(int n, const int *piv, int *perm)
         if (piv[k] >= 0 && piv[k] < n) std::swap(perm[k], perm[piv[k]]);
 }
 
-// What solve_refine reads of a rotor's pivots at its order.
+// The row permutation that solve_refine reads, after the pivots and info.
 const int *solve_pivots(vlm_ctx *ctx, int ir)
 {
-    const int n = ctx->aic_n[ir];
-    return ctx->piv[ir] + (n > SOLVE_WAVE_N2 ? n + 1 : 0);
+    return ctx->piv[ir] + ctx->aic_n[ir] + 1;
 }
 
 }  // namespace
@@ -720,8 +716,8 @@ int vlm_lu_solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, 
     if (!ctx || n <= 0 || !A || !LU || !ipiv || !rhs || !x) return VLM_ERR_ARG;
     for (int k = 0; k < n; ++k)
         if (ipiv[k] < 0 || ipiv[k] >= n) return fail(ctx, VLM_ERR_ARG, "pivot out of range");
-    std::vector<int> perm(ipiv, ipiv + n);
-    if (n > SOLVE_WAVE_N2) compose_pivots(n, ipiv, perm.data());
+    std::vector<int> perm((size_t)n);
+    compose_pivots(n, ipiv, perm.data());
     VLM_DEVICE(ctx);
     const size_t nn = (size_t)n * n;
     VLM_HIP(ctx->hostio.reserve(2 * nn));
