@@ -406,7 +406,7 @@ int mlp_forward_dev(vlm_ctx *ctx, int64_t m, const float *X, float *Y)
 
 // Gradient (and optionally one Adam step) on a device batch.
 int mlp_train_dev(vlm_ctx *ctx, int64_t m, const float *X, const float *T, int adam, float lr,
-                  float *loss_host, int keep_loss)
+                  float *loss_pin, int keep_loss)
 {
     Mlp *M = get_mlp(ctx);
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
@@ -415,8 +415,6 @@ int mlp_train_dev(vlm_ctx *ctx, int64_t m, const float *X, const float *T, int a
     const int rows = (int)(ntiles < MLP_ROWS ? ntiles : MLP_ROWS);
     VLM_HIP(M->part.reserve((size_t)rows * MLP_NP));
     VLM_HIP(M->loss.reserve((size_t)rows));
-    char *hp = nullptr;
-    if (loss_host) VLM_TRY(pin_take(ctx, sizeof(float), &hp));
     hipLaunchKernelGGL(mlp_train_tile_kernel, dim3((unsigned)rows), dim3(256), 0, ctx->stream,
                        M->params.p, m, X, T, M->part.p, M->loss.p);
     VLM_HIP(hipGetLastError());
@@ -427,19 +425,15 @@ int mlp_train_dev(vlm_ctx *ctx, int64_t m, const float *X, const float *T, int a
         bc1 = 1.f - std::pow(b1, (float)M->steps);
         bc2 = 1.f - std::pow(b2, (float)M->steps);
     }
-    const bool want_loss = loss_host || keep_loss;
+    const bool want_loss = loss_pin || keep_loss;
     float *lsum = want_loss ? M->lsum.p : M->lsum.p + 1;
     hipLaunchKernelGGL(mlp_grad_kernel, dim3((MLP_NP + 63) / 64 + 1), dim3(64 * GS), 0,
                        ctx->stream, M->params.p, M->part.p, rows, M->grad.p, M->mom.p, M->var.p,
                        adam, lr, b1, b2, bc1, bc2, 1e-8f, M->loss.p, lsum,
-                       reinterpret_cast<float *>(hp));
+                       loss_pin);
     VLM_HIP(hipGetLastError());
     if (want_loss) M->have_loss = true;
-    if (loss_host) {
-        VLM_TRY(sync_stream(ctx));
-        *loss_host = *reinterpret_cast<const float *>(hp);
-    }
-    return VLM_OK;
+    return loss_pin ? sync_stream(ctx) : VLM_OK;
 }
 
 // Loss of the last training call that kept it on the device (0 if none).
@@ -558,24 +552,27 @@ int vlm_mlp_forward(vlm_ctx *ctx, int64_t m, const float *x, float *y)
 }
 
 // A host batch where the training kernel reads it (each value once): in the
-// pinned arena up to MLP_DIRECT bytes, else in a device copy.
+// pinned arena up to MLP_DIRECT bytes, else in a device copy.  *loss receives
+// a pinned slot, taken with the batch (a later request may recycle the arena).
 static int batch_in(vlm_ctx *ctx, Mlp *M, int64_t m, const float *x, const float *t,
-                    const float **X, const float **T)
+                    const float **X, const float **T, float **loss)
 {
     const size_t nx = sizeof(float) * (size_t)m * MLP_IN, nt = sizeof(float) * (size_t)m * MLP_OUT;
-    if (nx + nt <= MLP_DIRECT) {
-        char *hp = nullptr;
-        VLM_TRY(pin_take(ctx, nx + nt, &hp));
-        std::memcpy(hp, x, nx);
-        std::memcpy(hp + nx, t, nt);
-        *X = reinterpret_cast<const float *>(hp);
-    } else {
+    const bool direct = nx + nt <= MLP_DIRECT;
+    if (!direct) {
         VLM_HIP(M->xin.reserve((size_t)m * (MLP_IN + MLP_OUT)));
         VLM_TRY(h2d(ctx, M->xin.p, x, nx));
         VLM_TRY(h2d(ctx, M->xin.p + m * MLP_IN, t, nt));
-        *X = M->xin.p;
     }
+    char *hp = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(float) + (direct ? nx + nt : 0), &hp));
+    if (direct) {
+        std::memcpy(hp, x, nx);
+        std::memcpy(hp + nx, t, nt);
+    }
+    *X = direct ? reinterpret_cast<const float *>(hp) : M->xin.p;
     *T = *X + m * MLP_IN;
+    *loss = reinterpret_cast<float *>(hp + (direct ? nx + nt : 0));
     return VLM_OK;
 }
 
@@ -587,10 +584,10 @@ int vlm_mlp_loss_grad(vlm_ctx *ctx, int64_t m, const float *x, const float *t, f
     Mlp *M = get_mlp(ctx);
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
     const float *X, *T;
-    VLM_TRY(batch_in(ctx, M, m, x, t, &X, &T));
-    float l = 0.f;
-    VLM_TRY(mlp_train_dev(ctx, m, X, T, 0, 0.f, &l));
-    if (loss) *loss = l;
+    float *l = nullptr;
+    VLM_TRY(batch_in(ctx, M, m, x, t, &X, &T, &l));
+    VLM_TRY(mlp_train_dev(ctx, m, X, T, 0, 0.f, l));
+    if (loss) *loss = *l;
     if (grad) return d2h(ctx, grad, M->grad.p, MLP_NP * sizeof(float));
     return VLM_OK;
 }
@@ -603,10 +600,10 @@ int vlm_mlp_train_step(vlm_ctx *ctx, int64_t m, const float *x, const float *t, 
     Mlp *M = get_mlp(ctx);
     if (!M) return fail(ctx, VLM_ERR_ALLOC, "mlp allocation failed");
     const float *X, *T;
-    VLM_TRY(batch_in(ctx, M, m, x, t, &X, &T));
-    float l = 0.f;
-    VLM_TRY(mlp_train_dev(ctx, m, X, T, 1, lr, &l));
-    if (loss) *loss = l;
+    float *l = nullptr;
+    VLM_TRY(batch_in(ctx, M, m, x, t, &X, &T, &l));
+    VLM_TRY(mlp_train_dev(ctx, m, X, T, 1, lr, l));
+    if (loss) *loss = *l;
     return VLM_OK;
 }
 

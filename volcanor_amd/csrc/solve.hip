@@ -318,9 +318,9 @@ __global__ void map_gam_kernel(const double *x, double *wg, int per_blade, int n
 // 96).  The workgroup has SOLVE_STAGE threads so that the staging copy keeps
 // many loads in flight; after it every wave but the first leaves.
 // Bound by the instructions of that wave, one every four cycles: a column of
-// a substitution is two readlanes (x_j), two writelanes (x_j kept, so that
-// rows already solved may be overwritten and need no mask) and R FMAs, and U
-// is scaled by its diagonal off that chain.  Order 90 with three
+// a substitution is two readlanes (x_j), a select (x_j kept, so that rows
+// already solved may be overwritten and need no mask) and R FMAs, and U is
+// scaled by its diagonal off that chain.  Order 90 with three
 // corrections takes 38 us; with masks, a division per column and the row
 // swaps in the wave it took 56.
 constexpr int SOLVE_STAGE = 512;

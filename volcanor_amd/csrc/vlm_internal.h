@@ -442,10 +442,11 @@ int d2h_deferred(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);
 int defer(vlm_ctx *ctx, std::initializer_list<vlm_ctx::Deferred> d);
 int wait_deferred(vlm_ctx *ctx);
 int mlp_forward_dev(vlm_ctx *ctx, int64_t m, const float *X, float *Y);
-// Training step on a device batch; loss_host downloads the loss (and
-// synchronises), keep_loss only sums it on the device for mlp_read_loss.
+// Training step on a batch in device or pinned memory; the loss goes to
+// loss_pin (a pinned slot: the call then synchronises), or with keep_loss
+// only to the device for mlp_read_loss.
 int mlp_train_dev(vlm_ctx *ctx, int64_t m, const float *X, const float *T, int adam, float lr,
-                  float *loss_host, int keep_loss = 0);
+                  float *loss_pin, int keep_loss = 0);
 int mlp_read_loss(vlm_ctx *ctx, float *loss);
 
 }  // namespace vlm
