@@ -152,8 +152,8 @@ def bench_microbench(args):
                    "precision": args.precision},
         "roofline": roofline(kms, nl, pairs, PEAK_FP64_VALU if prec == vlm.FP64
                              else PEAK_FP32_VALU,
-                             "bs_fp64_kernel<256>" if prec == vlm.FP64 else "bs_mixed_kernel<256>",
-                             "micro:bs_fp64_kernel<256>" if prec == vlm.FP64 else None),
+                             "bs_fp64_kernel" if prec == vlm.FP64 else "bs_mixed_kernel<2>",
+                             "micro:bs_fp64_kernel" if prec == vlm.FP64 else None),
     }
     if not args.no_cpu:
         from oracle import oracle as orc
@@ -308,7 +308,7 @@ def bench_rotor(args):
     prim = "fp64"
     P = runs[prim]["st"]
     value = P.bs_pairs_all / P.wall_steps_tail
-    traffic_key = f"{args.workload}_tail{K}:bs_fp64_kernel<256>"
+    traffic_key = f"{args.workload}_tail{K}:bs_fp64_kernel"
     out = {
         "metric": "Biot-Savart pair-interactions/s",
         "value": value, "unit": "pairs/s", "n_gpus": 1, "steps": K, "warmup": W,
@@ -325,7 +325,7 @@ def bench_rotor(args):
                                    f"{args.warmup if args.warmup is not None else '(unset)'} "
                                    "does not shorten the case")},
         "roofline": roofline(P.bs_kernel_ms, P.bs_launches, P.bs_pairs, PEAK_FP64_VALU,
-                             "bs_fp64_kernel<256>", traffic_key),
+                             "bs_fp64_kernel", traffic_key),
         "pairs_timed": {"all_launches": P.bs_pairs_all, "launches": int(P.bs_launches_all),
                         "work_queue_kernel": P.bs_pairs,
                         "work_queue_launches": int(P.bs_launches)},

@@ -103,10 +103,10 @@ int vlm_filament_vind(vlm_ctx *ctx, int64_t nfil, const double *a,
  * forbid hipMalloc).  a, b, p, v are device pointers to 3 x n arrays (as
  * above), gam and rc device arrays of nfil.  The call only enqueues work on
  * the context's stream; v holds the result once the stream reaches it
- * (vlm_synchronize).  All intermediate data lives in a 64 MiB device array
- * of the library, one per GPU, held until the process ends: about 120 B per
- * filament plus 72 B per point plus 24 B per point for each chunk of
- * partial sums must fit, else VLM_ERR_ARG with a message.  Calls that
+ * (vlm_synchronize).  All intermediate data lives in a 192 MiB device array
+ * of the library, one per GPU, held until the process ends; 120 B per
+ * filament plus 72 B per point must fit in 64 MiB, else VLM_ERR_ARG with a
+ * message.  Calls that
  * overlap on one GPU share that array and race: serialise them. */
 int vlm_filament_vind_noalloc(vlm_ctx *ctx, int64_t nfil, const double *a,
                               const double *b, const double *gam,
@@ -289,7 +289,7 @@ int vlm_rotor_get_velocity(vlm_ctx *ctx, int ir, int which, double *velN,
  * (rotor_calcAIC, classdef.f90:4151-4179); cp and ncap are 3 x N with
  * N = nb*nc*ns in the reference's row order.  The matrix is assembled,
  * factorised (LU, partial pivoting; blocked with an MFMA-FP64 trailing
- * update above order 256) and kept on the
+ * update) and kept on the
  * device; A (N x N column-major) is copied out when non-NULL. */
 int vlm_rotor_calc_aic(vlm_ctx *ctx, int ir, const double *cp,
                        const double *ncap, double *A);
