@@ -706,6 +706,7 @@ int vlm_lu_factor(vlm_ctx *ctx, int n, double *A, int *ipiv)
     VLM_TRY(d2h(ctx, piv.data(), dp, sizeof(int) * (n + 1)));
     std::memcpy(ipiv, piv.data(), sizeof(int) * n);
     const int info = piv[n];
+    release_large(ctx);
     if (info != 0) return fail(ctx, VLM_ERR_SINGULAR, "matrix is singular (zero pivot)");
     return VLM_OK;
 }
@@ -727,7 +728,9 @@ int vlm_lu_solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, 
     VLM_TRY(h2d(ctx, dA, A, sizeof(double) * nn));
     VLM_TRY(h2d(ctx, dLU, LU, sizeof(double) * nn));
     VLM_TRY(h2d(ctx, dp, perm.data(), sizeof(int) * n));
-    return solve_refine(ctx, n, dA, dLU, dp, rhs, x, max_iter, tol, iters);
+    VLM_TRY(solve_refine(ctx, n, dA, dLU, dp, rhs, x, max_iter, tol, iters));
+    release_large(ctx);
+    return VLM_OK;
 }
 
 }  // extern "C"

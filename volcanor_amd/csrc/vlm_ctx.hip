@@ -220,6 +220,11 @@ int pin_take(vlm_ctx *ctx, size_t bytes, char **out)
     return VLM_OK;
 }
 
+void release_large(vlm_ctx *ctx)
+{
+    if (ctx->hostio.n * sizeof(double) > KEEP_BYTES) ctx->hostio.release();
+}
+
 static int piece_event(vlm_ctx *ctx, int slot)
 {
     if (!ctx->io_ev[slot])
@@ -442,7 +447,10 @@ int vlm_filament_vind(vlm_ctx *ctx, int64_t nfil, const double *a, const double 
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
     VLM_TRY(bs_eval(ctx, ctx->seg_view, nfil, ctx->tgt.p, m, m, ctx->out.p, accumulate));
-    return points_to_host(ctx, m, ctx->out.p, m, v);
+    VLM_TRY(points_to_host(ctx, m, ctx->out.p, m, v));
+    release_large(ctx);
+    if (sizeof(double) * REC64_N * (size_t)nfil > KEEP_BYTES) ctx->seg.release();
+    return VLM_OK;
 }
 
 int vlm_fset_create(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b,
@@ -457,6 +465,7 @@ int vlm_fset_create(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b
         delete fs;
         return rc_;
     }
+    release_large(ctx);
     fs->n = nfil;
     ctx->fsets.push_back(fs);
     *fset = (int)ctx->fsets.size() - 1;

@@ -85,6 +85,14 @@ struct SegList {
     DBuf<double> soa, rec64, grp;
     DBuf<float> rec32, near32;
     DBuf<long long> count;
+    void release()
+    {
+        soa.release();
+        rec64.release();
+        grp.release();
+        rec32.release();
+        near32.release();
+    }
     // Room for n segments in the given formats.
     hipError_t reserve(int64_t n, int formats, SegPtrs *out)
     {
@@ -431,6 +439,10 @@ void mlp_release(vlm_ctx *ctx);
 // Kernels may read and write the arena themselves, which spares a small
 // call the copies' launches.
 constexpr size_t PIN_PIECE = (size_t)2 << 20;
+// Copies of host data that a call leaves in the context for the next one are
+// given back above this size (the call has synchronised, or hipFree waits).
+constexpr size_t KEEP_BYTES = (size_t)1 << 30;
+void release_large(vlm_ctx *ctx);
 int pin_take(vlm_ctx *ctx, size_t bytes, char **out);
 int h2d(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);
 int d2h(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);
