@@ -65,7 +65,9 @@ inline size_t ws_size(size_t n)
 //   soa (9): ax ay az g | r0x r0y r0z qq | n0
 // with g = gam / (4 pi), r0 = b - a, n0 = |r0|^2, q = rc^2 n0, qq = q^2 and
 // c the centre of the group's bounding box.  The last group is padded with
-// records of zero circulation and length (qq = 1, so that they give 0).
+// records of zero circulation and length that start where its last segment
+// does (qq = 1): the distance to that point is positive wherever the group is
+// far, so that they give 0 for every target.
 // count: device int64 with the number of valid segments.
 constexpr int GRP = 32;
 constexpr int SOA_N = 9, REC64_N = 16, REC32_N = 16, NEAR32_N = 8, GRPH_N = 4;
@@ -297,8 +299,8 @@ constexpr double kEps = 2.220446049250313080847263336181640625e-16;  // epsilon(
 
 // Writes the records of one group's GRP consecutive segments: lane l of a
 // 32-lane half wave (every lane active) holds segment k (the group's first
-// plus l); lanes with valid = false write the padding record (none in the
-// structure of arrays).  The far radius: a target further than |a - c| + 2 |r0|
+// plus l); lanes with valid = false hold the last valid segment and write the
+// padding record (none in the structure of arrays).  The far radius: a target further than |a - c| + 2 |r0|
 // from the centre, for every segment, has |r1| >= 2 |r0| for all of them.
 // It is infinite (never far) for a group that holds a segment with
 // q <= 1e-18 (the far pair has no zero-denominator guard) or is wider than
@@ -350,7 +352,7 @@ __device__ __forceinline__ void write_group_records(const Slot &s, bool valid, i
                          g * (r0y * lz - r0z * ly), g * (r0z * lx - r0x * lz),
                          g * (r0x * ly - r0y * lx), 0.0};
     if (!valid)
-        for (int i = 0; i < REC64_N; ++i) v[i] = i == 11 ? 1.0 : 0.0;
+        for (int i = 3; i < REC64_N; ++i) v[i] = i == 11 ? 1.0 : 0.0;
     double2 *o64 = reinterpret_cast<double2 *>(L.rec64 + (size_t)k * REC64_N);
 #pragma unroll
     for (int i = 0; i < REC64_N / 2; ++i) o64[i] = make_double2(v[2 * i], v[2 * i + 1]);
