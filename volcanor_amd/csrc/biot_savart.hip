@@ -152,9 +152,9 @@ __device__ __forceinline__ bool pair32(float phx, float phy, float phz, float pl
     return nearp;
 }
 
-// FP64 pair of a group that every target of the wave is far from (see
-// write_group_records): |r1| >= 2 |r0| and qq > 0, so none of pair64's
-// guards can act, and
+// FP64 pair of a group that every target of the wave is far from and within
+// 2^24 core radii of (see write_group_records): |r1| >= 2 |r0| and qq > 0, so
+// the clamps of pair64 and a zero denominator cannot occur, and
 //   n2 = n1 + n0 - 2 d1        (terms at most 2.25 n1, n2 >= n1 / 4)
 //   c2 = n0 n1 - d1^2          (Lagrange's identity)
 //   sum of s c = (sum of s r0) x q - sum of s r0 x (a - c)
@@ -165,7 +165,9 @@ __device__ __forceinline__ bool pair32(float phx, float phy, float phz, float pl
 // cancelling d1 j1 - d2 j2 is shared by n2, so the error against 64-bit
 // references is no larger (quad-precision emulation, relative 2-norm over 60
 // targets: 1.6e-15 against 6.3e-15 on a rotor wake, 2.2e-15 against 6.7e-15
-// on helices).
+// on helices).  pair64's zero for |r1 x r2| <= eps has no counterpart: the
+// pair's velocity is itself below rounding there (d1 j1 - d2 j2 is rounding
+// over a denominator of at least 32 eps n0 n1).
 __device__ __forceinline__ void pair64_far(double px, double py, double pz, const d8 &u,
                                            const d8 &v, double &Sx, double &Sy, double &Sz,
                                            double &Tx, double &Ty, double &Tz)
@@ -193,7 +195,7 @@ __device__ __forceinline__ void pair64_far(double px, double py, double pz, cons
 // once per group): rounding q and a - c costs eps (|p - c| + |a - c|) <=
 // eps (|r1| + 2 R) for a group of radius R, and groups wider than 64 of
 // their longest segments are never far.  25 vector instructions, two of
-// them v_rsq_f32.
+// them v_rsq_f32.  For targets within 2^10 core radii.
 __device__ __forceinline__ void pair32_far(const float *q, float4 a, float4 b, float4 c, float4 d,
                                            float *S, float *T)
 {
@@ -216,6 +218,29 @@ __device__ __forceinline__ void pair32_far(const float *q, float4 a, float4 b, f
     T[2] += w * d.z;
 }
 
+// The far pair at any distance: c2 from the cross product, the velocity
+// summed directly (32 vector instructions).
+__device__ __forceinline__ void pair32_cross(const float *q, float4 a, float4 b, float g, float *v)
+{
+    const float r1x = q[0] - a.x, r1y = q[1] - a.y, r1z = q[2] - a.z;
+    const float n0 = a.w;
+    const float cx = b.y * r1z - b.z * r1y;
+    const float cy = b.z * r1x - b.x * r1z;
+    const float cz = b.x * r1y - b.y * r1x;
+    const float c2 = cx * cx + cy * cy + cz * cz;
+    const float n1 = r1x * r1x + r1y * r1y + r1z * r1z;
+    const float d1 = b.x * r1x + b.y * r1y + b.z * r1z;
+    const float n2 = __builtin_fmaf(-2.0f, d1, n1 + n0);
+    const float d2 = d1 - n0;
+    const float den = __builtin_fmaf(c2, c2, b.w);
+    const float j1 = __builtin_amdgcn_rsqf(n1 * den);
+    const float j2 = __builtin_amdgcn_rsqf(n2 * den);
+    const float w = g * (d1 * j1 - d2 * j2);
+    v[0] += cx * w;
+    v[1] += cy * w;
+    v[2] += cz * w;
+}
+
 // One group for NK targets per lane, all far: records from the wave's LDS
 // copy (broadcast reads), sums folded into FP64 once per group.
 template <int NK>
@@ -235,6 +260,26 @@ __device__ __forceinline__ void group32_far(const float4 *buf, const float (&q)[
         v[k][1] += (double)((S[k][2] * q[k][0] - S[k][0] * q[k][2]) - T[k][1]);
         v[k][2] += (double)((S[k][0] * q[k][1] - S[k][1] * q[k][0]) - T[k][2]);
     }
+}
+
+// The same where a target may be past the distance that pair32_far is
+// accurate to.
+template <int NK>
+__device__ __forceinline__ void group32_cross(const float4 *buf, const float (&q)[NK][3],
+                                              double (&v)[NK][3])
+{
+    float s[NK][3] = {};
+#pragma unroll 2
+    for (int j = 0; j < GRP; ++j) {
+        const float4 a = buf[4 * j], b = buf[4 * j + 1];
+        const float g = buf[4 * j + 2].w;
+#pragma unroll
+        for (int k = 0; k < NK; ++k) pair32_cross(q[k], a, b, g, s[k]);
+    }
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) v[k][d] += (double)s[k][d];
 }
 
 struct BsArgs {
@@ -300,8 +345,8 @@ __global__ __launch_bounds__(BS_BLOCK, 8) void bs_fp64_kernel(BsArgs a)
         for (int64_t g = it.g0; g < it.g1; ++g) {
             const cdptr h = (cdptr)a.grp + g * GRPH_N;
             const double qx = px - h[0], qy = py - h[1], qz = pz - h[2];
-            const bool far = qx * qx + qy * qy + qz * qz > h[3];
-            if (__ballot(!far) == 0) {
+            const double d2 = qx * qx + qy * qy + qz * qz;
+            if (__ballot(!(d2 > h[3] && d2 <= h[4])) == 0) {
                 cd8ptr r = (cd8ptr)(a.rec64 + g * (GRP * REC64_N));
                 double Sx = 0, Sy = 0, Sz = 0, Tx = 0, Ty = 0, Tz = 0;
 #pragma unroll 2
@@ -371,7 +416,7 @@ __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
             n1 = src[gn * (GRP * 4) + 64];
             const cdptr h = (cdptr)a.grp + g * GRPH_N;
             float q[NT][3];
-            unsigned near = 0;   // bit k: a target of the k-th 64 is not far
+            unsigned odd = 0;   // bit k: the k-th 64 targets cannot all take the short pair
 #pragma unroll
             for (int k = 0; k < NT; ++k) {
                 double d2 = 0.0;
@@ -381,10 +426,22 @@ __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
                     d2 += x * x;
                     q[k][d] = (float)x;
                 }
+                if (__ballot(!(d2 > h[3] && d2 <= h[5])) != 0) odd |= 1u << k;
+            }
+            if (odd == 0) {
+                group32_far<NT>(buf, q, v);
+                continue;
+            }
+            unsigned near = 0;   // bit k: one of them is not far
+#pragma unroll
+            for (int k = 0; k < NT; ++k) {
+                double d2 = 0.0;
+#pragma unroll
+                for (int d = 0; d < 3; ++d) d2 += (p[k][d] - h[d]) * (p[k][d] - h[d]);
                 if (__ballot(!(d2 > h[3])) != 0) near |= 1u << k;
             }
             if (near == 0) {
-                group32_far<NT>(buf, q, v);
+                group32_cross<NT>(buf, q, v);
                 continue;
             }
 #pragma unroll
@@ -392,7 +449,8 @@ __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
                 if (!(near >> k & 1u)) {
                     const float qk[1][3] = {{q[k][0], q[k][1], q[k][2]}};
                     double vk[1][3] = {{v[k][0], v[k][1], v[k][2]}};
-                    group32_far<1>(buf, qk, vk);
+                    if (odd >> k & 1u) group32_cross<1>(buf, qk, vk);
+                    else group32_far<1>(buf, qk, vk);
                     for (int d = 0; d < 3; ++d) v[k][d] = vk[0][d];
                     continue;
                 }

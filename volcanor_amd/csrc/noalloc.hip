@@ -22,7 +22,7 @@
 namespace vlm {
 // Inputs are accepted up to 64 MiB at 120 B per filament and 72 B per point
 // (the sizes of an earlier layout, kept as the limit of the call).  The
-// records take 225 B per filament, so the array is 64 MiB x 225 / 120 plus
+// records take 226 B per filament, so the array is 64 MiB x 226 / 120 plus
 // room for chunks.
 constexpr size_t NOALLOC_ACCEPTED_BYTES = (size_t)64 << 20;
 constexpr size_t NOALLOC_SCRATCH_BYTES = (size_t)192 << 20;
@@ -90,7 +90,7 @@ int vlm_filament_vind_noalloc(vlm_ctx *ctx, int64_t nfil, const double *a, const
     // m targets need) | count | counter |
     // targets | partials.  The sizes accepted are those of the
     // documented 64 MiB at 120 B per filament and 72 B per point; the array
-    // itself is larger (225 B per filament, group records included).
+    // itself is larger (226 B per filament, group records included).
     const int64_t cap = nfil > 0 ? nfil : 1, gcap = (cap + GRP - 1) / GRP, rcap = gcap * GRP;
     const int fmt = bs_formats(ctx, m, nfil);
     const size_t osoa = 0;

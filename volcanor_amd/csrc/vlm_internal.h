@@ -59,7 +59,9 @@ inline size_t ws_size(size_t n)
 //   rec32 (16 floats):  a - c(3) n0 | r0(3) qq | g r0(3) g | g r0 x (a - c)(3) q
 //   near32 (8 floats):  a_hi(3) q' | a_lo(3) -   (a = a_hi + a_lo; q' = q, or
 //                       infinity for q <= 1e-18)
-//   grp (4 doubles per group): centre c, squared far radius
+//   grp (8 doubles per group): centre c, squared far radius, the squared
+//                       distances up to which the far pair's c2 is accurate
+//                       in FP64 and in FP32 (below), -, -
 // Launches of few pairs put segments on lanes instead and read one
 // structure of arrays (stride cap):
 //   soa (9): ax ay az g | r0x r0y r0z qq | n0
@@ -70,7 +72,9 @@ inline size_t ws_size(size_t n)
 // far, so that they give 0 for every target.
 // count: device int64 with the number of valid segments.
 constexpr int GRP = 32;
-constexpr int SOA_N = 9, REC64_N = 16, REC32_N = 16, NEAR32_N = 8, GRPH_N = 4;
+constexpr int SOA_N = 9, REC64_N = 16, REC32_N = 16, NEAR32_N = 8, GRPH_N = 8;
+// |r1| up to rc times these: see write_group_records.
+constexpr double FAR_CORE64 = 16777216.0, FAR_CORE32 = 1024.0;   // 2^24, 2^10
 
 // What a list holds; a launch with m targets needs bs_formats(m, its segments).
 enum { SEG_SOA = 1, SEG_REC = 2, SEG_F32 = 4, SEG_ALL = 7 };
@@ -341,11 +345,13 @@ __device__ __forceinline__ void write_group_records(const Slot &s, bool valid, i
     const double l2 = 2.0 * sqrt(n0);
     float ex = valid ? (float)((sqrt(lx * lx + ly * ly + lz * lz) + l2) * 1.000001) : 0.f;
     float lmax = valid ? (float)l2 : 0.f;
+    float rmin = valid ? (float)(fabs(s.rc) * 0.999999) : inf;
     if (valid && !(q > 1e-18)) ex = inf;
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) {
         ex = fmaxf(ex, __shfl_xor(ex, o, 32));
         lmax = fmaxf(lmax, __shfl_xor(lmax, o, 32));
+        rmin = fminf(rmin, __shfl_xor(rmin, o, 32));
     }
     if (!(ex <= 32.0f * lmax)) ex = inf;
     double v[REC64_N] = {s.ax, s.ay, s.az, g, r0x, r0y, r0z, n0, g * r0x, g * r0y, g * r0z, q * q,
@@ -360,6 +366,8 @@ __device__ __forceinline__ void write_group_records(const Slot &s, bool valid, i
         double2 *h = reinterpret_cast<double2 *>(L.grp + (size_t)(k / GRP) * GRPH_N);
         h[0] = make_double2(cx, cy);
         h[1] = make_double2(cz, (double)ex * (double)ex);
+        const double l64 = fmax(rmin * FAR_CORE64 - ex, 0.0), l32 = fmax(rmin * FAR_CORE32 - ex, 0.0);
+        h[2] = make_double2(l64 * l64, l32 * l32);
     }
     if (!L.rec32) return;
     const float hx = (float)s.ax, hy = (float)s.ay, hz = (float)s.az, qf = (float)q;
