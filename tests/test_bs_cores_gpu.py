@@ -51,3 +51,25 @@ def test_fp64_small_cores_off_the_axis(n, dist, rc):
     v, w = ctx.filament_vind(a, b, g, r, p), orc.filament_sum(a, b, g, r, p)
     ctx.close()
     assert np.max(np.linalg.norm(v - w, axis=1)) <= n * 8 * 2.0**-53 / rc / (4 * np.pi)
+
+
+@pytest.mark.parametrize("shuffle", [False, True])
+def test_mixed_tiles_of_near_and_far_targets(shuffle):
+    """Every pair of halves of a 128-target tile: beside the chain, within
+    2^10 core radii of it and past them; and (shuffled) every target order.
+    Near pairs obey the same bound."""
+    from volcanor_amd import vlm
+    rng = np.random.default_rng(11)
+    n, rc = 40, 1e-3
+    a, b, g, r, p = _axis_case(n, 0.01, rc, (0.0, 0.0), (-3.0, 0.4), 18 * 64 + 30, 7)
+    radii = {"near": (-2.0, -0.9), "far": (-0.3, -0.1), "past": (0.3, 0.6)}
+    pairs = [x for q in radii for s in radii for x in (q, s)] + ["near"]
+    scale = np.concatenate([10.0 ** rng.uniform(*radii[q], size=64) for q in pairs])[:len(p)]
+    p = p * scale[:, None]
+    if shuffle:
+        p = p[rng.permutation(len(p))]
+    ctx = vlm.Context(0)
+    ctx.set_precision(vlm.MIXED)
+    v, w = ctx.filament_vind(a, b, g, r, p), orc.filament_sum(a, b, g, r, p)
+    ctx.close()
+    assert np.max(np.linalg.norm(v - w, axis=1)) <= n * 4 * 2.0**-24 / rc / (4 * np.pi)

@@ -47,7 +47,6 @@ constexpr int BS_BLOCK = 256;
 // constant address space: a load from a wave-uniform address becomes a
 // scalar load.  The records are written by earlier launches only.
 typedef const double __attribute__((address_space(4))) *cdptr;
-typedef const float __attribute__((address_space(4))) *cfptr;
 typedef const long long __attribute__((address_space(4))) *clptr;
 // Whole FP64 records as vectors: one s_load_dwordx16 per eight doubles
 // (field by field the compiler issues five smaller loads: 5.38 against
@@ -117,20 +116,19 @@ __device__ __forceinline__ void pair64(double px, double py, double pz, double a
     vz += cz * s;
 }
 
-// FP32 pair on split coordinates (r: rec32, n: near32).  Returns true for
-// near-singular pairs, whose contribution is left to the FP64 recompute
-// (zero here): targets inside the core and, for segments without a core,
-// every target nearby (c2^2 underflows in FP32 long before the exact guard
-// acts, and den with it).  Same evaluation order as pair64:
+// FP32 pair on split coordinates (a, b: near32; r: r0 and qq, n0).  Returns
+// true for near-singular pairs, whose contribution is left to the FP64
+// recompute (zero here): targets inside the core and, for segments without a
+// core, every target nearby (c2^2 underflows in FP32 long before the exact
+// guard acts, and den with it).  Same evaluation order as pair64:
 // d1 / sqrt(n1 den) - d2 / sqrt(n2 den).
-__device__ __forceinline__ bool pair32(float phx, float phy, float phz, float plx, float ply,
-                                       float plz, cfptr r, cfptr n, float &vx, float &vy,
-                                       float &vz)
+__device__ __forceinline__ bool pair32(const float *ph, const float *pl, float4 a, float4 b,
+                                       float4 r, float n0, float *v)
 {
-    const float r1x = (phx - n[0]) + (plx - n[4]);
-    const float r1y = (phy - n[1]) + (ply - n[5]);
-    const float r1z = (phz - n[2]) + (plz - n[6]);
-    const float r0x = r[4], r0y = r[5], r0z = r[6], n0 = r[3], q = n[3];
+    const float r1x = (ph[0] - a.x) + (pl[0] - b.x);
+    const float r1y = (ph[1] - a.y) + (pl[1] - b.y);
+    const float r1z = (ph[2] - a.z) + (pl[2] - b.z);
+    const float r0x = r.x, r0y = r.y, r0z = r.z, q = b.w;
     const float r2x = r1x - r0x, r2y = r1y - r0y, r2z = r1z - r0z;
     const float cx = r0y * r1z - r0z * r1y;
     const float cy = r0z * r1x - r0x * r1z;
@@ -141,14 +139,14 @@ __device__ __forceinline__ bool pair32(float phx, float phy, float phz, float pl
     const bool nearp = (c2 < NEAR_CORE2 * q) && (n1 + n2 < 4.0f * n0);
     const float d1 = r0x * r1x + r0y * r1y + r0z * r1z;
     const float d2 = d1 - n0;
-    const float den = __builtin_fmaf(c2, c2, r[7]);
+    const float den = __builtin_fmaf(c2, c2, r.w);
     const float j1 = __builtin_amdgcn_rsqf(__builtin_fmaxf(n1, EPS2F) * den);
     const float j2 = __builtin_amdgcn_rsqf(__builtin_fmaxf(n2, EPS2F) * den);
-    float s = r[11] * (d1 * j1 - d2 * j2);
+    float s = a.w * (d1 * j1 - d2 * j2);
     s = (c2 > EPS2F && !nearp) ? s : 0.0f;
-    vx += cx * s;
-    vy += cy * s;
-    vz += cz * s;
+    v[0] += cx * s;
+    v[1] += cy * s;
+    v[2] += cz * s;
     return nearp;
 }
 
@@ -165,9 +163,10 @@ __device__ __forceinline__ bool pair32(float phx, float phy, float phz, float pl
 // cancelling d1 j1 - d2 j2 is shared by n2, so the error against 64-bit
 // references is no larger (quad-precision emulation, relative 2-norm over 60
 // targets: 1.6e-15 against 6.3e-15 on a rotor wake, 2.2e-15 against 6.7e-15
-// on helices).  pair64's zero for |r1 x r2| <= eps has no counterpart: the
-// pair's velocity is itself below rounding there (d1 j1 - d2 j2 is rounding
-// over a denominator of at least 32 eps n0 n1).
+// on helices).  pair64's zero for |r1 x r2| <= eps has no counterpart: near
+// the axis the pair gives rounding (over a denominator of at least 32 eps
+// n0 n1), and segments so short that |r0| |r1| is of the order of eps keep
+// their value.
 __device__ __forceinline__ void pair64_far(double px, double py, double pz, const d8 &u,
                                            const d8 &v, double &Sx, double &Sy, double &Sz,
                                            double &Tx, double &Ty, double &Tz)
@@ -282,6 +281,44 @@ __device__ __forceinline__ void group32_cross(const float4 *buf, const float (&q
         for (int d = 0; d < 3; ++d) v[k][d] += (double)s[k][d];
 }
 
+// One group that is not far: the split coordinates from the wave's second LDS
+// copy, then the flagged pairs in FP64 from the records rec64 in memory.
+template <int NK>
+__device__ __forceinline__ void group32_near(const float4 *buf, const float4 *nbuf,
+                                             const double *rec64, const double (&p)[NK][3],
+                                             double (&v)[NK][3])
+{
+    float ph[NK][3], pl[NK][3], s[NK][3] = {};
+    unsigned mask[NK] = {};
+#pragma unroll
+    for (int k = 0; k < NK; ++k)
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+            ph[k][d] = (float)p[k][d];
+            pl[k][d] = (float)(p[k][d] - (double)ph[k][d]);
+        }
+#pragma unroll 4
+    for (int j = 0; j < GRP; ++j) {
+        const float4 a = nbuf[2 * j], b = nbuf[2 * j + 1], r = buf[4 * j + 1];
+        const float n0 = buf[4 * j].w;
+#pragma unroll
+        for (int k = 0; k < NK; ++k)
+            mask[k] |= (pair32(ph[k], pl[k], a, b, r, n0, s[k]) ? 1u : 0u) << j;
+    }
+#pragma unroll
+    for (int k = 0; k < NK; ++k) {
+#pragma unroll
+        for (int d = 0; d < 3; ++d) v[k][d] += (double)s[k][d];
+        while (mask[k]) {
+            const int j = __builtin_ctz(mask[k]);
+            mask[k] &= mask[k] - 1u;
+            const double *r = rec64 + j * REC64_N;
+            pair64(p[k][0], p[k][1], p[k][2], r[0], r[1], r[2], r[3], r[4], r[5], r[6], r[11],
+                   r[7], v[k][0], v[k][1], v[k][2]);
+        }
+    }
+}
+
 struct BsArgs {
     const double *rec64, *grp;
     const float *rec32, *near32;
@@ -343,10 +380,10 @@ __global__ __launch_bounds__(BS_BLOCK, 8) void bs_fp64_kernel(BsArgs a)
         const double px = a.t[tc], py = a.t[a.tstride + tc], pz = a.t[2 * a.tstride + tc];
         double vx = 0.0, vy = 0.0, vz = 0.0;
         for (int64_t g = it.g0; g < it.g1; ++g) {
-            const cdptr h = (cdptr)a.grp + g * GRPH_N;
+            const d8 h = *(cd8ptr)(a.grp + g * GRPH_N);
             const double qx = px - h[0], qy = py - h[1], qz = pz - h[2];
             const double d2 = qx * qx + qy * qy + qz * qz;
-            if (__ballot(!(d2 > h[3] && d2 <= h[4])) == 0) {
+            if (__ballot(!((d2 > h[3]) & (d2 <= h[4]))) == 0) {
                 cd8ptr r = (cd8ptr)(a.rec64 + g * (GRP * REC64_N));
                 double Sx = 0, Sy = 0, Sz = 0, Tx = 0, Ty = 0, Tz = 0;
 #pragma unroll 2
@@ -378,14 +415,16 @@ __global__ __launch_bounds__(BS_BLOCK, 8) void bs_fp64_kernel(BsArgs a)
 // group's records to its own 2 KB of LDS (the next group's are loaded while
 // this one is evaluated) and reads them back as broadcasts, each shared by
 // the NT targets of a lane.  Groups that are not far for all 64 NT targets
-// are tested again per 64; the near ones run pair32 with scalar operands,
-// and the lanes recompute their flagged pairs in FP64 after the group.
+// are tested again per 64; for the near ones the split coordinates follow
+// into another 1 KB, and the lanes recompute their flagged pairs in FP64
+// after the group.  With pair32 on scalar operands, one 64 at a time, a list
+// in no spatial order (every group near, 4.8e9 pairs) took 5.26 ms; so 4.44.
 template <int NT>
 __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
 {
-    __shared__ float4 lds[BS_BLOCK / 64][GRP * 4];
+    __shared__ float4 lds[BS_BLOCK / 64][GRP * 4], nlds[BS_BLOCK / 64][GRP * 2];
     const int lane = threadIdx.x & 63;
-    float4 *buf = lds[threadIdx.x >> 6];
+    float4 *buf = lds[threadIdx.x >> 6], *nbuf = nlds[threadIdx.x >> 6];
     const int64_t ngroups = (*(clptr)a.nseg + GRP - 1) / GRP;
     for (int item = first_item(); item < a.nitems; item = next_item(a, item)) {
         const Item it = item_of(a, item, ngroups);
@@ -426,7 +465,7 @@ __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
                     d2 += x * x;
                     q[k][d] = (float)x;
                 }
-                if (__ballot(!(d2 > h[3] && d2 <= h[5])) != 0) odd |= 1u << k;
+                if (__ballot(!((d2 > h[3]) & (d2 <= h[5]))) != 0) odd |= 1u << k;
             }
             if (odd == 0) {
                 group32_far<NT>(buf, q, v);
@@ -444,38 +483,22 @@ __global__ __launch_bounds__(BS_BLOCK, 5) void bs_mixed_kernel(BsArgs a)
                 group32_cross<NT>(buf, q, v);
                 continue;
             }
+            nbuf[lane] = reinterpret_cast<const float4 *>(a.near32)[g * (GRP * 2) + lane];
+            __builtin_amdgcn_wave_barrier();
+            const double *r64 = a.rec64 + g * (GRP * REC64_N);
+            if (near == (1u << NT) - 1u) {
+                group32_near<NT>(buf, nbuf, r64, p, v);
+                continue;
+            }
 #pragma unroll
             for (int k = 0; k < NT; ++k) {
-                if (!(near >> k & 1u)) {
-                    const float qk[1][3] = {{q[k][0], q[k][1], q[k][2]}};
-                    double vk[1][3] = {{v[k][0], v[k][1], v[k][2]}};
-                    if (odd >> k & 1u) group32_cross<1>(buf, qk, vk);
-                    else group32_far<1>(buf, qk, vk);
-                    for (int d = 0; d < 3; ++d) v[k][d] = vk[0][d];
-                    continue;
-                }
-                const double px = p[k][0], py = p[k][1], pz = p[k][2];
-                const float phx = (float)px, phy = (float)py, phz = (float)pz;
-                const float plx = (float)(px - (double)phx), ply = (float)(py - (double)phy),
-                            plz = (float)(pz - (double)phz);
-                cfptr r = (cfptr)a.rec32 + g * (GRP * REC32_N);
-                cfptr n = (cfptr)a.near32 + g * (GRP * NEAR32_N);
-                float tx = 0.f, ty = 0.f, tz = 0.f;
-                unsigned mask = 0u;
-                for (int j = 0; j < GRP; ++j, r += REC32_N, n += NEAR32_N) {
-                    const bool nearp = pair32(phx, phy, phz, plx, ply, plz, r, n, tx, ty, tz);
-                    mask |= (nearp ? 1u : 0u) << j;
-                }
-                v[k][0] += (double)tx;
-                v[k][1] += (double)ty;
-                v[k][2] += (double)tz;
-                while (mask) {
-                    const int j = __builtin_ctz(mask);
-                    mask &= mask - 1u;
-                    const double *s = a.rec64 + (g * GRP + j) * REC64_N;
-                    pair64(px, py, pz, s[0], s[1], s[2], s[3], s[4], s[5], s[6], s[11], s[7],
-                           v[k][0], v[k][1], v[k][2]);
-                }
+                const float qk[1][3] = {{q[k][0], q[k][1], q[k][2]}};
+                const double pk[1][3] = {{p[k][0], p[k][1], p[k][2]}};
+                double vk[1][3] = {{v[k][0], v[k][1], v[k][2]}};
+                if (near >> k & 1u) group32_near<1>(buf, nbuf, r64, pk, vk);
+                else if (odd >> k & 1u) group32_cross<1>(buf, qk, vk);
+                else group32_far<1>(buf, qk, vk);
+                for (int d = 0; d < 3; ++d) v[k][d] = vk[0][d];
             }
         }
         double *o = a.part + (size_t)it.chunk * 3 * a.m;

@@ -57,7 +57,7 @@ inline size_t ws_size(size_t n)
 // structures:
 //   rec64 (16 doubles): a(3) g | r0(3) n0 | g r0(3) qq | g r0 x (a - c)(3) -
 //   rec32 (16 floats):  a - c(3) n0 | r0(3) qq | g r0(3) g | g r0 x (a - c)(3) q
-//   near32 (8 floats):  a_hi(3) q' | a_lo(3) -   (a = a_hi + a_lo; q' = q, or
+//   near32 (8 floats):  a_hi(3) g | a_lo(3) q'   (a = a_hi + a_lo; q' = q, or
 //                       infinity for q <= 1e-18)
 //   grp (8 doubles per group): centre c, squared far radius, the squared
 //                       distances up to which the far pair's c2 is accurate
@@ -378,9 +378,9 @@ __device__ __forceinline__ void write_group_records(const Slot &s, bool valid, i
         o32[1] = make_float4((float)r0x, (float)r0y, (float)r0z, qf * qf);
         o32[2] = make_float4((float)v[8], (float)v[9], (float)v[10], (float)g);
         o32[3] = make_float4((float)v[12], (float)v[13], (float)v[14], qf);
-        on[0] = make_float4(hx, hy, hz, q > 1e-18 ? qf : inf);
+        on[0] = make_float4(hx, hy, hz, (float)g);
         on[1] = make_float4((float)(s.ax - (double)hx), (float)(s.ay - (double)hy),
-                            (float)(s.az - (double)hz), 0.f);
+                            (float)(s.az - (double)hz), q > 1e-18 ? qf : inf);
     } else {
         const float4 z = make_float4(0.f, 0.f, 0.f, 0.f);
         o32[0] = o32[2] = on[0] = on[1] = z;
