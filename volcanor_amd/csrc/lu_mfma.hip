@@ -386,6 +386,12 @@ __global__ __launch_bounds__(PT) void lu_panel_fast_kernel(int n, double *A, int
 }
 
 
+// A column whose candidates are all NaN pivots on its diagonal, as IDAMAX has
+// it, and the factors are NaN; above this order the factorisation has always
+// reported it as a zero pivot (but for a ragged last panel).
+constexpr int NAN_OK = 256;
+__device__ __forceinline__ bool nan_is_error(int n, int jb) { return n > NAN_OK && jb == NBMAX; }
+
 // Panel held in registers, masking design (the 32-column panels, up to
 // 1024 rows): W waves, lane t owns the physical panel rows t + 64 W q, RPT
 // of them (columns [k0, k0+JB)).  A pivot row stays in its lane and is
@@ -408,6 +414,7 @@ struct WideCtx {
     double *cinv;   // [2][W] 1 / candidate value
     int *ipiv, *info;
     int tid, lane, w, k0, m;
+    bool report;    // a column of NaNs counts as a zero pivot (see nan_is_error)
 };
 
 template <int JB, int W, int RPT, int C>
@@ -462,16 +469,32 @@ __device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT
     const double gv = __hiloint2double(__builtin_amdgcn_readfirstlane((int)r.hi),
                                        __builtin_amdgcn_readfirstlane((int)r.lo));
     const int gkey = __builtin_amdgcn_readfirstlane(r.key);
-    const int gw = gkey & 7;
-    const int lp = gkey >> 3;   // logical row of the pivot
+    int gw = gkey & 7;
+    int lp = gkey >> 3;   // logical row of the pivot
+    bool zero = gv == 0.0;
+    if (gkey == INT_MAX) {
+        // every candidate is NaN (the same in all waves): the diagonal's row,
+        // from the slot of wave 0
+#pragma unroll
+        for (int q = 0; q < RPT; ++q)
+            if (pos[q] == C) {
+                P.cinv[par * W] = 1.0 / a[q][C];
+#pragma unroll
+                for (int j = C; j < JB; ++j) P.cand[par * W * JB + j] = a[q][j];
+            }
+        __syncthreads();
+        gw = 0;
+        lp = C;
+        zero = P.report;
+    }
     if (P.tid == 0) {
         P.ipiv[P.k0 + C] = P.k0 + lp;
         // a zero column (every candidate 0: lp = C, no swap) is recorded
         // and left as it is, as DGETF2 does; the factorisation reports it
-        if (gv == 0.0 && *P.info == 0) *P.info = P.k0 + C + 1;
+        if (zero && *P.info == 0) *P.info = P.k0 + C + 1;
     }
     const double *prow = P.cand + (par * W + gw) * JB;
-    const double inv = gv == 0.0 ? 0.0 : P.cinv[par * W + gw];
+    const double inv = zero ? 0.0 : P.cinv[par * W + gw];
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
         if (pos[q] == lp) pos[q] = C;
@@ -552,7 +575,8 @@ __global__ __launch_bounds__(64 * W) void lu_panel_wide_kernel(int n, double *A,
         __builtin_amdgcn_sched_barrier(0);   // one column's addresses live at a time
     }
     __syncthreads();   // moved = 0 visible
-    WideCtx<JB, W> P{cand, rec, cinv, ipiv, info, tid, tid & 63, tid >> 6, k0, m};
+    WideCtx<JB, W> P{cand, rec, cinv, ipiv, info, tid, tid & 63, tid >> 6, k0, m,
+                     nan_is_error(n, JB)};
     wide_column<JB, W, RPT, 0>(a, pos, P);
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
@@ -589,21 +613,20 @@ __global__ __launch_bounds__(64 * W) void lu_panel_wide_kernel(int n, double *A,
 struct WaveCtx {
     int *ipiv, *info;
     int lane, k0, m, jb;
+    bool report;    // a column of NaNs counts as a zero pivot
 };
 
 template <int C>
 __device__ __forceinline__ void wave_column(double (&a)[NBMAX], int &pos, const WaveCtx &P)
 {
     if (C >= P.jb) return;
-    // candidates: rows at logical >= C; the row at C counts as zero if it
-    // holds a NaN, so that a column of zeros or NaNs pivots on its diagonal
-    const double x = fabs(a[C]);
-    const bool live = pos >= C && pos < P.m;
-    const bool cand = live && (x >= 0.0 || pos == C);
-    const double bv = x >= 0.0 ? x : 0.0;
+    // candidates: rows at logical >= C, but for NaNs
+    const double bv = fabs(a[C]);
+    const bool cand = pos >= C && pos < P.m && bv >= 0.0;
     const unsigned hi = cand ? (unsigned)__double2hiint(bv) : 0u;
     const unsigned M = wave_umax(hi);
     unsigned long long hit = __ballot(cand && hi == M);
+    bool nan = false;
     if (__popcll(hit) != 1) {
         const bool th = cand && hi == M;
         const unsigned lo = th ? (unsigned)__double2loint(bv) : 0u;
@@ -611,13 +634,15 @@ __device__ __forceinline__ void wave_column(double (&a)[NBMAX], int &pos, const 
         const bool top = th && lo == Ml;
         const int r = wave_min(top ? pos : INT_MAX);
         hit = __ballot(top && pos == r);
+        nan = hit == 0;   // every candidate is NaN: the diagonal's row
+        if (nan) hit = __ballot(pos == C);
     }
     const int wl = __ffsll((long long)hit) - 1;
     const int lp = __builtin_amdgcn_readlane(pos, wl);
     double u[NBMAX];
 #pragma unroll
     for (int j = C; j < NBMAX; ++j) u[j] = readlane_f64(a[j], wl);
-    const bool zero = u[C] == 0.0;
+    const bool zero = nan ? P.report : u[C] == 0.0;
     if (P.lane == 0) {
         P.ipiv[P.k0 + C] = P.k0 + lp;
         // a zero column (lp = C, no swap) is recorded and left as it is, as
@@ -658,7 +683,7 @@ __global__ __launch_bounds__(64, 1) void lu_panel_wave_kernel(int n, double *A, 
         const double x = col[ld * (c < jb ? c : jb - 1) + (lane < m ? lane : m - 1)];
         a[c] = (lane < m && c < jb) ? x : 0.0;
     }
-    const WaveCtx P{ipiv, info, lane, k0, m, jb};
+    const WaveCtx P{ipiv, info, lane, k0, m, jb, nan_is_error(n, jb)};
     wave_column<0>(a, pos, P);
 #pragma unroll
     for (int c = 0; c < NBMAX; ++c)
