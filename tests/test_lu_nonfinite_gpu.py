@@ -1,7 +1,8 @@
-"""LU of matrices that hold NaNs, on every panel kernel of the orders up to
-256: a column's candidates are its numbers, a column without any pivots on
-its diagonal, and the factors hold NaN exactly where the column-by-column
-algorithm has them.  Finite entries agree as those of finite matrices do."""
+"""LU of matrices that hold NaNs and infinities, on every panel kernel of the
+orders up to 256: a column's candidates are its numbers, a column without any
+pivots on its diagonal, and the factors hold NaN and infinities exactly where
+the column-by-column algorithm has them (finished rows are not touched).
+Finite entries agree as those of finite matrices do."""
 import numpy as np
 import pytest
 
@@ -38,13 +39,23 @@ def _check(A):
 
 
 @pytest.mark.parametrize("n", [1, 20, 64, 65, 100, 129, 200, 256])
-@pytest.mark.parametrize("where", ["entry", "all"])
+@pytest.mark.parametrize("where", ["entry", "column", "all"])
 def test_nan(n, where):
     A = np.random.default_rng(n).standard_normal((n, n))
     if where == "entry":
         A[n // 2, n // 3] = np.nan
+    elif where == "column":
+        A[:, 2 * n // 5] = np.nan
     else:
         A[:] = np.nan
+    _check(A)
+
+
+@pytest.mark.parametrize("n", [20, 64, 65, 100, 129, 200, 256])
+@pytest.mark.parametrize("row,col", [(0.5, 0.3), (0.1, 0.97), (0.9, 0.6)])
+def test_infinity(n, row, col):
+    A = np.random.default_rng(n).standard_normal((n, n))
+    A[int(row * n), int(col * n)] = -np.inf
     _check(A)
 
 

@@ -501,16 +501,22 @@ __device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT
         else if (pos[q] == C) pos[q] = lp;
     }
     double l[RPT];
+    int on[RPT];
 #pragma unroll
     for (int q = 0; q < RPT; ++q) {
         const bool upd = pos[q] > C && pos[q] < P.m;
         const double x = a[q][C];
         l[q] = upd ? x * inv : 0.0;
         a[q][C] = upd ? l[q] : x;
+        on[q] = upd ? -1 : 0;
     }
     // rank-1 update, CH pivot-row entries at a time (the scheduling barrier
     // keeps later entries' loads from piling up in registers when the
-    // panel fills them)
+    // panel fills them).  Finished rows and empty slots have l = 0; they see
+    // the entries with the high word cleared (a tiny number), as 0 times an
+    // infinite entry is not 0.  That costs 2-4% (7% with two rows per lane);
+    // a branch over those rows cost 7-9%, taking the finished rows from the
+    // candidates' slots in the end 4-5%.
     constexpr int CH = RPT >= 3 ? 4 : 16;
 #pragma unroll
     for (int j0 = C + 1; j0 < JB; j0 += CH) {
@@ -522,7 +528,9 @@ __device__ __forceinline__ void wide_column(double (&a)[RPT][JB], int (&pos)[RPT
             if (j0 + t < JB) {
                 const int j = j0 + t < JB ? j0 + t : 0;
 #pragma unroll
-                for (int q = 0; q < RPT; ++q) a[q][j] -= l[q] * u[t];
+                for (int q = 0; q < RPT; ++q)
+                    a[q][j] -= l[q] * __hiloint2double(__double2hiint(u[t]) & on[q],
+                                                       __double2loint(u[t]));
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -652,10 +660,12 @@ __device__ __forceinline__ void wave_column(double (&a)[NBMAX], int &pos, const 
     const double inv = zero ? 0.0 : 1.0 / u[C];
     pos = pos == lp ? C : (pos == C ? lp : pos);
     const bool upd = pos > C && pos < P.m;
-    const double l = upd ? a[C] * inv : 0.0;
-    a[C] = upd ? l : a[C];
+    const double l = a[C] * inv;
+    if (upd) {   // not the finished rows: 0 times an infinite entry is not 0
+        a[C] = l;
 #pragma unroll
-    for (int j = C + 1; j < NBMAX; ++j) a[j] -= l * u[j];
+        for (int j = C + 1; j < NBMAX; ++j) a[j] -= l * u[j];
+    }
     if constexpr (C + 1 < NBMAX) wave_column<C + 1>(a, pos, P);
 }
 
