@@ -226,37 +226,53 @@ __global__ __launch_bounds__(256) void lu_sweeps_kernel(int n, const double *LU,
         v = row < n ? rhs[perm[row]] : 0.0;
     }
     v -= (part[0][lane] + part[1][lane]) + (part[2][lane] + part[3][lane]);
+    if (row >= n) v = 0.0;
+    // A solved value is kept in y; the rows behind it go on being updated
+    // with what no one reads (a zero factor would turn them into NaN where a
+    // value is infinite).
     constexpr int SU = 8;   // columns whose LDS reads issue ahead of the chain
+    double y = 0.0;
     if (!back) {
         for (int j = 0; j < TB; j += SU) {
             double l[SU];
 #pragma unroll
-            for (int u = 0; u < SU; ++u) l[u] = lane > j + u ? D[lane + TB * (j + u)] : 0.0;
+            for (int u = 0; u < SU; ++u) l[u] = D[lane + TB * (j + u)];
 #pragma unroll
-            for (int u = 0; u < SU; ++u) v -= l[u] * readlane_d(v, j + u);
+            for (int u = 0; u < SU; ++u) {
+                const double xj = readlane_d(v, j + u);
+                y = lane == j + u ? xj : y;
+                v -= l[u] * xj;
+            }
         }
-        publish(w.y + row, v);
+        publish(w.y + row, y);
         return;
     }
-    const double d = D[lane + TB * lane], rd = 1.0 / d;
-    // v / d by the reciprocal and one correction of the remainder, or, where
-    // a reciprocal leaves the normal range, by division
-    const bool plain = __any(!(fabs(rd) < 1e300 && fabs(rd) > 1e-300)) != 0;
-    for (int j = TB - SU; j >= 0; j -= SU) {
-        double l[SU];
+    // v / d by the reciprocal and one correction of the remainder, or by
+    // division where a reciprocal leaves the normal range or a value is not
+    // finite (seen at the end, as the correction makes it NaN)
+    const double d = D[lane + TB * lane], rd = 1.0 / d, v0 = v;
+    bool plain = __any(!(fabs(rd) < 1e300 && fabs(rd) > 1e-300)) != 0;
+    for (;;) {
+        v = v0;
+        for (int j = TB - SU; j >= 0; j -= SU) {
+            double l[SU];
 #pragma unroll
-        for (int u = 0; u < SU; ++u) l[u] = lane < j + u ? D[lane + TB * (j + u)] : 0.0;
+            for (int u = 0; u < SU; ++u) l[u] = D[lane + TB * (j + u)];
 #pragma unroll
-        for (int u = SU - 1; u >= 0; --u) {
-            const double g = v * rd;
-            double e = __builtin_fma(__builtin_fma(-g, d, v), rd, g);
-            if (plain) e = v / d;
-            v = lane == j + u ? e : v;
-            v -= l[u] * readlane_d(v, j + u);
+            for (int u = SU - 1; u >= 0; --u) {
+                const double g = v * rd;
+                double e = __builtin_fma(__builtin_fma(-g, d, v), rd, g);
+                if (plain) e = v / d;
+                const double xj = readlane_d(e, j + u);
+                y = lane == j + u ? xj : y;
+                v -= l[u] * xj;
+            }
         }
+        if (plain || !__any(!(fabs(y) < __builtin_inf()))) break;
+        plain = true;
     }
-    publish(w.z + row, v);
-    if (row < n) x[row] = acc ? x[row] + v : v;
+    publish(w.z + row, y);
+    if (row < n) x[row] = acc ? x[row] + y : y;
 }
 
 // r = b - A x and its maximum norm: RROWS rows per workgroup, the columns
