@@ -41,3 +41,17 @@ def test_zero_on_the_diagonal(n, row):
     np.testing.assert_array_equal(np.isposinf(x), np.isposinf(ref))
     np.testing.assert_array_equal(np.isneginf(x), np.isneginf(ref))
     np.testing.assert_allclose(x[k + 1:], ref[k + 1:], rtol=1e-10, atol=1e-12)
+
+
+@pytest.mark.parametrize("n", [40, 90, 97, 130])
+def test_a_residual_of_nans_ends_the_refinement(n):
+    from volcanor_amd import vlm
+    rng = np.random.default_rng(n)
+    A = np.asfortranarray(0.5 * rng.standard_normal((n, n)) / np.sqrt(n) + 2.0 * np.eye(n))
+    b = rng.standard_normal(n)
+    b[0] = np.nan
+    ctx = vlm.Context(0)
+    LU, piv = ctx.lu_factor(A)
+    x, it = ctx.lu_solve_refine(A, LU, piv, b, max_iter=3)
+    ctx.close()
+    assert np.all(np.isnan(x)) and it == 0

@@ -308,7 +308,8 @@ __global__ __launch_bounds__(RROWS * RSL) void residual_kernel(int n, const doub
     for (int k = 0; k < RSL; ++k) t += part[k][l];
     t = i < n ? b[i] - t : 0.0;
     if (i < n) r[i] = t;
-    unsigned long long m = (unsigned long long)__double_as_longlong(fabs(t));
+    // NaNs do not count
+    unsigned long long m = t == t ? (unsigned long long)__double_as_longlong(fabs(t)) : 0ull;
     for (int o = 16; o > 0; o >>= 1) {
         const unsigned long long v = __shfl_xor(m, o, 32);
         m = v > m ? v : m;
