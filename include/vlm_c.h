@@ -412,16 +412,21 @@ int vlm_predictor_errors(vlm_ctx *ctx, double *mlp_rel_rms, double *base_rel_rms
                          int64_t *judged_steps);
 
 /* ---- kernel timing ----------------------------------------------------- */
-/* When enabled, every work-queue Biot-Savart launch (1024 targets or more)
- * is bracketed by HIP events on the context stream.  vlm_profile_get returns the summed kernel time (ms),
- * the launch count and the algorithmic pair count since the last reset. */
+/* When enabled, every launch of the grouped (work-queue) Biot-Savart kernels
+ * is bracketed by HIP events on the context stream: all launches but those of
+ * few pairs, which are the ones with fewer than 192 targets in waves of 64
+ * less than four fifths full, and those of at most 1.6e7 pairs up to 400
+ * targets or 3e6 pairs up to 2048 targets; in mixed precision none of 1024
+ * targets or more counts as few.  vlm_profile_get returns the summed kernel
+ * time (ms), the launch count and the algorithmic pair count since the last
+ * reset. */
 int vlm_profile_enable(vlm_ctx *ctx, int enable);
 int vlm_profile_reset(vlm_ctx *ctx);
 int vlm_profile_get(vlm_ctx *ctx, double *bs_ms, int64_t *bs_launches,
                     double *pairs);
-/* Pair count of every Biot-Savart launch since the last reset, the
- * small-target launches (fewer than 1024 targets: collocation points,
- * bound vortices, loads) included, and the number of those launches. */
+/* Pair count of every Biot-Savart launch since the last reset, those of few
+ * pairs (collocation points, bound vortices, loads) included, and the number
+ * of those launches. */
 int vlm_profile_get_all(vlm_ctx *ctx, double *pairs, int64_t *launches);
 /* Device time of the LU factorisations (lu_factor on the device, events
  * around the whole factorisation) since the last reset, their count and

@@ -887,8 +887,7 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
     const int grid = (int)(need < cap ? need : cap);
     a.round_robin = len < LEN_MID || need <= cap;
     Timer tm{};
-    const bool timed = prof && m >= MIXED_MIN;
-    if (timed) {
+    if (prof) {
         VLM_HIP(hipEventCreate(&tm.a));
         VLM_HIP(hipEventCreate(&tm.b));
         VLM_HIP(hipEventRecord(tm.a, ctx->stream));
@@ -898,9 +897,11 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
     else
         hipLaunchKernelGGL(bs_fp64_kernel, dim3(grid), dim3(BS_BLOCK), 0, ctx->stream, a);
     VLM_HIP(hipGetLastError());
-    if (timed) VLM_HIP(hipEventRecord(tm.b, ctx->stream));
-    if (prof) VLM_TRY(profile_count(ctx, seg.count, m, timed ? 0 : 1, timed ? &tm : nullptr));
-    return launch_reduce(ctx, part, nchunks, m, out, o, accumulate, counter);
+    const hipError_t e = prof ? hipEventRecord(tm.b, ctx->stream) : hipSuccess;
+    // before any return: the reduction leaves the work counter at 0
+    VLM_TRY(launch_reduce(ctx, part, nchunks, m, out, o, accumulate, counter));
+    VLM_HIP(e);
+    return prof ? profile_count(ctx, seg.count, m, 0, &tm) : VLM_OK;
 }
 
 }  // namespace vlm

@@ -178,14 +178,14 @@ struct Rotor {
     size_t nvf() const { return 3u * d.nb * (size_t)(d.nFwake > 0 ? d.nFwake : 0); }
 };
 
-// One profiled Biot-Savart launch: events around the work-queue kernel
-// (a, b; null for the small-target kernel, which is counted but not timed)
+// One profiled Biot-Savart launch: events around the grouped kernel (a, b;
+// null for launches of few pairs, which are counted but not timed: bs_formats)
 // and the target count; pairs = targets x the device segment count, which
 // is copied to the pinned slot of the same index without a synchronisation.
 struct Timer {
     hipEvent_t a, b;
     double pairs;
-    int kind = 0;  // 0 work-queue kernel (timed), 1 small-target kernel
+    int kind = 0;  // 0 grouped kernel (timed), 1 kernel of few pairs
 };
 
 struct Mlp;

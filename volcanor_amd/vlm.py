@@ -534,7 +534,7 @@ class Context:
 
     def profile_get_all(self):
         """(pairs, launches) of every Biot-Savart launch since the reset,
-        small-target launches included."""
+        those of few pairs included."""
         pairs, n = C.c_double(), C.c_int64()
         self._chk(self.lib.vlm_profile_get_all(self.h, C.byref(pairs), C.byref(n)))
         return pairs.value, n.value
