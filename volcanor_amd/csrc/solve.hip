@@ -711,6 +711,7 @@ int vlm_lu_factor(vlm_ctx *ctx, int n, double *A, int *ipiv)
 {
     if (!ctx || n <= 0 || !A || !ipiv) return VLM_ERR_ARG;
     VLM_DEVICE(ctx);
+    const Trim trim{ctx};
     const size_t nn = (size_t)n * n;
     VLM_HIP(ctx->hostio.reserve(nn));
     VLM_HIP(ctx->hostio_i.reserve((size_t)n + 1));
@@ -723,7 +724,6 @@ int vlm_lu_factor(vlm_ctx *ctx, int n, double *A, int *ipiv)
     VLM_TRY(d2h(ctx, piv.data(), dp, sizeof(int) * (n + 1)));
     std::memcpy(ipiv, piv.data(), sizeof(int) * n);
     const int info = piv[n];
-    release_large(ctx);
     if (info != 0) return fail(ctx, VLM_ERR_SINGULAR, "matrix is singular (zero pivot)");
     return VLM_OK;
 }
@@ -737,6 +737,7 @@ int vlm_lu_solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, 
     std::vector<int> perm((size_t)n);
     compose_pivots(n, ipiv, perm.data());
     VLM_DEVICE(ctx);
+    const Trim trim{ctx};
     const size_t nn = (size_t)n * n;
     VLM_HIP(ctx->hostio.reserve(2 * nn));
     VLM_HIP(ctx->hostio_i.reserve((size_t)n + 1));
@@ -745,9 +746,7 @@ int vlm_lu_solve_refine(vlm_ctx *ctx, int n, const double *A, const double *LU, 
     VLM_TRY(h2d(ctx, dA, A, sizeof(double) * nn));
     VLM_TRY(h2d(ctx, dLU, LU, sizeof(double) * nn));
     VLM_TRY(h2d(ctx, dp, perm.data(), sizeof(int) * n));
-    VLM_TRY(solve_refine(ctx, n, dA, dLU, dp, rhs, x, max_iter, tol, iters));
-    release_large(ctx);
-    return VLM_OK;
+    return solve_refine(ctx, n, dA, dLU, dp, rhs, x, max_iter, tol, iters);
 }
 
 }  // extern "C"

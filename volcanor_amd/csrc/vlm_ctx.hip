@@ -220,9 +220,16 @@ int pin_take(vlm_ctx *ctx, size_t bytes, char **out)
     return VLM_OK;
 }
 
-void release_large(vlm_ctx *ctx)
+Trim::~Trim()
 {
-    if (ctx->hostio.n * sizeof(double) > KEEP_BYTES) ctx->hostio.release();
+    for (auto *b : {&ctx->hostio, &ctx->tgt, &ctx->out})
+        if (b->n * sizeof(double) > KEEP_BYTES) b->release();
+    // (wake passes have partial sums of up to 400 MB)
+    if (ctx->part.n * sizeof(double) > 4 * KEEP_BYTES) ctx->part.release();
+    if (ctx->seg.bytes() > KEEP_BYTES) {
+        ctx->seg.release();
+        ctx->seg_view = SegPtrs();
+    }
 }
 
 static int piece_event(vlm_ctx *ctx, int slot)
@@ -280,29 +287,53 @@ int d2h(vlm_ctx *ctx, void *dst, const void *src, size_t bytes)
     return sync_stream(ctx);
 }
 
+// Points of a piece: whole workgroups, and whole 64-byte lines.
+constexpr int64_t PIECE_POINTS = (int64_t)(PIN_PIECE / (3 * sizeof(double))) / 256 * 256;
+
 int points_to_device(vlm_ctx *ctx, int64_t m, const double *p, double *soa, int64_t stride)
 {
-    char *h = nullptr;
-    VLM_TRY(pin_take(ctx, sizeof(double) * 3 * m, &h));
-    std::memcpy(h, p, sizeof(double) * 3 * m);
-    hipLaunchKernelGGL(aos_to_soa_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m,
-                       reinterpret_cast<const double *>(h), soa, stride);
-    VLM_HIP(hipGetLastError());
+    const int64_t piece = std::min(m, PIECE_POINTS);
+    char *hp = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(double) * 3 * (m > piece ? 2 * piece : m), &hp));
+    for (int64_t k = 0, i = 0; i < m; ++k, i += piece) {
+        const int64_t n = std::min(piece, m - i);
+        double *h = reinterpret_cast<double *>(hp) + (k & 1) * 3 * piece;
+        if (k >= 2) VLM_HIP(hipEventSynchronize(ctx->io_ev[k & 1]));
+        std::memcpy(h, p + 3 * i, sizeof(double) * 3 * n);
+        hipLaunchKernelGGL(aos_to_soa_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream, n, h,
+                           soa + i, stride);
+        VLM_HIP(hipGetLastError());
+        if (m > piece) VLM_TRY(piece_event(ctx, k & 1));
+    }
     return VLM_OK;
 }
 
 int points_to_host(vlm_ctx *ctx, int64_t m, const double *soa, int64_t stride, double *p,
                    bool deferred = false)
 {
-    char *h = nullptr;
-    VLM_TRY(pin_take(ctx, sizeof(double) * 3 * m, &h));
-    hipLaunchKernelGGL(soa_to_aos_kernel, dim3(nblk(m)), dim3(256), 0, ctx->stream, m, soa,
-                       stride, reinterpret_cast<double *>(h));
-    VLM_HIP(hipGetLastError());
-    if (deferred) return defer(ctx, {{p, h, sizeof(double) * 3 * m}});
-    VLM_TRY(sync_stream(ctx));
-    std::memcpy(p, h, sizeof(double) * 3 * m);
-    return VLM_OK;
+    // a deferred result waits in the arena as a whole
+    const int64_t piece = deferred ? m : std::min(m, PIECE_POINTS);
+    const int64_t np = m > 0 ? (m + piece - 1) / piece : 0;
+    char *hp = nullptr;
+    VLM_TRY(pin_take(ctx, sizeof(double) * 3 * (m > piece ? 2 * piece : m), &hp));
+    double *h = reinterpret_cast<double *>(hp);
+    for (int64_t k = 0; k <= np; ++k) {
+        if (k < np) {
+            const int64_t n = std::min(piece, m - k * piece);
+            hipLaunchKernelGGL(soa_to_aos_kernel, dim3(nblk(n)), dim3(256), 0, ctx->stream, n,
+                               soa + k * piece, stride, h + (k & 1) * 3 * piece);
+            VLM_HIP(hipGetLastError());
+            if (deferred) return defer(ctx, {{p, hp, sizeof(double) * 3 * m}});
+            if (np > 1) VLM_TRY(piece_event(ctx, k & 1));
+        }
+        if (k > 0) {
+            if (np > 1) VLM_HIP(hipEventSynchronize(ctx->io_ev[(k - 1) & 1]));
+            else VLM_TRY(sync_stream(ctx));
+            std::memcpy(p + 3 * (k - 1) * piece, h + ((k - 1) & 1) * 3 * piece,
+                        sizeof(double) * 3 * std::min(piece, m - (k - 1) * piece));
+        }
+    }
+    return np > 1 ? sync_stream(ctx) : VLM_OK;
 }
 
 }  // namespace vlm
@@ -410,6 +441,7 @@ int vlm_filament_vind(vlm_ctx *ctx, int64_t nfil, const double *a, const double 
     if (!p || !v || (nfil > 0 && (!a || !b || !gam || !rc)))
         return fail(ctx, VLM_ERR_ARG, "null buffer");
     VLM_HIP(hipSetDevice(ctx->device));
+    const Trim trim{ctx};
     const int formats = bs_formats(ctx, m, nfil);
     VLM_HIP(ctx->tgt.reserve(ws_size<double>((size_t)3 * m)));
     VLM_HIP(ctx->seg.reserve(std::max<int64_t>(nfil, 4096), formats, &ctx->seg_view));
@@ -447,10 +479,7 @@ int vlm_filament_vind(vlm_ctx *ctx, int64_t nfil, const double *a, const double 
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
     if (accumulate) VLM_TRY(points_to_device(ctx, m, v, ctx->out.p, m));
     VLM_TRY(bs_eval(ctx, ctx->seg_view, nfil, ctx->tgt.p, m, m, ctx->out.p, accumulate));
-    VLM_TRY(points_to_host(ctx, m, ctx->out.p, m, v));
-    release_large(ctx);
-    if (sizeof(double) * REC64_N * (size_t)nfil > KEEP_BYTES) ctx->seg.release();
-    return VLM_OK;
+    return points_to_host(ctx, m, ctx->out.p, m, v);
 }
 
 int vlm_fset_create(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b,
@@ -459,13 +488,13 @@ int vlm_fset_create(vlm_ctx *ctx, int64_t nfil, const double *a, const double *b
     if (!ctx || !fset) return VLM_ERR_ARG;
     if (nfil <= 0 || !a || !b || !gam || !rc) return fail(ctx, VLM_ERR_ARG, "empty filament set");
     VLM_HIP(hipSetDevice(ctx->device));
+    const Trim trim{ctx};
     FSet *fs = new FSet();
     int rc_ = upload_fset(ctx, nfil, a, b, gam, rc, SEG_ALL, fs->seg, &fs->view);
     if (rc_ != VLM_OK) {
         delete fs;
         return rc_;
     }
-    release_large(ctx);
     fs->n = nfil;
     ctx->fsets.push_back(fs);
     *fset = (int)ctx->fsets.size() - 1;

@@ -99,6 +99,10 @@ struct SegList {
         rec32.release();
         near32.release();
     }
+    size_t bytes() const
+    {
+        return sizeof(double) * (soa.n + rec64.n + grp.n) + sizeof(float) * (rec32.n + near32.n);
+    }
     // Room for n segments in the given formats.
     hipError_t reserve(int64_t n, int formats, SegPtrs *out)
     {
@@ -449,10 +453,15 @@ void mlp_release(vlm_ctx *ctx);
 // Kernels may read and write the arena themselves, which spares a small
 // call the copies' launches.
 constexpr size_t PIN_PIECE = (size_t)2 << 20;
-// Copies of host data that a call leaves in the context for the next one are
-// given back above this size (the call has synchronised, or hipFree waits).
-constexpr size_t KEEP_BYTES = (size_t)1 << 30;
-void release_large(vlm_ctx *ctx);
+// What a call on host data leaves in the context for the next one (copies of
+// its filaments, points, results and matrices, its segment list and partial
+// sums) is given back above this size, buffer by buffer, when the call ends
+// with or without an error (hipFree waits for the device).
+constexpr size_t KEEP_BYTES = (size_t)256 << 20;
+struct Trim {
+    vlm_ctx *ctx;
+    ~Trim();
+};
 int pin_take(vlm_ctx *ctx, size_t bytes, char **out);
 int h2d(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);
 int d2h(vlm_ctx *ctx, void *dst, const void *src, size_t bytes);

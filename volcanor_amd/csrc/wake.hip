@@ -2289,6 +2289,7 @@ int vlm_rotor_induced_velocity(vlm_ctx *ctx, int ir, int set, int64_t m, const d
     if (set < VLM_SET_WING || set > VLM_SET_WAKE_PRED) return fail(ctx, VLM_ERR_ARG, "bad set");
     if (m <= 0) return VLM_OK;
     if (!p || !v) return fail(ctx, VLM_ERR_ARG, "null buffer");
+    const Trim trim{ctx};
     Sources src = {{ir, set}};
     int64_t nest = 0;
     VLM_TRY(build_sources(ctx, src, bs_formats(ctx, m, expected(ctx, src)), &nest));
@@ -2360,6 +2361,7 @@ static int induced_terms(vlm_ctx *ctx, int nterms, const int *ir, const int *set
     }
     if (m <= 0) return VLM_OK;
     if (!p || !v) return fail(ctx, VLM_ERR_ARG, "null buffer");
+    const Trim trim{ctx};
     VLM_HIP(ctx->tgt.reserve(ws_size<double>((size_t)3 * m)));
     VLM_HIP(ctx->out.reserve(ws_size<double>((size_t)3 * m)));
     VLM_TRY(points_to_device(ctx, m, p, ctx->tgt.p, m));
