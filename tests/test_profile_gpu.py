@@ -7,8 +7,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("m,n,mixed,timed", [
-    (300, 100000, False, True), (300, 2000, False, False), (640, 4688, False, True),
-    (640, 4687, False, False), (1200, 2000, False, False), (1200, 2000, True, True),
+    (300, 100001, False, True), (300, 2000, False, False), (640, 46876, False, True),
+    (640, 46875, False, False), (1200, 2000, False, False), (1200, 2000, True, True),
     (2049, 10, False, True), (20, 200000, False, False), (700, 100000, True, True)])
 def test_timed_launches(m, n, mixed, timed):
     from volcanor_amd import vlm

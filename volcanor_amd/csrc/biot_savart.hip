@@ -38,6 +38,8 @@
 //           reference's exact-zero guards act).
 //           Launches with fewer than 1024 targets (collocation points, judge
 //           samples) run in FP64 in both modes.
+#include <algorithm>
+
 #include "vlm_internal.h"
 
 namespace vlm {
@@ -327,7 +329,7 @@ struct BsArgs {
     double *part;
     int *counter;
     int64_t m, tstride;
-    int nchunks, ntiles, nitems, round_robin;
+    int nchunks, ntiles, nitems, nwaves, round_robin;
 };
 
 // Work items of both kernels: a wave takes 64 NT targets (NT per lane) and
@@ -362,11 +364,10 @@ __device__ __forceinline__ int first_item()
 }
 __device__ __forceinline__ int next_item(const BsArgs &a, int item)
 {
-    const int nwaves = (int)gridDim.x * (BS_BLOCK / 64);
-    if (a.round_robin) return item + nwaves;
+    if (a.round_robin) return item + a.nwaves;
     int next = 0;
     if ((threadIdx.x & 63) == 0) next = atomicAdd(a.counter, 1);
-    return nwaves + __builtin_amdgcn_readfirstlane(next);
+    return a.nwaves + __builtin_amdgcn_readfirstlane(next);
 }
 
 __global__ __launch_bounds__(BS_BLOCK, 8) void bs_fp64_kernel(BsArgs a)
@@ -540,22 +541,48 @@ struct TermTab {
     int64_t off[TERM_MAX];
 };
 
+// The only list of a launch, from segment 0.
+struct OneList {
+    int nchunks;
+};
+
+// The list that a block works on, its first chunk, its chunks and its start.
+struct ListChunks {
+    int k, first, n;
+    int64_t off;
+};
+
+__device__ __forceinline__ ListChunks chunks_of(const OneList &l, int)
+{
+    return {0, 0, l.nchunks, 0};
+}
+
+__device__ __forceinline__ ListChunks chunks_of(const TermTab &tt, int blk)
+{
+    int k = 0;
+    while (k + 1 < tt.n && blk >= tt.chunk0[k + 1]) ++k;
+    return {k, tt.chunk0[k], tt.chunk0[k + 1] - tt.chunk0[k], tt.off[k]};
+}
+
+// Lists: OneList or TermTab.  One list has a kernel of its own for its short
+// argument block, which the host writes across the bus at each launch: with
+// the table, and with the grid's size taken from the implicit arguments (256
+// bytes more), 50 segments at 1000 points took 8.4 us a call, so 6.1.
+template <typename Lists>
 __global__ __launch_bounds__(SM_BLOCK) void bs_small_kernel(const double *s64, int64_t S,
-                                                            const long long *counts, TermTab tt,
+                                                            const long long *counts, Lists lists,
                                                             const double *t, int64_t m,
                                                             int64_t tstride, double *part)
 {
     __shared__ double red[3 * SM_T][SM_BLOCK / 64];
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    int k = 0;
-    while (k + 1 < tt.n && (int)blockIdx.x >= tt.chunk0[k + 1]) ++k;
-    const int64_t nseg = counts[k];
-    const int nchunks = tt.chunk0[k + 1] - tt.chunk0[k];
-    const int64_t len = (nseg + nchunks - 1) / nchunks;
-    const int64_t s0 = (int64_t)((int)blockIdx.x - tt.chunk0[k]) * len;
+    const ListChunks c = chunks_of(lists, (int)blockIdx.x);
+    const int64_t nseg = counts[c.k];
+    const int64_t len = (nseg + c.n - 1) / c.n;
+    const int64_t s0 = (int64_t)((int)blockIdx.x - c.first) * len;
     const int64_t s1 = min(nseg, s0 + len);
     const int64_t g0 = (int64_t)blockIdx.y * SM_T;
-    s64 += tt.off[k];
+    s64 += c.off;
     double px[SM_T], py[SM_T], pz[SM_T], vx[SM_T], vy[SM_T], vz[SM_T];
 #pragma unroll
     for (int q = 0; q < SM_T; ++q) {
@@ -748,17 +775,20 @@ int profile_count(vlm_ctx *ctx, const long long *nseg_dev, int64_t m, int kind, 
 
 // bs_small_kernel has segments on its lanes, so no lane idles however few the
 // targets and short lists spread over the device, but every pair is the long
-// one.  Whole calls, small against 64 targets per wave, us:
-//   m    20 x 2e5      54   92    90 x 2e5     92  108   192 x 1e5     67   59
-//   m   200 x 2000     22   27   300 x 4e4     46   50   300 x 1e5     82   81
-//   m   300 x 2000     22   27   400 x 4e4     54   56   512 x 4e4     61   57
-//   m   600 x 2000     24   27   600 x 8000    36   35   192 x 4e5    229  151
-//   m  1200 x 500      24   27  1200 x 2000    28   31   400 x 4e5    357  306
+// one.  Sums over resident sets, us, small against 64 targets per wave, on
+// helices and on a rotor wake with a grid of points through it:
+//                 helices      wake                    helices      wake
+//   m   200 x 80000   48  54   48  54    200 x 200000   112 116  115 118
+//   m   200 x 400000 220 219  223 213    300 x 133333   100  93  100  94
+//   m   500 x 32000   42  47   45  45    500 x  80000    94  81  102  85
+//   m  1000 x  9000   26  30   28  28   1000 x  24000    56  66   59  65
+//   m  1000 x 40000   86  80   95  86   2048 x  11719    54  66   55  61
+//   m  2048 x 19531   84  88   88  81   2048 x  39063   158 143  170 149
+// Whole calls on host arrays, 20 x 2e5: 54 against 92, 90 x 2e5: 92, 108.
 static bool few_pairs(int64_t m, int64_t nseg)
 {
     if (m < 192 && 5 * m < 4 * 64 * ((m + 63) / 64)) return true;   // waves not 4/5 full
-    if (nseg > 16000000 || m > 2048) return false;
-    return m * nseg <= (m <= 400 ? 16000000 : 3000000);
+    return m <= 2048 && nseg <= 60000000 && m * nseg <= (m <= 256 ? 60000000 : 30000000);
 }
 
 int bs_formats(const vlm_ctx *ctx, int64_t m, int64_t nseg)
@@ -776,8 +806,9 @@ int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, cons
     const int64_t max_chunks = ws ? (int64_t)(ws->part_cap / (3 * (size_t)m)) : INT32_MAX;
     if (max_chunks < terms.n) return fail(ctx, VLM_ERR_ARG, "workspace too small for the targets");
     // per list about 2048 blocks of at least 8 segments per lane; short
-    // lists are split down to 2 per lane, up to 16 chunks (their loads wait
-    // on each other; more chunks only feed the reduction)
+    // lists are split down to 2 per lane (their loads wait on each other), up
+    // to 16 chunks (more only feed the reduction) and 512 blocks (2 per CU:
+    // 600 targets x 6666 segments 17 us with 450 blocks, 21 with 1950)
     const int64_t groups = (m + SM_T - 1) / SM_T;
     TermTab tt;
     tt.n = terms.n;
@@ -786,7 +817,7 @@ int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, cons
     for (int k = 0; k < terms.n; ++k) {
         int64_t nc = (2048 + groups - 1) / groups;
         const int64_t c2 = terms.est[k] / (2 * SM_BLOCK), c8 = terms.est[k] / (8 * SM_BLOCK);
-        const int64_t maxc = c8 > 16 ? c8 : (c2 > 16 ? 16 : c2);
+        const int64_t maxc = std::max(c8, std::min<int64_t>({16, c2, 512 / groups}));
         if (nc > maxc) nc = maxc;
         if (nc > max_chunks / terms.n) nc = max_chunks / terms.n;
         if (nc < 1) nc = 1;
@@ -800,11 +831,22 @@ int bs_eval_terms(vlm_ctx *ctx, const SegPtrs &seg, const TermLists &terms, cons
         VLM_HIP(ctx->part.reserve(ws_size<double>((size_t)nchunks * 3 * (size_t)m)));
         part = ctx->part.p;
     }
-    hipLaunchKernelGGL(bs_small_kernel, dim3(nchunks, (unsigned)groups), dim3(SM_BLOCK), 0,
-                       ctx->stream, seg.soa, seg.cap, seg.count, tt, t, m, tstride, part);
-    hipLaunchKernelGGL(bs_reduce_terms_kernel, dim3((unsigned)((m + 63) / 64), 3),
-                       dim3(64 * RT_W), 0, ctx->stream, part, tt, m, out,
-                       aos ? OutMap{1, 3} : OutMap{tstride, 1}, accumulate);
+    const dim3 grid(nchunks, (unsigned)groups);
+    const OutMap o = aos ? OutMap{1, 3} : OutMap{tstride, 1};
+    if (tt.n == 1 && tt.off[0] == 0 && !tt.neg) {
+        hipLaunchKernelGGL(bs_small_kernel<OneList>, grid, dim3(SM_BLOCK), 0, ctx->stream, seg.soa,
+                           seg.cap, seg.count, OneList{nchunks}, t, m, tstride, part);
+        // the sums of bs_reduce_terms_kernel
+        if (nchunks > RT_S)
+            reduce_as<64, RT_S>(ctx, part, nchunks, m, out, o, accumulate, nullptr);
+        else
+            reduce_as<64, 1>(ctx, part, nchunks, m, out, o, accumulate, nullptr);
+    } else {
+        hipLaunchKernelGGL(bs_small_kernel<TermTab>, grid, dim3(SM_BLOCK), 0, ctx->stream,
+                           seg.soa, seg.cap, seg.count, tt, t, m, tstride, part);
+        hipLaunchKernelGGL(bs_reduce_terms_kernel, dim3((unsigned)((m + 63) / 64), 3),
+                           dim3(64 * RT_W), 0, ctx->stream, part, tt, m, out, o, accumulate);
+    }
     VLM_HIP(hipGetLastError());
     if (ctx->profile && !ws)
         for (int k = 0; k < terms.n; ++k)
@@ -885,6 +927,7 @@ int bs_eval(vlm_ctx *ctx, const SegPtrs &seg, int64_t nseg_est, const double *t,
     a.nitems = (int)nitems;
     const int64_t need = (nitems + BS_BLOCK / 64 - 1) / (BS_BLOCK / 64);
     const int grid = (int)(need < cap ? need : cap);
+    a.nwaves = grid * (BS_BLOCK / 64);
     a.round_robin = len < LEN_MID || need <= cap;
     Timer tm{};
     if (prof) {
