@@ -416,7 +416,7 @@ int vlm_predictor_errors(vlm_ctx *ctx, double *mlp_rel_rms, double *base_rel_rms
  * is bracketed by HIP events on the context stream: all launches but those of
  * few pairs, which are the ones with fewer than 192 targets in waves of 64
  * less than four fifths full, and those of at most 6e7 pairs up to 256
- * targets or 3e7 pairs up to 2048 targets; in mixed precision none of 1024 targets or more counts as few.  vlm_profile_get returns the summed kernel
+ * targets or 3e7 pairs below 2048 targets; in mixed precision none of 1024 targets or more counts as few.  vlm_profile_get returns the summed kernel
  * time (ms), the launch count and the algorithmic pair count since the last
  * reset. */
 int vlm_profile_enable(vlm_ctx *ctx, int enable);

@@ -1,5 +1,5 @@
 """Launches of few pairs (segments on lanes) and grouped ones on both sides of
-the lines between them, 6e7 pairs up to 256 targets and 3e7 up to 2048, and where short lists are
+the lines between them, 6e7 pairs up to 256 targets and 3e7 below 2048, and where short lists are
 split (at most 512 blocks, 16 chunks, 2 segments per lane), against the FP64
 oracle; a list alone sums like the same list among others, to the bit."""
 import numpy as np
@@ -11,7 +11,7 @@ from tests.test_bs_groups_gpu import _chain
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("m,n", [(2048, 14648), (2048, 14649), (400, 75000), (400, 75001),
+@pytest.mark.parametrize("m,n", [(2047, 14655), (2047, 14656), (2048, 10), (400, 75000), (400, 75001),
                                  (192, 312500), (192, 312501), (257, 116731), (257, 116732), (1000, 50), (600, 6666),
                                  (128, 8192), (129, 8191), (2047, 511), (300, 13333)])
 def test_both_sides_match_oracle(m, n):

@@ -785,10 +785,11 @@ int profile_count(vlm_ctx *ctx, const long long *nseg_dev, int64_t m, int kind, 
 //   m  1000 x 40000   86  80   95  86   2048 x  11719    54  66   55  61
 //   m  2048 x 19531   84  88   88  81   2048 x  39063   158 143  170 149
 // Whole calls on host arrays, 20 x 2e5: 54 against 92, 90 x 2e5: 92, 108.
+// From 2048 targets on every launch is a grouped (and so a timed) one.
 static bool few_pairs(int64_t m, int64_t nseg)
 {
     if (m < 192 && 5 * m < 4 * 64 * ((m + 63) / 64)) return true;   // waves not 4/5 full
-    return m <= 2048 && nseg <= 60000000 && m * nseg <= (m <= 256 ? 60000000 : 30000000);
+    return m < 2048 && nseg <= 60000000 && m * nseg <= (m <= 256 ? 60000000 : 30000000);
 }
 
 int bs_formats(const vlm_ctx *ctx, int64_t m, int64_t nseg)
