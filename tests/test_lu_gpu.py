@@ -1,4 +1,4 @@
-"""AIC assembly, LU factorisation (single-workgroup and MFMA blocked paths)
+"""AIC assembly, LU factorisation (panels of every width, MFMA updates)
 and the refined circulation solve against the oracle and LAPACK."""
 import numpy as np
 import pytest
@@ -22,8 +22,9 @@ def _matrix(n, seed):
 
 @pytest.mark.parametrize("n", [40, 256, 257, 777])
 def test_lu_factor_matches_oracle(n):
-    """n <= 256 runs the one-workgroup path, n > 256 the blocked path whose
-    trailing update runs on MFMA; 257 and 777 leave ragged last panels."""
+    """40: panels of one wave; 256 and 257: panels of four and eight waves
+    first, the trailing update on MFMA; 257 and 777 leave ragged last panels
+    (1 and 9 columns)."""
     A = _matrix(n, n)
     LU, piv = _ctx().lu_factor(A)
     LUo, pivo, info = orc.lu_factor(A)
@@ -84,7 +85,7 @@ def test_triangular_solve_matches_oracle(n):
 
 @pytest.mark.parametrize("n,col", [(50, 16), (300, 100), (1300, 260)])
 def test_lu_zero_pivot_is_an_error(n, col):
-    """50: one-workgroup path; 300: the zero column in a 32-column panel held
+    """50: the one-wave panel; 300: the zero column in a 32-column panel held
     in registers (masking design); 1300: column 260 lies in the 16-column
     panel at 256, of 1044 rows (retiring design), where every candidate is 0
     and retired or empty slots must lose the tie to the live rows."""

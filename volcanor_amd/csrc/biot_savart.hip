@@ -20,10 +20,10 @@
 // depth 4, but FP64 and FP32 MFMA run no faster than the vector units here
 // (64 and 32 cycles per 16x16x4) and do not overlap with them (16 FMAs and
 // one MFMA take the sum of both times).  Measured against pair64 for every
-// pair with LDS broadcasts: 4.0e9 pairs on helices 6.6 -> 5.1 ms, a
-// quad-rotor wake pass (1.58e10 pairs) 25.7 -> 20.0 ms (7.9e11 pairs/s);
-// mixed, 2e10 pairs on helices 14.7 -> 11.4 ms (1.75e12 pairs/s), a rotor
-// wake pass (2.2e9 pairs) 2.00 -> 1.49 ms.
+// pair with LDS broadcasts: 4.0e9 pairs on helices 6.5 -> 5.15 ms, a
+// quad-rotor wake pass (1.58e10 pairs) 25.4 -> 19.9 ms (8.0e11 pairs/s);
+// mixed, 2e10 pairs on helices 14.7 -> 11.3 ms (1.78e12 pairs/s), a rotor
+// wake pass (2.2e9 pairs) 2.00 -> 1.46 ms.
 //
 // Precision modes
 //   FP64  : FP64 throughout; 1/sqrt via v_rsq_f64 plus one third-order

@@ -7,7 +7,8 @@
 //
 // Right-looking blocked LU.  Panels are 32 columns wide where the panel has
 // at most 1024 rows, 16 columns above that.
-//   1. panel: one workgroup (one wave up to 256 rows) factorises A[k:n, k:k+jb] column by column,
+//   1. panel: one workgroup (of 1, 2, 4 and 8 waves up to 64, 128, 256 and
+//      2560 rows, 16 above) factorises A[k:n, k:k+jb] column by column,
 //      the panel in registers; rows never move during the panel, each lane
 //      tracks the logical position of its rows, and one barrier per column
 //      publishes every wave's pivot candidate with its row.  16-column
@@ -613,9 +614,9 @@ __global__ __launch_bounds__(64 * W) void lu_panel_wide_kernel(int n, double *A,
 // and no step leaves the wave: the pivot by a DPP maximum and ballots, its
 // row by readlane (scalar operands of the update), no LDS and no barrier.
 // The arithmetic per element is that of the panels above.  Bound by the
-// chain of one column; 18 us for 32 columns, where 2, 4 and 8 waves of the
-// panel above (one row per lane: 128, 256, 512 rows) take 24, 29 and 37 us
-// for their LDS round trips and barrier.  With two and three rows per lane
+// chain of one column; 18 us for 32 columns (21 with a cold instruction
+// cache), where 2, 4 and 8 waves of the panel above (one row per lane: 128,
+// 256, 512 rows) take 25, 30 and 39 us for their LDS round trips and barrier.  With two and three rows per lane
 // it took 38 and 53 us, so taller panels stay above.  Takes any width jb <=
 // NBMAX, so the last columns of a matrix need no other kernel.
 struct WaveCtx {
