@@ -311,7 +311,8 @@ constexpr double kEps = 2.220446049250313080847263336181640625e-16;  // epsilon(
 // padding record (none in the structure of arrays).  The far radius: a target further than |a - c| + 2 |r0|
 // from the centre, for every segment, has |r1| >= 2 |r0| for all of them.
 // It is infinite (never far) for a group that holds a segment with
-// q <= 1e-18 (the far pair has no zero-denominator guard) or is wider than
+// q <= 1e-18 (the far pair has no zero-denominator guard) or an infinite
+// circulation (the moments would turn it into NaN), or is wider than
 // 64 of its longest segments (32 consecutive records can jump between wake
 // rows; a chain of 32 connected segments spans 34), whose centred
 // coordinates would lose accuracy against |r1|.
@@ -350,7 +351,7 @@ __device__ __forceinline__ void write_group_records(const Slot &s, bool valid, i
     float ex = valid ? (float)((sqrt(lx * lx + ly * ly + lz * lz) + l2) * 1.000001) : 0.f;
     float lmax = valid ? (float)l2 : 0.f;
     float rmin = valid ? (float)(fabs(s.rc) * 0.999999) : inf;
-    if (valid && !(q > 1e-18)) ex = inf;
+    if (valid && !(q > 1e-18 && fabs(g) < __builtin_inf())) ex = inf;
 #pragma unroll
     for (int o = 16; o > 0; o >>= 1) {
         ex = fmaxf(ex, __shfl_xor(ex, o, 32));
